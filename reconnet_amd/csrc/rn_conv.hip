@@ -714,51 +714,94 @@ __global__ __launch_bounds__(256) void k_out_dgrad(const float* __restrict__ dy,
 }
 
 // ---------------------------------------------------------------------------
-// weight gradients of the narrow layers (reduction over pixels, VALU):
+// weight gradients of the narrow layers (reduction over pixels, FP32 MFMA):
 // mode 0 (layer 1): part[t][c] = sum_p x[p + off_t] dz1[p][c], part[9][c] = sum_p dz1[p][c]
-// mode 1 (layer 5): part[t][c] = sum_p dy[p] a4[p + off_t][c], part[9][0] = sum_p dy[p]
-// one workgroup: 8 groups of 32 lanes (lane = channel c), partials per workgroup
+// mode 1 (layer 5): part[t][c] = sum_p dy[p] a4[p + off_t][c] = sum_q a4[q][c] dy[q - off_t],
+//                   part[9][0] = sum_p dy[p]
+//
+// Both are products of the 32-channel tensor's columns with the image's 9
+// shifts, K = pixels: v_mfma_f32_16x16x4f32 takes 4 adjacent pixels, A = 16
+// channels (lane l: channel pair l % 16 of pixel l / 16, one 4-byte load whose
+// halves feed an even-channel and an odd-channel tile, widened to FP32
+// exactly), B = the shifts (lane l: shift l % 16 of that pixel; column 9 is 1
+// and gives the channel sums, columns 10 .. 15 are 0).  Nothing is rounded
+// below FP32 and no LDS is needed.  A wave takes 64 pixels of one image row at
+// a time, 16 steps whose loads are independent.
+//
+// Bound: the 64 bytes per pixel of the tensor, read once: 89 us for 16 x 512^2
+// (3.0 TB/s; 56 us at the 4.8 TB/s of a large copy, the two matrix tiles alone
+// 27 us).  With 32 lanes of 2-byte loads and 10 FMAs per pixel: 1.60 ms.
 // ---------------------------------------------------------------------------
+typedef uint32_t U32a2 __attribute__((aligned(2)));   // a channel pair: 2-byte aligned like the tensor
+
+constexpr int kNarrowPx = 64;          // pixels of a wave's chunk
+
 __global__ __launch_bounds__(256) void k_wgrad_narrow(const float* __restrict__ img, const uint16_t* __restrict__ act,
-                                                      float* __restrict__ part, int B, int H, int W, int mode)
+                                                      float* __restrict__ part, int H, int W, int chunks_per_row,
+                                                      int nchunk, int mode)
 {
-    __shared__ float red[8][10 * 32];
-    const int c = threadIdx.x & 31, grp = threadIdx.x >> 5;
-    const long npx = (long)B * H * W;
-    float acc[10];
-    #pragma unroll
-    for (int t = 0; t < 10; ++t) acc[t] = 0.0f;
-    for (long p = (long)blockIdx.x * 8 + grp; p < npx; p += (long)gridDim.x * 8) {
-        const int xw = (int)(p % W), yh = (int)((p / W) % H);
-        const long base = p - (long)yh * W - xw;
-        if (mode == 0) {
-            const float d = bf2f(act[p * 32 + c]);
+    __shared__ float red[4][320];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int n = lane & 15, k = lane >> 4;
+    // shift of column n (mode 1 reads the image at q - off_t)
+    const int sg = mode == 0 ? 1 : -1;
+    const int oy = n < 9 ? sg * (n / 3 - 1) : 0, ox = n < 9 ? sg * (n % 3 - 1) : 0;
+    const uint32_t fixed = n == 9 ? 0x3f800000u : 0u;               // 1.0f
+    f32x4 ev = f32x4{0, 0, 0, 0}, od = f32x4{0, 0, 0, 0};
+    float sum = 0.0f;                  // lanes n = 4 (shift 0): the image's sum
+    for (int ch = (int)blockIdx.x * 4 + wv; ch < nchunk; ch += (int)gridDim.x * 4) {
+        const int row = ch / chunks_per_row;                        // image * H + y
+        const int c0 = (ch - row * chunks_per_row) * kNarrowPx;
+        const int y = row % H + oy;
+        const bool rok = y >= 0 && y < H, tap = n < 9 && rok;
+        const float* src = img + (long)(rok ? row + oy : row) * W;  // the shift's image row
+        const uint16_t* a = act + (long)row * W * 32 + 2 * n;
+        // loads without branches (columns clamped into the row, dropped by
+        // selects), 8 steps in flight
+        #pragma unroll
+        for (int s0 = 0; s0 < kNarrowPx / 4; s0 += 8) {
+            if (c0 + 4 * s0 >= W) break;
+            uint32_t u[8];
+            float v[8];
             #pragma unroll
-            for (int t = 0; t < 9; ++t) {
-                const int yy = yh + t / 3 - 1, xx = xw + t % 3 - 1;
-                if (yy >= 0 && yy < H && xx >= 0 && xx < W) acc[t] = fmaf(img[base + (long)yy * W + xx], d, acc[t]);
+            for (int s = 0; s < 8; ++s) {
+                const int px = c0 + 4 * (s0 + s) + k;
+                u[s] = *reinterpret_cast<const U32a2*>(a + (long)min(px, W - 1) * 32);
+                v[s] = src[min(max(px + ox, 0), W - 1)];
             }
-            acc[9] += d;
-        } else {
-            const float d = img[p];
             #pragma unroll
-            for (int t = 0; t < 9; ++t) {
-                const int yy = yh + t / 3 - 1, xx = xw + t % 3 - 1;
-                if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-                    acc[t] = fmaf(d, bf2f(act[(base + (long)yy * W + xx) * 32 + c]), acc[t]);
+            for (int s = 0; s < 8; ++s) {
+                const int px = c0 + 4 * (s0 + s) + k;
+                const bool in = px < W;
+                // masks, not selects: a select would sink its load under a branch
+                const uint32_t inside = in ? 0xffffffffu : 0u;
+                const uint32_t mok = (in && tap && px + ox >= 0 && px + ox < W) ? 0xffffffffu : 0u;
+                const uint32_t w = u[s] & inside;
+                const float f = __uint_as_float((__float_as_uint(v[s]) & mok) | (fixed & inside));
+                sum += f;
+                ev = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w << 16), f, ev, 0, 0, 0);
+                od = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w & 0xffff0000u), f, od, 0, 0, 0);
             }
-            acc[9] += d;
         }
     }
+    // D on lane l, register i: shift l % 16, channel pair 4 (l / 16) + i
     #pragma unroll
-    for (int t = 0; t < 10; ++t) red[grp][t * 32 + c] = acc[t];
-    __syncthreads();
-    for (int i = threadIdx.x; i < 320; i += blockDim.x) {
-        float s = 0.0f;
-        #pragma unroll
-        for (int gidx = 0; gidx < 8; ++gidx) s += red[gidx][i];
-        part[(long)blockIdx.x * 320 + i] = s;
+    for (int i = 0; i < 4; ++i) {
+        if (n < 10) {
+            red[wv][n * 32 + 2 * (4 * k + i)] = ev[i];
+            red[wv][n * 32 + 2 * (4 * k + i) + 1] = od[i];
+        }
     }
+    if (mode != 0) {
+        // the image's sum over the four pixel groups of the shift-0 lanes, in place of the channel sums
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (lane == 4) red[wv][288] = sum;
+    }
+    __syncthreads();
+    const int no = mode == 0 ? 320 : 289;       // the gradient's entries
+    for (int i = threadIdx.x; i < no; i += 256)
+        part[(long)blockIdx.x * no + i] = (red[0][i] + red[1][i]) + (red[2][i] + red[3][i]);
 }
 
 // bias gradient of a 32-channel NHWC tensor: part[wg][c] = sum_p dz[p][c]
@@ -1008,12 +1051,17 @@ void conv_out_dgrad(const float* dy, const float* w5, const uint16_t* a4, uint16
 void wgrad_narrow(const float* img, const uint16_t* act, float* grad, int B, int H, int W, int mode, DevBuf& work,
                   hipStream_t st)
 {
-    const long npx = (long)B * H * W;
-    const int blocks = grid_for(npx, 8 * 64, 1024);
+    const int chunks_per_row = cdiv(W, kNarrowPx);
+    RN_REQUIRE(B > 0 && H > 0 && W > 0 && (long)B * H * chunks_per_row + 4096 < 0x7fffffffL,
+               "wgrad_narrow: bad batch or image size");
+    const int nchunk = B * H * chunks_per_row;
+    // 4 workgroups per CU (16 waves of 16 loads in flight each), whole rounds of chunks
+    const int blocks = grid_for(nchunk, 4, 1024);
     work.ensure((size_t)blocks * 320 * sizeof(float));
-    hipLaunchKernelGGL(k_wgrad_narrow, dim3(blocks), dim3(256), 0, st, img, act, work.as<float>(), B, H, W, mode);
+    hipLaunchKernelGGL(k_wgrad_narrow, dim3(blocks), dim3(256), 0, st, img, act, work.as<float>(), H, W,
+                       chunks_per_row, nchunk, mode);
     check_launch("wgrad_narrow");
-    reduce_rows(work.as<float>(), grad, blocks, 320, st);
+    reduce_rows(work.as<float>(), grad, blocks, mode == 0 ? 320 : 289, st);
 }
 
 void bias_grad(const uint16_t* dz, float* grad, long npx, DevBuf& work, hipStream_t st)

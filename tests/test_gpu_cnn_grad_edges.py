@@ -1,0 +1,42 @@
+"""Weight-gradient kernels of the prior at the edges of their tiles: small
+integers, where every product and partial sum is exact in FP32, so each kernel
+must equal the FP64 sum over pixels bit for bit."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# widths around a 4-pixel step, a 32-pixel tile and a 64-pixel chunk; single rows and columns
+SHAPES = [(1, 1, 1), (1, 1, 3), (2, 3, 4), (1, 2, 31), (1, 5, 33), (3, 2, 63), (1, 7, 65), (2, 70, 36), (1, 3, 129)]
+
+
+def _shift_sums(img, act):
+    """[9][ci] sums over p of img[p + off_t] act[p], zero outside the image."""
+    B, H, W = img.shape
+    p = np.pad(img, ((0, 0), (1, 1), (1, 1)))
+    return np.stack([np.einsum("bhw,bhwc->c", p[:, t // 3:t // 3 + H, t % 3:t % 3 + W], act) for t in range(9)])
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("mode", [0, 1])
+def test_narrow_gradients(shape, mode):
+    from reconnet_amd.cnn import _p, _sigs, _st
+
+    B, H, W = shape
+    rng = np.random.default_rng(100 * W + 10 * H + mode)
+    img = rng.integers(-3, 4, shape).astype(np.float64)
+    act = rng.integers(-3, 4, shape + (32,)).astype(np.float64)
+    x = torch.from_numpy(img).float().cuda()
+    a = torch.from_numpy(act).cuda().to(torch.bfloat16)
+    g = torch.full((320,), 7.0, device="cuda")     # mode 1 writes 289 entries and no more
+    assert _sigs().rn_cnn_wgrad_narrow(_p(x), _p(a), _p(g), B, H, W, mode, _st()) == 0
+    g = g.cpu().double().numpy()
+    want = _shift_sums(img, act)
+    # mode 1: the tensor is shifted instead, the image's shifts in reverse
+    assert np.array_equal(g[:288].reshape(9, 32), want if mode == 0 else want[::-1])
+    if mode == 0:
+        assert np.array_equal(g[288:], act.sum((0, 1, 2)))
+    else:
+        assert g[288] == img.sum() and (g[289:] == 7.0).all()
