@@ -244,6 +244,9 @@ int rn_cnn_bias_grad(const unsigned short* dz, float* grad, long npx, void* stre
 /* grad[9][32 out][32 in] = sum_p dz[p][out] in[p + tap][in]  (MFMA) */
 int rn_cnn_wgrad_mid(const unsigned short* in, const unsigned short* dz, float* grad, int B, int H, int W,
         void* stream);
+/* rn_cnn_wgrad_mid and the layer's bias gradient gbias[32] = sum_p dz[p] in one pass over both tensors */
+int rn_cnn_wgrad_mid_bias(const unsigned short* in, const unsigned short* dz, float* grad, float* gbias,
+        int B, int H, int W, void* stream);
 
 /* Batches of 2D fan slices of uneven size (no reference counterpart).  dims
  * [nslices][4] = (nx, ny, nu, nview); geo [nslices][6] = (dx, dy, da, off_a,

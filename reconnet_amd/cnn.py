@@ -34,6 +34,7 @@ def _sigs():
         ("rn_cnn_wgrad_narrow", [_P, _P, _P, ci, ci, ci, ci, _P]),
         ("rn_cnn_bias_grad", [_P, _P, cl, _P]),
         ("rn_cnn_wgrad_mid", [_P, _P, _P, ci, ci, ci, _P]),
+        ("rn_cnn_wgrad_mid_bias", [_P, _P, _P, _P, ci, ci, ci, _P]),
     ]:
         fn = getattr(h, name)
         fn.restype = ci
@@ -147,7 +148,6 @@ class PriorCNN:
         x, acts = self._cache
         dy = dy.contiguous().float()
         B, H, W = x.shape
-        npx = B * H * W
         g = {}
         buf = torch.empty(9 * 32 + 32, dtype=torch.float32, device=x.device)
         check(h.rn_cnn_wgrad_narrow(_p(dy), _p(acts[3]), _p(buf), B, H, W, 1, _st()), "rn_cnn_wgrad_narrow")
@@ -158,9 +158,8 @@ class PriorCNN:
         for k in (4, 3, 2):
             a_in = acts[k - 2]
             gw = torch.empty(9, 32, 32, dtype=torch.float32, device=x.device)
-            check(h.rn_cnn_wgrad_mid(_p(a_in), _p(dz), _p(gw), B, H, W, _st()), "rn_cnn_wgrad_mid")
             gb = torch.empty(32, dtype=torch.float32, device=x.device)
-            check(h.rn_cnn_bias_grad(_p(dz), _p(gb), npx, _st()), "rn_cnn_bias_grad")
+            check(h.rn_cnn_wgrad_mid_bias(_p(a_in), _p(dz), _p(gw), _p(gb), B, H, W, _st()), "rn_cnn_wgrad_mid_bias")
             g["w%d" % k], g["b%d" % k] = gw, gb
             nz = torch.empty_like(dz)
             check(h.rn_cnn_conv_mid(_p(dz), _p(self.wd[k]), None, _p(a_in), _p(nz), B, H, W, 0, _st()),

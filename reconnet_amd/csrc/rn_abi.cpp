@@ -865,7 +865,16 @@ extern "C" int rn_cnn_wgrad_mid(const uint16_t* in, const uint16_t* dz, float* g
 {
     return guarded_status("rn_cnn_wgrad_mid", [&] {
         RN_REQUIRE(in && dz && grad && B > 0 && H > 0 && W > 0, "invalid argument");
-        wgrad_mid(in, dz, grad, B, H, W, conv_work(), static_cast<hipStream_t>(stream));
+        wgrad_mid(in, dz, grad, nullptr, B, H, W, conv_work(), static_cast<hipStream_t>(stream));
+    });
+}
+
+extern "C" int rn_cnn_wgrad_mid_bias(const uint16_t* in, const uint16_t* dz, float* grad, float* gbias, int B, int H,
+                                     int W, void* stream)
+{
+    return guarded_status("rn_cnn_wgrad_mid_bias", [&] {
+        RN_REQUIRE(in && dz && grad && gbias && B > 0 && H > 0 && W > 0, "invalid argument");
+        wgrad_mid(in, dz, grad, gbias, B, H, W, conv_work(), static_cast<hipStream_t>(stream));
     });
 }
 

@@ -34,7 +34,8 @@ void wgrad_narrow(const float* img, const uint16_t* act, float* grad, int B, int
                   hipStream_t st);
 // grad[c] = sum_p dz[p][c]
 void bias_grad(const uint16_t* dz, float* grad, long npx, DevBuf& work, hipStream_t st);
-// grad[t][co][ci] = sum_p dz[p][co] in[p + off_t][ci]   (MFMA)
-void wgrad_mid(const uint16_t* in, const uint16_t* dz, float* grad, int B, int H, int W, DevBuf& work, hipStream_t st);
+// grad[t][co][ci] = sum_p dz[p][co] in[p + off_t][ci]   (MFMA); gbias[co] = sum_p dz[p][co] if not null
+void wgrad_mid(const uint16_t* in, const uint16_t* dz, float* grad, float* gbias, int B, int H, int W, DevBuf& work,
+               hipStream_t st);
 
 } // namespace rn

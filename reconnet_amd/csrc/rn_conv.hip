@@ -6,15 +6,15 @@
 // product accumulates in FP32.
 //
 // The 32 -> 32 layers (forward and data gradient) run on gfx950 BF16 matrix
-// cores: v_mfma_f32_16x16x32_bf16 with A = weights (16 output channels x 32
-// input channels of one tap) and B = 16 consecutive pixels x 32 input
-// channels; 9 taps x 2 channel tiles = 18 MFMAs per 16-pixel segment.  The
-// weight gradient of those layers is an MFMA GEMM over pixels with LDS
-// transposes.  The 1 -> 32 and 32 -> 1 layers (K = 9, N = 1) are VALU kernels.
+// cores (v_mfma_f32_32x32x16_bf16, A = weights, B = pixels); their weight
+// gradient is an MFMA GEMM over pixels whose operands are transposed by the LDS
+// reads themselves.  The 1 -> 32 layer and its and the 32 -> 1 layer's weight
+// gradients use FP32 (VALU, FP32 MFMA), the 32 -> 1 layer split weights on MFMA.
 
 #include "rn_conv.h"
 #include "rn_tune.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rn {
@@ -821,101 +821,144 @@ __global__ __launch_bounds__(256) void k_bias_grad(const uint16_t* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// 32 -> 32 weight gradient on MFMA:
-//   dW[t][co][ci] = sum_p dz[p][co] in[p + off_t][ci]
-// GEMM with M = co, N = ci, K = pixels.  Each wave takes 32-pixel row chunks;
-// per chunk it transposes dz into LDS as [co][px] and the 3 x 34 input pixels
-// into 9 shifted copies [t][ci][px], so every fragment is one aligned 16-byte
-// LDS read.  All waves of a workgroup run the same number of chunk rounds
-// (out-of-range chunks contribute zeros) so block barriers are uniform.
+// 32 -> 32 weight gradient on MFMA, with the layer's bias gradient:
+//   dW[t][co][ci] = sum_p dz[p][co] in[p + off_t][ci],  db[co] = sum_p dz[p][co]
+// GEMM with M = co, N = ci, K = pixels (v_mfma_f32_32x32x16_bf16).  A wave
+// walks L rows of a 32-column strip.  Per step it stages one input row (34
+// pixels) and one dz row (32 pixels) as they lie in memory, 64 bytes per pixel,
+// in its own LDS rows; both operands need 8 pixels of one channel per lane, and
+// ds_read_b64_tr_b16 delivers exactly that from the staged rows (a group of 16
+// lanes reads 4 pixels x 16 channels and gets it transposed), so a tap's column
+// shift is only another first pixel and nothing is copied or transposed by
+// VALU work.  The dz fragments of three rows stay in registers, so each staged
+// row feeds all 9 taps.  The next row is loaded into registers while this one
+// is used.  No barrier: a wave touches only its own rows.
+//
+// Bound: one pass over both tensors: 125 us for 16 x 512^2 (4.3 TB/s; 112 us at
+// the 4.8 TB/s of a large copy, the matrix cores need 36 us).  With nine shifted transposed
+// copies written to LDS 2 bytes at a time it took 0.51 ms, and the bias
+// gradient another 0.22 ms in a kernel of its own.
 // ---------------------------------------------------------------------------
-constexpr int WG_WAVES = 4;
-constexpr int LDS_PER_WAVE = 32 * 32 + 9 * 32 * 32;   // bf16 elements
+constexpr int kWgIn = 34 * 32, kWgDz = 32 * 32;          // bf16 elements of a wave's staged rows
+constexpr int kWgOut = 9 * 1024 + 32;                    // gradient entries of a partial
 
-__global__ __launch_bounds__(256) void k_wgrad_mid(const uint16_t* __restrict__ in, const uint16_t* __restrict__ dz,
-                                                   float* __restrict__ part, int B, int H, int W)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// 16 pixels x 32 channels from LDS rows of 32 channels, transposed: this lane
+// holds channel lane % 32 of pixels 8 (lane / 32) .. + 7.  `row` points at the
+// lane's own read address within the first pixel's row (tr_lane).
+__device__ __forceinline__ bf16x8 tr_frag(const uint16_t* row)
 {
-    extern __shared__ uint16_t lds[];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int r16 = lane & 15, g4 = lane >> 4;
-    uint16_t* dzT = lds + wv * LDS_PER_WAVE;        // [32 co][32 px]
-    uint16_t* inS = dzT + 32 * 32;                  // [9 t][32 ci][32 px]
-    const int chunks_per_row = (W + 31) / 32;
-    const long nchunk = (long)B * H * chunks_per_row;
-    const long stride = (long)gridDim.x * WG_WAVES;
-    f32x4 acc[9][2][2];
+    typedef __attribute__((address_space(3))) s16x4 Lds;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds*)row);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds*)(row + 4 * 32));
+    const short v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    bf16x8 r;
+    __builtin_memcpy(&r, v, sizeof(r));
+    return r;
+}
+
+// element offset of a lane's read: pixel 8 (lane / 32) + (lane % 16) / 4, channels 16 ((lane / 16) % 2) + 4 (lane % 4) ..
+__device__ __forceinline__ int tr_lane(int lane)
+{
+    return (8 * (lane >> 5) + ((lane & 15) >> 2)) * 32 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+}
+
+__global__ __launch_bounds__(256, 2) void k_wgrad_mid(const uint16_t* __restrict__ in, const uint16_t* __restrict__ dz,
+                                                      float* __restrict__ part, int H, int W, int L, int nxs, int nys,
+                                                      int nitems)
+{
+    constexpr int kStage = 4 * (kWgIn + kWgDz) * (int)sizeof(uint16_t), kRed = kWgOut * (int)sizeof(float);
+    __shared__ __align__(16) char smem[kStage > kRed ? kStage : kRed];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    uint16_t* inS = reinterpret_cast<uint16_t*>(smem) + wv * (kWgIn + kWgDz);   // [34 px][32 ci]
+    uint16_t* dzS = inS + kWgIn;                                               // [32 px][32 co]
+    const int tl = tr_lane(lane);
+    f32x16 acc[9], accb = zero16();
     #pragma unroll
-    for (int t = 0; t < 9; ++t)
+    for (int t = 0; t < 9; ++t) acc[t] = zero16();
+    bf16x8 ones;
+    #pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+    const int px = lane >> 2, c8 = 8 * (lane & 3);        // this lane's 16-byte chunk of 16 pixels
+    for (int it = (int)blockIdx.x * 4 + wv; it < nitems; it += (int)gridDim.x * 4) {
+        const int ys = it % nys, t = it / nys, xs = t % nxs;
+        const int x0 = xs * 32, y0 = ys * L, y1 = min(y0 + L, H);
+        const long img = (long)(t / nxs) * H * W;
+        uint4 vi[3], vd[2];
+        // input row r (zero outside the image) and dz row r + 1 (zero outside this item's rows)
+        auto load = [&](int r) {
+            const bool rok = r >= 0 && r < H, dok = r + 1 >= y0 && r + 1 < y1;
+            #pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int x = x0 - 1 + px + 16 * k;
+                vi[k] = make_uint4(0, 0, 0, 0);
+                if (rok && x >= 0 && x < W && px + 16 * k < 34)
+                    vi[k] = *reinterpret_cast<const uint4*>(in + (img + (long)r * W + x) * 32 + c8);
+            }
+            #pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int x = x0 + px + 16 * k;
+                vd[k] = make_uint4(0, 0, 0, 0);
+                if (dok && x < W) vd[k] = *reinterpret_cast<const uint4*>(dz + (img + (long)(r + 1) * W + x) * 32 + c8);
+            }
+        };
+        bf16x8 d0[2], d1[2], d2[2];      // dz rows r - 1, r, r + 1: pixels 0 .. 15 and 16 .. 31
         #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int kc = 0; kc < 2; ++kc) d0[kc] = d1[kc] = as_bf16x8(make_uint4(0, 0, 0, 0));
+        load(y0 - 1);
+        for (int r = y0 - 1; r <= y1; ++r) {
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             #pragma unroll
-            for (int b = 0; b < 2; ++b) acc[t][a][b] = f32x4{0, 0, 0, 0};
-    const long rounds = (nchunk + stride - 1) / stride;
-    for (long rd = 0; rd < rounds; ++rd) {
-        const long ch = rd * stride + (long)blockIdx.x * WG_WAVES + wv;
-        const bool live = ch < nchunk;
-        long bimg = 0; int yh = 0, x0 = 0;
-        if (live) {
-            x0 = (int)(ch % chunks_per_row) * 32;
-            const long by = ch / chunks_per_row;
-            yh = (int)(by % H);
-            bimg = by / H;
-        }
-        // dz chunk -> dzT[co][px]
-        for (int j = lane; j < 128; j += 64) {
-            const int px = j >> 2, c8 = (j & 3) * 8;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (live && x0 + px < W) v = *reinterpret_cast<const uint4*>(dz + ((bimg * H + yh) * W + x0 + px) * 32 + c8);
-            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+            for (int k = 0; k < 3; ++k)
+                if (px + 16 * k < 34) *reinterpret_cast<uint4*>(inS + (px + 16 * k) * 32 + c8) = vi[k];
             #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                dzT[(c8 + e) * 32 + px] = (uint16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff));
-        }
-        // input rows yh-1..yh+1, pixels x0-1..x0+32 -> inS[t][ci][px_out], px_out = px_in - dx
-        for (int j = lane; j < 3 * 34 * 4; j += 64) {
-            const int r = j / 136, rem = j % 136, pin = rem >> 2, c8 = (rem & 3) * 8;
-            const int yy = yh + r - 1, xx = x0 + pin - 1;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (live && yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = *reinterpret_cast<const uint4*>(in + ((bimg * H + yy) * W + xx) * 32 + c8);
-            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+            for (int k = 0; k < 2; ++k) *reinterpret_cast<uint4*>(dzS + (px + 16 * k) * 32 + c8) = vd[k];
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (r < y1) load(r + 1);
             #pragma unroll
-            for (int dx = 0; dx < 3; ++dx) {
-                const int po = pin - dx;
-                if (po < 0 || po >= 32) continue;
-                uint16_t* dst = inS + ((r * 3 + dx) * 32 + c8) * 32 + po;
+            for (int kc = 0; kc < 2; ++kc) {
+                d2[kc] = tr_frag(dzS + 16 * kc * 32 + tl);
+                accb = mfma32(d2[kc], ones, accb);
+            }
+            #pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
                 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    dst[e * 32] = (uint16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff));
-            }
-        }
-        __syncthreads();
-        bf16x8 af[2];
-        #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-            af[mt] = as_bf16x8(*reinterpret_cast<const uint4*>(dzT + (16 * mt + r16) * 32 + 8 * g4));
-        #pragma unroll
-        for (int t = 0; t < 9; ++t) {
+                for (int kc = 0; kc < 2; ++kc) {
+                    const bf16x8 f = tr_frag(inS + (16 * kc + dx) * 32 + tl);
+                    acc[dx] = mfma32(d2[kc], f, acc[dx]);             // input row above the dz row
+                    acc[3 + dx] = mfma32(d1[kc], f, acc[3 + dx]);
+                    acc[6 + dx] = mfma32(d0[kc], f, acc[6 + dx]);     // below
+                }
             #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const bf16x8 bfrag = as_bf16x8(*reinterpret_cast<const uint4*>(inS + (t * 32 + 16 * nt + r16) * 32 + 8 * g4));
-                acc[t][0][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0], bfrag, acc[t][0][nt], 0, 0, 0);
-                acc[t][1][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[1], bfrag, acc[t][1][nt], 0, 0, 0);
+            for (int kc = 0; kc < 2; ++kc) {
+                d0[kc] = d1[kc];
+                d1[kc] = d2[kc];
             }
         }
-        __syncthreads();
     }
-    // partial of this wave: part[wave][t][co][ci], D lane layout n = ci = 16 nt + r16, m = co = 16 mt + 4 g4 + i
-    float* dst = part + ((long)blockIdx.x * WG_WAVES + wv) * 9216;
-    #pragma unroll
-    for (int t = 0; t < 9; ++t)
+    // the four waves' sums in LDS, wave after wave (a fixed order), then one partial per workgroup;
+    // D on this lane, register i: co = 8 (i / 4) + 4 (lane / 32) + i % 4, ci = lane % 32
+    float* red = reinterpret_cast<float*>(smem);
+    for (int w = 0; w < 4; ++w) {
+        __syncthreads();
+        if (w != wv) continue;
         #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int i = 0; i < 16; ++i) {
+            const int co = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
             #pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-                #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    dst[(t * 32 + 16 * mt + 4 * g4 + i) * 32 + 16 * nt + r16] = acc[t][mt][nt][i];
+            for (int t = 0; t < 9; ++t) {
+                float& q = red[t * 1024 + co * 32 + (lane & 31)];
+                q = w == 0 ? acc[t][i] : q + acc[t][i];
+            }
+            if ((lane & 31) == 0) {
+                float& q = red[9 * 1024 + co];
+                q = w == 0 ? accb[i] : q + accb[i];
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kWgOut; i += 256) part[(long)blockIdx.x * kWgOut + i] = red[i];
 }
 
 // out[i] = sum_r part[r][i]: a workgroup takes 32 adjacent columns (128-byte
@@ -926,8 +969,10 @@ __global__ __launch_bounds__(256) void k_wgrad_mid(const uint16_t* __restrict__ 
 // (624 us on average over the eight reductions of a 16 x 512^2 backward).
 constexpr int kRedCols = 32, kRedGroups = 32;
 
+// Columns n0 and up go to out2 (the bias behind a layer's weights; dropped if null).
 __global__ __launch_bounds__(kRedCols * kRedGroups) void k_reduce_rows(const float* __restrict__ part,
-                                                                       float* __restrict__ out, int nrows, int n)
+                                                                       float* __restrict__ out, int nrows, int n,
+                                                                       int n0, float* __restrict__ out2)
 {
     __shared__ float red[kRedGroups][kRedCols];
     const int c = threadIdx.x % kRedCols, grp = threadIdx.x / kRedCols;
@@ -943,13 +988,14 @@ __global__ __launch_bounds__(kRedCols * kRedGroups) void k_reduce_rows(const flo
     float t = 0.0f;
     #pragma unroll
     for (int g = 0; g < kRedGroups; ++g) t += red[g][c];
-    out[i] = t;
+    if (i < n0) out[i] = t;
+    else if (out2 != nullptr) out2[i - n0] = t;
 }
 
-void reduce_rows(const float* part, float* out, int nrows, int n, hipStream_t st)
+void reduce_rows(const float* part, float* out, int nrows, int n, hipStream_t st, int n0 = -1, float* out2 = nullptr)
 {
     hipLaunchKernelGGL(k_reduce_rows, dim3((unsigned)cdiv(n, kRedCols)), dim3(kRedCols * kRedGroups), 0, st, part,
-                       out, nrows, n);
+                       out, nrows, n, n0 < 0 ? n : n0, out2);
     check_launch("reduce_rows");
 }
 
@@ -1073,15 +1119,23 @@ void bias_grad(const uint16_t* dz, float* grad, long npx, DevBuf& work, hipStrea
     reduce_rows(work.as<float>(), grad, blocks, 32, st);
 }
 
-void wgrad_mid(const uint16_t* in, const uint16_t* dz, float* grad, int B, int H, int W, DevBuf& work, hipStream_t st)
+void wgrad_mid(const uint16_t* in, const uint16_t* dz, float* grad, float* gbias, int B, int H, int W, DevBuf& work,
+               hipStream_t st)
 {
-    const long nchunk = (long)B * H * ((W + 31) / 32);
-    const int blocks = grid_for(nchunk, WG_WAVES * 8, 1024);
-    work.ensure((size_t)blocks * WG_WAVES * 9216 * sizeof(float));
-    const size_t lds = (size_t)WG_WAVES * LDS_PER_WAVE * sizeof(uint16_t);
-    hipLaunchKernelGGL(k_wgrad_mid, dim3(blocks), dim3(256), lds, st, in, dz, work.as<float>(), B, H, W);
+    const int nxs = cdiv(W, 32);
+    RN_REQUIRE(B > 0 && H > 0 && W > 0 && (long)B * nxs * H < (1L << 30), "wgrad_mid: bad batch or image size");
+    // rows per item: one round of 2048 waves (2 per SIMD) where the batch has
+    // that many strips of at least 8 rows, at most 64 rows (the two halo rows
+    // of an item are read twice)
+    const int L = (int)std::min<long>(64, std::max<long>(8, ((long)B * nxs * H + 2047) / 2048));
+    const int nys = cdiv(H, L);
+    const int nitems = B * nxs * nys;
+    const int blocks = grid_for(nitems, 4, 512);
+    work.ensure((size_t)blocks * kWgOut * sizeof(float));
+    hipLaunchKernelGGL(k_wgrad_mid, dim3(blocks), dim3(256), 0, st, in, dz, work.as<float>(), H, W, L, nxs, nys,
+                       nitems);
     check_launch("wgrad_mid");
-    reduce_rows(work.as<float>(), grad, blocks * WG_WAVES, 9216, st);
+    reduce_rows(work.as<float>(), grad, blocks, kWgOut, st, 9216, gbias);
 }
 
 } // namespace rn

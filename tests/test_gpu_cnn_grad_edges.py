@@ -40,3 +40,21 @@ def test_narrow_gradients(shape, mode):
         assert np.array_equal(g[288:], act.sum((0, 1, 2)))
     else:
         assert g[288] == img.sum() and (g[289:] == 7.0).all()
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(5, 300, 40)])    # the last: several 64-row items per strip
+def test_mid_gradients(shape):
+    from reconnet_amd.cnn import _p, _sigs, _st
+
+    B, H, W = shape
+    rng = np.random.default_rng(100 * W + 10 * H + 5)
+    a = rng.integers(-2, 3, shape + (32,)).astype(np.float64)
+    d = rng.integers(-2, 3, shape + (32,)).astype(np.float64)
+    at, dt = (torch.from_numpy(v).cuda().to(torch.bfloat16) for v in (a, d))
+    g, gb = torch.empty(9, 32, 32, device="cuda"), torch.empty(32, device="cuda")
+    assert _sigs().rn_cnn_wgrad_mid_bias(_p(at), _p(dt), _p(g), _p(gb), B, H, W, _st()) == 0
+    p = np.pad(a, ((0, 0), (1, 1), (1, 1), (0, 0)))
+    want = np.stack([np.tensordot(d, p[:, t // 3:t // 3 + H, t % 3:t % 3 + W], ((0, 1, 2), (0, 1, 2)))
+                     for t in range(9)])
+    assert np.array_equal(g.cpu().double().numpy(), want)
+    assert np.array_equal(gb.cpu().double().numpy(), d.sum((0, 1, 2)))
