@@ -53,6 +53,7 @@ struct FanK {
     // line lies between them).  Computed in FP64.
     const float4* dray;
     const int* vwide;    // [nview] 1: every Siddon line interval of the view has a positive FP32 width
+    int dwide;           // 1: every DD footprint (dray) has a positive FP32 width on every image line
     int unit_angle;      // 1: |rx / (ry + dso)| < 1 for every pixel centre and view (image well inside the circle)
 };
 
@@ -95,8 +96,6 @@ void launch_siddon_fan_bp_f64(const FanK& g, const double* prj_vu, double* img_x
 // pixel-driven gathers (exact transposes of the two FPs above)
 void launch_siddon_fan_bp(const FanK& g, const float* prj_vu, float* img_xy, int nslices,
                           int view0, int nviews, bool accumulate, hipStream_t st);
-void launch_dd_fan_adj(const FanK& g, const float* prj_vu, float* img_xy, int nslices,
-                       int view0, int nviews, bool accumulate, hipStream_t st);
 // reference-parity DD BP (DDBPFanKernelX/Y) on a pre-weighted vu sinogram
 void launch_dd_fan_bp(const FanK& g, const float* wprj_vu, float* img_xy, int nslices, bool fbp,
                       hipStream_t st);
@@ -148,6 +147,11 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
 // reference-parity DD BP of a quad pre-weighted sinogram [q][view][nu] into plain images
 void launch_dd_fan_bp_q(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, bool fbp,
                         hipStream_t st);
+// exact DD adjoint of quad sinograms [q][nview][nu] multiplied by the rays' length
+// per line (launch_pack_quads_len) into plain images
+void launch_dd_fan_adj(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, hipStream_t st);
+// plain sinograms [s][nu][nview] -> quads [q][nview][nu] of value x sray.z
+void launch_pack_quads_len(const FanK& g, const float* in, float4* q, int nslices, hipStream_t st);
 // plain [s][n1][n2] -> quads [q][n1][n2] (if q_same) and (if q_tr) the transposed quads [q][n2][n1];
 // padded: lines of the padded layout (pitch qpitch(n2), resp. qpitch(n1); the
 // pad cells are left as they are)

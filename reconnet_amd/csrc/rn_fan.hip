@@ -430,25 +430,59 @@ __global__ __launch_bounds__(BX * BY, G >= 8 ? 4 : 1) void k_siddon_fan_bp_ql(Fa
     }
 }
 
-template <int BX, int BY, int S, bool UNIT>
-__global__ __launch_bounds__(BX * BY) void k_dd_fan_adj(FanK g, const float* __restrict__ prj,
-                                                    float* __restrict__ img, int view0, int nviews, int ns,
-                                                    int accumulate)
+// Exact DD adjoint (dd_adj_tile): a workgroup takes an 8 x 8-pixel tile of G
+// groups of 4 slices with 1 wave, or with kDdAdjSegs waves that walk one view
+// segment each (tiles x groups too few to fill the chip); the segments' sums
+// are added in LDS in segment order, the order of the one-wave shape.
+//
+// Bound: VALU (about 70 instructions per wave and view, 22 per candidate bin and
+// 4 per bin and group).  For 32 slices of 256^2, 360 views, 512 bins of 1.4 mm
+// pixels the per-slice gathers of the plain layout, S slices per lane, took
+// 1.69 ms.
+template <int G, int CAP, bool WIDE>
+__global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const float4* __restrict__ wprj,
+                                                                   float* __restrict__ img, int ns)
 {
-    const int iy = blockIdx.x * BX + threadIdx.x;
-    const int ix = blockIdx.y * BY + threadIdx.y;
-    const int s0 = blockIdx.z * S;
-    const int nsl = min(S, ns - s0);
-    if (ix >= g.nx || iy >= g.ny) return;
-    const long sstride = (long)nviews * g.nu;
-    float acc[S];
-    dd_adj_pixel_slices<UNIT, S>(g, prj + s0 * sstride, sstride, nsl, view0, nviews, ix, iy, acc);
-    const long plane = (long)g.nx * g.ny;
+    extern __shared__ float4 dyn4[];
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
+    const int iy = blockIdx.x * 8 + (lane & 7), ix = blockIdx.y * 8 + (lane >> 3);
+    const bool inside = ix < g.nx && iy < g.ny;
+    const int nquads = (ns + 3) / 4;
+    const int q0 = blockIdx.z * G;
+    const int nq = min(G, nquads - q0);
+    const long sstride = (long)g.nview * g.nu;
+    const int per = kDdAdjSegs / nw;
+    float4 tot[G];
+    dd_adj_tile<G, CAP, 3, WIDE>(g, wprj + q0 * sstride, sstride, nq, 0, g.nview, wv * per, (wv + 1) * per, ix, iy,
+                                 inside, lane, dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
+    if (nw > 1) {
+        float4* red = dyn4 + nw * DdAdjStage<G, CAP>::kFloat4;
+        for (int w = 0; w < nw; ++w) {
+            if (w == wv) {
+                #pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    float4 v = tot[k];
+                    if (w > 0) {
+                        const float4 r = red[k * 64 + lane];
+                        v = make_float4(r.x + v.x, r.y + v.y, r.z + v.z, r.w + v.w);
+                    }
+                    red[k * 64 + lane] = tot[k] = v;
+                }
+            }
+            __syncthreads();
+        }
+        if (wv != nw - 1) return;
+    }
+    if (!inside) return;
+    const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
     #pragma unroll
-    for (int q = 0; q < S; ++q) {
-        if (q >= nsl) break;
-        float* o = img + (long)(s0 + q) * plane + (long)ix * g.ny + iy;
-        *o = accumulate ? *o + acc[q] : acc[q];
+    for (int k = 0; k < G; ++k) {
+        if (k >= nq) break;
+        const int s = 4 * (q0 + k);
+        const float v[4] = {tot[k].x, tot[k].y, tot[k].z, tot[k].w};
+        #pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (s + c < ns) img[(long)(s + c) * plane + pix] = v[c];
     }
 }
 
@@ -725,9 +759,10 @@ __global__ __launch_bounds__(BX * BY) void k_pixel_fan_bp(FanK g, const float* _
 // q_same[q][i][j] = (in[4q][i][j], .., in[4q+3][i][j]) (zero past nslices) and,
 // if q_tr, q_tr[q][j][i] = the same value; 32 x 32 tiles through LDS.  Output
 // lines have pitch p_same / p_tr and start off cells into the line.
+// len (optional): the transposed values times len[j][i].z.
 __global__ __launch_bounds__(256) void k_pack_quads(const float* __restrict__ in, float4* __restrict__ q_same,
                                                     float4* __restrict__ q_tr, int n1, int n2, int ns, int p_same,
-                                                    int p_tr, int off)
+                                                    int p_tr, int off, const float4* __restrict__ len)
 {
     __shared__ float4 tile[32][33];
     const int j0 = blockIdx.x * 32, i0 = blockIdx.y * 32, q = blockIdx.z;
@@ -751,7 +786,11 @@ __global__ __launch_bounds__(256) void k_pack_quads(const float* __restrict__ in
     __syncthreads();
     for (int r = ty; r < 32; r += 8) {
         const int j = j0 + r, i = i0 + tx;
-        if (i < n1 && j < n2) q_tr[(long)q * n2 * p_tr + (long)j * p_tr + off + i] = tile[tx][r];
+        if (i < n1 && j < n2) {
+            float4 f = tile[tx][r];
+            if (len != nullptr) f = vscale(f, len[(long)j * n1 + i].z);
+            q_tr[(long)q * n2 * p_tr + (long)j * p_tr + off + i] = f;
+        }
     }
 }
 
@@ -957,6 +996,21 @@ void FanTables::build(const FanGeo& g, const float* deg_host, hipStream_t st)
         for (int kb = 0; kb < nu; kb++)
             dray[(size_t)v * nu + kb] = make_float4((float)eA[kb], (float)eB[kb], (float)eA[kb + 1], (float)eB[kb + 1]);
     }
+    // 1 if every footprint has a positive FP32 width on every image line: the
+    // edges' distance, affine in the line, has one sign and exceeds the
+    // rounding of the two end points by a wide margin
+    k.dwide = 1;
+    for (int v = 0; v < nview && k.dwide; v++) {
+        const double h = 0.5 * (cls[v] == 0 ? g.ny : g.nx);
+        for (int kb = 0; kb < nu && k.dwide; kb++) {
+            const float4 d = dray[(size_t)v * nu + kb];
+            const double dA = (double)d.z - d.x, dB = (double)d.w - d.y;
+            const double w0 = dA - dB * h, w1 = dA + dB * h;
+            const double emax = std::max(std::fabs((double)d.x), std::fabs((double)d.z)) +
+                                std::max(std::fabs((double)d.y), std::fabs((double)d.w)) * h + 1.0;
+            if (!(w0 * w1 > 0 && std::min(std::fabs(w0), std::fabs(w1)) > 1e-6 * emax && emax < 1e30)) k.dwide = 0;
+        }
+    }
     dray_.alloc(dray.size() * sizeof(float4));
     RN_HIP_CHECK(hipMemcpyAsync(dray_.get(), dray.data(), dray.size() * sizeof(float4), hipMemcpyHostToDevice, st));
     RN_HIP_CHECK(hipStreamSynchronize(st));
@@ -1034,16 +1088,13 @@ void go_siddon_bp(const FanK& g, const float* prj, float* img, int ns, int view0
                        dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns, acc);
 }
 
-template <int BX, int BY, int S>
-void go_dd_adj(const FanK& g, const float* prj, float* img, int ns, int view0, int nviews, int acc, hipStream_t st)
+template <int G, int CAP>
+void go_dd_adj(const FanK& g, const float4* wprj, float* img, int ns, int nw, hipStream_t st)
 {
-    const dim3 grd(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(ns, S));
-    if (g.unit_angle)
-        hipLaunchKernelGGL((k_dd_fan_adj<BX, BY, S, true>), grd, dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns,
-                           acc);
-    else
-        hipLaunchKernelGGL((k_dd_fan_adj<BX, BY, S, false>), grd, dim3(BX, BY), 0, st, g, prj, img, view0, nviews,
-                           ns, acc);
+    const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G)), blk(64, nw);
+    const size_t lds = ((size_t)nw * DdAdjStage<G, CAP>::kFloat4 + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    if (g.dwide) hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, true>), grd, blk, lds, st, g, wprj, img, ns);
+    else hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, false>), grd, blk, lds, st, g, wprj, img, ns);
 }
 
 template <int BX, int BY, int S>
@@ -1083,8 +1134,10 @@ const GatherFn kSidBp[] = {go_siddon_bp<16, 16, 3, 1>, go_siddon_bp<8, 8, 3, 1>,
                            go_siddon_bp<8, 8, 3, 8>,   go_siddon_bp<8, 8, 2, 16>,  go_siddon_bp<16, 16, 2, 16>};
 constexpr int kNSidFp = sizeof(kSidFp) / sizeof(kSidFp[0]);
 constexpr int kNSidBp = sizeof(kSidBp) / sizeof(kSidBp[0]);
-const GatherFn kDdAdj[] = {go_dd_adj<16, 16, 1>, go_dd_adj<8, 32, 1>, go_dd_adj<32, 8, 1>, go_dd_adj<8, 8, 1>,
-                           go_dd_adj<16, 16, 2>, go_dd_adj<8, 8, 2>,  go_dd_adj<16, 16, 4>, go_dd_adj<8, 8, 4>};
+using DdAdjFn = void (*)(const FanK&, const float4*, float*, int, int, hipStream_t);
+// groups of 4 slices per lane 1, 2, 4, 8; windows of 32 and 24 bins
+const DdAdjFn kDdAdj[] = {go_dd_adj<1, 32>, go_dd_adj<1, 24>, go_dd_adj<2, 32>, go_dd_adj<2, 24>,
+                          go_dd_adj<4, 32>, go_dd_adj<4, 24>, go_dd_adj<8, 32>, go_dd_adj<8, 24>};
 constexpr int kNDdAdj = sizeof(kDdAdj) / sizeof(kDdAdj[0]);
 const DdBpFn kDdBp[] = {go_dd_bp<16, 16, 1>, go_dd_bp<8, 32, 1>, go_dd_bp<32, 8, 1>, go_dd_bp<8, 8, 1>,
                        go_dd_bp<8, 8, 4>,   go_dd_bp<16, 16, 4>, go_dd_bp<8, 8, 8>, go_dd_bp<16, 16, 8>,
@@ -1331,15 +1384,32 @@ void launch_siddon_fan_bp(const FanK& g, const float* prj_vu, float* img_xy, int
     check_launch("siddon_fan_bp");
 }
 
-void launch_dd_fan_adj(const FanK& g, const float* prj_vu, float* img_xy, int nslices,
-                       int view0, int nviews, bool accumulate, hipStream_t st)
+void launch_dd_fan_adj(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, hipStream_t st)
 {
     if (nslices <= 0) return;
-    require_offsets32(g, nviews, sizeof(float));
-    const int c = tune_choose({TK_DD_ADJ, g.nx, g.ny, g.nu, nviews, nslices}, kNDdAdj, [&](int i) {
-        kDdAdj[i](g, prj_vu, img_xy, nslices, view0, nviews, 0, st);
-    }, st, !accumulate);
-    kDdAdj[c](g, prj_vu, img_xy, nslices, view0, nviews, accumulate ? 1 : 0, st);
+    const int nquads = cdiv(nslices, 4);
+    RN_REQUIRE((long)g.nx * g.ny * 4L < 0x7fffffffL && (long)g.nview * g.nu * 16L < 0x7fffffffL,
+               "image plane, ray table or sinogram of one slice exceeds 2 GiB");
+    // one wave per tile and view segment while one wave per tile would leave
+    // fewer than 4 waves per SIMD (1024 SIMDs): 128^2 x 180 views, one slice,
+    // 256 us with one wave per tile
+    const int nw = (long)cdiv(g.nx, 8) * cdiv(g.ny, 8) * nquads < 4096 ? kDdAdjSegs : 1;
+    // candidates in the order of preference for this batch: the fewest groups
+    // per lane that hold it first, then fewer; more groups than that last.
+    // Groups are addressed with 32-bit byte offsets: G of them have to fit.
+    int order[kNDdAdj], n = 0;
+    auto add = [&](int lg) {
+        if (lg > 0 && ((long)g.nview * g.nu * 16L << lg) >= 0x7fffffffL) return;
+        order[n++] = 2 * lg;
+        order[n++] = 2 * lg + 1;
+    };
+    int best = 0;
+    while (best < 3 && (1 << best) < nquads) ++best;
+    for (int lg = best; lg >= 0; --lg) add(lg);
+    for (int lg = best + 1; lg < 4; ++lg) add(lg);
+    const int c = tune_choose({TK_DD_ADJ, g.nx, g.ny, g.nu, g.nview, nslices}, n,
+                              [&](int i) { kDdAdj[order[i]](g, wprj_q, img_xy, nslices, nw, st); }, st, true);
+    kDdAdj[order[c]](g, wprj_q, img_xy, nslices, nw, st);
     check_launch("dd_fan_adj");
 }
 
@@ -1400,8 +1470,18 @@ void launch_pack_quads(const float* in, float4* q_same, float4* q_tr, int n1, in
     if (nslices <= 0 || n1 <= 0 || n2 <= 0) return;
     dim3 grd(cdiv(n2, 32), cdiv(n1, 32), cdiv(nslices, 4));
     hipLaunchKernelGGL(k_pack_quads, grd, dim3(256), 0, st, in, q_same, q_tr, n1, n2, nslices,
-                       padded ? qpitch(n2) : n2, padded ? qpitch(n1) : n1, padded ? kQPadL : 0);
+                       padded ? qpitch(n2) : n2, padded ? qpitch(n1) : n1, padded ? kQPadL : 0,
+                       (const float4*)nullptr);
     check_launch("pack_quads");
+}
+
+void launch_pack_quads_len(const FanK& g, const float* in, float4* q, int nslices, hipStream_t st)
+{
+    if (nslices <= 0) return;
+    dim3 grd(cdiv(g.nview, 32), cdiv(g.nu, 32), cdiv(nslices, 4));
+    hipLaunchKernelGGL(k_pack_quads, grd, dim3(256), 0, st, in, (float4*)nullptr, q, g.nu, g.nview, nslices, g.nview,
+                       g.nu, 0, g.sray);
+    check_launch("pack_quads_len");
 }
 
 void launch_permute_rows(const float* in, float* out, const int* perm, int rows, int cols, int batch,

@@ -901,59 +901,181 @@ __device__ __forceinline__ T siddon_bp_pixel(const FanK& g, const T* __restrict_
 // the reference DD BP is not the adjoint of its FP).  The pixel enters line
 // iy (or ix), its lower edge, and line iy + 1 (or ix + 1), its upper edge,
 // with weight 1/2 each (each line averages two rows); on each it takes, from
-// every bin whose footprint meets its segment, the FP's weight
-// L_k overlap / width from the same edge-ray table.  One pass over the
-// candidate bins serves both lines: the bins whose centre lies within half a
-// bin of the angles the pixel's disc spans (bin_range plus half a bin; the
-// others have zero overlap).  S slices share the weights (slice q's
-// view-major sinogram `sstride` elements after prj; q >= nsl re-reads the last).
-template <bool UNIT, int S>
-__device__ __forceinline__ void dd_adj_pixel_slices(const FanK& g, const float* __restrict__ prj, long sstride,
-                                                    int nsl, int view0, int nviews, int ix, int iy,
-                                                    float (&acc)[S])
+// every bin whose footprint meets its segment, the FP's share overlap / width
+// from the same edge rays.  One pass over the candidate bins serves both
+// lines: the bins whose centre lies within half a bin of the angles the
+// pixel's disc spans (bin_range plus half a bin; the others have zero overlap).
+//
+// A wave takes an 8 x 8-pixel tile of G groups of 4 interleaved slices
+// (float4 sinograms [view][nu], already multiplied by the rays' length per
+// line) and stages, per view, the tile's bin window in its own LDS rows: the
+// groups' values and the window's bin edges, (A, B) of one edge ray per entry,
+// each edge shared by the two bins it separates.  As in k_siddon_fan_bp_ql: CAP
+// bins at a time, the first chunk loaded one view ahead into registers, wider
+// windows in further chunks, no barrier (a wave touches only its rows), rows
+// cleared at the start so that lanes without a bin read zeros or an earlier
+// view's bins with weight 0, never unwritten memory.
+//
+// The views are summed in kDdAdjSegs fixed segments whose sums are then added
+// in order, whatever the launch shape: one wave may walk all of them, or one
+// wave each, with the same bits.
+constexpr int kDdAdjSegs = 8;
+
+template <int G, int CAP>
+struct DdAdjStage {
+    static constexpr int kVals = G * CAP;                  // float4: the groups' bins
+    static constexpr int kEdges = (CAP + 2) / 2;           // float4: CAP + 1 edges of 8 bytes
+    static constexpr int kFloat4 = kVals + kEdges;         // LDS of one wave
+};
+
+// Shares of the bins t0 .. t1 (relative to the staged window, t0 >= 0 where
+// t1 >= t0; empty otherwise) of lines lr and lr + 1 in cell [cell, cell + 1],
+// applied to the G groups.  up: 1/2 if the upper line exists, else 0.  WIDE:
+// every footprint of the geometry has a positive FP32 width (FanK::dwide).
+template <int G, int CAP, int NB, bool WIDE>
+__device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, float lr, float cell, float up,
+                                              float4 (&acc)[G])
 {
+    const float2* edge = reinterpret_cast<const float2*>(st + G * CAP);
+    const float c1 = cell + 1.0f, lu = lr + 1.0f;
+    const int ts = t1 >= t0 ? t0 : 0;
+    float2 e = edge[ts];
+    float a0 = fmaf(e.y, lr, e.x), a1 = fmaf(e.y, lu, e.x);
+    float q0 = __builtin_amdgcn_fmed3f(a0, cell, c1), q1 = __builtin_amdgcn_fmed3f(a1, cell, c1);
+    auto share = [&](float ea, float eb, float qa, float qb) {
+        const float w = eb - ea, ov = qb - qa;             // one sign: the edges are monotone
+        if (WIDE) return ov * __builtin_amdgcn_rcpf(w);
+        const float lo = fminf(ea, eb);
+        return w != 0.0f ? ov * __builtin_amdgcn_rcpf(w) : ((lo >= cell && lo < c1) ? 1.0f : 0.0f);
+    };
+    // bin at slot t, its upper edge at slot t + 1
+    auto bin = [&](int t, bool on) {
+        e = edge[t + 1];
+        const float b0 = fmaf(e.y, lr, e.x), b1 = fmaf(e.y, lu, e.x);
+        const float p0 = __builtin_amdgcn_fmed3f(b0, cell, c1), p1 = __builtin_amdgcn_fmed3f(b1, cell, c1);
+        const float s0 = share(a0, b0, q0, p0), s1 = share(a1, b1, q1, p1);
+        const float w = on ? fmaf(up, s1, 0.5f * s0) : 0.0f;
+        #pragma unroll
+        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], w);
+        a0 = b0; a1 = b1; q0 = p0; q1 = p1;
+    };
+    #pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const bool on = t0 + j <= t1;
+        bin(on ? t0 + j : 0, on);
+    }
+    for (int t = t0 + NB; t <= t1; ++t) bin(t, true);
+}
+
+// Views [nviews seg0 / kDdAdjSegs, nviews seg1 / kDdAdjSegs) of the G groups at
+// P (groups sstride cells apart, groups k >= nq read group nq - 1 and are
+// discarded by the caller) for this lane's pixel (ix, iy); lanes outside the
+// image (inside = false) stage only.  st: this wave's DdAdjStage LDS.  tot
+// receives the ordered sum of the segments' sums.  Byte offsets from P stay
+// below 2^31 (checked on the host).
+template <int G, int CAP, int NB, bool WIDE>
+__device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restrict__ P, long sstride, int nq,
+                                            int view0, int nviews, int seg0, int seg1, int ix, int iy, bool inside,
+                                            int lane, float4* st, float4 (&tot)[G])
+{
+    using S = DdAdjStage<G, CAP>;
+    static_assert(CAP <= 64, "one load for the edges and one more");
+    constexpr int kLoads = (G * CAP + 63) / 64;
+    for (int i = lane; i < S::kFloat4; i += 64) st[i] = vzero<float4>();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const int cx = min(ix, g.nx - 1), cy = min(iy, g.ny - 1);
+    const float xc = ((float)cx - 0.5f * (g.nx - 1)) * g.dx, yc = ((float)cy - 0.5f * (g.ny - 1)) * g.dy;
+    const float rpix = 0.5f * sqrtf(g.dx * g.dx + g.dy * g.dy);
     const float inv_da = 1.0f / g.da;
     const float ainv = fabsf(inv_da);
+    const float yr = (float)cy - 0.5f * g.ny, xr = (float)cx - 0.5f * g.nx;
+    const float upx = cy + 1 < g.ny ? 0.5f : 0.0f, upy = cx + 1 < g.nx ? 0.5f : 0.0f;
+    int bj[kLoads];
+    unsigned roff[kLoads];
+    bool has[kLoads];
     #pragma unroll
-    for (int q = 0; q < S; ++q) acc[q] = 0.0f;
-    const float* pq[S];
+    for (int j = 0; j < kLoads; ++j) {
+        const int i = j * 64 + lane, r = i / CAP;
+        bj[j] = i % CAP;
+        has[j] = r < G;
+        roff[j] = (unsigned)(min(r, nq - 1) * sstride) * 16u;
+    }
+    float4 acc[G], rg[kLoads];
+    float2 re;
     #pragma unroll
-    for (int q = 0; q < S; ++q) pq[q] = prj + (long)min(q, nsl - 1) * sstride;
-    const float xc = ((float)ix - 0.5f * (g.nx - 1)) * g.dx, yc = ((float)iy - 0.5f * (g.ny - 1)) * g.dy;
-    const float rpix = 0.5f * sqrtf(g.dx * g.dx + g.dy * g.dy);
-    for (int vi = 0; vi < nviews; ++vi) {
-        const int view = view0 + vi;
-        const float ct = g.vcos[view], st = g.vsin[view];
-        const float4* __restrict__ dr = g.dray + (long)view * g.nu;
-        const float4* __restrict__ sr = g.sray + (long)view * g.nu;
-        const long row = (long)vi * g.nu;
-        const bool isx = g.vcls[view] == 0;
-        const int l0 = isx ? iy : ix;
-        const int nl = isx ? g.ny : g.nx;
-        const float fcell = (float)(isx ? ix : iy);
-        const float up = l0 + 1 < nl ? 0.5f : 0.0f;     // the upper edge's line exists
-        const float rx = xc * ct + yc * st, ry = -xc * st + yc * ct;
+    for (int q = 0; q < G; ++q) tot[q] = acc[q] = vzero<float4>();
+    // the pixel's candidate bins of view row vi (empty outside the image or the detector)
+    auto range = [&](int vi, int& k0, int& k1) {
+        const float ct = g.vcos[view0 + vi], sn = g.vsin[view0 + vi];
+        const float rx = xc * ct + yc * sn, ry = -xc * sn + yc * ct;
         const float d0 = ry + g.dso;
-        const float uc = g.cu - g.off_a - atan_fast<UNIT>(rx * __builtin_amdgcn_rcpf(d0)) * inv_da;
-        const float sn = fminf(rpix * __builtin_amdgcn_rsqf(fmaf(rx, rx, d0 * d0)), 1.0f);
-        const float hw = sn * fmaf(2.0f, sn, 1.0f) * ainv + 0.52f + RN_ATAN_FAST_ERR * ainv;
-        const int k0 = max((int)ceilf(uc - hw), 0), k1 = min((int)floorf(uc + hw), g.nu - 1);
-        const float lr = (float)l0 - 0.5f * (float)nl;
-        for (int k = k0; k <= k1; ++k) {
-            const float4 d = dr[k];
-            float sh[2];
-            #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float le = lr + (float)e;
-                const float ea = fmaf(d.y, le, d.x), eb = fmaf(d.w, le, d.z);
-                const float lo = fminf(ea, eb), hi = fmaxf(ea, eb), w = hi - lo;
-                const float ov = fmaxf(fminf(hi, fcell + 1.0f) - fmaxf(lo, fcell), 0.0f);
-                const bool pos = w > 0.0f;
-                sh[e] = pos ? ov * __builtin_amdgcn_rcpf(w) : ((lo >= fcell && lo < fcell + 1.0f) ? 1.0f : 0.0f);
+        const float z = rx * __builtin_amdgcn_rcpf(d0);
+        const float uc = g.cu - g.off_a - (g.unit_angle ? atan_fast<true>(z) : atan_fast<false>(z)) * inv_da;
+        const float sr = fminf(rpix * __builtin_amdgcn_rsqf(fmaf(rx, rx, d0 * d0)), 1.0f);
+        const float hw = sr * fmaf(2.0f, sr, 1.0f) * ainv + 0.52f + RN_ATAN_FAST_ERR * ainv;
+        k0 = max((int)ceilf(uc - hw), 0);
+        k1 = min((int)floorf(uc + hw), g.nu - 1);
+        if (!inside || k1 < k0) { k0 = g.nu; k1 = -1; }
+    };
+    // loads of the CAP bins from `base` of view row vi and of their CAP + 1 edges
+    // (edge e is the first edge of bin e, the last one the second edge of the
+    // last bin), and their LDS handover
+    auto issue = [&](int vi, int base) {
+        #pragma unroll
+        for (int j = 0; j < kLoads; ++j)
+            if (has[j]) rg[j] = ld_at(P, roff[j] + (unsigned)(vi * g.nu + min(base + bj[j], g.nu - 1)) * 16u);
+        if (lane < CAP + 1) {
+            const int e = min(base + lane, g.nu);
+            const float2* d2 = reinterpret_cast<const float2*>(g.dray);
+            re = ld_at(d2, (unsigned)((view0 + vi) * g.nu) * 16u + (e < g.nu ? (unsigned)e * 16u : (unsigned)g.nu * 16u - 8u));
+        }
+    };
+    auto handover = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        #pragma unroll
+        for (int j = 0; j < kLoads; ++j)
+            if (has[j]) st[j * 64 + lane] = rg[j];
+        if (lane < CAP + 1) reinterpret_cast<float2*>(st + S::kVals)[lane] = re;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    };
+    const int vend = (int)((long)nviews * seg1 / kDdAdjSegs);
+    int vi = (int)((long)nviews * seg0 / kDdAdjSegs);
+    int k0 = g.nu, k1 = -1;
+    if (vi < vend) range(vi, k0, k1);
+    int wlo = wave_min(k0), whi = wave_max(k1);
+    if (vi < vend && whi >= wlo) issue(vi, wlo);
+    for (int seg = seg0; seg < seg1; ++seg) {
+        const int send = (int)((long)nviews * (seg + 1) / kDdAdjSegs);
+        for (; vi < send; ++vi) {
+            const bool any = whi >= wlo;
+            const int nch = any ? (whi - wlo) / CAP + 1 : 1;   // an empty window: one chunk of weight-0 reads
+            if (any) handover();
+            int n0 = g.nu, n1 = -1, nlo = g.nu, nhi = -1;
+            if (vi + 1 < vend) {
+                range(vi + 1, n0, n1);
+                nlo = wave_min(n0);
+                nhi = wave_max(n1);
             }
-            const float wk = fmaf(up, sh[1], 0.5f * sh[0]) * sr[k].z;
-            #pragma unroll
-            for (int q = 0; q < S; ++q) acc[q] = fmaf(pq[q][row + k], wk, acc[q]);
+            const bool pre = nhi >= nlo;
+            if (pre && nch == 1) issue(vi + 1, nlo);
+            const bool xv = g.vcls[view0 + vi] == 0;
+            const float lr = xv ? yr : xr, up = xv ? upx : upy;
+            const float cell = xv ? (float)cx : (float)cy;
+            dd_adj_gather<G, CAP, NB, WIDE>(st, k0 - wlo, min(k1 - wlo, CAP - 1), lr, cell, up, acc);
+            for (int c = 1; c < nch; ++c) {
+                const int base = wlo + c * CAP;
+                issue(vi, base);
+                handover();
+                dd_adj_gather<G, CAP, NB, WIDE>(st, max(k0 - base, 0), min(k1 - base, CAP - 1), lr, cell, up, acc);
+            }
+            if (pre && nch > 1) issue(vi + 1, nlo);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            k0 = n0; k1 = n1; wlo = nlo; whi = nhi;
+        }
+        #pragma unroll
+        for (int q = 0; q < G; ++q) {
+            vadd(tot[q], acc[q]);
+            acc[q] = vzero<float4>();
         }
     }
 }

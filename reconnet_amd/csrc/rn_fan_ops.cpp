@@ -168,7 +168,7 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
         Q = w.ry.as<float>();
     }
     float* W = w.sino.as<float>();   // [slice][nview][nu]
-    launch_transpose(Q, W, g.nu, g.nview, ns, st);
+    if (kind != FanBP::DDAdjoint) launch_transpose(Q, W, g.nu, g.nview, ns, st);
     float* out = direct_out ? img_ref : w.rx.as<float>();
     switch (kind) {
     case FanBP::DD:
@@ -192,7 +192,10 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
         break;
     }
     case FanBP::DDAdjoint:
-        launch_dd_fan_adj(t.k, W, out, ns, 0, g.nview, false, st);
+        // transposed, interleaved and multiplied by the rays' length per line in one pass
+        w.quad.ensure((size_t)cdiv(ns, 4) * sino * sizeof(float4));
+        launch_pack_quads_len(t.k, Q, w.quad.as<float4>(), ns, st);
+        launch_dd_fan_adj(t.k, w.quad.as<float4>(), out, ns, st);
         break;
     case FanBP::Siddon:
         launch_siddon_fan_bp(t.k, W, out, ns, 0, g.nview, false, st);

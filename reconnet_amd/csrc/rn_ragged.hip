@@ -82,11 +82,10 @@ __global__ __launch_bounds__(256) void k_ragged_fp(const RagSlice* __restrict__ 
     }
 }
 
-// S: the descriptors' slice bound (kRagSidBp for Siddon, kRagS for the DD adjoint)
-template <bool SIDDON, int S>
-__global__ __launch_bounds__(256) void k_ragged_bp(const RagSlice* __restrict__ sl, int nsl, int total,
-                                                   int* __restrict__ counter)
+__global__ __launch_bounds__(256) void k_ragged_siddon_bp(const RagSlice* __restrict__ sl, int nsl, int total,
+                                                          int* __restrict__ counter)
 {
+    constexpr int S = kRagSidBp;
     const int lane = threadIdx.x & 63;
     for (;;) {
         const int item = next_item(counter, lane);
@@ -97,15 +96,46 @@ __global__ __launch_bounds__(256) void k_ragged_bp(const RagSlice* __restrict__ 
         if (ix < d.g.nx && iy < d.g.ny) {
             const long plane = (long)d.g.nx * d.g.ny, sino = (long)d.g.nu * d.g.nview;
             float acc[S];
-            if (SIDDON)
-                siddon_bp_pixel_slices<float, 4, S>(d.g, d.pa, sino, d.nsl, 0, d.g.nview, ix, iy, acc);
-            else if (d.g.unit_angle)
-                dd_adj_pixel_slices<true, S>(d.g, d.pa, sino, d.nsl, 0, d.g.nview, ix, iy, acc);
-            else
-                dd_adj_pixel_slices<false, S>(d.g, d.pa, sino, d.nsl, 0, d.g.nview, ix, iy, acc);
+            siddon_bp_pixel_slices<float, 4, S>(d.g, d.pa, sino, d.nsl, 0, d.g.nview, ix, iy, acc);
             #pragma unroll
             for (int q = 0; q < S; ++q)
                 if (q < d.nsl) d.out[q * plane + (long)ix * d.g.ny + iy] = acc[q];
+        }
+    }
+}
+
+// DD adjoint: pa holds the descriptor's kRagS slices as kRagS / 4 interleaved
+// groups (multiplied by the rays' length per line); a wave takes one tile and
+// stages its bin windows in its own LDS rows (dd_adj_tile).
+__global__ __launch_bounds__(256, 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl, int total,
+                                                          int* __restrict__ counter)
+{
+    constexpr int G = kRagS / 4, CAP = 32;
+    __shared__ float4 stage[4 * DdAdjStage<G, CAP>::kFloat4];
+    const int lane = threadIdx.x & 63;
+    float4* st = stage + (threadIdx.x >> 6) * DdAdjStage<G, CAP>::kFloat4;
+    for (;;) {
+        const int item = __builtin_amdgcn_readfirstlane(next_item(counter, lane));
+        if (item >= total) break;
+        const RagSlice& d = sl[__builtin_amdgcn_readfirstlane(find_slice(sl, nsl, item))];
+        const int local = item - d.item0;
+        const int ix = (local / d.tiles) * 8 + (lane >> 3), iy = (local % d.tiles) * 8 + (lane & 7);
+        const bool inside = ix < d.g.nx && iy < d.g.ny;
+        const long plane = (long)d.g.nx * d.g.ny, sino = (long)d.g.nu * d.g.nview;
+        const float4* P = reinterpret_cast<const float4*>(d.pa);
+        const int nq = (d.nsl + 3) / 4;
+        float4 tot[G];
+        if (d.g.dwide)
+            dd_adj_tile<G, CAP, 3, true>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, ix, iy, inside, lane, st, tot);
+        else
+            dd_adj_tile<G, CAP, 3, false>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, ix, iy, inside, lane, st, tot);
+        if (!inside) continue;
+        #pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const float v[4] = {tot[k].x, tot[k].y, tot[k].z, tot[k].w};
+            #pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (4 * k + c < d.nsl) d.out[(4 * k + c) * plane + (long)ix * d.g.ny + iy] = v[c];
         }
     }
 }
@@ -129,7 +159,7 @@ struct RaggedBatch::Impl {
     std::vector<int> first, count;   // descriptor k: slices first[k] .. first[k] + count[k] - 1
     std::vector<int> order;          // descriptors by decreasing cost
     long img_total = 0, sino_total = 0;
-    DevBuf desc, counter, wa, wb, wc;
+    DevBuf desc, counter, wa, wb, wc, wq;
     std::vector<RagSlice> host;
 };
 
@@ -159,6 +189,10 @@ void RaggedBatch::setup(const std::vector<FanGeo>& geos, const std::vector<const
     p_->img_total = io;
     p_->sino_total = so;
     // runs of consecutive slices with one geometry and angle set, in chunks of kRagS
+    // (one chunk's interleaved groups of 4 slices are addressed with 32-bit byte offsets)
+    auto fits = [&](int s, int count) {
+        return (long)((count + 3) / 4) * geos[s].nu * geos[s].nview * 16L < 0x7fffffffL;
+    };
     auto same = [&](int a, int b) {
         const FanGeo& x = geos[a];
         const FanGeo& y = geos[b];
@@ -170,7 +204,8 @@ void RaggedBatch::setup(const std::vector<FanGeo>& geos, const std::vector<const
     p_->first.clear();
     p_->count.clear();
     for (int s = 0; s < n; s++) {
-        if (!p_->count.empty() && p_->count.back() < kRagS && same(p_->first.back(), s)) {
+        if (!p_->count.empty() && p_->count.back() < kRagS && same(p_->first.back(), s) &&
+            fits(s, p_->count.back() + 1)) {
             ++p_->count.back();
         } else {
             p_->first.push_back(s);
@@ -190,6 +225,13 @@ void RaggedBatch::setup(const std::vector<FanGeo>& geos, const std::vector<const
     p_->wa.alloc(io * sizeof(float));
     p_->wb.alloc(std::max(io, so) * sizeof(float));
     p_->wc.alloc(io * sizeof(float));
+    // the DD adjoint's interleaved sinograms: whole groups of 4 slices per descriptor
+    long qo = 0;
+    for (int k = 0; k < nd; k++) {
+        const FanGeo& g = geos[p_->first[k]];
+        qo += (long)((p_->count[k] + 3) / 4) * g.nu * g.nview;
+    }
+    p_->wq.alloc(qo * sizeof(float4));
 }
 
 int RaggedBatch::size() const { return (int)p_->tables.size(); }
@@ -253,6 +295,7 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
 {
     const int nd = (int)p_->first.size();
     float* V = p_->wb.as<float>();   // view-major copies of the sinograms
+    float4* Q = p_->wq.as<float4>();
     p_->host.clear();
     const int chunk = siddon ? kRagSidBp : kRagS;
     int item = 0;
@@ -260,13 +303,14 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
         const int s = p_->first[p_->order[k]], cnt = p_->count[p_->order[k]];
         const FanGeo& g = p_->tables[s].geo;
         float* v = V + p_->sino_off[s];
-        launch_transpose(prj + p_->sino_off[s], v, g.nu, g.nview, cnt, st);
+        if (siddon) launch_transpose(prj + p_->sino_off[s], v, g.nu, g.nview, cnt, st);
+        else launch_pack_quads_len(p_->tables[s].k, prj + p_->sino_off[s], Q, cnt, st);
         const long plane = (long)g.nx * g.ny, sino = (long)g.nu * g.nview;
         for (int c0 = 0; c0 < cnt; c0 += chunk) {
             RagSlice d{};
             d.g = p_->tables[s].k;
             d.nsl = std::min(chunk, cnt - c0);
-            d.pa = v + c0 * sino;
+            d.pa = siddon ? v + c0 * sino : reinterpret_cast<const float*>(Q);    // one chunk for the DD adjoint
             d.pb = nullptr;
             d.out = img + p_->img_off[s] + c0 * plane;
             d.tiles = cdiv(g.ny, 8);
@@ -275,15 +319,16 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
             item += d.nitems;
             p_->host.push_back(d);
         }
+        Q += (long)((cnt + 3) / 4) * sino;
     }
     const int nbd = (int)p_->host.size();
     RN_HIP_CHECK(hipMemcpyAsync(p_->desc.get(), p_->host.data(), nbd * sizeof(RagSlice), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, p_->counter.as<int>());
     if (siddon)
-        hipLaunchKernelGGL((k_ragged_bp<true, kRagSidBp>), dim3(persistent_blocks()), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_ragged_siddon_bp, dim3(persistent_blocks()), dim3(256), 0, st,
                            p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
     else
-        hipLaunchKernelGGL((k_ragged_bp<false, kRagS>), dim3(persistent_blocks()), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_ragged_dd_adj, dim3(persistent_blocks()), dim3(256), 0, st,
                            p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
     check_launch("ragged_bp");
     RN_HIP_CHECK(hipStreamSynchronize(st));
