@@ -435,10 +435,11 @@ __global__ __launch_bounds__(BX * BY, G >= 8 ? 4 : 1) void k_siddon_fan_bp_ql(Fa
 // segment each (tiles x groups too few to fill the chip); the segments' sums
 // are added in LDS in segment order, the order of the one-wave shape.
 //
-// Bound: VALU (about 70 instructions per wave and view, 22 per candidate bin and
-// 4 per bin and group).  For 32 slices of 256^2, 360 views, 512 bins of 1.4 mm
-// pixels the per-slice gathers of the plain layout, S slices per lane, took
-// 1.69 ms.
+// Bound: VALU (about 100 instructions per wave and view for the bin range, its
+// window and the staging, 20 per candidate bin and 4 per bin and group).  32
+// slices of 256^2, 360 views, 512 bins: 0.44 ms (1.69 ms with per-slice gathers
+// from memory, S slices per lane); one slice 0.12 ms; one slice of 128^2, 180
+// views 32 us (256 us).
 template <int G, int CAP, bool WIDE>
 __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const float4* __restrict__ wprj,
                                                                    float* __restrict__ img, int ns)
@@ -998,7 +999,8 @@ void FanTables::build(const FanGeo& g, const float* deg_host, hipStream_t st)
     }
     // 1 if every footprint has a positive FP32 width on every image line: the
     // edges' distance, affine in the line, has one sign and exceeds the
-    // rounding of the two end points by a wide margin
+    // rounding of the two end points by a wide margin (and the product of two
+    // widths stays in range)
     k.dwide = 1;
     for (int v = 0; v < nview && k.dwide; v++) {
         const double h = 0.5 * (cls[v] == 0 ? g.ny : g.nx);
@@ -1008,7 +1010,7 @@ void FanTables::build(const FanGeo& g, const float* deg_host, hipStream_t st)
             const double w0 = dA - dB * h, w1 = dA + dB * h;
             const double emax = std::max(std::fabs((double)d.x), std::fabs((double)d.z)) +
                                 std::max(std::fabs((double)d.y), std::fabs((double)d.w)) * h + 1.0;
-            if (!(w0 * w1 > 0 && std::min(std::fabs(w0), std::fabs(w1)) > 1e-6 * emax && emax < 1e30)) k.dwide = 0;
+            if (!(w0 * w1 > 0 && std::min(std::fabs(w0), std::fabs(w1)) > 1e-6 * emax && emax < 1e15)) k.dwide = 0;
         }
     }
     dray_.alloc(dray.size() * sizeof(float4));
@@ -1088,10 +1090,17 @@ void go_siddon_bp(const FanK& g, const float* prj, float* img, int ns, int view0
                        dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns, acc);
 }
 
+// One wave per tile and view segment while one wave per tile would leave the
+// 1024 SIMDs fewer than 8 waves each (32 slices of 256^2, 16 per lane, are 2048
+// waves: 0.62 ms by one wave per tile, 0.45 by eight).
+constexpr long kDdAdjWaves = 8192;
+
 template <int G, int CAP>
-void go_dd_adj(const FanK& g, const float4* wprj, float* img, int ns, int nw, hipStream_t st)
+void go_dd_adj(const FanK& g, const float4* wprj, float* img, int ns, hipStream_t st)
 {
-    const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G)), blk(64, nw);
+    const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
+    const int nw = (long)grd.x * grd.y * grd.z < kDdAdjWaves ? kDdAdjSegs : 1;
+    const dim3 blk(64, nw);
     const size_t lds = ((size_t)nw * DdAdjStage<G, CAP>::kFloat4 + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     if (g.dwide) hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, true>), grd, blk, lds, st, g, wprj, img, ns);
     else hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, false>), grd, blk, lds, st, g, wprj, img, ns);
@@ -1134,7 +1143,7 @@ const GatherFn kSidBp[] = {go_siddon_bp<16, 16, 3, 1>, go_siddon_bp<8, 8, 3, 1>,
                            go_siddon_bp<8, 8, 3, 8>,   go_siddon_bp<8, 8, 2, 16>,  go_siddon_bp<16, 16, 2, 16>};
 constexpr int kNSidFp = sizeof(kSidFp) / sizeof(kSidFp[0]);
 constexpr int kNSidBp = sizeof(kSidBp) / sizeof(kSidBp[0]);
-using DdAdjFn = void (*)(const FanK&, const float4*, float*, int, int, hipStream_t);
+using DdAdjFn = void (*)(const FanK&, const float4*, float*, int, hipStream_t);
 // groups of 4 slices per lane 1, 2, 4, 8; windows of 32 and 24 bins
 const DdAdjFn kDdAdj[] = {go_dd_adj<1, 32>, go_dd_adj<1, 24>, go_dd_adj<2, 32>, go_dd_adj<2, 24>,
                           go_dd_adj<4, 32>, go_dd_adj<4, 24>, go_dd_adj<8, 32>, go_dd_adj<8, 24>};
@@ -1390,10 +1399,6 @@ void launch_dd_fan_adj(const FanK& g, const float4* wprj_q, float* img_xy, int n
     const int nquads = cdiv(nslices, 4);
     RN_REQUIRE((long)g.nx * g.ny * 4L < 0x7fffffffL && (long)g.nview * g.nu * 16L < 0x7fffffffL,
                "image plane, ray table or sinogram of one slice exceeds 2 GiB");
-    // one wave per tile and view segment while one wave per tile would leave
-    // fewer than 4 waves per SIMD (1024 SIMDs): 128^2 x 180 views, one slice,
-    // 256 us with one wave per tile
-    const int nw = (long)cdiv(g.nx, 8) * cdiv(g.ny, 8) * nquads < 4096 ? kDdAdjSegs : 1;
     // candidates in the order of preference for this batch: the fewest groups
     // per lane that hold it first, then fewer; more groups than that last.
     // Groups are addressed with 32-bit byte offsets: G of them have to fit.
@@ -1408,8 +1413,8 @@ void launch_dd_fan_adj(const FanK& g, const float4* wprj_q, float* img_xy, int n
     for (int lg = best; lg >= 0; --lg) add(lg);
     for (int lg = best + 1; lg < 4; ++lg) add(lg);
     const int c = tune_choose({TK_DD_ADJ, g.nx, g.ny, g.nu, g.nview, nslices}, n,
-                              [&](int i) { kDdAdj[order[i]](g, wprj_q, img_xy, nslices, nw, st); }, st, true);
-    kDdAdj[order[c]](g, wprj_q, img_xy, nslices, nw, st);
+                              [&](int i) { kDdAdj[order[i]](g, wprj_q, img_xy, nslices, st); }, st, true);
+    kDdAdj[order[c]](g, wprj_q, img_xy, nslices, st);
     check_launch("dd_fan_adj");
 }
 

@@ -942,19 +942,23 @@ __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, 
     float2 e = edge[ts];
     float a0 = fmaf(e.y, lr, e.x), a1 = fmaf(e.y, lu, e.x);
     float q0 = __builtin_amdgcn_fmed3f(a0, cell, c1), q1 = __builtin_amdgcn_fmed3f(a1, cell, c1);
-    auto share = [&](float ea, float eb, float qa, float qb) {
-        const float w = eb - ea, ov = qb - qa;             // one sign: the edges are monotone
-        if (WIDE) return ov * __builtin_amdgcn_rcpf(w);
-        const float lo = fminf(ea, eb);
-        return w != 0.0f ? ov * __builtin_amdgcn_rcpf(w) : ((lo >= cell && lo < c1) ? 1.0f : 0.0f);
+    // 1/2 share on line lr + up x share on line lr + 1 (overlap and width have
+    // one sign: the edges are monotone); WIDE: both quotients by one reciprocal
+    auto weight = [&](float b0, float b1, float p0, float p1) {
+        const float w0 = b0 - a0, w1 = b1 - a1, v0 = p0 - q0, v1 = p1 - q1;
+        if (WIDE) return fmaf(0.5f * v0, w1, up * v1 * w0) * __builtin_amdgcn_rcpf(w0 * w1);
+        const float l0 = fminf(a0, b0), l1 = fminf(a1, b1);
+        const float s0 = w0 != 0.0f ? v0 * __builtin_amdgcn_rcpf(w0) : ((l0 >= cell && l0 < c1) ? 1.0f : 0.0f);
+        const float s1 = w1 != 0.0f ? v1 * __builtin_amdgcn_rcpf(w1) : ((l1 >= cell && l1 < c1) ? 1.0f : 0.0f);
+        return fmaf(up, s1, 0.5f * s0);
     };
     // bin at slot t, its upper edge at slot t + 1
     auto bin = [&](int t, bool on) {
         e = edge[t + 1];
         const float b0 = fmaf(e.y, lr, e.x), b1 = fmaf(e.y, lu, e.x);
         const float p0 = __builtin_amdgcn_fmed3f(b0, cell, c1), p1 = __builtin_amdgcn_fmed3f(b1, cell, c1);
-        const float s0 = share(a0, b0, q0, p0), s1 = share(a1, b1, q1, p1);
-        const float w = on ? fmaf(up, s1, 0.5f * s0) : 0.0f;
+        const float wt = weight(b0, b1, p0, p1);
+        const float w = on ? wt : 0.0f;
         #pragma unroll
         for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], w);
         a0 = b0; a1 = b1; q0 = p0; q1 = p1;
