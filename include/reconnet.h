@@ -278,9 +278,11 @@ int rn_tv_iso_sqs(const float* img, float* s1, float* s2, float* var, int nb, in
  * axis (x iff |C.x - S.x| >= |C.y - S.y|) the rectangle footprints of the
  * detector cells; its backward is the exact adjoint.  The Siddon kind is the
  * SiddonCone pair (SiddonCone.cu:117,196).  Device pointers, reference
- * layouts, caller stream.  A plan keeps one scratch buffer (the DD
- * backward's FP64 row sums, 8·nBatches·nChannels·nu·nview·(nv + 1) bytes):
- * calls on one plan must not overlap. */
+ * layouts, caller stream.  A plan keeps one scratch buffer (the DD backward's
+ * row windows, 4·nBatches·nChannels·nu·nview·(nv + 12) bytes, or its FP64 row
+ * sums, 8·nBatches·nChannels·nu·nview·(nv + 1) bytes, where a voxel covers more
+ * than 7 rows and while the launch shape is tuned): calls on one plan must not
+ * overlap. */
 enum { RN_CONE_DD = 0, RN_CONE_SIDDON = 1 };
 void* rn_cone_plan_create(int nx, int ny, int nz, float dx, float dy, float dz, float cx, float cy, float cz,
         int nu, int nview, int nv, float du, float dv, float off_u, float off_v,

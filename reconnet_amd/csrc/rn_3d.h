@@ -57,8 +57,9 @@ public:
     ArbGeo geo{};
 private:
     // vec_: C, U, V, S per view; cls_: main axis per view; views_, cols_:
-    // per-view and per-(view, column) constants of the table-driven adjoint
+    // per-view and per-(view, column) constants of the DD adjoint
     DevBuf vec_, cls_, views_, cols_;
+    double ds_max_ = 0.0;   // most detector rows a voxel covers along z
 };
 
 struct HelicalGeo {

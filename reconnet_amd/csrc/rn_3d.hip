@@ -879,124 +879,242 @@ __global__ __launch_bounds__(256) void k_dd_cone_rowsum(ArbGeo a, const float* _
     }
 }
 
-// Exact transpose of k_dd_cone_fp: voxel (ix, iy, iz) gathers, per view, the
-// cells whose footprint on its plane overlaps it, with the forward pass's
-// weight overlap / area * L.  A wave holds one (ix, iy) column of 64 voxels
-// along z, so the view's plane, the candidate detector columns and each
-// column's in-plane footprint [e1, e2] (the rays through its u edges, which
-// do not depend on v because the detector rows run along z) are
-// wave-uniform.  Candidate columns come from inverting the plane crossing of
-// the u-edge rays, u = (A - q Cc) / (q D - B) with q the in-plane slope of the
-// voxel edge.  Along a column the rows' z edges on plane p are affine in v,
-// z(v) = alpha + beta v (the forward pass's z-edge crossings), which gives
-// each lane its candidate rows and every row its footprint with a few FMAs.
-// Reference layouts.
-template <int ZPL>
-__global__ __launch_bounds__(256) void k_dd_cone_adj(ArbGeo a, Grid3K g, const float* __restrict__ prj,
-                                                     float* __restrict__ img, const float* Cp, const float* Up,
-                                                     const float* Vp, const float* Sp, const int* __restrict__ cls,
-                                                     int nC)
+// Row windows of the list-driven adjoint: len(row) q(row) of every (slice, view,
+// detector column) as floats with `pad` zero rows before and 4 after, pitch nvp.
+__global__ __launch_bounds__(256) void k_dd_cone_rows(ArbGeo a, const float* __restrict__ prj, const float* Cp,
+                                                      const float* Up, const float* Vp, const float* Sp, int nC,
+                                                      long n, int nvp, int pad, float* __restrict__ Q)
 {
-    const int iz = (blockIdx.x * 64 + (threadIdx.x & 63)) * ZPL;
-    const int iy = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + (int)(threadIdx.x >> 6));
-    const int ix = blockIdx.z % g.nx, bc = blockIdx.z / g.nx;
-    if (iz >= g.nz || iy >= g.ny) return;
-    const int cc = bc % nC, b = bc / nC;
-    const float* q = prj + (long)b * a.nu * a.nview * a.nv * nC + cc;
-    const float cu = (a.nu - 1) / 2.0f + a.off_u, cv = (a.nv - 1) / 2.0f + a.off_v;
-    const float margin = 0.05f;
-    const float fz = (float)iz;
-    const float idu = 1.0f / a.du, idv = 1.0f / a.dv, idz = 1.0f / g.dz;
-    float acc[ZPL];
-    #pragma unroll
-    for (int k = 0; k < ZPL; ++k) acc[k] = 0.f;
-    for (int view = 0; view < a.nview; ++view) {
-        const bool xv = cls[view] == 0;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const long col = i / nvp;
+    const int iv = (int)(i - col * nvp) - pad;
+    float f = 0.0f;
+    if (iv >= 0 && iv < a.nv) {
+        const int iu = (int)(col % a.nu);
+        const long rest = col / a.nu;
+        const int view = (int)(rest % a.nview);
+        const long bc = rest / a.nview;
+        const int cc = (int)(bc % nC), b = (int)(bc / nC);
         const F3 c = ld3(Cp, view), U = ld3(Up, view), V = ld3(Vp, view), s = ld3(Sp, view);
-        const int p = xv ? ix : iy, j = xv ? iy : ix;
-        const int nm = xv ? g.nx : g.ny, nn = xv ? g.ny : g.nx;
-        const float dm = xv ? g.dx : g.dy, dn = xv ? g.dy : g.dx;
-        const float idn = 1.0f / dn;
-        const float sm = xv ? s.x : s.y, sn = xv ? s.y : s.x;
-        const float cn = xv ? g.cy : g.cx;
-        const float cm = xv ? c.x : c.y, cnd = xv ? c.y : c.x, Um = xv ? U.x : U.y, Un = xv ? U.y : U.x;
-        // plane p, relative to the source along the main axis
-        const float mp = ((float)p + 0.5f - 0.5f * nm) * dm + (xv ? g.cx : g.cy) - sm;
+        const float uc = ((float)iu - ((a.nu - 1) / 2.0f + a.off_u)) * a.du;
+        const float lx = fmaf(uc, U.x, c.x) - s.x, ly = fmaf(uc, U.y, c.y) - s.y;
+        const float lzs = V.z * a.dv, lz_0 = fmaf(-((a.nv - 1) / 2.0f + a.off_v), lzs, fmaf(uc, U.z, c.z) - s.z);
+        const float lz = fmaf(lzs, (float)iv, lz_0);
+        f = sqrtf(fmaf(lz, lz, fmaf(lx, lx, ly * ly))) *
+            prj[((((long)b * a.nu + iu) * a.nview + view) * a.nv + iv) * nC + cc];
+    }
+    Q[i] = f;
+}
+
+// Exact transpose of k_dd_cone_fp: a voxel gathers, per view, the cells whose
+// footprint on its plane overlaps it, with the forward pass's weight
+// overlap / area * L.  The in-plane part (which detector columns meet the
+// column (x, y) of voxels, with what share) does not depend on z, and along a
+// detector column the rows' z edges on the plane are affine in z: the row
+// coordinate of z index zi is s(zi) = zi ibdv + c, so a voxel takes the rows it
+// covers, [s, s + |ibdv|], with weights clamp(s + |ibdv| - j, 0, 1) etc.
+//
+// A group of LZ lanes takes one (x, y); 64 / LZ of them share a wave.  Per batch
+// of LZ views each lane works out one view's columns and appends {share, c,
+// ibdv, row offset} to the group's list in LDS; then the group's lanes take LZ
+// consecutive voxels of the z range the batch reaches and walk the list: one
+// LDS broadcast, one load of 3 or 4 adjacent rows and 16 VALU instructions
+// per entry and lane.  The sums over the batch go to the group's z column in
+// LDS.
+//
+// Bound: VALU issue and the texture addresser alike (16-byte loads): 3.0 ms at
+// 256^2 x 128, 720 views, 64 x 512, and 0.11 ms for the row windows.  Why this
+// split: a cone detector's rows reach a quarter to a third of the z range, so
+// 64 lanes along z with every lane's 2 voxels tested per view and column left
+// 28 % of the lanes busy, the (x, y) geometry was repeated by every lane, and
+// FP64 row sums cost 3 16-byte loads per 2 voxels (13.1 ms).  16 lanes per
+// (x, y) cover that reach best (3.2 ms with 8, 4.4 with 32, 5.1 with 64).
+constexpr int kConeZB = 256;        // z voxels of a workgroup's columns
+constexpr int kConeCols = 4;        // list entries per view and round
+constexpr float kConeMaxDs = 7.0f;  // rows per voxel beyond which the row-sum tables are used
+
+// rows r0 .. r0 + NR - 1 of the window at byte offset off (r0 >= -pad, r0 + NR <= nv + 4)
+template <int NR>
+__device__ __forceinline__ void cone_rows(const char* __restrict__ Q, unsigned off, float (&v)[NR])
+{
+    typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float F2 __attribute__((ext_vector_type(2), aligned(4)));
+    if constexpr (NR == 4) {
+        const F4 x = *reinterpret_cast<const F4*>(Q + off);
+        v[0] = x[0]; v[1] = x[1]; v[2] = x[2]; v[3] = x[3];
+    } else {
+        static_assert(NR == 3, "3 or 4 rows");
+        const F2 x = *reinterpret_cast<const F2*>(Q + off);
+        v[0] = x[0]; v[1] = x[1];
+        v[2] = *reinterpret_cast<const float*>(Q + off + 8u);
+    }
+}
+
+// Sum over the list's n entries (a multiple of 4) for the voxel at z index fz.
+// NR = 3 or 4: every entry's |ibdv| <= NR - 1; NR = 0: any, in chunks of 4 rows.
+template <int NR>
+__device__ __forceinline__ float cone_list_sum(const float4* list, int n, const char* __restrict__ Q, float fz,
+                                               float lo, float hi, int chunks)
+{
+    float sum = 0.0f;
+    for (int i = 0; i < n; i += 4) {
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float4 e = list[i + k];
+            const float s = fmaf(fz, e.z, e.y), r0 = floorf(s);
+            const float f = s - r0, t = f + fabsf(e.z);
+            const unsigned off = __float_as_uint(e.w);
+            if constexpr (NR > 0) {
+                const int r = (int)__builtin_amdgcn_fmed3f(r0, lo, hi);
+                float v[NR];
+                cone_rows<NR>(Q, off + (unsigned)(r * 4), v);
+                float d = (fminf(t, 1.0f) - f) * v[0];
+                #pragma unroll
+                for (int j = 1; j < NR; ++j) d = fmaf(__builtin_amdgcn_fmed3f(t - (float)j, 0.0f, 1.0f), v[j], d);
+                sum = fmaf(e.x, d, sum);
+            } else {
+                float d = 0.0f;
+                for (int c = 0; c < chunks; ++c) {
+                    const int r = (int)__builtin_amdgcn_fmed3f(r0 + 4.0f * (float)c, lo, hi);
+                    float v[4];
+                    cone_rows<4>(Q, off + (unsigned)(r * 4), v);
+                    #pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float q = (float)(4 * c + j);
+                        const float w = __builtin_amdgcn_fmed3f(t - q, 0.0f, 1.0f);
+                        d = fmaf(c + j == 0 ? w - f : w, v[j], d);
+                    }
+                }
+                sum = fmaf(e.x, d, sum);
+            }
+        }
+    }
+    return sum;
+}
+
+// maximum over the wave's 64 lanes of a non-negative value
+__device__ __forceinline__ int wave_max_nn(int v)
+{
+    #pragma unroll
+    for (int d = 1; d < 64; d <<= 1) v = max(v, __shfl_xor(v, d));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+template <int LZ>
+__global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g, const float* __restrict__ Q, int nvp,
+                                                             int pad, float* __restrict__ img,
+                                                             const ConeView* __restrict__ views,
+                                                             const ConeColumn* __restrict__ cols, int nC)
+{
+    constexpr int NG = 64 / LZ;
+    __shared__ float4 lists[4][64 * kConeCols];
+    __shared__ float accs[4][NG * kConeZB];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int grp = lane / LZ, lg = lane % LZ;
+    const int iy0 = ((int)blockIdx.y * 4 + wv) * NG;
+    if (iy0 >= g.ny) return;                       // whole waves (no workgroup barrier below)
+    const int iy = iy0 + grp, ix = blockIdx.z % g.nx, bc = blockIdx.z / g.nx;
+    const int z0 = (int)blockIdx.x * kConeZB, z1 = min(z0 + kConeZB, g.nz);
+    float4* list = lists[wv] + grp * (LZ * kConeCols);
+    float* acc = accs[wv] + grp * kConeZB;
+    for (int z = lg; z < kConeZB; z += LZ) acc[z] = 0.0f;
+    const char* Qb = reinterpret_cast<const char*>(Q + (long)bc * a.nview * a.nu * nvp);
+    const float cu = (a.nu - 1) / 2.0f + a.off_u, idu = 1.0f / a.du;
+    const float margin = 0.05f;
+    const float fnv = (float)a.nv, lo = -(float)pad, fz0 = (float)z0, fz1 = (float)z1;
+    const unsigned long long gmask = LZ == 64 ? ~0ull : ((1ull << (LZ & 63)) - 1ull);
+    for (int vb = 0; vb < a.nview; vb += LZ) {
+        const int view = min(vb + lg, a.nview - 1);
+        const ConeView vw = views[view];
+        const int p = vw.xv ? ix : iy, j = vw.xv ? iy : ix;
+        const float mp = fmaf((float)p, vw.dm, vw.mp0);
         const float imp = __builtin_amdgcn_rcpf(mp);
-        // u of the rays through the voxel's two in-plane edges
-        const float cn0 = cn - 0.5f * nn * dn;
-        const float A = cnd - sn, Cc = cm - sm;
+        // u of the rays through the column's two in-plane edges
         float ulo = 3.0e38f, uhi = -3.0e38f;
         #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const float qe = (cn0 + (float)(j + e) * dn - sn) * imp;
-            const float u = (A - qe * Cc) * __builtin_amdgcn_rcpf(qe * Um - Un);
+            const float qe = fmaf((float)(j + e), vw.dn, vw.qn0) * imp;
+            const float u = fmaf(-qe, vw.Cc, vw.A) * __builtin_amdgcn_rcpf(fmaf(qe, vw.Um, -vw.Un));
             ulo = fminf(ulo, u);
             uhi = fmaxf(uhi, u);
         }
         const float flo = fmaxf(ulo * idu + cu - 0.5f - margin, -1.0f);
         const float fhi = fminf(uhi * idu + cu + 0.5f + margin, (float)a.nu);
-        if (!(fhi >= flo)) continue;                // also rejects NaN
-        const int u0 = max((int)ceilf(flo), 0), u1 = min((int)floorf(fhi), a.nu - 1);
-        for (int iu = u0; iu <= u1; ++iu) {
-            const float uc = ((float)iu - cu) * a.du;
-            // in-plane footprint of the column on plane p (index coordinates)
-            bool ok = true;
-            float ee[2];
+        int u0 = 0, ncol = 0;
+        if (fhi >= flo && vb + lg < a.nview && iy < g.ny) {       // false for NaN
+            u0 = max((int)ceilf(flo), 0);
+            ncol = max(min((int)floorf(fhi), a.nu - 1) - u0 + 1, 0);
+        }
+        const int maxcol = wave_max_nn(ncol);
+        for (int cb = 0; cb < maxcol; cb += kConeCols) {
+            int cnt = 0;
+            float zl = 3.0e38f, zh = -3.0e38f, dmax = 0.0f;
             #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float ue = fmaf(e ? 0.5f : -0.5f, a.du, uc);
-                const float em = fmaf(ue, Um, cm) - sm, eo = fmaf(ue, Un, cnd) - sn;
-                ok = ok && fabsf(em) > 1e-6f;
-                ee[e] = (fmaf(mp, eo * __builtin_amdgcn_rcpf(em), sn) - cn) * idn + 0.5f * nn;
-            }
-            const float e1 = fminf(ee[0], ee[1]), e2 = fmaxf(ee[0], ee[1]);
-            const float oe = fminf(e2, (float)(j + 1)) - fmaxf(e1, (float)j);
-            const float dpc = fmaf(uc, Um, cm) - sm;     // centre ray's main-axis run to the detector
-            if (!ok || !(fabsf(dpc) > 1e-6f) || !(oe > 0.f) || !(e2 > e1)) continue;
-            const float idpc = __builtin_amdgcn_rcpf(dpc);
-            const float lx = fmaf(uc, U.x, c.x) - s.x, ly = fmaf(uc, U.y, c.y) - s.y;
-            const float lxy2 = fmaf(lx, lx, ly * ly);
-            const float zc0 = fmaf(uc, U.z, c.z) - s.z;
-            // z edges of a row at detector height v: alpha + beta v (index
-            // coordinates); every row's footprint is |beta| dv high
-            const float alpha = (fmaf(mp, zc0 * idpc, s.z) - g.cz) * idz + 0.5f * g.nz;
-            const float beta = mp * V.z * idpc * idz;
-            if (!(fabsf(beta) > 0.f)) continue;
-            const float ib = __builtin_amdgcn_rcpf(beta);
-            const float va = (fz - alpha) * ib, vb = (fz + (float)ZPL - alpha) * ib;
-            const float glo = fmaxf(fminf(va, vb) * idv + cv - 0.5f - margin, -1.0f);
-            const float ghi = fminf(fmaxf(va, vb) * idv + cv + 0.5f + margin, (float)a.nv);
-            if (!(ghi >= glo)) continue;
-            const int v0 = max((int)ceilf(glo), 0), v1 = min((int)floorf(ghi), a.nv - 1);
-            // oe / (e2 - e1) / (|beta| dv) * dm / |dpc|: every factor of the weight but oz and the length
-            const float wcol = oe * __builtin_amdgcn_rcpf((e2 - e1) * fabsf(beta) * a.dv) * dm * fabsf(idpc);
-            // the row's z edges and the ray's z run are affine in the row
-            // index: z1 = z1_0 + beta dv iv, z2 = z1 + |beta| dv, lz = lz_0 + V.z dv iv
-            const float bdv = beta * a.dv, hb = 0.5f * a.dv;
-            const float z1_0 = fmaf(beta, -cv * a.dv - hb, alpha) + fminf(bdv, 0.f), zh = fabsf(bdv);
-            const float lzs = V.z * a.dv, lz_0 = fmaf(-cv, lzs, zc0);
-            const float* qcol = q + ((long)iu * a.nview + view) * a.nv * nC;
-            for (int iv = v0; iv <= v1; ++iv) {
-                const float fiv = (float)iv;
-                const float z1 = fmaf(bdv, fiv, z1_0), z2 = z1 + zh;
-                const float lz = fmaf(lzs, fiv, lz_0);
-                const float wv = wcol * __builtin_amdgcn_sqrtf(fmaf(lz, lz, lxy2)) * qcol[(long)iv * nC];
-                #pragma unroll
-                for (int k = 0; k < ZPL; ++k) {
-                    const float oz = fminf(z2, fz + (float)(k + 1)) - fmaxf(z1, fz + (float)k);
-                    if (oz > 0.f) acc[k] = fmaf(oz, wv, acc[k]);
+            for (int c = 0; c < kConeCols; ++c) {
+                bool on = cb + c < ncol;
+                float4 e = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (on) {
+                    const long ci = (long)view * a.nu + (u0 + cb + c);
+                    const ConeColumn col = cols[ci];
+                    // in-plane footprint of the column on plane p (index coordinates)
+                    const float ea = fmaf(mp, col.k0, vw.o), eb = fmaf(mp, col.k1, vw.o);
+                    const float e1 = fminf(ea, eb), e2 = fmaxf(ea, eb);
+                    const float oe = fminf(e2, (float)(j + 1)) - fmaxf(e1, (float)j);
+                    // row coordinate of z index zi: (zi - zA) / bdv = zi ibdv + s0
+                    const float zA = fmaf(mp, col.A1, vw.a0), ibdv = imp * col.T3;
+                    on = oe > 0.0f && e2 > e1 && fabsf(ibdv) <= kConeMaxDs && ibdv != 0.0f;
+                    // share of the column times dm / |dpc|
+                    e.x = oe * __builtin_amdgcn_rcpf(e2 - e1) * fabsf(col.W);
+                    e.y = fminf(ibdv, 0.0f) - zA * ibdv;
+                    e.z = ibdv;
+                    e.w = __uint_as_float((unsigned)(ci * nvp + pad) * 4u);
+                    const float zB = fmaf(fnv, __builtin_amdgcn_rcpf(ibdv), zA);
+                    if (on) {
+                        zl = fminf(zl, fminf(zA, zB));
+                        zh = fmaxf(zh, fmaxf(zA, zB));
+                        dmax = fmaxf(dmax, fabsf(ibdv));
+                    }
                 }
+                const unsigned long long gm = (__ballot(on) >> (grp * LZ)) & gmask;
+                if (on) list[cnt + __popcll(gm & ((1ull << lg) - 1ull))] = e;
+                cnt += __popcll(gm);
             }
+            const int n = (wave_max_nn(cnt) + 3) & ~3;
+            for (int i = cnt + lg; i < n; i += LZ) list[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            // the voxels the batch reaches, the same for the group's lanes
+            #pragma unroll
+            for (int d = 1; d < LZ; d <<= 1) {
+                zl = fminf(zl, __shfl_xor(zl, d));
+                zh = fmaxf(zh, __shfl_xor(zh, d));
+            }
+            #pragma unroll
+            for (int d = 1; d < 64; d <<= 1) dmax = fmaxf(dmax, __shfl_xor(dmax, d));
+            dmax = wave_uniform(dmax);
+            const int zs = (int)__builtin_amdgcn_fmed3f(zl - 1.0f, fz0, fz1);
+            const int ze = (int)__builtin_amdgcn_fmed3f(zh + 2.0f, fz0, fz1);
+            const int passes = wave_max_nn(max((ze - zs + LZ - 1) / LZ, 0));
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            for (int m = 0; m < passes; ++m) {
+                const int z = zs + m * LZ + lg;
+                const float fz = (float)z;
+                float v;
+                if (dmax <= 2.0f) v = cone_list_sum<3>(list, n, Qb, fz, lo, fnv, 0);
+                else if (dmax <= 3.0f) v = cone_list_sum<4>(list, n, Qb, fz, lo, fnv, 0);
+                else v = cone_list_sum<0>(list, n, Qb, fz, lo, fnv, ((int)dmax + 5) / 4);
+                if (z < ze) acc[z - z0] += v;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
     }
-    float* out = img + ((((long)b * g.nx + ix) * g.ny + iy) * g.nz + iz) * nC + cc;
-    #pragma unroll
-    for (int k = 0; k < ZPL; ++k)
-        if (iz + k < g.nz) out[(long)k * nC] = acc[k];
+    if (iy >= g.ny) return;
+    const int cc = bc % nC, b = bc / nC;
+    float* out = img + ((((long)b * g.nx + ix) * g.ny + iy) * g.nz) * nC + cc;
+    for (int z = z0 + lg; z < z1; z += LZ) out[(long)z * nC] = acc[z - z0];
 }
 
-// k_dd_cone_adj driven by tables: the rows' z footprints on a column's
+// The same from running row sums, for rows much finer than a voxel (and the
+// launch-shape tuner's other candidates): the rows' z footprints on a column's
 // plane tile z without gaps (row r covers [zA + r bdv, zA + (r + 1) bdv],
 // bdv = beta dv), so the sum over rows of the z overlap times len q is bdv
 // times the difference of the row sums, interpolated linearly within a row,
@@ -1402,7 +1520,8 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
     cls_.alloc(cls.size() * sizeof(int));
     RN_HIP_CHECK(hipMemcpyAsync(vec_.get(), h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice, st));
     RN_HIP_CHECK(hipMemcpyAsync(cls_.get(), cls.data(), cls.size() * sizeof(int), hipMemcpyHostToDevice, st));
-    // view and column tables of the table-driven DD adjoint, in double
+    // view and column tables of the DD adjoint, in double
+    ds_max_ = 0.0;
     std::vector<ConeView> vt(n);
     std::vector<ConeColumn> ct((size_t)n * g.nu);
     const double cu = (g.nu - 1) / 2.0 + g.off_u, cv = (g.nv - 1) / 2.0 + g.off_v;
@@ -1428,6 +1547,7 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
         w.o = (float)((Sn - gn) / dn + 0.5 * nn);
         w.a0 = (float)((Sz - g.cz) / g.dz + 0.5 * g.nz);
         w.pad = 0.f;
+        float t3 = 0.f;
         for (int iu = 0; iu < g.nu; iu++) {
             ConeColumn& k = ct[(size_t)v * g.nu + iu];
             k = ConeColumn{0.f, 0.f, 0.f, 0.f, 0.f, {0.f, 0.f, 0.f}};
@@ -1441,8 +1561,12 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
             k.k1 = (float)(e1n / e1m / dn);
             k.A1 = (float)(zr0 / dpc / g.dz);
             k.T3 = (float)(dpc * g.dz / (Vz * g.dv));
+            t3 = std::max(t3, std::fabs(k.T3));
             k.W = (float)(dm / std::fabs(dpc) * (Vz / dpc > 0 ? 1.0 : -1.0));
         }
+        // rows per voxel on the plane nearest to the source (unbounded if it lies between the planes)
+        const double m0 = w.mp0, m1 = w.mp0 + (nm - 1) * dm;
+        ds_max_ = std::max(ds_max_, m0 * m1 > 0 ? t3 / std::min(std::fabs(m0), std::fabs(m1)) : HUGE_VAL);
     }
     views_.alloc(vt.size() * sizeof(ConeView));
     cols_.alloc(ct.size() * sizeof(ConeColumn));
@@ -1487,18 +1611,36 @@ void ConePlan::dd_adj(int nB, int nC, const float* prj, float* img, DevBuf& work
     const ArbGeo& g = geo;
     RN_REQUIRE(nB > 0 && nC > 0 && (long)g.nx * nB * nC <= 65535, "cone batch too large for one launch");
     const float* v = vec_.as<float>();
-    // candidates 0-2: 1, 2 or 4 voxels per lane summing the rows one by one;
-    // 3-5: 1, 2 or 4 voxels per lane from the row-sum table
     const long ncols = (long)nB * nC * g.nu * g.nview;
     RN_REQUIRE((ncols + 3) / 4 < 0x7fffffffL, "dd_cone_adj: too many detector columns");
-    auto launch = [&](int c) {
-        const int zpl = 1 << (c % 3);
-        dim3 grd(cdiv(g.nz, 64 * zpl), cdiv(g.ny, 4), g.nx * nB * nC);
+    // candidates 0-2: one (x, y) per 16, 8 or 32 lanes walking lists of columns
+    // over row windows (up to kConeMaxDs rows per voxel: beyond, a voxel's rows
+    // are better taken from two row sums; the windows of one slice in 4 GiB);
+    // 3-5: 1, 2 or 4 voxels per lane from the row-sum table
+    const int pad = 8, nvp = pad + g.nv + 4;
+    const bool windows = ds_max_ <= kConeMaxDs && (long)g.nu * g.nview * nvp * 4L < (1L << 32);
+    const int first = windows ? 0 : 3;
+    auto launch = [&](int i) {
+        const int c = first + i;
         if (c < 3) {
-            auto k = c == 0 ? k_dd_cone_adj<1> : c == 1 ? k_dd_cone_adj<2> : k_dd_cone_adj<4>;
-            hipLaunchKernelGGL(k, grd, dim3(256), 0, st, g, grid_of(g), prj, img, v, v + 3 * g.nview,
-                               v + 6 * g.nview, v + 9 * g.nview, cls_.as<int>(), nC);
+            work.ensure((size_t)ncols * nvp * sizeof(float));
+            float* Q = work.as<float>();
+            const long n = ncols * nvp;
+            RN_REQUIRE((n + 255) / 256 < 0x7fffffffL, "dd_cone_adj: too many detector rows");
+            hipLaunchKernelGGL(k_dd_cone_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, prj, v,
+                               v + 3 * g.nview, v + 6 * g.nview, v + 9 * g.nview, nC, n, nvp, pad, Q);
+            check_launch("dd_cone_rows");
+            auto go = [&](auto kern, int lz) {
+                const dim3 grd(cdiv(g.nz, kConeZB), cdiv(g.ny, 4 * (64 / lz)), g.nx * nB * nC);
+                hipLaunchKernelGGL(kern, grd, dim3(256), 0, st, g, grid_of(g), Q, nvp, pad, img,
+                                   views_.as<ConeView>(), cols_.as<ConeColumn>(), nC);
+            };
+            if (c == 0) go(k_dd_cone_adj_list<16>, 16);
+            else if (c == 1) go(k_dd_cone_adj_list<8>, 8);
+            else go(k_dd_cone_adj_list<32>, 32);
         } else {
+            const int zpl = 1 << (c - 3);
+            const dim3 grd(cdiv(g.nz, 64 * zpl), cdiv(g.ny, 4), g.nx * nB * nC);
             work.ensure((size_t)ncols * (g.nv + 1) * sizeof(double));
             double* T = work.as<double>();
             hipLaunchKernelGGL(k_dd_cone_rowsum, dim3((unsigned)cdiv(ncols, 4)), dim3(256), 0, st, g, prj, v,
@@ -1510,7 +1652,8 @@ void ConePlan::dd_adj(int nB, int nC, const float* prj, float* img, DevBuf& work
         }
         check_launch("dd_cone_adj");
     };
-    const int c = tune_choose({TK_DD_CONE_ADJ, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC}, 6, launch, st, true);
+    const int c = tune_choose({TK_DD_CONE_ADJ, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC}, 6 - first, launch, st,
+                              true);
     launch(c);
 }
 

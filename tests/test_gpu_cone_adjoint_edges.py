@@ -1,0 +1,43 @@
+"""The list-driven cone DD adjoint against the FP64 oracle where its paths
+change: up to 2, 3 and more rows per voxel, detector columns much finer than a
+voxel (several list rounds), volumes taller than a workgroup's z block, fewer
+views than a batch, detector rows that run against z, and a source close enough
+that the row-sum tables take over (bar 1e-5 relative L2, the suite's parity bar)."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as orc
+from reconnet_amd.geometry import circular_cone_vectors
+from tests.helpers import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # nx, ny, nz, dz, nu, nv, du, dv, nview, dso, flip
+    (9, 14, 20, 1.0, 20, 12, 2.0, 1.0, 5, 300.0, False),        # < 2 rows per voxel
+    (17, 6, 11, 1.0, 30, 20, 1.3, 0.7, 33, 120.0, False),       # 2 to 3
+    (8, 8, 10, 2.0, 24, 40, 1.3, 0.8, 17, 120.0, True),         # 3 to 7, rows against z
+    (6, 7, 150, 0.5, 90, 30, 0.2, 1.0, 9, 120.0, False),        # fine columns, two z blocks
+    (8, 8, 6, 4.0, 20, 60, 1.3, 0.5, 8, 90.0, False),           # more than 7: row sums
+]
+
+
+@pytest.mark.parametrize("nx,ny,nz,dz,nu,nv,du,dv,nview,dso,flip", CASES)
+def test_cone_adjoint_paths(nx, ny, nz, dz, nu, nv, du, dv, nview, dso, flip):
+    from reconnet_amd._lib import autotune_pin
+    from reconnet_amd.torch_ops import ConePlan
+
+    ctr, u, v, src = circular_cone_vectors(nview, dso, 200.0 + dso, th0=0.3)
+    if flip:
+        v = -v
+    plan = ConePlan(nx, ny, nz, 1.0, 1.0, dz, nu, nv, du, dv, ctr, u, v, src, cx=0.3, cy=-0.2, cz=0.4, off_v=0.2)
+    geo = dict(dx=1.0, dy=1.0, dz=dz, du=du, dv=dv, off_u=0.0, off_v=0.2, cx=0.3, cy=-0.2, cz=0.4)
+    p = np.random.default_rng(nu + nv).uniform(0, 1, (1, nu, nview, nv, 1)).astype(np.float32)
+    ref = orc.dd_cone_adj(p, ctr, u, v, src, geo, (nx, ny, nz))
+    try:
+        for c in range(3):
+            autotune_pin("dd_cone_adj", c)
+            assert rel_l2(plan.backward(torch.from_numpy(p).cuda(), "dd").cpu().numpy(), ref) <= 1e-5, c
+    finally:
+        autotune_pin("dd_cone_adj", None)
