@@ -526,6 +526,307 @@ __global__ __launch_bounds__(256) void k_siddon_arb_bp(ArbGeo a, Grid3K g, int p
         if (iz + k < g.nz) out[(long)k * nC] = acc[k];
 }
 
+// Row windows of the cone backprojections: len(row) q(row) of every (slice, view,
+// detector column), len the length from the source to the cell centre, as floats
+// with kConePad zero rows before and 4 after (pitch nv + kConePad + 4).
+constexpr int kConePad = 8;
+
+__global__ __launch_bounds__(256) void k_cone_rows(ArbGeo a, const float* __restrict__ prj, const float* Cp,
+                                                      const float* Up, const float* Vp, const float* Sp, int nC,
+                                                      long n, float* __restrict__ Q)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int nvp = a.nv + kConePad + 4;
+    const long col = i / nvp;
+    const int iv = (int)(i - col * nvp) - kConePad;
+    float f = 0.0f;
+    if (iv >= 0 && iv < a.nv) {
+        const int iu = (int)(col % a.nu);
+        const long rest = col / a.nu;
+        const int view = (int)(rest % a.nview);
+        const long bc = rest / a.nview;
+        const int cc = (int)(bc % nC), b = (int)(bc / nC);
+        const F3 c = ld3(Cp, view), U = ld3(Up, view), V = ld3(Vp, view), s = ld3(Sp, view);
+        const float uc = ((float)iu - ((a.nu - 1) / 2.0f + a.off_u)) * a.du;
+        const float lx = fmaf(uc, U.x, c.x) - s.x, ly = fmaf(uc, U.y, c.y) - s.y;
+        const float lzs = V.z * a.dv, lz_0 = fmaf(-((a.nv - 1) / 2.0f + a.off_v), lzs, fmaf(uc, U.z, c.z) - s.z);
+        const float lz = fmaf(lzs, (float)iv, lz_0);
+        f = sqrtf(fmaf(lz, lz, fmaf(lx, lx, ly * ly))) *
+            prj[((((long)b * a.nu + iu) * a.nview + view) * a.nv + iv) * nC + cc];
+    }
+    Q[i] = f;
+}
+
+// NR adjacent rows of a window at byte offset off (rows -kConePad .. nv + 3)
+template <int NR>
+__device__ __forceinline__ void cone_rows(const char* __restrict__ Q, unsigned off, float (&v)[NR])
+{
+    typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float F2 __attribute__((ext_vector_type(2), aligned(4)));
+    if constexpr (NR == 4) {
+        const F4 x = *reinterpret_cast<const F4*>(Q + off);
+        v[0] = x[0]; v[1] = x[1]; v[2] = x[2]; v[3] = x[3];
+    } else {
+        static_assert(NR == 2 || NR == 3, "2, 3 or 4 rows");
+        const F2 x = *reinterpret_cast<const F2*>(Q + off);
+        v[0] = x[0]; v[1] = x[1];
+        if constexpr (NR == 3) v[2] = *reinterpret_cast<const float*>(Q + off + 8u);
+    }
+}
+
+// maximum over the wave's 64 lanes of a non-negative value
+__device__ __forceinline__ int wave_max_nn(int v)
+{
+    #pragma unroll
+    for (int d = 1; d < 64; d <<= 1) v = max(v, __shfl_xor(v, d));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Siddon backprojection of upright cone views from column lists: the transpose of
+// the walk as in siddon_rows_z_view, organised as k_dd_cone_adj_list.  A group of
+// LZ lanes takes one (x, y); per batch of LZ views each lane works out one view's
+// detector columns through (x, y) (FP64 ray set-up, the in-plane slab interval
+// [xy0, xy1] around the closest approach tp, the rows' affine coordinates) and
+// appends them to the group's list; then the group's lanes take LZ consecutive
+// voxels of the z range the batch reaches and walk the list.  A voxel's rows on
+// an entry are those whose ray meets it between the in-plane crossings: the row
+// coordinate (z - Sz) / (t dzs) - dz0 / dzs of its two z faces at t = tp + xy0
+// and tp + xy1.  Their chords, in t, are the overlap of the z slab's interval
+// with [xy0, xy1], measured from tp like the in-plane interval; the ray's length
+// is already in the row windows.  A chord beyond the detector point counts only
+// if the ray entered the grid before that point (g0 of the entry, in plane, and
+// the row's z entry).
+//
+// Bound: VALU issue (about 25 instructions per entry and 19 per row, 2 rows per
+// entry where a voxel covers less than 2).  190 x 177 x 99 voxels, 240 views, 49
+// x 323: 0.99 ms with 32 lanes per (x, y) (1.06 with 16, 1.28 with 8), and 22 us
+// for the row windows; 7.4 ms with 64 lanes along z testing every view, column
+// and row for 2 stacked voxels each (siddon_rows_z_view).
+constexpr int kSidCols = 2;          // list entries per view and round
+constexpr int kSidZB = 128;          // z voxels of a workgroup's columns
+
+struct SidEntry {
+    float xy0, xy1, tp, Sz;          // in-plane interval around tp; source height
+    float ia, ib, c;                 // rows: (z - Sz) ia - c at tp + xy0, ib at tp + xy1
+    unsigned off;                    // byte offset of the column's row 0
+    float dzc, dzs, g0, pad;         // row iv's ray rises dzc + (iv - cv) dzs (0 exactly on a
+                                     // centred detector's middle row); grid entry in plane
+};
+
+// Sum over the list's n entries for the voxel whose centre is zh + zl, half height h.
+// NR = 2, 3, 4: every entry's voxel meets at most NR rows; NR = 0: `chunks` x 4 rows.
+template <int NR, bool FAR>
+__device__ __forceinline__ float sid_list_sum(const float4* list, int n, const char* __restrict__ Q, float zh, float zl,
+                                              float h, float cv, float fnv, float glz, float ghz, int chunks)
+{
+    float sum = 0.0f;
+    #pragma unroll 2
+    for (int i = 0; i < n; ++i) {
+        const float4 A = list[3 * i], B = list[3 * i + 1], C = list[3 * i + 2];
+        // voxel centre above the source, as a float pair
+        const float w = zh - A.w, bb = w - zh;
+        const float wl = ((zh - (w - bb)) - (A.w + bb)) + zl;
+        const float ub = w - h, ut = w + h;
+        const float rmin = fminf(fminf(ub * B.x, ub * B.y), fminf(ut * B.x, ut * B.y)) - B.z;
+        const float r0 = ceilf(rmin - 1e-3f);
+        auto rows = [&](float rf, const float* v, int count) {
+            #pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (j >= count) break;
+                float dz = fmaf(C.y, (rf - cv) + (float)j, C.x), rz = fmaf(-A.z, dz, w) + wl;
+                // a level ray lies in the voxel with -h < rz <= h
+                const bool level = fabsf(dz) < 1e-30f;
+                dz = level ? 1e-30f : dz;
+                rz = level ? fmaf(-1e-6f, h, rz) : rz;
+                const float inv = __builtin_amdgcn_rcpf(dz);
+                const float m = rz * inv, k = h * inv;
+                const float q0 = __builtin_amdgcn_fmed3f(m - k, A.x, A.y), q1 = __builtin_amdgcn_fmed3f(m + k, A.x, A.y);
+                float ch = fabsf(q1 - q0);
+                if (FAR) {
+                    const float gz = fminf((glz - A.w) * inv, (ghz - A.w) * inv);
+                    if (fminf(q0, q1) >= 1.0f - A.z && !(fmaxf(C.z, gz) < 1.0f)) ch = 0.0f;
+                }
+                // a row that misses the voxel adds nothing, whatever its value
+                sum = ch > 0.0f ? fmaf(ch, v[j], sum) : sum;
+            }
+        };
+        const float lo = -(float)kConePad;
+        if constexpr (NR > 0) {
+            const float rf = __builtin_amdgcn_fmed3f(r0, lo, fnv);
+            float v[NR];
+            cone_rows<NR>(Q, __float_as_uint(B.w) + (unsigned)((int)rf * 4), v);
+            rows(rf, v, NR);
+        } else {
+            for (int c = 0; c < chunks; ++c) {
+                const float rf = __builtin_amdgcn_fmed3f(r0 + 4.0f * (float)c, lo, fnv);
+                float v[4];
+                cone_rows<4>(Q, __float_as_uint(B.w) + (unsigned)((int)rf * 4), v);
+                rows(rf, v, 4);
+            }
+        }
+    }
+    return sum;
+}
+
+template <int LZ>
+__global__ __launch_bounds__(256, 4) void k_siddon_cone_bp_list(ArbGeo a, Grid3K g, const float* __restrict__ Q,
+                                                                float* __restrict__ img, const float* Cp,
+                                                                const float* Up, const float* Vp, const float* Sp,
+                                                                const float4* __restrict__ vt, int nC)
+{
+    constexpr int NG = 64 / LZ, kCap = LZ * kSidCols;
+    static_assert(sizeof(SidEntry) == 48, "three float4 per entry");
+    __shared__ float4 lists[4][NG * kCap * 3];
+    __shared__ float accs[4][NG * kSidZB];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int grp = lane / LZ, lg = lane % LZ;
+    const int iy0 = ((int)blockIdx.y * 4 + wv) * NG;
+    if (iy0 >= g.ny) return;                       // whole waves (no workgroup barrier below)
+    const int iy = iy0 + grp, ix = blockIdx.z % g.nx, bc = blockIdx.z / g.nx;
+    const int z0 = (int)blockIdx.x * kSidZB, z1 = min(z0 + kSidZB, g.nz);
+    float4* list = lists[wv] + grp * kCap * 3;
+    float* acc = accs[wv] + grp * kSidZB;
+    for (int z = lg; z < kSidZB; z += LZ) acc[z] = 0.0f;
+    const int nvp = a.nv + kConePad + 4;
+    const char* Qb = reinterpret_cast<const char*>(Q + (long)bc * a.nview * a.nu * nvp);
+    const float vlx = g.cx + (ix - g.nx / 2.0f) * g.dx, vly = g.cy + (iy - g.ny / 2.0f) * g.dy;
+    const double vcx = g.cx + (ix + 0.5 - g.nx / 2.0) * g.dx, vcy = g.cy + (iy + 0.5 - g.ny / 2.0) * g.dy;
+    const float hx = 0.5f * g.dx, hy = 0.5f * g.dy, hz = 0.5f * g.dz;
+    const float glx = g.cx - g.nx / 2.0f * g.dx, ghx = g.cx + g.nx / 2.0f * g.dx;
+    const float gly = g.cy - g.ny / 2.0f * g.dy, ghy = g.cy + g.ny / 2.0f * g.dy;
+    const float glz = g.cz - g.nz / 2.0f * g.dz, ghz = g.cz + g.nz / 2.0f * g.dz;
+    const float cu = (a.nu - 1) / 2.0f + a.off_u, cv = (a.nv - 1) / 2.0f + a.off_v;
+    const float fz0 = (float)z0, fz1 = (float)z1, fnv = (float)a.nv, idz = 1.0f / g.dz;
+    const unsigned long long gmask = LZ == 64 ? ~0ull : ((1ull << (LZ & 63)) - 1ull);
+    for (int vb = 0; vb < a.nview; vb += LZ) {
+        const int view = min(vb + lg, a.nview - 1);
+        const F3 Cv = ld3(Cp, view), Uv = ld3(Up, view), Vv = ld3(Vp, view), Sv = ld3(Sp, view);
+        const float4 t0v = vt[4 * view], t1v = vt[4 * view + 1];
+        // columns whose centre ray can meet the voxel column: its corners on the detector
+        float umin = INFINITY, umax = -INFINITY;
+        bool ok = vb + lg < a.nview && iy < g.ny;
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float wxk = vlx + ((k & 1) ? g.dx : 0.0f) - Sv.x, wyk = vly + ((k & 2) ? g.dy : 0.0f) - Sv.y;
+            const float den = fmaf(wxk, t0v.x, wyk * t0v.y);
+            ok = ok && (den * t0v.w > 0.f);
+            const float u = fmaf(t0v.w * __builtin_amdgcn_rcpf(den), fmaf(wxk, t1v.x, wyk * t1v.y), t1v.w);
+            umin = fminf(umin, u); umax = fmaxf(umax, u);
+        }
+        int u0 = 0, ncol = 0;
+        if (ok) {
+            const float fu0 = umin / a.du + cu, fu1 = umax / a.du + cu;
+            u0 = max((int)ceilf(fminf(fu0, fu1) - 1e-3f), 0);
+            ncol = max(min((int)floorf(fmaxf(fu0, fu1) + 1e-3f), a.nu - 1) - u0 + 1, 0);
+        }
+        const int maxcol = wave_max_nn(ncol);
+        const float dzs = Vv.z * a.dv, dzc = (float)((double)Cv.z - Sv.z), dz0 = fmaf(-cv, dzs, dzc);
+        const float idzs = 1.0f / dzs;
+        for (int cb = 0; cb < maxcol; cb += kSidCols) {
+            int cnt = 0;
+            float zl = 3.0e38f, zh = -3.0e38f, wmax = 0.0f;
+            bool far = false;
+            #pragma unroll
+            for (int c = 0; c < kSidCols; ++c) {
+                bool on = cb + c < ncol;
+                SidEntry e{};
+                if (on) {
+                    const int iu = u0 + cb + c;
+                    const double uc = (double)(iu - cu) * a.du;
+                    const double wx = vcx - Sv.x, wy = vcy - Sv.y;
+                    const double dxd = fma((double)Uv.x, uc, (double)Cv.x) - Sv.x;
+                    const double dyd = fma((double)Uv.y, uc, (double)Cv.y) - Sv.y;
+                    const float dx = (float)dxd, dy = (float)dyd;
+                    // tp: the column's in-plane closest approach to the voxel
+                    const float tp = (float)(wx * dxd + wy * dyd) * __builtin_amdgcn_rcpf(fmaf(dx, dx, dy * dy));
+                    const float rx = (float)fma(-(double)tp, dxd, wx), ry = (float)fma(-(double)tp, dyd, wy);
+                    float xy0 = -tp, xy1 = INFINITY, g0 = -INFINITY;      // from the source on
+                    if (dx != 0.f) {
+                        const float inv = __builtin_amdgcn_rcpf(dx);
+                        const float a0 = (rx - hx) * inv, a1 = (rx + hx) * inv;
+                        xy0 = fmaxf(xy0, fminf(a0, a1)); xy1 = fminf(xy1, fmaxf(a0, a1));
+                        g0 = fmaxf(g0, fminf((glx - Sv.x) * inv, (ghx - Sv.x) * inv));
+                    } else if (!(rx > -hx && rx <= hx)) {
+                        xy1 = -INFINITY;
+                    }
+                    if (dy != 0.f) {
+                        const float inv = __builtin_amdgcn_rcpf(dy);
+                        const float a0 = (ry - hy) * inv, a1 = (ry + hy) * inv;
+                        xy0 = fmaxf(xy0, fminf(a0, a1)); xy1 = fminf(xy1, fmaxf(a0, a1));
+                        g0 = fmaxf(g0, fminf((gly - Sv.y) * inv, (ghy - Sv.y) * inv));
+                    } else if (!(ry > -hy && ry <= hy)) {
+                        xy1 = -INFINITY;
+                    }
+                    const float ta = tp + xy0, tb = tp + xy1;
+                    on = xy1 > xy0 && ta > 0.0f;       // (ta > 0: the source lies off the grid, checked on the host)
+                    if (on) {
+                        e.xy0 = xy0; e.xy1 = xy1; e.tp = tp; e.Sz = Sv.z;
+                        e.ia = idzs / ta; e.ib = idzs / tb; e.c = dz0 * idzs;
+                        e.off = (unsigned)(((long)view * a.nu + iu) * nvp + kConePad) * 4u;
+                        e.dzc = dzc; e.dzs = dzs; e.g0 = g0;
+                        far = far || xy1 > 1.0f - tp;
+                        // the voxels the rows' rays reach and the rows of one voxel
+                        const float d1 = fmaf(dzs, fnv - 1.0f, dz0);
+                        const float p = fminf(fminf(ta * dz0, tb * dz0), fminf(ta * d1, tb * d1));
+                        const float q = fmaxf(fmaxf(ta * dz0, tb * dz0), fmaxf(ta * d1, tb * d1));
+                        zl = fminf(zl, fmaf(Sv.z - g.cz + p, idz, 0.5f * g.nz));
+                        zh = fmaxf(zh, fmaf(Sv.z - g.cz + q, idz, 0.5f * g.nz));
+                        const float ds = fabsf(g.dz * e.ia);
+                        wmax = fmaxf(wmax, fmaf(fmaf(fmaxf(fabsf(dz0), fabsf(d1)), fabsf(idzs), ds + 1.0f),
+                                                (tb - ta) / ta, ds));
+                    }
+                }
+                const unsigned long long gm = (__ballot(on) >> (grp * LZ)) & gmask;
+                if (on) {
+                    float4* d = list + 3 * (cnt + __popcll(gm & ((1ull << lg) - 1ull)));
+                    d[0] = make_float4(e.xy0, e.xy1, e.tp, e.Sz);
+                    d[1] = make_float4(e.ia, e.ib, e.c, __uint_as_float(e.off));
+                    d[2] = make_float4(e.dzc, e.dzs, e.g0, 0.0f);
+                }
+                cnt += __popcll(gm);
+            }
+            const int n = wave_max_nn(cnt);
+            // entries past the group's count: an empty interval on row 0 of the first column
+            for (int i = cnt + lg; i < n; i += LZ) {
+                list[3 * i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                list[3 * i + 1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                list[3 * i + 2] = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+            }
+            #pragma unroll
+            for (int d = 1; d < LZ; d <<= 1) {
+                zl = fminf(zl, __shfl_xor(zl, d));
+                zh = fmaxf(zh, __shfl_xor(zh, d));
+            }
+            #pragma unroll
+            for (int d = 1; d < 64; d <<= 1) wmax = fmaxf(wmax, __shfl_xor(wmax, d));
+            wmax = wave_uniform(wmax) + 4e-3f;         // rows' rounding and the margin of the first row
+            const bool anyfar = __any(far);
+            const int zs = (int)__builtin_amdgcn_fmed3f(zl - 1.0f, fz0, fz1);
+            const int ze = (int)__builtin_amdgcn_fmed3f(zh + 2.0f, fz0, fz1);
+            const int passes = wave_max_nn(max((ze - zs + LZ - 1) / LZ, 0));
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            for (int m = 0; m < passes; ++m) {
+                const int z = zs + m * LZ + lg;
+                const double zc = g.cz + (z + 0.5 - g.nz / 2.0) * g.dz;
+                const float ch = (float)zc, cl = (float)(zc - ch);
+                float v;
+                if (anyfar) v = sid_list_sum<0, true>(list, n, Qb, ch, cl, hz, cv, fnv, glz, ghz, ((int)wmax + 4) / 4);
+                else if (wmax < 2.0f) v = sid_list_sum<2, false>(list, n, Qb, ch, cl, hz, cv, fnv, glz, ghz, 0);
+                else if (wmax < 3.0f) v = sid_list_sum<3, false>(list, n, Qb, ch, cl, hz, cv, fnv, glz, ghz, 0);
+                else if (wmax < 4.0f) v = sid_list_sum<4, false>(list, n, Qb, ch, cl, hz, cv, fnv, glz, ghz, 0);
+                else v = sid_list_sum<0, false>(list, n, Qb, ch, cl, hz, cv, fnv, glz, ghz, ((int)wmax + 4) / 4);
+                if (z < ze) acc[z - z0] += v;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+    }
+    if (iy >= g.ny) return;
+    const int cc = bc % nC, b = bc / nC;
+    float* out = img + ((((long)b * g.nx + ix) * g.ny + iy) * g.nz) * nC + cc;
+    for (int z = z0 + lg; z < z1; z += LZ) out[(long)z * nC] = acc[z - z0];
+}
+
 // ---- DD tomosynthesis ----
 
 // average over [x1,x2] x [y1,y2] of a [ny][nx] plane (zero outside)
@@ -879,34 +1180,6 @@ __global__ __launch_bounds__(256) void k_dd_cone_rowsum(ArbGeo a, const float* _
     }
 }
 
-// Row windows of the list-driven adjoint: len(row) q(row) of every (slice, view,
-// detector column) as floats with `pad` zero rows before and 4 after, pitch nvp.
-__global__ __launch_bounds__(256) void k_dd_cone_rows(ArbGeo a, const float* __restrict__ prj, const float* Cp,
-                                                      const float* Up, const float* Vp, const float* Sp, int nC,
-                                                      long n, int nvp, int pad, float* __restrict__ Q)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const long col = i / nvp;
-    const int iv = (int)(i - col * nvp) - pad;
-    float f = 0.0f;
-    if (iv >= 0 && iv < a.nv) {
-        const int iu = (int)(col % a.nu);
-        const long rest = col / a.nu;
-        const int view = (int)(rest % a.nview);
-        const long bc = rest / a.nview;
-        const int cc = (int)(bc % nC), b = (int)(bc / nC);
-        const F3 c = ld3(Cp, view), U = ld3(Up, view), V = ld3(Vp, view), s = ld3(Sp, view);
-        const float uc = ((float)iu - ((a.nu - 1) / 2.0f + a.off_u)) * a.du;
-        const float lx = fmaf(uc, U.x, c.x) - s.x, ly = fmaf(uc, U.y, c.y) - s.y;
-        const float lzs = V.z * a.dv, lz_0 = fmaf(-((a.nv - 1) / 2.0f + a.off_v), lzs, fmaf(uc, U.z, c.z) - s.z);
-        const float lz = fmaf(lzs, (float)iv, lz_0);
-        f = sqrtf(fmaf(lz, lz, fmaf(lx, lx, ly * ly))) *
-            prj[((((long)b * a.nu + iu) * a.nview + view) * a.nv + iv) * nC + cc];
-    }
-    Q[i] = f;
-}
-
 // Exact transpose of k_dd_cone_fp: a voxel gathers, per view, the cells whose
 // footprint on its plane overlaps it, with the forward pass's weight
 // overlap / area * L.  The in-plane part (which detector columns meet the
@@ -933,23 +1206,6 @@ __global__ __launch_bounds__(256) void k_dd_cone_rows(ArbGeo a, const float* __r
 constexpr int kConeZB = 256;        // z voxels of a workgroup's columns
 constexpr int kConeCols = 4;        // list entries per view and round
 constexpr float kConeMaxDs = 7.0f;  // rows per voxel beyond which the row-sum tables are used
-
-// rows r0 .. r0 + NR - 1 of the window at byte offset off (r0 >= -pad, r0 + NR <= nv + 4)
-template <int NR>
-__device__ __forceinline__ void cone_rows(const char* __restrict__ Q, unsigned off, float (&v)[NR])
-{
-    typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
-    typedef float F2 __attribute__((ext_vector_type(2), aligned(4)));
-    if constexpr (NR == 4) {
-        const F4 x = *reinterpret_cast<const F4*>(Q + off);
-        v[0] = x[0]; v[1] = x[1]; v[2] = x[2]; v[3] = x[3];
-    } else {
-        static_assert(NR == 3, "3 or 4 rows");
-        const F2 x = *reinterpret_cast<const F2*>(Q + off);
-        v[0] = x[0]; v[1] = x[1];
-        v[2] = *reinterpret_cast<const float*>(Q + off + 8u);
-    }
-}
 
 // Sum over the list's n entries (a multiple of 4) for the voxel at z index fz.
 // NR = 3 or 4: every entry's |ibdv| <= NR - 1; NR = 0: any, in chunks of 4 rows.
@@ -993,17 +1249,9 @@ __device__ __forceinline__ float cone_list_sum(const float4* list, int n, const 
     return sum;
 }
 
-// maximum over the wave's 64 lanes of a non-negative value
-__device__ __forceinline__ int wave_max_nn(int v)
-{
-    #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) v = max(v, __shfl_xor(v, d));
-    return __builtin_amdgcn_readfirstlane(v);
-}
-
 template <int LZ>
-__global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g, const float* __restrict__ Q, int nvp,
-                                                             int pad, float* __restrict__ img,
+__global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g, const float* __restrict__ Q,
+                                                             float* __restrict__ img,
                                                              const ConeView* __restrict__ views,
                                                              const ConeColumn* __restrict__ cols, int nC)
 {
@@ -1019,10 +1267,11 @@ __global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g,
     float4* list = lists[wv] + grp * (LZ * kConeCols);
     float* acc = accs[wv] + grp * kConeZB;
     for (int z = lg; z < kConeZB; z += LZ) acc[z] = 0.0f;
+    const int nvp = a.nv + kConePad + 4;
     const char* Qb = reinterpret_cast<const char*>(Q + (long)bc * a.nview * a.nu * nvp);
     const float cu = (a.nu - 1) / 2.0f + a.off_u, idu = 1.0f / a.du;
     const float margin = 0.05f;
-    const float fnv = (float)a.nv, lo = -(float)pad, fz0 = (float)z0, fz1 = (float)z1;
+    const float fnv = (float)a.nv, lo = -(float)kConePad, fz0 = (float)z0, fz1 = (float)z1;
     const unsigned long long gmask = LZ == 64 ? ~0ull : ((1ull << (LZ & 63)) - 1ull);
     for (int vb = 0; vb < a.nview; vb += LZ) {
         const int view = min(vb + lg, a.nview - 1);
@@ -1068,7 +1317,7 @@ __global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g,
                     e.x = oe * __builtin_amdgcn_rcpf(e2 - e1) * fabsf(col.W);
                     e.y = fminf(ibdv, 0.0f) - zA * ibdv;
                     e.z = ibdv;
-                    e.w = __uint_as_float((unsigned)(ci * nvp + pad) * 4u);
+                    e.w = __uint_as_float((unsigned)(ci * nvp + kConePad) * 4u);
                     const float zB = fmaf(fnv, __builtin_amdgcn_rcpf(ibdv), zA);
                     if (on) {
                         zl = fminf(zl, fminf(zA, zB));
@@ -1412,6 +1661,33 @@ bool arb_rows_along_z(const float* detU, const float* detV, int nview)
     return true;
 }
 
+float arb_rows_per_voxel(const ArbGeo& g, const float* C, const float* U, const float* V, const float* S)
+{
+    if (!C || !S || !arb_rows_along_z(U, V, g.nview)) return 0.0f;
+    double most = 0.0;
+    for (int v = 0; v < g.nview; v++) {
+        const double dzs = std::fabs((double)V[3 * v + 2] * g.dv);
+        // t of the grid's in-plane corners on the view's rays (1 on the detector): affine in (x, y)
+        const double nx = U[3 * v + 1], ny = -(double)U[3 * v];
+        const double A = (C[3 * v] - (double)S[3 * v]) * nx + (C[3 * v + 1] - (double)S[3 * v + 1]) * ny;
+        double t = HUGE_VAL;
+        for (int k = 0; k < 4; k++) {
+            const double x = g.cx + ((k & 1) ? 0.5 : -0.5) * g.nx * g.dx, y = g.cy + ((k & 2) ? 0.5 : -0.5) * g.ny * g.dy;
+            t = std::min(t, ((x - S[3 * v]) * nx + (y - S[3 * v + 1]) * ny) / A);
+        }
+        // the nearest voxel's rows: its height at t, plus what its in-plane
+        // extent shifts the steepest row
+        const double run = std::fabs(A) / std::sqrt(nx * nx + ny * ny);      // source to detector line
+        const double dt = std::hypot((double)g.dx, (double)g.dy) / run;
+        const double cz = std::fabs((double)C[3 * v + 2] - S[3 * v + 2]);
+        const double steep = cz / dzs + 0.5 * g.nv + std::fabs((double)g.off_v) + 1.0;
+        const double w = g.dz / (t * dzs) + steep * dt / t;
+        if (!(t > 0.02) || !(w <= 1e6)) return 0.0f;
+        most = std::max(most, w);
+    }
+    return (float)most;
+}
+
 void siddon_arb_fp(const ArbGeo& g, bool parallel, int nB, int nC, const float* img, float* prj,
                    const float* detCenter, const float* detU, const float* detV, const float* srcOrDir,
                    DevBuf& work, hipStream_t st)
@@ -1445,13 +1721,47 @@ void siddon_arb_bp(const ArbGeo& g, bool parallel, int nB, int nC, const float* 
         check_launch("siddon_arb_bp");
         return;
     }
-    // upright cone views: 1, 2 or 4 voxels per lane (the launch-shape tuner)
+    // upright cone views: column lists with one (x, y) per 16, 8 or 32 lanes where
+    // a voxel meets few rows (and the windows of one slice fit 4 GiB), else 1, 2
+    // or 4 voxels per lane testing every view
+    const int nvp = g.nv + kConePad + 4;
+    const long n = (long)nB * nC * g.nu * g.nview * nvp;
+    const bool lists = g.rows_per_voxel > 0 && g.rows_per_voxel <= kConeMaxDs &&
+                       (long)g.nu * g.nview * nvp * 4L < (1L << 32) && (n + 255) / 256 < 0x7fffffffL;
+    if (lists) {
+        const size_t vt_bytes = (size_t)g.nview * 4 * sizeof(float4);
+        if (work.size() < vt_bytes + (size_t)n * sizeof(float)) {
+            // (the view table above was written to the buffer that is replaced)
+            work.ensure(vt_bytes + (size_t)n * sizeof(float));
+            vt = work.as<float4>();
+            hipLaunchKernelGGL(k_siddon_arb_views, dim3(cdiv(g.nview, 256)), dim3(256), 0, st, g, grid_of(g), 0,
+                               detCenter, detU, detV, srcOrDir, vt);
+            check_launch("siddon_arb_views");
+        }
+        float* Q = reinterpret_cast<float*>(static_cast<char*>(work.get()) + vt_bytes);
+        hipLaunchKernelGGL(k_cone_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, prj, detCenter, detU,
+                           detV, srcOrDir, nC, n, Q);
+        check_launch("cone_rows");
+    }
     auto launch = [&](int c) {
-        const int zpl = 1 << c;
-        dim3 grd(cdiv(g.nz, 64 * zpl), cdiv(g.ny, 4), g.nx * nB * nC);
-        auto k = c == 0 ? k_siddon_arb_bp<true, 1> : c == 1 ? k_siddon_arb_bp<true, 2> : k_siddon_arb_bp<true, 4>;
-        hipLaunchKernelGGL(k, grd, dim3(256), 0, st, g, grid_of(g), 0, prj, img, detCenter, detU, detV, srcOrDir, vt, nC);
-        check_launch("siddon_arb_bp");
+        if (lists) {
+            const float* Q = reinterpret_cast<const float*>(vt + (size_t)g.nview * 4);
+            auto go = [&](auto kern, int lz) {
+                const dim3 grd(cdiv(g.nz, kSidZB), cdiv(g.ny, 4 * (64 / lz)), g.nx * nB * nC);
+                hipLaunchKernelGGL(kern, grd, dim3(256), 0, st, g, grid_of(g), Q, img, detCenter, detU, detV, srcOrDir,
+                                   vt, nC);
+            };
+            if (c == 0) go(k_siddon_cone_bp_list<16>, 16);
+            else if (c == 1) go(k_siddon_cone_bp_list<8>, 8);
+            else go(k_siddon_cone_bp_list<32>, 32);
+        } else {
+            const int zpl = 1 << c;
+            dim3 grd(cdiv(g.nz, 64 * zpl), cdiv(g.ny, 4), g.nx * nB * nC);
+            auto k = c == 0 ? k_siddon_arb_bp<true, 1> : c == 1 ? k_siddon_arb_bp<true, 2> : k_siddon_arb_bp<true, 4>;
+            hipLaunchKernelGGL(k, grd, dim3(256), 0, st, g, grid_of(g), 0, prj, img, detCenter, detU, detV, srcOrDir,
+                               vt, nC);
+        }
+        check_launch("siddon_cone_bp");
     };
     const int c = tune_choose({TK_SIDDON_CONE_BP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC}, 3, launch, st, true);
     launch(c);
@@ -1547,7 +1857,6 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
         w.o = (float)((Sn - gn) / dn + 0.5 * nn);
         w.a0 = (float)((Sz - g.cz) / g.dz + 0.5 * g.nz);
         w.pad = 0.f;
-        float t3 = 0.f;
         for (int iu = 0; iu < g.nu; iu++) {
             ConeColumn& k = ct[(size_t)v * g.nu + iu];
             k = ConeColumn{0.f, 0.f, 0.f, 0.f, 0.f, {0.f, 0.f, 0.f}};
@@ -1561,11 +1870,13 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
             k.k1 = (float)(e1n / e1m / dn);
             k.A1 = (float)(zr0 / dpc / g.dz);
             k.T3 = (float)(dpc * g.dz / (Vz * g.dv));
-            t3 = std::max(t3, std::fabs(k.T3));
             k.W = (float)(dm / std::fabs(dpc) * (Vz / dpc > 0 ? 1.0 : -1.0));
         }
-        // rows per voxel on the plane nearest to the source (unbounded if it lies between the planes)
+        // rows per voxel on the plane nearest to the source (unbounded if it lies
+        // between the planes); the main-axis run to the detector is affine in the column
         const double m0 = w.mp0, m1 = w.mp0 + (nm - 1) * dm;
+        const double t3 = std::max(std::fabs(-cu * g.du * Um + Cm - Sm), std::fabs((g.nu - 1 - cu) * g.du * Um + Cm - Sm)) *
+                          g.dz / std::fabs(Vz * g.dv);
         ds_max_ = std::max(ds_max_, m0 * m1 > 0 ? t3 / std::min(std::fabs(m0), std::fabs(m1)) : HUGE_VAL);
     }
     views_.alloc(vt.size() * sizeof(ConeView));
@@ -1575,6 +1886,7 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
     RN_HIP_CHECK(hipStreamSynchronize(st));
     geo = g;
     geo.rows_z = arb_rows_along_z(U, V, n) ? 1 : 0;
+    geo.rows_per_voxel = arb_rows_per_voxel(g, C, U, V, S);
 }
 
 void ConePlan::dd_fp(int nB, int nC, const float* img, float* prj, hipStream_t st) const
@@ -1617,7 +1929,7 @@ void ConePlan::dd_adj(int nB, int nC, const float* prj, float* img, DevBuf& work
     // over row windows (up to kConeMaxDs rows per voxel: beyond, a voxel's rows
     // are better taken from two row sums; the windows of one slice in 4 GiB);
     // 3-5: 1, 2 or 4 voxels per lane from the row-sum table
-    const int pad = 8, nvp = pad + g.nv + 4;
+    const int nvp = g.nv + kConePad + 4;
     const bool windows = ds_max_ <= kConeMaxDs && (long)g.nu * g.nview * nvp * 4L < (1L << 32);
     const int first = windows ? 0 : 3;
     auto launch = [&](int i) {
@@ -1627,12 +1939,12 @@ void ConePlan::dd_adj(int nB, int nC, const float* prj, float* img, DevBuf& work
             float* Q = work.as<float>();
             const long n = ncols * nvp;
             RN_REQUIRE((n + 255) / 256 < 0x7fffffffL, "dd_cone_adj: too many detector rows");
-            hipLaunchKernelGGL(k_dd_cone_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, prj, v,
-                               v + 3 * g.nview, v + 6 * g.nview, v + 9 * g.nview, nC, n, nvp, pad, Q);
-            check_launch("dd_cone_rows");
+            hipLaunchKernelGGL(k_cone_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, prj, v,
+                               v + 3 * g.nview, v + 6 * g.nview, v + 9 * g.nview, nC, n, Q);
+            check_launch("cone_rows");
             auto go = [&](auto kern, int lz) {
                 const dim3 grd(cdiv(g.nz, kConeZB), cdiv(g.ny, 4 * (64 / lz)), g.nx * nB * nC);
-                hipLaunchKernelGGL(kern, grd, dim3(256), 0, st, g, grid_of(g), Q, nvp, pad, img,
+                hipLaunchKernelGGL(kern, grd, dim3(256), 0, st, g, grid_of(g), Q, img,
                                    views_.as<ConeView>(), cols_.as<ConeColumn>(), nC);
             };
             if (c == 0) go(k_dd_cone_adj_list<16>, 16);

@@ -1,4 +1,4 @@
-"""The list-driven cone DD adjoint against the FP64 oracle where its paths
+"""The list-driven cone backprojections against the FP64 oracle where their paths
 change: up to 2, 3 and more rows per voxel, detector columns much finer than a
 voxel (several list rounds), volumes taller than a workgroup's z block, fewer
 views than a batch, detector rows that run against z, and a source close enough
@@ -41,3 +41,50 @@ def test_cone_adjoint_paths(nx, ny, nz, dz, nu, nv, du, dv, nview, dso, flip):
             assert rel_l2(plan.backward(torch.from_numpy(p).cuda(), "dd").cpu().numpy(), ref) <= 1e-5, c
     finally:
         autotune_pin("dd_cone_adj", None)
+
+
+SIDDON = [  # nx, ny, nz, dz, nu, nv, du, dv, nview, dso, det (distance of the detector behind the axis), flip
+    (9, 14, 20, 1.0, 20, 13, 2.0, 1.6, 5, 300.0, 200.0, False),     # < 2 rows, a level row
+    (17, 6, 11, 1.0, 30, 20, 1.3, 0.8, 33, 120.0, 80.0, False),     # 2 to 3
+    (8, 8, 10, 2.0, 24, 40, 1.3, 1.0, 17, 120.0, 80.0, True),       # 3 to 4, rows against z
+    (8, 9, 12, 2.0, 24, 41, 1.3, 0.6, 7, 120.0, 80.0, False),       # 4 to 7, a level row
+    (6, 7, 150, 0.5, 90, 30, 0.2, 1.0, 9, 120.0, 80.0, False),      # fine columns, two z blocks
+    (16, 12, 9, 1.0, 40, 21, 0.6, 0.7, 11, 90.0, 3.0, False),       # the detector inside the volume
+    (8, 8, 6, 4.0, 20, 60, 1.3, 0.5, 8, 90.0, 80.0, False),         # more than 7 rows: tested view by view
+]
+
+
+@pytest.mark.parametrize("nx,ny,nz,dz,nu,nv,du,dv,nview,dso,det,flip", SIDDON)
+def test_siddon_cone_backprojection_paths(nx, ny, nz, dz, nu, nv, du, dv, nview, dso, det, flip):
+    from reconnet_amd._lib import autotune_pin
+    from reconnet_amd.torch_ops import ConePlan
+
+    ctr, u, v, src = circular_cone_vectors(nview, dso, det + dso, th0=0.3)
+    if flip:
+        v = -v
+    plan = ConePlan(nx, ny, nz, 1.0, 1.0, dz, nu, nv, du, dv, ctr, u, v, src, cx=0.3, cy=-0.2)
+    geo = dict(dx=1.0, dy=1.0, dz=dz, du=du, dv=dv, off_u=0.0, off_v=0.0, cx=0.3, cy=-0.2, cz=0.0)
+    p = np.random.default_rng(nu + nv).uniform(0, 1, (1, nu, nview, nv, 2)).astype(np.float32)
+    ref = orc.siddon_cone_bp(p, ctr, u, v, src, geo, (nx, ny, nz))
+    try:
+        for c in range(3):
+            autotune_pin("siddon_cone_bp", c)
+            assert rel_l2(plan.backward(torch.from_numpy(p).cuda(), "siddon").cpu().numpy(), ref) <= 1e-5, c
+    finally:
+        autotune_pin("siddon_cone_bp", None)
+
+
+def test_siddon_cone_backprojection_keeps_a_nan_in_its_rays():
+    # a NaN detector cell reaches the voxels its ray meets (the forward
+    # projection of each has the cell non-zero) and no others
+    from reconnet_amd.torch_ops import ConePlan
+
+    vecs = circular_cone_vectors(6, 120.0, 200.0, th0=0.3)
+    plan = ConePlan(10, 10, 12, 1.0, 1.0, 1.0, 24, 18, 1.3, 1.0, *vecs)
+    p = torch.rand((1, 24, 6, 18, 1), device="cuda")
+    p[0, 11, 2, 7, 0] = float("nan")
+    got = torch.isnan(plan.backward(p, "siddon"))
+    q = torch.zeros_like(p)
+    q[0, 11, 2, 7, 0] = 1.0
+    assert torch.equal(got, plan.backward(q, "siddon") > 0)
+    assert bool(got.any())
