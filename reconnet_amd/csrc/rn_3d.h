@@ -63,9 +63,9 @@ public:
     void siddon_bp(int nB, int nC, const float* prj, float* img, DevBuf& work, hipStream_t st) const;
     ArbGeo geo{};
 private:
-    // vec_: C, U, V, S per view; cls_: main axis per view; views_, cols_:
-    // per-view and per-(view, column) constants of the DD adjoint
-    DevBuf vec_, cls_, views_, cols_;
+    // vec_: C, U, V, S per view; views_, cols_: per-view (main axis included)
+    // and per-(view, column) constants of the DD pair
+    DevBuf vec_, views_, cols_;
     double ds_max_ = 0.0;   // most detector rows a voxel covers along z
 };
 

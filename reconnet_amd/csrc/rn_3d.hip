@@ -948,175 +948,7 @@ __global__ __launch_bounds__(256) void k_dd_tomo_bp(ArbGeo a, Grid3K g, const fl
 // forward value is sum_p (rectangle average of plane p) * L; the adjoint
 // gathers, per voxel, exactly those weights (overlap area / rectangle area * L).
 
-struct ConeRay {
-    float a[4], b[4];   // e1, e2, z1, z2 = a + b * plane
-    float L;
-    bool ok;
-};
-
-__device__ __forceinline__ ConeRay cone_ray(const ArbGeo& a, const Grid3K& g, const F3& c, const F3& U, const F3& V,
-                                            const F3& s, bool xv, int iu, int iv)
-{
-    ConeRay r;
-    const float uc = (iu - a.off_u - (a.nu - 1) / 2.0f) * a.du, vc = (iv - a.off_v - (a.nv - 1) / 2.0f) * a.dv;
-    auto P = [&](float u, float v) {
-        return F3{fmaf(v, V.x, fmaf(u, U.x, c.x)), fmaf(v, V.y, fmaf(u, U.y, c.y)), fmaf(v, V.z, fmaf(u, U.z, c.z))};
-    };
-    const F3 pc = P(uc, vc);
-    const F3 pts[4] = {P(uc - 0.5f * a.du, vc), P(uc + 0.5f * a.du, vc), P(uc, vc - 0.5f * a.dv), P(uc, vc + 0.5f * a.dv)};
-    // main axis m, in-plane axis n (plane coordinate of plane 0 and its step)
-    const float sm = xv ? s.x : s.y, sn = xv ? s.y : s.x;
-    const float dm = xv ? g.dx : g.dy, dn = xv ? g.dy : g.dx;
-    const float cn = xv ? g.cy : g.cx;
-    const int nn = xv ? g.ny : g.nx, nm = xv ? g.nx : g.ny;
-    const float m0 = (0.5f - 0.5f * nm) * dm + (xv ? g.cx : g.cy);
-    const float dpc = (xv ? pc.x : pc.y) - sm;
-    r.ok = fabsf(dpc) > 1e-6f;
-    const float lx = pc.x - s.x, ly = pc.y - s.y, lz = pc.z - s.z;
-    r.L = dm * sqrtf(fmaf(lx, lx, fmaf(ly, ly, lz * lz))) / fabsf(dpc);
-    #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float em = (xv ? pts[e].x : pts[e].y) - sm;
-        const float eo = e < 2 ? (xv ? pts[e].y : pts[e].x) - sn : pts[e].z - s.z;
-        const float k = eo / em;                                  // slope along the main axis
-        const float so = e < 2 ? sn : s.z, co = e < 2 ? cn : g.cz, d = e < 2 ? dn : g.dz;
-        const float no = e < 2 ? (float)nn : (float)g.nz;
-        r.b[e] = k * dm / d;
-        r.a[e] = (fmaf(m0 - sm, k, so) - co) / d + 0.5f * no;
-        r.ok = r.ok && fabsf(em) > 1e-6f;
-    }
-    return r;
-}
-
-// vol, prj: reference layouts [b][nx][ny][nz][c], [b][nu][nview][nv][c]
-// XCD > 0: 1-D grid (padded to a multiple of XCD) renumbered so that each XCD
-// walks a contiguous range of (row block, column, view): the adjacent detector
-// columns of a view, whose footprints share plane cells, meet in one L2.
-// OFF32: the 2 x 2 path addresses a plane's cells as a wave-uniform plane
-// base plus 32-bit byte offsets from 24-bit multiplies (byte strides below
-// 2^24, one slice's volume below 4 GiB: checked on the host).
-template <int XCD, bool OFF32>
-__global__ __launch_bounds__(64) void k_dd_cone_fp(ArbGeo a, Grid3K g, const float* __restrict__ vol,
-                                                   float* __restrict__ prj, const float* Cp, const float* Up,
-                                                   const float* Vp, const float* Sp, const int* __restrict__ cls,
-                                                   int nC, int nblocks)
-{
-    int bx, iu, bz;
-    if (XCD > 0) {
-        const int per = gridDim.x / XCD;
-        const int l = (blockIdx.x % XCD) * per + blockIdx.x / XCD;
-        if (l >= nblocks) return;
-        const int nvb = (a.nv + 63) / 64;
-        bx = l % nvb;
-        iu = (l / nvb) % a.nu;
-        bz = l / (nvb * a.nu);
-    } else {
-        bx = blockIdx.x;
-        iu = blockIdx.y;
-        bz = blockIdx.z;
-    }
-    const int iv = bx * 64 + threadIdx.x;
-    const int view = bz % a.nview, bc = bz / a.nview;
-    if (iv >= a.nv) return;
-    const bool xv = cls[view] == 0;
-    ConeRay r = cone_ray(a, g, ld3(Cp, view), ld3(Up, view), ld3(Vp, view), ld3(Sp, view), xv, iu, iv);
-    const int nm = xv ? g.nx : g.ny, nn = xv ? g.ny : g.nx;
-    const long sP = xv ? (long)g.ny * g.nz : g.nz, sJ = xv ? g.nz : (long)g.ny * g.nz;
-    const int c = bc % nC, b = bc / nC;
-    const float* base = vol + (long)b * g.nx * g.ny * g.nz * nC + c;   // reference layout, channel innermost
-    float acc = 0.f;
-    // the in-plane edges do not depend on the row (detV = (0, 0, v)): the
-    // wave's, in scalar registers
-    #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        r.a[e] = wave_uniform(r.a[e]);
-        r.b[e] = wave_uniform(r.b[e]);
-    }
-    // footprints at most one cell wide and high on every plane (the widths
-    // are affine in the plane index: the end planes bound them): at most 2 x
-    // 2 cells, taken without loops
-    const float wl = nm - 1.0f;
-    const bool small = fmaxf(fabsf(r.a[1] - r.a[0]), fabsf(fmaf(r.b[1] - r.b[0], wl, r.a[1] - r.a[0]))) <= 1.0f &&
-                       fmaxf(fabsf(r.a[3] - r.a[2]), fabsf(fmaf(r.b[3] - r.b[2], wl, r.a[3] - r.a[2]))) <= 1.0f;
-    if (r.ok && small) {
-        // the two edges of a pair never cross between planes (the footprint
-        // would vanish): order each pair once
-        const bool se = r.a[0] > r.a[1], sz = r.a[2] > r.a[3];
-        const float ea1 = se ? r.a[1] : r.a[0], eb1 = se ? r.b[1] : r.b[0];
-        const float ea2 = se ? r.a[0] : r.a[1], eb2 = se ? r.b[0] : r.b[1];
-        const float za1 = sz ? r.a[3] : r.a[2], zb1 = sz ? r.b[3] : r.b[2];
-        const float za2 = sz ? r.a[2] : r.a[3], zb2 = sz ? r.b[2] : r.b[3];
-        for (int p = 0; p < nm; ++p) {
-            const float fp = (float)p;
-            const float e1 = fmaf(eb1, fp, ea1), e2 = fmaf(eb2, fp, ea2);
-            const float le = fmaxf(e1, 0.f), he = fminf(e2, (float)nn);
-            if (!(he > le)) continue;
-            const float z1 = fmaf(zb1, fp, za1), z2 = fmaf(zb2, fp, za2);
-            const float lz = fmaxf(z1, 0.f), hz = fminf(z2, (float)g.nz);
-            const float area = (e2 - e1) * (z2 - z1);
-            if (!(hz > lz) || !(area > 0.f)) continue;
-            // cells j0, j0 + 1 and k0, k0 + 1; a second cell's share is 0 when
-            // the footprint ends in the first (its index is then clamped)
-            const int j0 = (int)le, k0 = (int)lz;
-            const float oe0 = fminf(he, (float)(j0 + 1)) - le, oe1 = fmaxf(he - (float)(j0 + 1), 0.f);
-            const float oz0 = fminf(hz, (float)(k0 + 1)) - lz, oz1 = fmaxf(hz - (float)(k0 + 1), 0.f);
-            const int j1 = min(j0 + 1, nn - 1), k1 = min(k0 + 1, g.nz - 1);
-            const float* P = base + p * sP * nC;
-            float v00, v01, v10, v11;
-            if (OFF32) {
-                const unsigned sj4 = (unsigned)(sJ * nC * 4), sk4 = (unsigned)(nC * 4);
-                const unsigned oj0 = __umul24((unsigned)j0, sj4), oj1 = __umul24((unsigned)j1, sj4);
-                const unsigned ok0 = __umul24((unsigned)k0, sk4), ok1 = __umul24((unsigned)k1, sk4);
-                const char* Pc = reinterpret_cast<const char*>(P);
-                v00 = *reinterpret_cast<const float*>(Pc + (oj0 + ok0));
-                v01 = *reinterpret_cast<const float*>(Pc + (oj0 + ok1));
-                v10 = *reinterpret_cast<const float*>(Pc + (oj1 + ok0));
-                v11 = *reinterpret_cast<const float*>(Pc + (oj1 + ok1));
-            } else {
-                v00 = P[(j0 * sJ + k0) * nC];
-                v01 = P[(j0 * sJ + k1) * nC];
-                v10 = P[(j1 * sJ + k0) * nC];
-                v11 = P[(j1 * sJ + k1) * nC];
-            }
-            const float sum = fmaf(fmaf(v01, oz1, v00 * oz0), oe0, fmaf(v11, oz1, v10 * oz0) * oe1);
-            acc = fmaf(sum, __builtin_amdgcn_rcpf(area), acc);
-        }
-        acc *= r.L;
-    } else if (r.ok) {
-        for (int p = 0; p < nm; ++p) {
-            const float fp = (float)p;
-            float e1 = fmaf(r.b[0], fp, r.a[0]), e2 = fmaf(r.b[1], fp, r.a[1]);
-            float z1 = fmaf(r.b[2], fp, r.a[2]), z2 = fmaf(r.b[3], fp, r.a[3]);
-            if (e1 > e2) { const float t = e1; e1 = e2; e2 = t; }
-            if (z1 > z2) { const float t = z1; z1 = z2; z2 = t; }
-            const float area = (e2 - e1) * (z2 - z1);
-            const float le = fmaxf(e1, 0.f), he = fminf(e2, (float)nn);
-            const float lz = fmaxf(z1, 0.f), hz = fminf(z2, (float)g.nz);
-            if (!(area > 0.f) || !(he > le) || !(hz > lz)) continue;
-            const float* P = base + p * sP * nC;
-            const int j0 = (int)le, j1 = min((int)he, nn - 1), k0 = (int)lz, k1 = min((int)hz, g.nz - 1);
-            float sum = 0.f;
-            for (int j = j0; j <= j1; ++j) {
-                const float oe = fminf(he, (float)(j + 1)) - fmaxf(le, (float)j);
-                if (oe <= 0.f) continue;
-                float row = 0.f;
-                for (int k = k0; k <= k1; ++k) {
-                    const float oz = fminf(hz, (float)(k + 1)) - fmaxf(lz, (float)k);
-                    row = fmaf(P[(j * sJ + k) * nC], fmaxf(oz, 0.f), row);
-                }
-                sum = fmaf(row, oe, sum);
-            }
-            acc += sum / area;
-        }
-        acc *= r.L;
-    }
-    prj[((((long)b * a.nu + iu) * a.nview + view) * a.nv + iv) * nC + c] = acc;
-}
-
-// Tables of the table-driven cone DD adjoint (k_dd_cone_adj_tab).
-// Row sums: per (slice, view, detector column) the nv + 1 FP64 sums
-// G[r] = sum over rows below r of len(row) q(row), len the length of the ray
-// through the cell centre (the adjoint's row weight).
+// Tables of the cone DD pair, built in double on the host with the plan.
 // ConeView: per view the constants of the plane-crossing geometry, resolved
 // for the view's main axis m (x or y; n the other in-plane axis, p the plane
 // index along m and j the voxel index along n).
@@ -1138,6 +970,188 @@ struct alignas(16) ConeView {
 // k0 = k1 = 0 (an empty footprint) and W = 0.
 struct alignas(32) ConeColumn { float k0, k1, A1, T3, W, pad[3]; };
 
+// A group of LV lanes takes LV detector rows of one column; 64 / LV columns share
+// a wave.  Per batch of LV planes each lane works out one plane's in-plane
+// footprint [e1, e2] (the rows run along z, so it is the same for every row) and
+// appends {offsets of cell rows j and j + 1, their shares / area, plane} to the
+// group's list in LDS, one entry per pair of cells; then every lane walks the
+// list with its own z footprint, z1 = a0 + mp (A1 + row / T3), |mp / T3| high:
+// one LDS broadcast, two loads of 2 adjacent cells (3 where the footprint is
+// over one voxel high) and 17 VALU instructions per entry.  A batch whose
+// footprints leave the volume along z, or are over two voxels high, sums
+// cell by cell within clamped bounds instead.
+//
+// Bound: instruction issue and the texture addresser alike: 3.5 ms at 256^2 x
+// 128, 720 views, 64 x 512 (5.9 ms with the in-plane footprint worked out by every
+// lane on every plane and four 4-byte loads).
+//
+// vol, prj: reference layouts [b][nx][ny][nz][c], [b][nu][nview][nv][c].  xcd: the
+// 1-D grid (a multiple of 8) is renumbered so that each XCD walks a contiguous
+// range of (column, row block, view): adjacent columns, whose footprints share
+// cells, meet in one L2.  OFF32: byte offsets within one slice's volume below
+// 4 GiB; C1: one channel (adjacent cells load as a pair).
+template <int LV, bool OFF32, bool C1>
+__global__ __launch_bounds__(256) void k_dd_cone_fp(ArbGeo a, Grid3K g, const float* __restrict__ vol,
+                                                    float* __restrict__ prj, const float* Cp, const float* Up,
+                                                    const float* Vp, const float* Sp,
+                                                    const ConeView* __restrict__ views,
+                                                    const ConeColumn* __restrict__ cols, int nC, int ncg, int nrb,
+                                                    int nblocks, int xcd)
+{
+    typedef float F2 __attribute__((ext_vector_type(2), aligned(4)));
+    constexpr int NG = 64 / LV;
+    __shared__ float4 ents[4][64];
+    __shared__ float emps[4][64];
+    int l = blockIdx.x;
+    if (xcd > 0) {
+        l = (l % xcd) * ((int)gridDim.x / xcd) + l / xcd;
+        if (l >= nblocks) return;
+    }
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int grp = lane / LV, lg = lane % LV;
+    const int iu0 = ((l % ncg) * 4 + wv) * NG;
+    if (iu0 >= a.nu) return;                       // whole waves (no workgroup barrier below)
+    const int rb = (l / ncg) % nrb, bz = l / (ncg * nrb);
+    const int view = bz % a.nview, bc = bz / a.nview;
+    const int cc = bc % nC, b = bc / nC;
+    const int iu = iu0 + grp, iv = rb * LV + lg;
+    const bool live = iu < a.nu && iv < a.nv;
+    const float fiv = (float)min(iv, a.nv - 1);
+    const ConeView vw = views[view];
+    const ConeColumn col = cols[(long)view * a.nu + min(iu, a.nu - 1)];
+    const int nm = vw.xv ? g.nx : g.ny, nn = vw.xv ? g.ny : g.nx;
+    const char* base = reinterpret_cast<const char*>(vol + (long)b * g.nx * g.ny * g.nz * nC + cc);
+    const float iT3 = col.T3 != 0.0f ? 1.0f / col.T3 : 0.0f, aT3 = fabsf(iT3);
+    // z edges of this lane's row: a0 + mp sl0 and a0 + mp sl1
+    const float sl0 = fmaf(fiv, iT3, col.A1), sl1 = fmaf(fiv + 1.0f, iT3, col.A1);
+    const float fnz = (float)g.nz;
+    const unsigned long long gmask = LV == 64 ? ~0ull : ((1ull << (LV & 63)) - 1ull);
+    float4* ent = ents[wv] + grp * LV;
+    float* emp = emps[wv] + grp * LV;
+    // cell k of the row of cells along z that an entry's word names (a byte
+    // offset, or the row's number where byte offsets do not fit 32 bits)
+    auto cell = [&](float word, int k) -> const char* {
+        const unsigned o = __float_as_uint(word);
+        if (OFF32) return base + (unsigned)(o + (C1 ? (unsigned)k * 4u : __umul24((unsigned)k, (unsigned)nC * 4u)));
+        return base + ((size_t)o * g.nz + k) * nC * 4;
+    };
+    auto ld = [](const char* p) { return *reinterpret_cast<const float*>(p); };
+    float acc = 0.0f;
+    for (int pb = 0; pb < nm; pb += LV) {
+        const int p = pb + lg;
+        const float mp = fmaf((float)p, vw.dm, vw.mp0);
+        const float ea = fmaf(mp, col.k0, vw.o), eb = fmaf(mp, col.k1, vw.o);
+        const float e1 = fminf(ea, eb), e2 = fmaxf(ea, eb);
+        const float le = fmaxf(e1, 0.0f), he = fminf(e2, (float)nn);
+        const float area = (e2 - e1) * fabsf(mp) * aT3;
+        int j0 = 0, pairs = 0;
+        if (p < nm && he > le && area > 0.0f && col.W != 0.0f) {
+            j0 = (int)le;
+            pairs = (min((int)he, nn - 1) - j0) / 2 + 1;
+        }
+        const float ia = __builtin_amdgcn_rcpf(area);
+        const int rounds = wave_max_nn(pairs);
+        // the batch's z footprints over all of the wave's rows: affine in mp
+        const float mpA = fmaf((float)pb, vw.dm, vw.mp0), mpB = fmaf((float)(min(pb + LV, nm) - 1), vw.dm, vw.mp0);
+        const float za = fmaf(mpA, sl0, vw.a0), zb = fmaf(mpB, sl0, vw.a0), zc = fmaf(mpA, sl1, vw.a0),
+                    zd = fmaf(mpB, sl1, vw.a0);
+        const float zlo = fminf(fminf(za, zb), fminf(zc, zd)), zhi = fmaxf(fmaxf(za, zb), fmaxf(zc, zd));
+        const float hmax = fmaxf(fabsf(mpA), fabsf(mpB)) * aT3;
+        const bool in = mpA * mpB > 0.0f && zlo >= 0.01f;
+        const bool two = __all(in && zhi <= fnz - 1.01f && hmax <= 1.0f);
+        const bool three = __all(in && zhi <= fnz - 2.01f && hmax <= 2.0f);
+        const float sl = mpA * iT3 > 0.0f ? sl0 : sl1;       // the lower edge's
+        for (int r = 0; r < rounds; ++r) {
+            const bool on = r < pairs;
+            const int j = j0 + 2 * r;
+            const float fj = (float)j;
+            const float oa = fminf(he, fj + 1.0f) - fmaxf(le, fj), ob = fmaxf(fminf(he, fj + 2.0f) - fmaxf(le, fj + 1.0f), 0.0f);
+            const unsigned long long gm = (__ballot(on) >> (grp * LV)) & gmask;
+            const int cnt = __popcll(gm), n = (wave_max_nn(cnt) + 3) & ~3;
+            if (on) {
+                const int pos = __popcll(gm & ((1ull << lg) - 1ull));
+                const int k = min(j + 1, nn - 1);
+                const unsigned r1 = (unsigned)(vw.xv ? p * g.ny + j : j * g.ny + p);
+                const unsigned r2 = (unsigned)(vw.xv ? p * g.ny + k : k * g.ny + p);
+                const unsigned m = OFF32 ? (unsigned)g.nz * (unsigned)nC * 4u : 1u;
+                ent[pos] = make_float4(__uint_as_float(r1 * m), __uint_as_float(r2 * m), oa * ia, ob * ia);
+                emp[pos] = mp;
+            }
+            // entries past the group's count: no weight, on a plane of the batch
+            for (int i = cnt + lg; i < n; i += LV) {
+                ent[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                emp[i] = mpA;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (two) {
+                for (int i = 0; i < n; i += 4) {
+                    #pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float4 e = ent[i + k];
+                        const float m = emp[i + k];
+                        const float z1 = fmaf(m, sl, vw.a0), fl = floorf(z1), h = fabsf(m) * aT3;
+                        const float w1 = fmaxf((z1 - fl) + h - 1.0f, 0.0f), w0 = h - w1;
+                        const char *pa = cell(e.x, (int)fl), *pb2 = cell(e.y, (int)fl);
+                        float a0, a1, b0, b1;
+                        if (C1) {
+                            const F2 x = *reinterpret_cast<const F2*>(pa), y = *reinterpret_cast<const F2*>(pb2);
+                            a0 = x[0]; a1 = x[1]; b0 = y[0]; b1 = y[1];
+                        } else {
+                            a0 = ld(pa); a1 = ld(pa + 4 * nC); b0 = ld(pb2); b1 = ld(pb2 + 4 * nC);
+                        }
+                        acc = fmaf(e.z, fmaf(a1, w1, a0 * w0), acc);
+                        acc = fmaf(e.w, fmaf(b1, w1, b0 * w0), acc);
+                    }
+                }
+            } else if (three) {
+                for (int i = 0; i < n; i += 4) {
+                    #pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float4 e = ent[i + k];
+                        const float m = emp[i + k];
+                        const float z1 = fmaf(m, sl, vw.a0), fl = floorf(z1), h = fabsf(m) * aT3;
+                        const float t = (z1 - fl) + h;
+                        const float w1 = __builtin_amdgcn_fmed3f(t - 1.0f, 0.0f, 1.0f), w2 = fmaxf(t - 2.0f, 0.0f);
+                        const float w0 = (h - w1) - w2;
+                        const char *pa = cell(e.x, (int)fl), *pb2 = cell(e.y, (int)fl);
+                        const float sa = fmaf(ld(pa + 8 * nC), w2, fmaf(ld(pa + 4 * nC), w1, ld(pa) * w0));
+                        const float sb = fmaf(ld(pb2 + 8 * nC), w2, fmaf(ld(pb2 + 4 * nC), w1, ld(pb2) * w0));
+                        acc = fmaf(e.w, sb, fmaf(e.z, sa, acc));
+                    }
+                }
+            } else {
+                for (int i = 0; i < n; ++i) {
+                    const float4 e = ent[i];
+                    const float m = emp[i];
+                    const float y0 = fmaf(m, sl0, vw.a0), y1 = fmaf(m, sl1, vw.a0);
+                    const float lz = fmaxf(fminf(y0, y1), 0.0f), hz = fminf(fmaxf(y0, y1), fnz);
+                    if (!(hz > lz)) continue;
+                    const int k1 = min((int)hz, g.nz - 1);
+                    float sa = 0.0f, sb = 0.0f;
+                    for (int k = (int)lz; k <= k1; ++k) {
+                        const float oz = fmaxf(fminf(hz, (float)(k + 1)) - fmaxf(lz, (float)k), 0.0f);
+                        sa = fmaf(ld(cell(e.x, k)), oz, sa);
+                        sb = fmaf(ld(cell(e.y, k)), oz, sb);
+                    }
+                    acc = fmaf(e.w, sb, fmaf(e.z, sa, acc));
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+    }
+    if (!live) return;
+    // path length per plane: dm / |main-axis run| times the ray's length to the cell
+    const F3 c = ld3(Cp, view), U = ld3(Up, view), V = ld3(Vp, view), s = ld3(Sp, view);
+    const float uc = (iu - a.off_u - (a.nu - 1) / 2.0f) * a.du, vc = (iv - a.off_v - (a.nv - 1) / 2.0f) * a.dv;
+    const float lx = fmaf(vc, V.x, fmaf(uc, U.x, c.x)) - s.x, ly = fmaf(vc, V.y, fmaf(uc, U.y, c.y)) - s.y,
+                lz = fmaf(vc, V.z, fmaf(uc, U.z, c.z)) - s.z;
+    prj[((((long)b * a.nu + iu) * a.nview + view) * a.nv + iv) * nC + cc] =
+        acc * fabsf(col.W) * sqrtf(fmaf(lx, lx, fmaf(ly, ly, lz * lz)));
+}
+
+// Row sums of the adjoint's second form: per (slice, view, detector column) the
+// nv + 1 FP64 sums G[r] = sum over rows below r of len(row) q(row), len the
+// length of the ray through the cell centre (the adjoint's row weight).
 // Row sums: one wave per (slice, view, column), in table order; lanes take
 // 64 rows at a time, an FP64 inclusive scan across the wave, then a carry.
 __global__ __launch_bounds__(256) void k_dd_cone_rowsum(ArbGeo a, const float* __restrict__ prj, const float* Cp,
@@ -1827,9 +1841,7 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
     std::copy(V, V + 3 * n, h.begin() + 6 * n);
     std::copy(S, S + 3 * n, h.begin() + 9 * n);
     vec_.alloc(h.size() * sizeof(float));
-    cls_.alloc(cls.size() * sizeof(int));
     RN_HIP_CHECK(hipMemcpyAsync(vec_.get(), h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice, st));
-    RN_HIP_CHECK(hipMemcpyAsync(cls_.get(), cls.data(), cls.size() * sizeof(int), hipMemcpyHostToDevice, st));
     // view and column tables of the DD adjoint, in double
     ds_max_ = 0.0;
     std::vector<ConeView> vt(n);
@@ -1894,24 +1906,28 @@ void ConePlan::dd_fp(int nB, int nC, const float* img, float* prj, hipStream_t s
     const ArbGeo& g = geo;
     RN_REQUIRE(nB > 0 && nC > 0 && (long)g.nview * nB * nC <= 65535, "cone batch too large for one launch");
     const float* v = vec_.as<float>();
-    const long nblocks = (long)cdiv(g.nv, 64) * g.nu * g.nview * nB * nC;
+    // byte offsets in 32 bits, channel strides by 24-bit multiplies
+    const bool off32 = (long)g.nx * g.ny * g.nz * nC * 4 < (1L << 32) && g.nz < (1 << 24) && nC < (1 << 22);
+    RN_REQUIRE((long)g.nx * g.ny < 0x7fffffffL, "dd_cone_fp: volume too large in plane");
+    // rows per group of lanes: the split with the fewest idle lanes, wide first
+    int lv = 64;
+    for (int w : {32, 16})
+        if (cdiv(g.nv, w) * w < cdiv(g.nv, lv) * lv) lv = w;
+    const int ncg = cdiv(g.nu, 4 * (64 / lv)), nrb = cdiv(g.nv, lv);
+    const long nblocks = (long)ncg * nrb * g.nview * nB * nC;
     RN_REQUIRE(nblocks + 8 < 0x7fffffffL, "dd_cone_fp: grid too large");
-    // 32-bit cell offsets when every byte stride fits 24 bits and a slice's
-    // volume 4 GiB
-    const bool off32 = (long)std::max(g.ny, g.nx) * g.nz * nC * 4 < (1L << 24) &&
-                       (long)g.nx * g.ny * g.nz * nC * 4 < (1L << 32);
     auto launch = [&](int c) {
-        if (c == 0) {
-            const long n8 = (nblocks + 7) / 8 * 8;
-            auto k = off32 ? k_dd_cone_fp<8, true> : k_dd_cone_fp<8, false>;
-            hipLaunchKernelGGL(k, dim3((unsigned)n8), dim3(64), 0, st, g, grid_of(g), img, prj, v, v + 3 * g.nview,
-                               v + 6 * g.nview, v + 9 * g.nview, cls_.as<int>(), nC, (int)nblocks);
-        } else {
-            dim3 grd(cdiv(g.nv, 64), g.nu, g.nview * nB * nC);
-            auto k = off32 ? k_dd_cone_fp<0, true> : k_dd_cone_fp<0, false>;
-            hipLaunchKernelGGL(k, grd, dim3(64), 0, st, g, grid_of(g), img, prj, v, v + 3 * g.nview, v + 6 * g.nview,
-                               v + 9 * g.nview, cls_.as<int>(), nC, (int)nblocks);
-        }
+        const int xcd = c == 0 ? 8 : 0;
+        const unsigned n = (unsigned)(c == 0 ? (nblocks + 7) / 8 * 8 : nblocks);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(n), dim3(256), 0, st, g, grid_of(g), img, prj, v, v + 3 * g.nview,
+                               v + 6 * g.nview, v + 9 * g.nview, views_.as<ConeView>(), cols_.as<ConeColumn>(), nC, ncg,
+                               nrb, (int)nblocks, xcd);
+        };
+        auto pick = [&](auto k64, auto k32, auto k16) { lv == 64 ? go(k64) : lv == 32 ? go(k32) : go(k16); };
+        if (!off32) pick(k_dd_cone_fp<64, false, false>, k_dd_cone_fp<32, false, false>, k_dd_cone_fp<16, false, false>);
+        else if (nC == 1) pick(k_dd_cone_fp<64, true, true>, k_dd_cone_fp<32, true, true>, k_dd_cone_fp<16, true, true>);
+        else pick(k_dd_cone_fp<64, true, false>, k_dd_cone_fp<32, true, false>, k_dd_cone_fp<16, true, false>);
         check_launch("dd_cone_fp");
     };
     const int c = tune_choose({TK_DD_CONE_FP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC}, 2, launch, st, true);

@@ -1,4 +1,4 @@
-"""The list-driven cone backprojections against the FP64 oracle where their paths
+"""The list-driven cone projectors against the FP64 oracle where their paths
 change: up to 2, 3 and more rows per voxel, detector columns much finer than a
 voxel (several list rounds), volumes taller than a workgroup's z block, fewer
 views than a batch, detector rows that run against z, and a source close enough
@@ -88,3 +88,30 @@ def test_siddon_cone_backprojection_keeps_a_nan_in_its_rays():
     q[0, 11, 2, 7, 0] = 1.0
     assert torch.equal(got, plan.backward(q, "siddon") > 0)
     assert bool(got.any())
+
+
+FORWARD = [  # nx, ny, nz, dz, nu, nv, du, dv, nview, dso, channels
+    (9, 14, 40, 1.0, 20, 12, 1.0, 1.0, 5, 300.0, 1),       # z footprints under a voxel, inside the volume
+    (9, 14, 40, 0.6, 20, 17, 1.0, 1.2, 5, 300.0, 2),       # one to two voxels; 32 rows a group
+    (17, 6, 9, 0.3, 30, 70, 1.3, 1.4, 33, 120.0, 1),       # over two, and out of the volume; 16 rows a group
+    (70, 67, 12, 1.0, 9, 33, 9.0, 1.0, 7, 200.0, 1),       # cells several voxels wide, two plane batches
+    (8, 8, 10, 2.0, 300, 40, 0.1, 0.8, 3, 120.0, 1),       # columns much finer than a voxel
+]
+
+
+@pytest.mark.parametrize("nx,ny,nz,dz,nu,nv,du,dv,nview,dso,nc", FORWARD)
+def test_cone_forward_paths(nx, ny, nz, dz, nu, nv, du, dv, nview, dso, nc):
+    from reconnet_amd._lib import autotune_pin
+    from reconnet_amd.torch_ops import ConePlan
+
+    vecs = circular_cone_vectors(nview, dso, 200.0 + dso, th0=0.3)
+    plan = ConePlan(nx, ny, nz, 1.0, 1.0, dz, nu, nv, du, dv, *vecs, cx=0.3, cy=-0.2, cz=0.4, off_v=0.2)
+    geo = dict(dx=1.0, dy=1.0, dz=dz, du=du, dv=dv, off_u=0.0, off_v=0.2, cx=0.3, cy=-0.2, cz=0.4)
+    x = np.random.default_rng(nu + nv).uniform(0, 1, (1, nx, ny, nz, nc)).astype(np.float32)
+    ref = orc.dd_cone_fp(x, *vecs, geo, nu, nv)
+    try:
+        for c in range(2):
+            autotune_pin("dd_cone_fp", c)
+            assert rel_l2(plan.forward(torch.from_numpy(x).cuda(), "dd").cpu().numpy(), ref) <= 1e-5, c
+    finally:
+        autotune_pin("dd_cone_fp", None)
