@@ -39,8 +39,6 @@ struct FanK {
     const float* vcos;   // [nview] cos t
     const float* vsin;   // [nview] sin t
     const int* vcls;     // [nview] 0 = X view, 1 = Y view
-    const float* esin;   // [nu+1] sin of bin-edge angles (edge e = a_e + da/2 of bin e)
-    const float* ecos;
     const float* bsin;   // [nu] sin of bin-centre angles
     const float* bcos;
     // [nview][nu] line of the ray through bin centre k, in image coordinates:

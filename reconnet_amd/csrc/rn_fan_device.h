@@ -42,29 +42,6 @@ __device__ __forceinline__ float4 vscale(float4 v, float f) { return make_float4
 // geometry helpers
 // ---------------------------------------------------------------------------
 
-// Ray of detector angle a (sin sa, cos ca) in view t (cos ct, sin st):
-// X views:  X(Y) = A + B (Y - ny/2)   (absolute image coordinates)
-__device__ __forceinline__ void xline(const FanK& g, float ct, float st, float sa, float ca,
-                                      float& A, float& B, float& cu)
-{
-    cu = ca * ct + sa * st;            // cos(a - t)
-    const float su = sa * ct - ca * st;  // sin(a - t)
-    const float inv = 1.0f / cu;
-    A = 0.5f * g.nx + (g.dso / g.dx) * sa * inv;
-    B = (g.dy / g.dx) * su * inv;
-}
-
-// Y views:  Y(X) = A + B (X - nx/2)
-__device__ __forceinline__ void yline(const FanK& g, float ct, float st, float sa, float ca,
-                                      float& A, float& B, float& su)
-{
-    const float cu = ca * ct + sa * st;
-    su = sa * ct - ca * st;
-    const float inv = 1.0f / su;
-    A = 0.5f * g.ny - (g.dso / g.dy) * sa * inv;
-    B = (g.dx / g.dy) * cu * inv;
-}
-
 // acc[q] += scale * the average of row q (`rboff` bytes after the
 // wave-uniform base rows[q]) over one interval [lo, hi] of its n
 // piecewise-constant cells (zero outside [0, n)): the cells, their overlaps and the
