@@ -258,6 +258,65 @@ __global__ __launch_bounds__(BX * BY) void k_siddon_fan_bp_q(FanK g, const float
     }
 }
 
+// A lane's G groups of 4 slices of pixel (ix, iy): stored to the plain images
+// img, or with UPD the OS-SQS update applied to them instead (sqs_update_core per
+// slice, the arithmetic of k_sqs_update_q): the current image and its 4-neighbours
+// are read as float4 groups from the interleaved copy u.Qold, the normaliser from
+// u.D4, and the new image goes to u.Xn and, as float4 per group, to the other
+// interleaved copies u.Qxy, u.Qyx (the launch reads none of the buffers it writes).
+template <int G, bool UPD>
+__device__ __forceinline__ void store_or_update(const FanK& g, const float4 (&acc)[G], float* __restrict__ img,
+                                                const SqsUpd& u, int ix, int iy, int q0, int nq, int ns)
+{
+    const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
+    #pragma unroll
+    for (int k = 0; k < G; ++k) {
+        if (k >= nq) break;
+        const int s = 4 * (q0 + k);
+        float v[4] = {acc[k].x, acc[k].y, acc[k].z, acc[k].w};
+        if constexpr (UPD) {
+            const int pxy = qpitch(g.ny), pyx = qpitch(g.nx);
+            const float4* qo = u.Qold + (long)(q0 + k) * g.nx * pxy;
+            const long c0 = (long)ix * pxy + kQPadL + iy;
+            const float4 xc = qo[c0];
+            // neighbours for the TV terms (padded lines: iy - 1 and iy + 1 stay inside
+            // the line; the border cases below use the pixel value itself, as the
+            // plain update)
+            float4 xl = xc, xr = xc, yl = xc, yr = xc;
+            if (u.beta2 != 0.0f) {
+                if (ix > 0) xl = qo[c0 - pxy];
+                if (ix < g.nx - 1) xr = qo[c0 + pxy];
+                yl = qo[c0 - 1];
+                yr = qo[c0 + 1];
+            }
+            const float4 d4 = u.D4[(long)(q0 + k) * plane + pix];
+            const float xs[4] = {xc.x, xc.y, xc.z, xc.w}, xls[4] = {xl.x, xl.y, xl.z, xl.w};
+            const float xrs[4] = {xr.x, xr.y, xr.z, xr.w}, yls[4] = {yl.x, yl.y, yl.z, yl.w};
+            const float yrs[4] = {yr.x, yr.y, yr.z, yr.w}, ds[4] = {d4.x, d4.y, d4.z, d4.w};
+            #pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float x = xs[c];
+                const float dx0 = ix == 0 ? x : x - xls[c], dx1 = ix == g.nx - 1 ? x : x - xrs[c];
+                const float dy0 = iy == 0 ? x : x - yls[c], dy1 = iy == g.ny - 1 ? x : x - yrs[c];
+                float xn = 0.0f;
+                if (s + c < ns) {
+                    xn = sqs_update_core(x, dx0, dx1, dy0, dy1, v[c], ds[c], u.step, u.beta2, u.eps, u.lb, u.ub,
+                                         u.crop);
+                    u.Xn[(long)(s + c) * plane + pix] = xn;
+                }
+                v[c] = xn;
+            }
+            const float4 f = make_float4(v[0], v[1], v[2], v[3]);
+            u.Qxy[(long)(q0 + k) * g.nx * pxy + (long)ix * pxy + kQPadL + iy] = f;
+            u.Qyx[(long)(q0 + k) * g.ny * pyx + (long)iy * pyx + kQPadL + ix] = f;
+        } else {
+            #pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (s + c < ns) img[(long)(s + c) * plane + pix] = v[c];
+        }
+    }
+}
+
 // k_siddon_fan_bp_q with each wave's bin window staged in LDS.  Per view the
 // wave's 64 pixels need the bins [wlo, whi] (the lane minimum and maximum of
 // their ranges); the G groups' values and the view's ray table over CAP bins
@@ -276,12 +335,8 @@ __global__ __launch_bounds__(BX * BY) void k_siddon_fan_bp_q(FanK g, const float
 // group rows are addressed as 32-bit byte offsets from the groups' base (the
 // launcher checks that G groups fit).
 //
-// UPD: the epilogue applies the OS-SQS update to the backprojected gradient
-// instead of storing it (sqs_update_core per slice, the arithmetic of
-// k_sqs_update_q): the current image and its 4-neighbours are read as float4
-// groups from the interleaved copy u.Qold, the normaliser from u.D4, and the
-// new image goes to u.Xn and, as float4 per group, to the other interleaved
-// copies u.Qxy, u.Qyx (this launch reads none of the buffers it writes).
+// UPD: the epilogue applies the OS-SQS update instead of storing the gradient
+// (store_or_update).
 template <int BX, int BY, int NB, int G, int CAP, bool UPD = false>
 __global__ __launch_bounds__(BX * BY, G >= 8 ? 4 : 1) void k_siddon_fan_bp_ql(FanK g, const float4* __restrict__ prj,
                                                           float* __restrict__ img, int view0, int nviews, int ns,
@@ -380,54 +435,40 @@ __global__ __launch_bounds__(BX * BY, G >= 8 ? 4 : 1) void k_siddon_fan_bp_ql(Fa
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         k0 = n0; k1 = n1; wlo = nlo; whi = nhi;
     }
-    if (!inside) return;
-    const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
-    #pragma unroll
-    for (int k = 0; k < G; ++k) {
-        if (k >= nq) break;
-        const int s = 4 * (q0 + k);
-        float v[4] = {acc[k].x, acc[k].y, acc[k].z, acc[k].w};
-        if (UPD) {
-            const int pxy = qpitch(g.ny), pyx = qpitch(g.nx);
-            const float4* qo = u.Qold + (long)(q0 + k) * g.nx * pxy;
-            const long c0 = (long)ix * pxy + kQPadL + iy;
-            const float4 xc = qo[c0];
-            // neighbours for the TV terms (padded lines: iy - 1 and iy + 1 stay inside
-            // the line; the border cases below use the pixel value itself, as the
-            // plain update)
-            float4 xl = xc, xr = xc, yl = xc, yr = xc;
-            if (u.beta2 != 0.0f) {
-                if (ix > 0) xl = qo[c0 - pxy];
-                if (ix < g.nx - 1) xr = qo[c0 + pxy];
-                yl = qo[c0 - 1];
-                yr = qo[c0 + 1];
-            }
-            const float4 d4 = u.D4[(long)(q0 + k) * plane + pix];
-            const float xs[4] = {xc.x, xc.y, xc.z, xc.w}, xls[4] = {xl.x, xl.y, xl.z, xl.w};
-            const float xrs[4] = {xr.x, xr.y, xr.z, xr.w}, yls[4] = {yl.x, yl.y, yl.z, yl.w};
-            const float yrs[4] = {yr.x, yr.y, yr.z, yr.w}, ds[4] = {d4.x, d4.y, d4.z, d4.w};
-            #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const float x = xs[c];
-                const float dx0 = ix == 0 ? x : x - xls[c], dx1 = ix == g.nx - 1 ? x : x - xrs[c];
-                const float dy0 = iy == 0 ? x : x - yls[c], dy1 = iy == g.ny - 1 ? x : x - yrs[c];
-                float xn = 0.0f;
-                if (s + c < ns) {
-                    xn = sqs_update_core(x, dx0, dx1, dy0, dy1, v[c], ds[c], u.step, u.beta2, u.eps, u.lb, u.ub,
-                                         u.crop);
-                    u.Xn[(long)(s + c) * plane + pix] = xn;
-                }
-                v[c] = xn;
-            }
-            const float4 f = make_float4(v[0], v[1], v[2], v[3]);
-            u.Qxy[(long)(q0 + k) * g.nx * pxy + (long)ix * pxy + kQPadL + iy] = f;
-            u.Qyx[(long)(q0 + k) * g.ny * pyx + (long)iy * pyx + kQPadL + ix] = f;
-        } else {
-            #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (s + c < ns) img[(long)(s + c) * plane + pix] = v[c];
+    if (inside) store_or_update<G, UPD>(g, acc, img, u, ix, iy, q0, nq, ns);
+}
+
+// Quad-layout Siddon BP for launches with few tiles: an 8 x 8-pixel tile of one
+// group of 4 slices per workgroup, whose VS waves take one part of the views each
+// (gathers from memory, as k_siddon_fan_bp_q); their sums are added in LDS in wave
+// order and the last wave stores or updates.
+//
+// Bound: the latency of a wave's view loop (about 0.7 us per view).  One slice,
+// k_siddon_fan_bp_q -> VS = 4: 256^2, 30 views 23 -> 11 us (1024 -> 4096 waves);
+// 512^2, 96 views 74 -> 67 us, 288 views 254 -> 195 us; and the update is in the
+// epilogue instead of a launch of its own.
+template <int NB, int VS, bool UPD>
+__global__ __launch_bounds__(64 * VS) void k_siddon_fan_bp_qv(FanK g, const float4* __restrict__ prj,
+                                                              float* __restrict__ img, int view0, int nviews, int ns,
+                                                              SqsUpd u)
+{
+    __shared__ float4 red[64];
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int iy = blockIdx.x * 8 + (lane & 7), ix = blockIdx.y * 8 + (lane >> 3), q0 = blockIdx.z;
+    const int v0 = (int)((long)nviews * wv / VS), v1 = (int)((long)nviews * (wv + 1) / VS);
+    const bool inside = ix < g.nx && iy < g.ny;
+    float4 acc[1] = {vzero<float4>()};
+    if (inside)
+        siddon_bp_pixel_slices<float4, NB, 1>(g, prj + ((long)q0 * nviews + v0) * g.nu, 0, 1, view0 + v0, v1 - v0, ix,
+                                              iy, acc);
+    for (int w = 0; w < VS; ++w) {
+        if (w == wv) {
+            if (w > 0) vadd(acc[0], red[lane]);
+            red[lane] = acc[0];
         }
+        __syncthreads();
     }
+    if (wv == VS - 1 && inside) store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
 }
 
 // Exact DD adjoint (dd_adj_tile): a workgroup takes an 8 x 8-pixel tile of G
@@ -1221,6 +1262,20 @@ void go_siddon_bp_ql(const FanK& g, const float4* prj, float* img, int ns, int v
                        view0, nviews, ns, SqsUpd{});
 }
 
+template <int NB, int VS>
+void go_siddon_bp_qv(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_siddon_fan_bp_qv<NB, VS, false>), dim3(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(ns, 4)),
+                       dim3(64, VS), 0, st, g, prj, img, view0, nviews, ns, SqsUpd{});
+}
+
+template <int NB, int VS>
+void go_siddon_bp_qvu(const FanK& g, const float4* prj, int ns, int view0, int nviews, const SqsUpd& u, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_siddon_fan_bp_qv<NB, VS, true>), dim3(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(ns, 4)),
+                       dim3(64, VS), 0, st, g, prj, nullptr, view0, nviews, ns, u);
+}
+
 template <int BX, int BY, int NB, int G, int CAP>
 void go_siddon_bp_qlu(const FanK& g, const float4* prj, int ns, int view0, int nviews, const SqsUpd& u,
                       hipStream_t st)
@@ -1251,16 +1306,35 @@ const SidBpQFn kSidBpQ[] = {go_siddon_bp_ql<8, 8, 2, 8, 24>,  go_siddon_bp_ql<8,
                             go_siddon_bp_q<16, 16, 2, 4>,     go_siddon_bp_q<8, 8, 2, 4>,
                             go_siddon_bp_q<8, 8, 2, 2>,       go_siddon_bp_q<16, 16, 2, 2>,
                             go_siddon_bp_q<8, 8, 2, 1>,       go_siddon_bp_q<16, 16, 2, 1>,
-                            go_siddon_bp_q<8, 8, 3, 4>,       go_siddon_bp_q<8, 8, 3, 2>};
+                            go_siddon_bp_q<8, 8, 3, 4>,       go_siddon_bp_q<8, 8, 3, 2>,
+                            go_siddon_bp_qv<2, 4>,            go_siddon_bp_qv<2, 8>,
+                            go_siddon_bp_qv<2, 2>};
 constexpr int kNSidFpQ = sizeof(kSidFpQ) / sizeof(kSidFpQ[0]);
 constexpr int kNSidBpQ = sizeof(kSidBpQ) / sizeof(kSidBpQ[0]);
 constexpr int kNSidBpStaged = 7;   // the first seven are k_siddon_fan_bp_ql
+constexpr int kNSidBpSplit = 3;    // the last three k_siddon_fan_bp_qv
 using SidBpQUFn = void (*)(const FanK&, const float4*, int, int, int, const SqsUpd&, hipStream_t);
 // the staged shapes of kSidBpQ, in the same order, with the OS-SQS update in the epilogue
 const SidBpQUFn kSidBpQU[kNSidBpStaged] = {
     go_siddon_bp_qlu<8, 8, 2, 8, 24>, go_siddon_bp_qlu<8, 32, 2, 8, 24>, go_siddon_bp_qlu<8, 8, 2, 8, 32>,
     go_siddon_bp_qlu<8, 8, 2, 8, 21>, go_siddon_bp_qlu<8, 8, 2, 8, 16>, go_siddon_bp_qlu<8, 8, 2, 4, 24>,
     go_siddon_bp_qlu<8, 8, 2, 2, 32>};
+const SidBpQUFn kSidBpQVU[kNSidBpSplit] = {go_siddon_bp_qvu<2, 4>, go_siddon_bp_qvu<2, 8>, go_siddon_bp_qvu<2, 2>};
+
+// Candidate i of the interleaved BP for this launch: in listed order, or for one
+// group of slices the view-split shapes first (the staged shapes carry up to 8
+// groups per lane: 43 against 10 us for one slice of 256^2, 30 views); the
+// staged shapes only where 8 groups' rows fit 32-bit offsets.
+struct SidBpOrder {
+    int first, n, shift;
+    SidBpOrder(const FanK& g, int nslices, int nviews)
+    {
+        first = 9L * nviews * g.nu * 16L < 0x7fffffffL ? 0 : kNSidBpStaged;
+        n = kNSidBpQ - first;
+        shift = nslices <= 4 ? n - kNSidBpSplit : 0;
+    }
+    int operator[](int i) const { return first + (i + shift) % n; }
+};
 
 } // namespace
 
@@ -1335,11 +1409,10 @@ void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, i
 {
     if (nslices <= 0 || nviews <= 0) return;
     require_offsets32(g, nviews, sizeof(float4));
-    // the LDS-staged candidates address 8 groups' rows with 32-bit offsets
-    const int first = 9L * nviews * g.nu * 16L < 0x7fffffffL ? 0 : kNSidBpStaged;
-    const int c = first + tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, kNSidBpQ - first,
-                                      [&](int i) { kSidBpQ[first + i](g, prj_q, img_xy, nslices, view0, nviews, st); },
-                                      st, true);
+    const SidBpOrder order(g, nslices, nviews);
+    const int c = order[tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, order.n,
+                                    [&](int i) { kSidBpQ[order[i]](g, prj_q, img_xy, nslices, view0, nviews, st); }, st,
+                                    true)];
     kSidBpQ[c](g, prj_q, img_xy, nslices, view0, nviews, st);
     check_launch("siddon_fan_bp_q");
 }
@@ -1349,11 +1422,16 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
 {
     if (nslices <= 0 || nviews <= 0) return false;
     require_offsets32(g, nviews, sizeof(float4));
-    const int first = 9L * nviews * g.nu * 16L < 0x7fffffffL ? 0 : kNSidBpStaged;
+    const SidBpOrder order(g, nslices, nviews);
     // the launch shape is tuned on the plain backprojection (img_xy as its output)
-    const int c = first + tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, kNSidBpQ - first,
-                                      [&](int i) { kSidBpQ[first + i](g, prj_q, img_xy, nslices, view0, nviews, st); },
-                                      st, true);
+    const int c = order[tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, order.n,
+                                    [&](int i) { kSidBpQ[order[i]](g, prj_q, img_xy, nslices, view0, nviews, st); }, st,
+                                    true)];
+    if (c >= kNSidBpQ - kNSidBpSplit) {
+        kSidBpQVU[c - (kNSidBpQ - kNSidBpSplit)](g, prj_q, nslices, view0, nviews, u, st);
+        check_launch("siddon_fan_bp_q_update");
+        return true;
+    }
     if (c < kNSidBpStaged) {
         kSidBpQU[c](g, prj_q, nslices, view0, nviews, u, st);
         check_launch("siddon_fan_bp_q_update");

@@ -72,9 +72,10 @@ private:
     FanTables t_;
     int ns_ = 0, npers_ = 0, nsub_ = 0;
     DevBuf B_, W_, D_, X_[2], Xyx_, R_, G_, red_;
-    // interleaved layout (groups of 4 slices as float4), used for 4 or more
-    // slices unless RECONNET_SQS_INTERLEAVE=0: images in both orientations,
-    // measurement, weights and the subset residual
+    // interleaved layout (groups of 4 slices as float4, the last one padded),
+    // used unless RECONNET_SQS_INTERLEAVE=0 (below 4 slices only while its padded
+    // planes fit 32-bit offsets): images in both orientations, measurement,
+    // weights and the subset residual
     bool quads_ = false;
     // one FP launch over the whole subset (default), or one per view class
     // (RECONNET_SQS_FP_SPLIT=1)

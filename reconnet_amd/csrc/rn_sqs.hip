@@ -378,7 +378,17 @@ void OsSqs::setup(const FanGeo& g, const float* deg_host, int nslices, int nview
     X_[1].ensure(ns_ * plane * sizeof(float));
     G_.ensure(ns_ * plane * sizeof(float));
     const char* env = std::getenv("RECONNET_SQS_INTERLEAVE");
-    quads_ = ns_ >= 4 && !(env && env[0] == '0');
+    // Interleaved layout: also for 1 to 3 slices, whose empty components are
+    // carried along: a crossing's two or three cells come with one load either
+    // way, and the forward projection may then split a ray's lines over lanes, the
+    // backprojection its views over waves with the update in its epilogue.  ms per
+    // pass, plain -> interleaved: 64^2 1 slice (6 subsets) 0.18 -> 0.08; 256^2 1 and
+    // 3 slices (12) 0.70 -> 0.36, 0.76 -> 0.36; 512^2 1, 2, 3 slices (12) 1.80, 2.20,
+    // 2.58 -> 1.21, 1.22, 1.23; 512^2 3 slices (4) 1.99 -> 1.15.  Fewer than 4 slices
+    // keep the plain layout where only its planes meet the 2 GiB offsets.
+    const bool fits = (long)std::max(g.nx * (long)qpitch(g.ny), g.ny * (long)qpitch(g.nx)) * 16L < 0x7fffffffL &&
+                      (long)npers_ * g.nu * 16L < 0x7fffffffL;
+    quads_ = (ns_ >= 4 || fits) && !(env && env[0] == '0');
     const char* split = std::getenv("RECONNET_SQS_FP_SPLIT");
     fp_split_ = split && split[0] == '1';
     if (quads_) {
