@@ -116,10 +116,13 @@ __host__ __device__ constexpr int qpitch(int n) { return n + kQPadL + kQPadR; }
 void launch_siddon_fan_fp_residual_q(const FanK& g, const float4* Qyx, const float4* Qxy, float4* res_q,
                                      int nslices, int view0, int nviews, const float4* meas_q, const float4* w_q,
                                      int res_vstride, int res_voff, hipStream_t st);
+// Siddon FP of the same quad images into plain sinograms [s][nviews][nu]
+void launch_siddon_fan_fp_q(const FanK& g, const float4* Qyx, const float4* Qxy, float* prj_vu, int nslices,
+                            int view0, int nviews, hipStream_t st);
 // out[b][j][:] = in[b][perm[j]][:] for a batch of (rows x cols) matrices (perm: device, rows entries)
 void launch_permute_rows(const float* in, float* out, const int* perm, int rows, int cols, int batch,
                          hipStream_t st);
-// Siddon BP gather of a quad subset sinogram [q][view][nu] into plain images [s][nx][ny]
+// Siddon BP gather of a quad sinogram [q][view][nu] into plain images [s][nx][ny]
 void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, int nslices, int view0,
                             int nviews, hipStream_t st);
 // The OS-SQS update applied to a backprojected subset gradient: the current
@@ -155,6 +158,17 @@ void launch_pack_quads_len(const FanK& g, const float* in, float4* q, int nslice
 // pad cells are left as they are)
 void launch_pack_quads(const float* in, float4* q_same, float4* q_tr, int n1, int n2, int nslices, bool padded,
                        hipStream_t st);
+// plain images [s][n1][n2] -> both padded quad orientations, q_same [q][n1][qpitch(n2)]
+// and q_tr [q][n2][qpitch(n1)], pad cells zeroed; avg: of the averaged planes
+// (in[i-1][j] + in[i][j]) / 2 in q_same and (in[i][j-1] + in[i][j]) / 2 in q_tr
+void launch_pack_planes(const float* in, float4* q_same, float4* q_tr, int n1, int n2, int nslices, bool avg,
+                        hipStream_t st);
+// the padded quad planes of one slice group fit 32-bit byte offsets
+inline bool qplanes_fit32(int nx, int ny)
+{
+    const long a = (long)nx * qpitch(ny), b = (long)ny * qpitch(nx);
+    return (a > b ? a : b) * 16L < 0x7fffffffL;
+}
 
 // ---- layout helpers ----
 // out[b][c][r] = in[b][r][c] for a batch of (rows x cols) matrices

@@ -56,6 +56,20 @@ std::vector<float> identity(int n)
     return I;
 }
 
+// One size for every operation on ns slices, so that a plan that has run one of
+// them allocates nothing in the others.
+void ensure_work(FanWork& w, const FanGeo& g, int ns)
+{
+    const size_t plane = (size_t)g.nx * g.ny, sino = (size_t)g.nu * g.nview;
+    const size_t big = (size_t)ns * std::max(plane, sino) * sizeof(float);
+    w.rx.ensure(big);
+    w.ry.ensure(big);
+    w.sino.ensure(big);
+    // quad sinograms, or both padded quad orientations of the images
+    const size_t qplanes = ns >= 4 ? (size_t)g.ny * qpitch(g.nx) + (size_t)g.nx * qpitch(g.ny) : 0;
+    w.quad.ensure((size_t)cdiv(ns, 4) * std::max(sino, qplanes) * sizeof(float4));
+}
+
 } // namespace
 
 std::vector<float> fp_mix_matrix(const FanGeo& g, FanFP kind)
@@ -99,10 +113,7 @@ void fan_forward(const FanTables& t, FanFP kind, int nB, int nC, const float* im
     const std::vector<float> M = fp_mix_matrix(g, kind);
     const bool direct_in = (g.nz == 1 && g.nv == 1 && is_identity_1(M, nB, nC));
     const bool direct_out = (g.nv * nC == 1);
-    const size_t big = (size_t)ns * std::max(plane, sino) * sizeof(float);
-    w.rx.ensure(big);
-    w.ry.ensure(big);
-    w.sino.ensure(big);
+    ensure_work(w, g, ns);
 
     const float* P = img_ref;
     if (!direct_in) {
@@ -112,20 +123,21 @@ void fan_forward(const FanTables& t, FanFP kind, int nB, int nC, const float* im
         P = w.planes.as<float>();
     }
     float* out_vu = w.sino.as<float>();
-    if (kind == FanFP::DD && ns >= 4) {
-        // groups of 4 slices interleaved, padded lines (zero pads):
-        // QY[q][x][pad + y] = (P[x-1][y] + P[x][y]) / 2,  QX[q][y][pad + x] = (P[x][y-1] + P[x][y]) / 2
-        const size_t qx = (size_t)g.ny * qpitch(g.nx), qy = (size_t)g.nx * qpitch(g.ny);
-        const int nq = cdiv(ns, 4);
-        w.qdd.ensure((qx + qy) * nq * sizeof(float4));
-        float4* QX = w.qdd.as<float4>();
-        float4* QY = QX + qx * nq;
-        launch_fill(w.qdd.as<float>(), 0.0f, (qx + qy) * nq * 4, st);
-        launch_avg_prev(P, w.ry.as<float>(), g.nx, g.ny, ns, 0, st);
-        launch_pack_quads(w.ry.as<float>(), QY, nullptr, g.nx, g.ny, ns, true, st);
-        launch_avg_prev(P, w.rx.as<float>(), g.nx, g.ny, ns, 1, st);
-        launch_pack_quads(w.rx.as<float>(), nullptr, QX, g.nx, g.ny, ns, true, st);
-        launch_dd_fan_fp_q(t.k, QX, QY, out_vu, ns, 0, g.nview, st);
+    // Interleaved from 4 slices (Siddon: while the padded planes fit 32-bit offsets).
+    // Siddon, one-slice layout -> interleaved, FP and BP in ms: 64^2 4 slices 0.019,
+    // 0.068 -> 0.017, 0.019; 256^2 4 slices 0.077, 0.29 -> 0.056, 0.090; 512^2 4, 5
+    // and 32 slices 0.52, 1.22 -> 0.37, 0.79; 0.93, 1.73 -> 0.67, 1.17; 3.6, 5.7 -> 2.7,
+    // 2.0.  Fewer slices keep the one-slice layout, whose bits do not depend on the
+    // launch shape.
+    if (ns >= 4 && (kind == FanFP::DD || qplanes_fit32(g.nx, g.ny))) {
+        // groups of 4 slices interleaved, padded lines (zero pads), the images or (DD)
+        // their averaged planes: QY[q][x][pad + y] of P or (P[x-1][y] + P[x][y]) / 2,
+        // QX[q][y][pad + x] of P or (P[x][y-1] + P[x][y]) / 2
+        float4* QX = w.quad.as<float4>();
+        float4* QY = QX + (size_t)g.ny * qpitch(g.nx) * cdiv(ns, 4);
+        launch_pack_planes(P, QY, QX, g.nx, g.ny, ns, kind == FanFP::DD, st);
+        if (kind == FanFP::DD) launch_dd_fan_fp_q(t.k, QX, QY, out_vu, ns, 0, g.nview, st);
+        else launch_siddon_fan_fp_q(t.k, QX, QY, out_vu, ns, 0, g.nview, st);
     } else if (kind == FanFP::DD) {
         // RY[x][y] = (P[x-1][y] + P[x][y]) / 2 ;  RX = transpose((P[x][y-1] + P[x][y]) / 2)
         launch_avg_prev(P, w.ry.as<float>(), g.nx, g.ny, ns, 0, st);
@@ -156,10 +168,7 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
     const std::vector<float> M = bp_mix_matrix(g, kind);
     const bool direct_in = (g.nz == 1 && g.nv == 1 && is_identity_1(M, nB, nC));
     const bool direct_out = (g.nz * nC == 1);
-    const size_t big = (size_t)ns * std::max(plane, sino) * sizeof(float);
-    w.rx.ensure(big);
-    w.ry.ensure(big);
-    w.sino.ensure(big);
+    ensure_work(w, g, ns);
 
     const float* Q = prj_ref;   // [slice][nu][nview]
     if (!direct_in) {
@@ -168,7 +177,8 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
         Q = w.ry.as<float>();
     }
     float* W = w.sino.as<float>();   // [slice][nview][nu]
-    if (kind != FanBP::DDAdjoint) launch_transpose(Q, W, g.nu, g.nview, ns, st);
+    const bool quads = kind == FanBP::Siddon && ns >= 4;   // transposed and interleaved in one pass
+    if (kind != FanBP::DDAdjoint && !quads) launch_transpose(Q, W, g.nu, g.nview, ns, st);
     float* out = direct_out ? img_ref : w.rx.as<float>();
     switch (kind) {
     case FanBP::DD:
@@ -183,7 +193,6 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
         }
         if (ns >= 4) {
             // groups of 4 slices interleaved: one float4 load per bin and group
-            w.quad.ensure((size_t)cdiv(ns, 4) * sino * sizeof(float4));
             launch_pack_quads(P, w.quad.as<float4>(), nullptr, g.nview, g.nu, ns, false, st);
             launch_dd_fan_bp_q(t.k, w.quad.as<float4>(), out, ns, fbp, st);
         } else {
@@ -193,12 +202,16 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
     }
     case FanBP::DDAdjoint:
         // transposed, interleaved and multiplied by the rays' length per line in one pass
-        w.quad.ensure((size_t)cdiv(ns, 4) * sino * sizeof(float4));
         launch_pack_quads_len(t.k, Q, w.quad.as<float4>(), ns, st);
         launch_dd_fan_adj(t.k, w.quad.as<float4>(), out, ns, st);
         break;
     case FanBP::Siddon:
-        launch_siddon_fan_bp(t.k, W, out, ns, 0, g.nview, false, st);
+        if (quads) {
+            launch_pack_quads(Q, nullptr, w.quad.as<float4>(), g.nu, g.nview, ns, false, st);
+            launch_siddon_fan_bp_q(t.k, w.quad.as<float4>(), out, ns, 0, g.nview, st);
+        } else {
+            launch_siddon_fan_bp(t.k, W, out, ns, 0, g.nview, false, st);
+        }
         break;
     case FanBP::Pixel:
         launch_pixel_fan_bp(t.k, W, out, ns, st);

@@ -386,8 +386,7 @@ void OsSqs::setup(const FanGeo& g, const float* deg_host, int nslices, int nview
     // 3 slices (12) 0.70 -> 0.36, 0.76 -> 0.36; 512^2 1, 2, 3 slices (12) 1.80, 2.20,
     // 2.58 -> 1.21, 1.22, 1.23; 512^2 3 slices (4) 1.99 -> 1.15.  Fewer than 4 slices
     // keep the plain layout where only its planes meet the 2 GiB offsets.
-    const bool fits = (long)std::max(g.nx * (long)qpitch(g.ny), g.ny * (long)qpitch(g.nx)) * 16L < 0x7fffffffL &&
-                      (long)npers_ * g.nu * 16L < 0x7fffffffL;
+    const bool fits = qplanes_fit32(g.nx, g.ny) && (long)npers_ * g.nu * 16L < 0x7fffffffL;
     quads_ = (ns_ >= 4 || fits) && !(env && env[0] == '0');
     const char* split = std::getenv("RECONNET_SQS_FP_SPLIT");
     fp_split_ = split && split[0] == '1';

@@ -12,7 +12,7 @@ namespace rn {
 
 bool TuneKey::operator<(const TuneKey& o) const
 {
-    return std::tie(kernel, a, b, c, d, e) < std::tie(o.kernel, o.a, o.b, o.c, o.d, o.e);
+    return std::tie(kernel, a, b, c, d, e, layout) < std::tie(o.kernel, o.a, o.b, o.c, o.d, o.e, o.layout);
 }
 
 namespace {

@@ -5,9 +5,10 @@
 // launch of a key the tuner times every candidate with HIP events on the
 // caller's stream (one warm-up and three timed runs each) and keeps the first
 // candidate within 3 % of the fastest (candidates are listed in order of
-// preference); later launches of the key reuse it.  Candidates differ only in the
-// block / tile shape of the launch: every output element is computed by the
-// same per-element code, so the choice never changes the results.
+// preference); later launches of the key reuse it.  Candidates compute every
+// output element by the same per-element code; those that split an element's
+// sum over lanes or waves (interleaved Siddon and DD kernels) may round it
+// differently in its last bits.
 //
 // Tuning is skipped (the first candidate, or the cached choice, is used) when
 // the stream is being captured into a graph, when the launch accumulates into
@@ -25,6 +26,7 @@ namespace rn {
 struct TuneKey {
     int kernel;
     int a, b, c, d, e;
+    int layout = 0;   // one kernel id with several candidate lists: 1 = interleaved slices
     bool operator<(const TuneKey& o) const;
 };
 
