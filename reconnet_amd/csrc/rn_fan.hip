@@ -328,6 +328,28 @@ __device__ __forceinline__ void store_or_update(const FanK& g, const float4 (&ac
     }
 }
 
+// Adds the G values per lane of a workgroup's nw waves in wave order through
+// red [G][64]; true in the wave that holds the sums (every wave calls it).
+template <int G>
+__device__ __forceinline__ bool add_waves(float4 (&v)[G], float4* red, int lane, int wv, int nw)
+{
+    if (nw == 1) return true;
+    for (int w = 0; w < nw; ++w) {
+        if (w == wv) {
+            #pragma unroll
+            for (int k = 0; k < G; ++k) {
+                if (w > 0) {
+                    const float4 r = red[k * 64 + lane];
+                    v[k] = make_float4(r.x + v[k].x, r.y + v[k].y, r.z + v[k].z, r.w + v[k].w);
+                }
+                red[k * 64 + lane] = v[k];
+            }
+        }
+        __syncthreads();
+    }
+    return wv == nw - 1;
+}
+
 // k_siddon_fan_bp_q with each wave's bin window staged in LDS.  Per view the
 // wave's 64 pixels need the bins [wlo, whi] (the lane minimum and maximum of
 // their ranges); the G groups' values and the view's ray table over CAP bins
@@ -472,14 +494,7 @@ __global__ __launch_bounds__(64 * VS) void k_siddon_fan_bp_qv(FanK g, const floa
     if (inside)
         siddon_bp_pixel_slices<float4, NB, 1>(g, prj + ((long)q0 * nviews + v0) * g.nu, 0, 1, view0 + v0, v1 - v0, ix,
                                               iy, acc);
-    for (int w = 0; w < VS; ++w) {
-        if (w == wv) {
-            if (w > 0) vadd(acc[0], red[lane]);
-            red[lane] = acc[0];
-        }
-        __syncthreads();
-    }
-    if (wv == VS - 1 && inside) store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
+    if (add_waves<1>(acc, red, lane, wv, VS) && inside) store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
 }
 
 // Exact DD adjoint (dd_adj_tile): a workgroup takes an 8 x 8-pixel tile of G
@@ -508,35 +523,8 @@ __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const
     float4 tot[G];
     dd_adj_tile<G, CAP, 3, WIDE>(g, wprj + q0 * sstride, sstride, nq, 0, g.nview, wv * per, (wv + 1) * per, ix, iy,
                                  inside, lane, dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
-    if (nw > 1) {
-        float4* red = dyn4 + nw * DdAdjStage<G, CAP>::kFloat4;
-        for (int w = 0; w < nw; ++w) {
-            if (w == wv) {
-                #pragma unroll
-                for (int k = 0; k < G; ++k) {
-                    float4 v = tot[k];
-                    if (w > 0) {
-                        const float4 r = red[k * 64 + lane];
-                        v = make_float4(r.x + v.x, r.y + v.y, r.z + v.z, r.w + v.w);
-                    }
-                    red[k * 64 + lane] = tot[k] = v;
-                }
-            }
-            __syncthreads();
-        }
-        if (wv != nw - 1) return;
-    }
-    if (!inside) return;
-    const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
-    #pragma unroll
-    for (int k = 0; k < G; ++k) {
-        if (k >= nq) break;
-        const int s = 4 * (q0 + k);
-        const float v[4] = {tot[k].x, tot[k].y, tot[k].z, tot[k].w};
-        #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (s + c < ns) img[(long)(s + c) * plane + pix] = v[c];
-    }
+    if (add_waves<G>(tot, dyn4 + nw * DdAdjStage<G, CAP>::kFloat4, lane, wv, nw) && inside)
+        store_or_update<G, false>(g, tot, img, SqsUpd{}, ix, iy, q0, nq, ns);
 }
 
 // PreweightBPKernelX/Y: length factor for the iterative (non-FBP) DD BP.
@@ -554,7 +542,8 @@ __global__ void k_dd_preweight(FanK g, const float* __restrict__ prj, float* __r
     wprj[i] = prj[i] * f;
 }
 
-// Reference-parity DD BP (DDBPFanKernelX/Y): pixel edges projected through
+// Reference-parity DD BP (DDBPFanKernelX/Y) of geometries without FanK::tile: pixel
+// edges projected through
 // atan, average of the (pre-weighted) detector row over the footprint.  One
 // lane per pixel of S consecutive slices (grid z counts groups of S): the
 // footprint and the FBP weight are computed once for the S slices (their
@@ -629,135 +618,123 @@ __global__ __launch_bounds__(BX * BY) void k_dd_fan_bp_q(FanK g, const float4* _
     for (int k = 0; k < G; ++k) rows[k] = wprj + (long)(q0 + min(k, nq - 1)) * sstride;
     float4 acc[G];
     dd_bp_pixel<float4, G>(g, rows, ix, iy, fbp, acc);
-    const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
-    #pragma unroll
-    for (int k = 0; k < G; ++k) {
-        if (k >= nq) break;
-        const int s = 4 * (q0 + k);
-        const float v[4] = {acc[k].x, acc[k].y, acc[k].z, acc[k].w};
-        #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (s + c < ns) img[(long)(s + c) * plane + pix] = v[c];
-    }
+    store_or_update<G, false>(g, acc, img, SqsUpd{}, ix, iy, q0, nq, ns);
 }
 
-// k_dd_fan_bp_q with each wave's bin window staged in LDS (as
-// k_siddon_fan_bp_ql): per view the wave's 64 pixels read the bins [wlo, whi]
-// of the G groups' pre-weighted rows; those CAP bins from wlo are loaded once
-// per wave with coalesced dwordx4 loads, issued one view ahead into
-// registers, written to the wave's own LDS rows and averaged from there with
-// the arithmetic of dd_bp_pixel.  Views whose window is wider than CAP bins
-// read the rows directly.
-template <int BX, int BY, int G, int CAP, int NB>
-__global__ __launch_bounds__(BX * BY, G >= 8 ? 4 : 1) void k_dd_fan_bp_ql(FanK g, const float4* __restrict__ wprj,
-                                                      float* __restrict__ img, int ns, int fbp)
+// The footprint of the lane's pixel in one view of a TileProj batch (l: the view's
+// lane): [lo, hi] relative to the tile's first bin, between the projections of the
+// pixel's edges along x (X views) or y, and the view's weight over the footprint's
+// width, kr / (r / r0)^2 / (hi - lo) with fbp, else 1 / (hi - lo).  FanK::tile keeps
+// the width above 1e-3 bins.
+__device__ __forceinline__ void dd_bp_footprint(const FanK& g, const TileProj& tp, int l, int cls, float inv_da, int fbp,
+                                                float& lo, float& hi, float& k)
 {
-    static_assert((BX * BY) % 64 == 0, "whole waves");
+    const float P = lane_f(tp.P, l), Q = lane_f(tp.Q, l), u0 = lane_f(tp.u0, l);
+    const float en = cls == 0 ? P * (0.5f * g.dx) : Q * (0.5f * g.dy);
+    const float ed = cls == 0 ? -Q * (0.5f * g.dx) : P * (0.5f * g.dy);
+    const float num = fmaf(P, tp.px, Q * tp.py), den = fmaf(P, tp.py, fmaf(-Q, tp.px, 1.0f));
+    auto bin = [&](float nn, float dd) {
+        const float z = nn * __builtin_amdgcn_rcpf(dd), s = z * z;   // atan z to 2e-8 at |z| = 0.1
+        return fmaf(z * inv_da, -fmaf(s, fmaf(s, 0.2f, -1.0f / 3.0f), 1.0f), u0);
+    };
+    const float b1 = bin(num - en, den - ed), b2 = bin(num + en, den + ed);
+    lo = fminf(b1, b2);
+    hi = fmaxf(b1, b2);
+    const float w = hi - lo;
+    k = fbp ? lane_f(tp.kr, l) * __builtin_amdgcn_rcpf(fmaf(num, num, den * den) * w) : __builtin_amdgcn_rcpf(w);
+}
+
+// The DD BP of an 8 x 8-pixel tile of G interleaved slice groups, for geometries
+// with FanK::tile.  The views are split evenly over the workgroup's nw waves; the
+// waves' sums are added in LDS in wave order.  Per view the tile's bins of the G
+// groups' pre-weighted rows, CAP at a time, are loaded once per wave with coalesced
+// dwordx4 loads, issued one step (a view, or a further CAP bins of it) ahead into
+// registers, written to the wave's own LDS rows and averaged from there by every
+// pixel.  One gather code for every step (no branch around the accumulators, which
+// would cost copies of them): the step before the first adds zeros times the
+// cleared rows.  A wave touches only its own rows and the LDS instructions of one
+// wave execute in order, so the steps need no barrier; the fences keep the compiler
+// from moving LDS accesses across the handovers.  The group rows are addressed as
+// 32-bit byte offsets from the groups' base (the launcher checks that G groups fit).
+//
+// Bound: LDS reads (three bins of 8 groups per pixel and view are 192 clocks of a
+// wave's 757) and VALU (195 instructions).  32 slices of 512^2, 1152 views, 736 bins,
+// FBP: 2.27 -> 1.70 ms; before, every pixel's two edges went through atanf and the
+// window was the lanes' minimum and maximum (386 instructions), and batches that fill
+// no 8 groups or tiles that fill no chip read the bins per pixel from memory
+// (256^2, 360 views, 1 and 32 slices: 0.20 -> 0.07, 0.39 -> 0.17 ms).
+template <int G, int CAP>
+__global__ __launch_bounds__(512, 4) void k_dd_fan_bp_tile(FanK g, const float4* __restrict__ wprj,
+                                                           float* __restrict__ img, int ns, int fbp)
+{
+    extern __shared__ float4 dyn4[];
     constexpr int kLoads = (G * CAP + 63) / 64;
-    __shared__ float4 stage[(BX * BY / 64) * G * CAP];
-    const int tid = threadIdx.y * BX + threadIdx.x;
-    const int lane = tid & 63;
-    float4* st = stage + (tid >> 6) * G * CAP;
-    const int iy = blockIdx.x * BX + threadIdx.x;
-    const int ix = blockIdx.y * BY + threadIdx.y;
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
+    const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
+    float4* st = dyn4 + wv * G * CAP;
+    for (int i = lane; i < G * CAP; i += 64) st[i] = vzero<float4>();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const bool inside = ix < g.nx && iy < g.ny;   // lanes outside stage but gather nothing
-    const int nquads = (ns + 3) / 4;
-    const int q0 = blockIdx.z * G;
-    const int nq = min(G, nquads - q0);
+    const int q0 = blockIdx.z * G, nq = min(G, (ns + 3) / 4 - q0);
     const long sstride = (long)g.nview * g.nu;
     const float4* P = wprj + q0 * sstride;
-    const float4* rows[G];
     float4 acc[G];
     #pragma unroll
-    for (int q = 0; q < G; ++q) {
-        rows[q] = P + (long)min(q, nq - 1) * sstride;
-        acc[q] = vzero<float4>();
-    }
+    for (int q = 0; q < G; ++q) acc[q] = vzero<float4>();
     // staging load j of this lane: element i = 64 j + lane, row i / CAP, bin
     // i % CAP (LDS slot i)
     int bj[kLoads];
-    const float4* src[kLoads];
-    bool has[kLoads];
+    unsigned roff[kLoads];
     #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-        const int i = j * 64 + lane, r = i / CAP;
+        const int i = j * 64 + lane;
         bj[j] = i % CAP;
-        has[j] = r < G;
-        src[j] = P + (long)min(r, nq - 1) * sstride;
+        roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
     }
-    const int cx = min(ix, g.nx - 1), cy = min(iy, g.ny - 1);
-    const float x = (cx - 0.5f * (g.nx - 1)) * g.dx, y = (cy - 0.5f * (g.ny - 1)) * g.dy;
     const float inv_da = 1.0f / g.da;
-    const float boff = 0.5f * g.nu - g.off_a;
-    // the footprint [lo, hi] of the pixel in view `view` (dd_bp_pixel), its
-    // bins and FBP weight
-    auto geom = [&](int view, float& lo, float& hi, float& fw, int& m0, int& m1) {
-        const float ct = g.vcos[view], sn = g.vsin[view];
-        const float rx = x * ct + y * sn, ry = -x * sn + y * ct;
-        float ex, ey;
-        if (g.vcls[view] == 0) { ex = 0.5f * g.dx * ct; ey = -0.5f * g.dx * sn; }
-        else                   { ex = 0.5f * g.dy * sn; ey = 0.5f * g.dy * ct; }
-        const float b1 = boff - atanf((rx - ex) * __builtin_amdgcn_rcpf(ry - ey + g.dso)) * inv_da;
-        const float b2 = boff - atanf((rx + ex) * __builtin_amdgcn_rcpf(ry + ey + g.dso)) * inv_da;
-        lo = fminf(b1, b2);
-        hi = fmaxf(b1, b2);
-        const float d = g.dso + ry;
-        fw = g.dso * g.dso * __builtin_amdgcn_rcpf(fmaf(rx, rx, d * d));
-        seg_avg_bins(g.nu, lo, hi, m0, m1);
-        if (!inside) { m0 = g.nu; m1 = -1; }
-    };
+    TileProj tp;
+    tp.init(g, lane);
     float4 rg[kLoads];
-    auto issue = [&](int view, int wlo) {
-        #pragma unroll
-        for (int j = 0; j < kLoads; ++j)
-            if (has[j]) rg[j] = ld_at(src[j], (unsigned)(view * g.nu + min(wlo + bj[j], g.nu - 1)) * 16u);
-    };
-    float lo, hi, fw;
-    int m0, m1;
-    geom(0, lo, hi, fw, m0, m1);
-    int wlo = wave_min(m0), whi = wave_max(m1);
-    if (whi >= wlo && whi - wlo < CAP) issue(0, wlo);
-    for (int view = 0; view < g.nview; ++view) {
-        const bool any = whi >= wlo;            // some lane reads a bin of this view
-        const bool staged = whi - wlo < CAP;
-        if (any && staged) {
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            #pragma unroll
-            for (int j = 0; j < kLoads; ++j)
-                if (has[j]) st[j * 64 + lane] = rg[j];
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        }
-        float nlo_f = 0.0f, nhi_f = 0.0f, nfw = 1.0f;
-        int n0 = g.nu, n1 = -1, nlo = g.nu, nhi = -1;
-        if (view + 1 < g.nview) {
-            geom(view + 1, nlo_f, nhi_f, nfw, n0, n1);
-            nlo = wave_min(n0);
-            nhi = wave_max(n1);
-            if (nhi >= nlo && nhi - nlo < CAP) issue(view + 1, nlo);
-        }
-        if (any) {
-            const float sc = fbp ? fw : 1.0f;
-            if (staged) {
-                // lanes outside the image read nothing: their interval is made empty
-                seg_acc_staged<G, CAP, NB>(st, wlo, g.nu, inside ? lo : -2.0f, inside ? hi : -1.0f, sc, acc);
-            } else if (inside) {
-                seg_acc_rows<float4, G>(rows, (unsigned)(view * g.nu) * 16u, g.nu, lo, hi, sc, acc);
+    float lo = 0.0f, hi = -1.0f, k = 0.0f;   // the step's interval (relative to its first bin) and scale
+    const int v0 = (int)((long)g.nview * wv / nw), v1 = (int)((long)g.nview * (wv + 1) / nw);
+    int view = v0 - 1, base = 0, span = -1, off = 0;
+    for (bool more = true;;) {
+        const float l = lo, h = hi, kk = k;
+        if (off + CAP <= span) {
+            off += CAP;
+            lo -= (float)CAP;
+            hi -= (float)CAP;
+        } else {
+            off = 0;
+            do {
+                more = ++view < v1;
+                if (!more) break;
+                if (((view - v0) & 63) == 0) tp.batch(g, view, lane, tx, ty, 0.5 * g.nu - (double)g.off_a, 0.0f);
+                span = __builtin_amdgcn_readlane(tp.span, (view - v0) & 63);
+            } while (span < 0);
+            if (more) {
+                const int w = (view - v0) & 63;
+                base = __builtin_amdgcn_readlane(tp.base, w);
+                dd_bp_footprint(g, tp, w, g.vcls[view], inv_da, fbp, lo, hi, k);
+                hi = inside ? fminf(hi, (float)(g.nu - base)) : -1.0f;
             }
         }
+        if (more) {
+            #pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP)
+                    rg[j] = ld_at(P, roff[j] + (unsigned)(view * g.nu + min(base + off + bj[j], g.nu - 1)) * 16u);
+        }
+        seg_rel_staged<G, CAP>(st, l, h, (float)CAP, kk, acc);
+        if (!more) break;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        lo = nlo_f; hi = nhi_f; fw = nfw; wlo = nlo; whi = nhi;
-    }
-    if (!inside) return;
-    const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
-    #pragma unroll
-    for (int k = 0; k < G; ++k) {
-        if (k >= nq) break;
-        const int s = 4 * (q0 + k);
-        const float v[4] = {acc[k].x, acc[k].y, acc[k].z, acc[k].w};
         #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (s + c < ns) img[(long)(s + c) * plane + pix] = v[c];
+        for (int j = 0; j < kLoads; ++j)
+            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane] = rg[j];
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
+    if (add_waves<G>(acc, dyn4 + nw * G * CAP, lane, wv, nw) && inside)
+        store_or_update<G, false>(g, acc, img, SqsUpd{}, ix, iy, q0, nq, ns);
 }
 
 // bpFanKernel3D with isFBP = true (the only mode the reference launches).
@@ -1130,6 +1107,13 @@ void FanTables::build(const FanGeo& g, const float* deg_host, hipStream_t st)
     // pixel centres lie within R of the centre: |rx| / (dso - |ry|) <= R / (dso - R) < 1 if R < 0.45 dso
     const double R = 0.5 * std::sqrt((double)g.nx * g.dx * g.nx * g.dx + (double)g.ny * g.dy * g.ny * g.dy);
     k.unit_angle = R < 0.45 * (double)g.dso ? 1 : 0;
+    // the tiles' points (an incomplete tile reaches over the image) lie within Rt of the
+    // centre: half a tile over their distance from the source at most kTileMax, and
+    // the footprint of half a pixel, at least cos(72 deg) of it across the ray
+    // (45 deg of view, 27 of fan), over 1e-3 bins
+    const double hx = 4.0 * g.dx, hy = 4.0 * g.dy, ht = std::sqrt(hx * hx + hy * hy), Rt = R + 2.0 * ht;
+    k.tile = Rt < 0.45 * (double)g.dso && ht <= fan::kTileMax * ((double)g.dso - Rt) &&
+             0.3 * std::min(g.dx, g.dy) >= 1e-3 * std::fabs((double)g.da) * ((double)g.dso + Rt) ? 1 : 0;
 }
 
 bool FanTables::matches(const FanGeo& g, const float* deg_host) const
@@ -1199,9 +1183,10 @@ void go_siddon_bp(const FanK& g, const float* prj, float* img, int ns, int view0
                        dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns, acc);
 }
 
-// One wave per tile and view segment while one wave per tile would leave the
-// 1024 SIMDs fewer than 8 waves each (32 slices of 256^2, 16 per lane, are 2048
-// waves: 0.62 ms by one wave per tile, 0.45 by eight).
+// Eight waves per tile, one per view segment, while one would leave the 1024 SIMDs
+// fewer than 8 waves each (32 slices of 256^2, 16 per lane, are 2048 waves: DD
+// adjoint 0.62 ms by one wave per tile, 0.45 by eight; DD BP, one slice of 512^2,
+// 4096 waves: 0.73 by two, 0.65 by eight).
 constexpr long kDdAdjWaves = 8192;
 
 template <int G, int CAP>
@@ -1268,22 +1253,42 @@ void go_dd_bp_q(const FanK& g, const float4* wprj, float* img, int ns, int fbp, 
     hipLaunchKernelGGL((k_dd_fan_bp_q<BX, BY, G>), dim3(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(cdiv(ns, 4), G)),
                        dim3(BX, BY), 0, st, g, wprj, img, ns, fbp);
 }
-template <int BX, int BY, int G, int CAP, int NB = 2>
-void go_dd_bp_ql(const FanK& g, const float4* wprj, float* img, int ns, int fbp, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_dd_fan_bp_ql<BX, BY, G, CAP, NB>), dim3(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(cdiv(ns, 4), G)),
-                       dim3(BX, BY), 0, st, g, wprj, img, ns, fbp);
-}
 using DdBpQFn = void (*)(const FanK&, const float4*, float*, int, int, hipStream_t);
-// LDS-staged shapes only with 8 slice groups per lane: staged 4- and 2-group
-// kernels timed within a few per cent of the direct ones back to back, so the
-// tuner took them at times, but after the preweighting and packing launches
-// of a backward call they ran 0.496 and 0.639 ms against 0.410 ms (32 slices
-// of 256^2) and 3.4 and 5.3 ms against 2.4 ms (32 slices of 512^2)
-const DdBpQFn kDdBpQ[] = {go_dd_bp_ql<8, 8, 8, 24>, go_dd_bp_ql<8, 8, 8, 32>, go_dd_bp_ql<8, 32, 8, 32>,
-                          go_dd_bp_ql<8, 32, 8, 24>, go_dd_bp_q<8, 8, 4>,       go_dd_bp_q<16, 16, 2>,
-                          go_dd_bp_q<8, 8, 2>,       go_dd_bp_q<16, 16, 1>,     go_dd_bp_q<8, 8, 1>};
+const DdBpQFn kDdBpQ[] = {go_dd_bp_q<8, 8, 4>,   go_dd_bp_q<16, 16, 2>, go_dd_bp_q<8, 8, 2>,
+                          go_dd_bp_q<16, 16, 1>, go_dd_bp_q<8, 8, 1>};
 constexpr int kNDdBpQ = sizeof(kDdBpQ) / sizeof(kDdBpQ[0]);
+
+template <int G, int CAP>
+void go_dd_bp_tile(const FanK& g, const float4* wprj, float* img, int ns, int fbp, hipStream_t st)
+{
+    const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
+    const int nw = (long)grd.x * grd.y * grd.z < kDdAdjWaves ? 8 : 1;
+    const size_t lds = ((size_t)nw * G * CAP + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    hipLaunchKernelGGL((k_dd_fan_bp_tile<G, CAP>), grd, dim3(64, nw), lds, st, g, wprj, img, ns, fbp);
+}
+// groups of 4 slices per lane 1, 2, 4, 8; windows of 32 and 24 bins
+const DdBpQFn kDdBpTile[] = {go_dd_bp_tile<1, 32>, go_dd_bp_tile<1, 24>, go_dd_bp_tile<2, 32>, go_dd_bp_tile<2, 24>,
+                             go_dd_bp_tile<4, 32>, go_dd_bp_tile<4, 24>, go_dd_bp_tile<8, 32>, go_dd_bp_tile<8, 24>};
+
+// Candidates of a kernel with G = 1, 2, 4, 8 groups per lane, two each, in the order
+// of preference for this batch: the fewest groups per lane that hold it first, then
+// fewer; more groups than that last.  Groups are addressed with 32-bit byte offsets:
+// G of them have to fit.
+struct GroupOrder {
+    int idx[8], n = 0;
+    GroupOrder(const FanK& g, int nslices)
+    {
+        const int nquads = cdiv(nslices, 4);
+        auto add = [&](int lg) {
+            if (lg > 0 && ((long)g.nview * g.nu * 16L << lg) >= 0x7fffffffL) return;
+            idx[n++] = 2 * lg;
+            idx[n++] = 2 * lg + 1;
+        };
+        const int best = nquads > 4 ? 3 : nquads > 2 ? 2 : nquads - 1;
+        for (int lg = best; lg >= 0; lg--) add(lg);
+        for (int lg = best + 1; lg < 4; lg++) add(lg);
+    }
+};
 
 // The Siddon and DD gather kernels address one slice's image plane, ray table
 // and sinogram rows with 32-bit byte offsets.
@@ -1582,22 +1587,10 @@ void launch_dd_fan_adj(const FanK& g, const float4* wprj_q, float* img_xy, int n
     const int nquads = cdiv(nslices, 4);
     RN_REQUIRE((long)g.nx * g.ny * 4L < 0x7fffffffL && (long)g.nview * g.nu * 16L < 0x7fffffffL,
                "image plane, ray table or sinogram of one slice exceeds 2 GiB");
-    // candidates in the order of preference for this batch: the fewest groups
-    // per lane that hold it first, then fewer; more groups than that last.
-    // Groups are addressed with 32-bit byte offsets: G of them have to fit.
-    int order[kNDdAdj], n = 0;
-    auto add = [&](int lg) {
-        if (lg > 0 && ((long)g.nview * g.nu * 16L << lg) >= 0x7fffffffL) return;
-        order[n++] = 2 * lg;
-        order[n++] = 2 * lg + 1;
-    };
-    int best = 0;
-    while (best < 3 && (1 << best) < nquads) ++best;
-    for (int lg = best; lg >= 0; --lg) add(lg);
-    for (int lg = best + 1; lg < 4; ++lg) add(lg);
-    const int c = tune_choose({TK_DD_ADJ, g.nx, g.ny, g.nu, g.nview, nslices}, n,
-                              [&](int i) { kDdAdj[order[i]](g, wprj_q, img_xy, nslices, st); }, st, true);
-    kDdAdj[order[c]](g, wprj_q, img_xy, nslices, st);
+    const GroupOrder order(g, nslices);
+    const int c = tune_choose({TK_DD_ADJ, g.nx, g.ny, g.nu, g.nview, nslices}, order.n,
+                              [&](int i) { kDdAdj[order.idx[i]](g, wprj_q, img_xy, nslices, st); }, st, true);
+    kDdAdj[order.idx[c]](g, wprj_q, img_xy, nslices, st);
     check_launch("dd_fan_adj");
 }
 
@@ -1617,6 +1610,20 @@ void launch_dd_fan_bp(const FanK& g, const float* wprj_vu, float* img_xy, int ns
                               [&](int i) { kDdBp[i](g, wprj_vu, img_xy, nslices, fbp ? 1 : 0, st); }, st, true);
     kDdBp[c](g, wprj_vu, img_xy, nslices, fbp ? 1 : 0, st);
     check_launch("dd_fan_bp");
+}
+
+void launch_dd_fan_bp_tile(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, bool fbp, hipStream_t st)
+{
+    if (nslices <= 0) return;
+    require_offsets32(g, g.nview, nslices < 4 ? sizeof(float) : sizeof(float4));
+    const GroupOrder order(g, nslices);
+    // the kernel id of the layout the slices' count had without tiles
+    const int id = nslices < 4 ? (fbp ? TK_DD_FBP : TK_DD_BP) : (fbp ? TK_DD_FBP_Q : TK_DD_BP_Q);
+    const int c = tune_choose({id, g.nx, g.ny, g.nu, g.nview, nslices, 1}, order.n,
+                              [&](int i) { kDdBpTile[order.idx[i]](g, wprj_q, img_xy, nslices, fbp ? 1 : 0, st); }, st,
+                              true);
+    kDdBpTile[order.idx[c]](g, wprj_q, img_xy, nslices, fbp ? 1 : 0, st);
+    check_launch("dd_fan_bp_tile");
 }
 
 void launch_dd_fan_bp_q(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, bool fbp, hipStream_t st)

@@ -72,64 +72,36 @@ __device__ __forceinline__ void seg_acc_rows(const T* const (&rows)[S], unsigned
     }
 }
 
-// seg_acc_rows for G rows staged in LDS: row q of `st` holds bins wlo ..
-// wlo + CAP - 1 (CAP float4 entries).  The first NB bins of the interval are
-// taken without branches (a bin past its end with weight 0, its index
-// clamped into the interval), further bins in a loop.
-template <int G, int CAP, int NB>
-__device__ __forceinline__ void seg_acc_staged(const float4* st, int wlo, int n, float lo, float hi, float scale,
+// acc[q] += k * the integral over [lo, hi] (h0: the end of the row) of row q of G
+// staged rows (CAP entries from st + q CAP, the first one the interval's origin);
+// two bins without branches (a lane that does not meet one takes its first with
+// weight 0), further ones in a loop.
+template <int G, int CAP>
+__device__ __forceinline__ void seg_rel_staged(const float4* st, float lo, float hi, float h0, float k,
                                                float4 (&acc)[G])
 {
-    const float w = hi - lo;
-    const float l = fmaxf(lo, 0.0f), h = fminf(hi, (float)n);
-    const bool normal = h > l;
-    const bool point = !normal && !(w > 0.0f) && lo >= 0.0f && lo < (float)n;
-    // (an interval that reads nothing: m0 = wlo, m1 = wlo - 1, so that no
-    // float outside the int range is converted)
-    const int m0 = normal ? (int)l : (point ? (int)lo : wlo);
-    const int m1 = normal ? min((int)h, n - 1) : (point ? m0 : m0 - 1);
-    const int t0 = m0 - wlo, tl = max(m1 - wlo, 0);
-    const float k = normal ? scale / w : scale;
+    const float l = fmaxf(lo, 0.0f), h = fminf(hi, h0);
+    const bool on0 = h > l;
+    float f = floorf(l);
+    int t = on0 ? (int)f : 0;
+    const float c0 = on0 ? (fminf(h, f + 1.0f) - l) * k : 0.0f;
     #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int m = m0 + j;
-        const bool on = m <= m1;
-        const int t = on ? t0 + j : tl;
-        const float ov = normal ? fminf(h, (float)(m + 1)) - fmaxf(l, (float)m) : 1.0f;
-        const float c = on ? ov * k : 0.0f;
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], c0);
+    f += 1.0f;
+    const bool on1 = on0 && h > f;
+    const float c1 = on1 ? (fminf(h, f + 1.0f) - f) * k : 0.0f;
+    t += on1 ? 1 : 0;
+    #pragma unroll
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], c1);
+    f += 1.0f;
+    if (!on1) return;
+    while (h > f) {
+        ++t;
+        const float c = (fminf(h, f + 1.0f) - f) * k;
         #pragma unroll
         for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], c);
+        f += 1.0f;
     }
-    for (int m = m0 + NB; m <= m1; ++m) {
-        const float pl = fmaxf(l, (float)m), ph = fminf(h, (float)(m + 1));
-        const float c = (ph - pl) * k;
-        #pragma unroll
-        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + m - wlo], c);
-    }
-}
-
-// The bins seg_acc_rows reads for the interval [lo, hi] of a row of n bins:
-// m0 .. m1, or m0 = n, m1 = -1 when it reads none.
-__device__ __forceinline__ void seg_avg_bins(int n, float lo, float hi, int& m0, int& m1)
-{
-    const float w = hi - lo;
-    const float l = fmaxf(lo, 0.0f), h = fminf(hi, (float)n);
-    if (h > l) {
-        m0 = (int)l;
-        m1 = min((int)h, n - 1);
-    } else if (!(w > 0.0f) && lo >= 0.0f && lo < (float)n) {
-        m0 = m1 = (int)lo;
-    } else {
-        m0 = n;
-        m1 = -1;
-    }
-}
-
-// conservative half width (in bins) of the set of rays through a disc of
-// radius r at distance dist from the source:  asin(r/d) <= r/(d-r)
-__device__ __forceinline__ float half_width_bins(float r, float dist, float inv_da)
-{
-    return r * inv_da / fmaxf(dist - r, 1e-3f) + 0.02f;
 }
 
 // ---------------------------------------------------------------------------
@@ -726,6 +698,84 @@ __device__ __forceinline__ float atan_fast(float z)
     float r = p * t;
     if (inv) r = 1.5707963267948966f - r;
     return copysignf(r, z);
+}
+
+// The projection of an 8 x 8-pixel tile onto the detector: its centre's angle
+// th0 and distance r0 from the source once per view in FP64, every other point d
+// of the tile relative to it,
+//     theta(d) = th0 + atan(z),  z = (P dx + Q dy) / (1 + P dy - Q dx),
+// (P, Q) the tangential direction over r0: |z| is about half the tile over r0
+// (FanK::tile: at most 0.1, on the host), so FP32 gives the angle to about 1e-9
+// rad, an absolute bin coordinate in FP32 1e-7.  A wave owns a tile and works out
+// 64 views at a time, one per lane; a view's numbers then reach the wave as
+// scalars (v_readlane).  Bin coordinates are relative to `base`, the first bin the
+// tile can meet; base + span is the last (span < 0: the tile misses the detector).
+constexpr float kTileMax = 0.1f;
+
+// 1/15!, 1/14!, 1/13!, ..., 1/1!, 1/0!: sin and cos from the highest term down, in
+// memory so that the loop over them keeps no registers between batches
+__constant__ const double kTrig[16] = {
+    1.0 / 1307674368000.0, 1.0 / 87178291200.0, 1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0,
+    1.0 / 3628800.0, 1.0 / 362880.0, 1.0 / 40320.0, 1.0 / 5040.0, 1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0,
+    1.0 / 6.0, 1.0 / 2.0, 1.0, 1.0};
+
+struct TileProj {
+    float P, Q;         // per mm
+    float u0;           // bin coordinate of the centre minus base
+    float kr;           // dso^2 / r0^2
+    int base, span;
+    float px, py;       // this lane's pixel from the tile centre, mm
+
+    __device__ __forceinline__ void init(const FanK& g, int lane)
+    {
+        px = ((float)(lane >> 3) - 3.5f) * g.dx;
+        py = ((float)(lane & 7) - 3.5f) * g.dy;
+    }
+    // Views view .. view + 63 (this lane's: view + lane, clamped) of the tile whose
+    // first pixel is (tx, ty); ub: bin coordinate of angle 0; pad: bins added to
+    // the span on either side.
+    __device__ __forceinline__ void batch(const FanK& g, int view, int lane, int tx, int ty, double ub, float pad)
+    {
+        // (opaque, so that nothing of the tile is kept in registers between batches)
+        asm volatile("" : "+s"(tx), "+s"(ty));
+        const int v = min(view + lane, g.nview - 1);
+        const double c = g.vcos[v], s = g.vsin[v];
+        const double x = (tx + 3.5 - 0.5 * (g.nx - 1)) * (double)g.dx, y = (ty + 3.5 - 0.5 * (g.ny - 1)) * (double)g.dy;
+        const double rx = x * c + y * s, d = y * c - x * s + (double)g.dso;
+        const double r2 = rx * rx + d * d;
+        const float ir2 = 1.0f / (float)r2;
+        P = (float)(c * d + s * rx) * ir2;
+        Q = (float)(s * d - c * rx) * ir2;
+        kr = g.dso * g.dso * ir2;
+        // th0: an FP32 estimate t, then the small angle left, (rx cos t - d sin t) / r0,
+        // with sin t and cos t from their Taylor series (|t| < 0.5: terms past t^15
+        // are below 1e-18)
+        const double t = (double)atan_fast<true>((float)rx / (float)d), q = t * t;
+        double sn = kTrig[0], cn = kTrig[1];
+        #pragma unroll 1
+        for (int i = 2; i < 16; i += 2) {
+            sn = fma(sn, -q, kTrig[i]);
+            cn = fma(cn, -q, kTrig[i + 1]);
+        }
+        sn *= t;
+        const double th = t + (double)((float)(rx * cn - d * sn) * sqrtf(ir2));
+        const double u = ub - th / (double)g.da;
+        // the tile's corners lie within |P| 4 dx + |Q| 4 dy of z's numerator, the
+        // denominator within that (with dx and dy exchanged) of 1; atan z <= z
+        const float m = fabsf(P) * 4.0f * g.dx + fabsf(Q) * 4.0f * g.dy;
+        const float n = fabsf(P) * 4.0f * g.dy + fabsf(Q) * 4.0f * g.dx;
+        const double w = (double)(m / ((1.0f - n) * fabsf(g.da)) + pad + 0.02f);
+        const double lo = fmin(fmax(floor(u - w), 0.0), (double)g.nu);
+        const double hi = fmax(fmin(floor(u + w), (double)(g.nu - 1)), -1.0);
+        base = (int)lo;
+        span = (int)hi - base;
+        u0 = (float)(u - lo);
+    }
+};
+
+__device__ __forceinline__ float lane_f(float v, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
 // First and last bin whose centre ray can meet pixel (ix, iy) of view `view`:

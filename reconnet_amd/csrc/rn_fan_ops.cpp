@@ -177,7 +177,7 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
         Q = w.ry.as<float>();
     }
     float* W = w.sino.as<float>();   // [slice][nview][nu]
-    const bool quads = kind == FanBP::Siddon && ns >= 4;   // transposed and interleaved in one pass
+    const bool quads = kind == FanBP::Siddon && ns >= 4 && qplanes_fit32(g.nx, g.ny);   // transposed and interleaved in one pass
     if (kind != FanBP::DDAdjoint && !quads) launch_transpose(Q, W, g.nu, g.nview, ns, st);
     float* out = direct_out ? img_ref : w.rx.as<float>();
     switch (kind) {
@@ -191,7 +191,10 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
             launch_dd_preweight(t.k, W, w.ry.as<float>(), ns, st);
             P = w.ry.as<float>();
         }
-        if (ns >= 4) {
+        if (t.k.tile) {
+            launch_pack_quads(P, w.quad.as<float4>(), nullptr, g.nview, g.nu, ns, false, st);
+            launch_dd_fan_bp_tile(t.k, w.quad.as<float4>(), out, ns, fbp, st);
+        } else if (ns >= 4) {
             // groups of 4 slices interleaved: one float4 load per bin and group
             launch_pack_quads(P, w.quad.as<float4>(), nullptr, g.nview, g.nu, ns, false, st);
             launch_dd_fan_bp_q(t.k, w.quad.as<float4>(), out, ns, fbp, st);
