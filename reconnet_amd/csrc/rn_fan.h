@@ -52,7 +52,8 @@ struct FanK {
     const float4* dray;
     const int* vwide;    // [nview] 1: every Siddon line interval of the view has a positive FP32 width
     int dwide;           // 1: every DD footprint (dray) has a positive FP32 width on every image line
-    int tile;            // 1: the 8 x 8-pixel tiles are small seen from the source (TileProj)
+    int tile;            // 1: the 8 x 8-pixel tiles are small seen from the source (TileRange)
+    int tile_dd;         // 1: tile, and every pixel's DD footprint has a positive width (TileProj)
     int unit_angle;      // 1: |rx / (ry + dso)| < 1 for every pixel centre and view (image well inside the circle)
 };
 
@@ -141,7 +142,7 @@ struct SqsUpd {
     int crop;
 };
 // launch_siddon_fan_bp_q with the update fused into the backprojection's epilogue
-// when the chosen launch shape is one of the LDS-staged ones (returns true; img_xy
+// when the chosen launch shape is a tile one (returns true; img_xy
 // is then not written), else the plain backprojection into img_xy (returns false:
 // the caller applies the update)
 bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* img_xy, int nslices, int view0,
@@ -149,7 +150,7 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
 // reference-parity DD BP of a quad pre-weighted sinogram [q][view][nu] into plain images
 void launch_dd_fan_bp_q(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, bool fbp,
                         hipStream_t st);
-// the same for geometries with FanK::tile, any number of slices (the groups padded)
+// the same for geometries with FanK::tile_dd, any number of slices (the groups padded)
 void launch_dd_fan_bp_tile(const FanK& g, const float4* wprj_q, float* img_xy, int nslices, bool fbp,
                            hipStream_t st);
 // exact DD adjoint of quad sinograms [q][nview][nu] multiplied by the rays' length

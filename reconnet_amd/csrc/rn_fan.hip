@@ -350,151 +350,148 @@ __device__ __forceinline__ bool add_waves(float4 (&v)[G], float4* red, int lane,
     return wv == nw - 1;
 }
 
-// k_siddon_fan_bp_q with each wave's bin window staged in LDS.  Per view the
-// wave's 64 pixels need the bins [wlo, whi] (the lane minimum and maximum of
-// their ranges); the G groups' values and the view's ray table over CAP bins
-// at a time are loaded once per wave with coalesced dwordx4 loads and written
-// to the wave's own LDS rows, from which every pixel gathers its bins: a
-// fraction of the per-pixel gathers' vector-memory traffic.  The first CAP
-// bins of a view are loaded one view ahead into registers; a wider window
-// takes further chunks of CAP bins, loaded in turn (the next view's loads are
-// then issued after them).  Every view runs the one gather code (no branch
-// around the accumulators, which would cost copies of all of them).  A wave
-// touches only its own rows and the LDS instructions of one wave execute in
-// order, so no barrier is needed; the fences keep the compiler from moving
-// LDS accesses across the handovers.  A wave clears its rows at the start, so
-// that a view with an empty window (every lane then takes weight 0 from slot
-// 0) reads zeros or an earlier view's bins, never unwritten memory.  The
-// group rows are addressed as 32-bit byte offsets from the groups' base (the
-// launcher checks that G groups fit).
+// The Siddon BP of an 8 x 8-pixel tile of G interleaved slice groups, for geometries
+// with FanK::tile.  The views are split evenly over the workgroup's nw waves; the
+// waves' sums are added in LDS in wave order.  Per view the tile's bins of the G
+// groups and of the view's ray table, CAP at a time, are loaded once per wave with
+// coalesced dwordx4 loads, issued one step (a view, or a further CAP bins of it) ahead
+// into registers, written to the wave's own LDS rows and gathered from there by every
+// pixel: a fraction of the per-pixel gathers' vector-memory traffic.  One gather
+// code for every step (no branch around the accumulators, which would cost copies
+// of them): the step before the first takes no bin of the cleared rows.  A wave
+// touches only its own rows and the LDS instructions of one wave execute in order, so
+// the steps need no barrier; the fences keep the compiler from moving LDS accesses
+// across the handovers.  The group rows are addressed as 32-bit byte offsets from the
+// groups' base (the launcher checks that G groups fit).
 //
 // UPD: the epilogue applies the OS-SQS update instead of storing the gradient
 // (store_or_update).
-template <int BX, int BY, int NB, int G, int CAP, bool UPD = false>
-__global__ __launch_bounds__(BX * BY, G >= 8 ? 4 : 1) void k_siddon_fan_bp_ql(FanK g, const float4* __restrict__ prj,
-                                                          float* __restrict__ img, int view0, int nviews, int ns,
-                                                          SqsUpd u)
+//
+// Bound: LDS reads (nine per bin with 8 groups, 8 clocks each and shared by four
+// SIMDs) and VALU (about 200 instructions, 64 to 96 of them FMAs).  ms, before (bin
+// ranges per pixel through an atan, window as the lanes' minimum and maximum) ->
+// now: 32 slices of 512^2, 96 views 0.168 -> 0.153; 16 slices, 1152 views 1.50 ->
+// 1.27; 32 slices of 250^2, 360 views 0.40 -> 0.20; 6 slices of 256^2 0.28 -> 0.12.
+extern __shared__ float4 dyn4[];
+
+template <int G, int CAP, bool UPD>
+__global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const float4* __restrict__ prj,
+                                                               float* __restrict__ img, int view0, int nviews, int ns,
+                                                               SqsUpd u)
 {
-    static_assert((BX * BY) % 64 == 0 && CAP <= 64, "whole waves, one load for the ray table row");
+    static_assert(CAP <= 64, "one load for the ray table row");
     // LDS rows 0 .. G - 1: the groups; row G: the ray table
     constexpr int kRows = G + 1, kLoads = (G * CAP + 63) / 64;
-    __shared__ float4 stage[(BX * BY / 64) * kRows * CAP];
-    const int tid = threadIdx.y * BX + threadIdx.x;
-    const int lane = tid & 63;
-    float4* st = stage + (tid >> 6) * kRows * CAP;
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
+    const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
+    float4* st = dyn4 + wv * kRows * CAP;
     for (int i = lane; i < kRows * CAP; i += 64) st[i] = vzero<float4>();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int iy = blockIdx.x * BX + threadIdx.x;
-    const int ix = blockIdx.y * BY + threadIdx.y;
-    const bool inside = ix < g.nx && iy < g.ny;   // lanes outside stage and gather nothing
-    const int nquads = (ns + 3) / 4;
-    const int q0 = blockIdx.z * G;
-    const int nq = min(G, nquads - q0);
+    const bool inside = ix < g.nx && iy < g.ny;   // lanes outside stage but gather nothing
+    const int q0 = blockIdx.z * G, nq = min(G, (ns + 3) / 4 - q0);
     const long sstride = (long)nviews * g.nu;
     const float4* P = prj + q0 * sstride;
-    const int cx = min(ix, g.nx - 1), cy = min(iy, g.ny - 1);
-    const float xc = (cx - 0.5f * (g.nx - 1)) * g.dx, yc = (cy - 0.5f * (g.ny - 1)) * g.dy;
-    const float rpix = 0.5f * sqrtf(g.dx * g.dx + g.dy * g.dy);
-    const float inv_da = 1.0f / g.da;
-    const float yr = (float)cy - 0.5f * g.ny, xr = (float)cx - 0.5f * g.nx;
-    // group staging load j of this lane: element i = 64 j + lane of the group
-    // rows, that is group i / CAP, bin i % CAP of the chunk (LDS slot i), at
-    // byte offset roff[j] + (view row + bin) * 16 from P; the ray table row is
-    // one more load by the first CAP lanes
-    int bj[kLoads];
-    unsigned roff[kLoads];
-    bool has[kLoads];
-    #pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-        const int i = j * 64 + lane, r = i / CAP;
-        bj[j] = i % CAP;
-        has[j] = r < G;
-        roff[j] = (unsigned)(min(r, nq - 1) * sstride) * 16u;
-    }
-    const float4* const sray_v = g.sray + (long)view0 * g.nu;
+    const float4* const sray = g.sray + (long)view0 * g.nu;
+    const float yr = (float)iy - 0.5f * g.ny, xr = (float)ix - 0.5f * g.nx;
     float4 acc[G];
     #pragma unroll
     for (int q = 0; q < G; ++q) acc[q] = vzero<float4>();
+    // staging load j of this lane: element i = 64 j + lane of the group rows, that is
+    // group i / CAP, bin i % CAP of the window (LDS slot i); the ray table row is one
+    // more load by the first CAP lanes
+    int bj[kLoads];
+    unsigned roff[kLoads];
+    #pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+        const int i = j * 64 + lane;
+        bj[j] = i % CAP;
+        roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
+    }
+    TileRange tr;
+    tr.init(g, lane);
     float4 rg[kLoads], rr;
-    // the pixel's bins of view vi (empty outside the image or the detector)
-    auto range = [&](int vi, int& k0, int& k1) {
-        if (g.unit_angle) bin_range<true>(g, xc, yc, rpix, inv_da, view0 + vi, k0, k1);
-        else bin_range<false>(g, xc, yc, rpix, inv_da, view0 + vi, k0, k1);
-        if (!inside || k1 < k0) { k0 = g.nu; k1 = -1; }
-    };
-    // loads of the CAP bins from `base` of view vi, and their LDS handover
-    auto issue = [&](int vi, int base) {
-        #pragma unroll
-        for (int j = 0; j < kLoads; ++j)
-            if (has[j]) rg[j] = ld_at(P, roff[j] + (unsigned)(vi * g.nu + min(base + bj[j], g.nu - 1)) * 16u);
-        if (lane < CAP) rr = ld_at(sray_v, (unsigned)(vi * g.nu + min(base + lane, g.nu - 1)) * 16u);
-    };
-    auto handover = [&]() {
+    int t0 = 0, t1 = -1;   // the step's bins (relative to its first one)
+    float lr = 0.0f, cell = 0.0f;
+    const int v0 = (int)((long)nviews * wv / nw), v1 = (int)((long)nviews * (wv + 1) / nw);
+    int vi = v0 - 1, base = 0, span = -1, off = 0;
+    for (bool more = true;;) {
+        const int a0 = max(t0, 0), a1 = min(t1, CAP - 1);
+        const float l = lr, ce = cell;
+        if (off + CAP <= span) {
+            off += CAP;
+            t0 -= CAP;
+            t1 -= CAP;
+        } else {
+            off = 0;
+            do {
+                more = ++vi < v1;
+                if (!more) break;
+                if (((vi - v0) & 63) == 0) tr.batch(g, view0 + vi, lane, tx, ty, 0.0f);
+                span = __builtin_amdgcn_readlane(tr.span, (vi - v0) & 63);
+            } while (span < 0);
+            if (more) {
+                const int w = (vi - v0) & 63;
+                base = __builtin_amdgcn_readlane(tr.base, w);
+                tr.range(w, span, t0, t1);
+                if (!inside) t1 = -1;
+                const bool xv = g.vcls[view0 + vi] == 0;
+                lr = xv ? yr : xr;
+                cell = xv ? (float)ix : (float)iy;
+            }
+        }
+        if (more) {
+            #pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP)
+                    rg[j] = ld_at(P, roff[j] + (unsigned)(vi * g.nu + min(base + off + bj[j], g.nu - 1)) * 16u);
+            if (lane < CAP) rr = ld_at(sray, (unsigned)(vi * g.nu + min(base + off + lane, g.nu - 1)) * 16u);
+        }
+        siddon_gather_staged<G, CAP>(st, a0, a1, l, ce, acc);
+        if (!more) break;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
         for (int j = 0; j < kLoads; ++j)
-            if (has[j]) st[j * 64 + lane] = rg[j];
+            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane] = rg[j];
         if (lane < CAP) st[G * CAP + lane] = rr;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    };
-    int k0, k1;
-    range(0, k0, k1);
-    int wlo = wave_min(k0), whi = wave_max(k1);
-    if (whi >= wlo) issue(0, wlo);
-    for (int vi = 0; vi < nviews; ++vi) {
-        const bool any = whi >= wlo;
-        const int nch = any ? (whi - wlo) / CAP + 1 : 1;   // an empty window: one chunk of weight-0 reads
-        if (any) handover();
-        int n0 = g.nu, n1 = -1, nlo = g.nu, nhi = -1;
-        if (vi + 1 < nviews) {
-            range(vi + 1, n0, n1);
-            nlo = wave_min(n0);
-            nhi = wave_max(n1);
-        }
-        const bool pre = nhi >= nlo;
-        if (pre && nch == 1) issue(vi + 1, nlo);
-        const int view = view0 + vi;
-        const bool xv = g.vcls[view] == 0;
-        const float lr = xv ? yr : xr;
-        const float cell = xv ? (float)cx : (float)cy;
-        siddon_gather_staged<NB, G, CAP, false>(st, k0 - wlo, min(k1 - wlo, CAP - 1), lr, cell, acc);
-        for (int c = 1; c < nch; ++c) {
-            const int base = wlo + c * CAP;
-            issue(vi, base);
-            handover();
-            siddon_gather_staged<NB, G, CAP, false>(st, max(k0 - base, 0), min(k1 - base, CAP - 1), lr, cell, acc);
-        }
-        if (pre && nch > 1) issue(vi + 1, nlo);
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        k0 = n0; k1 = n1; wlo = nlo; whi = nhi;
     }
-    if (inside) store_or_update<G, UPD>(g, acc, img, u, ix, iy, q0, nq, ns);
+    if (add_waves<G>(acc, dyn4 + nw * kRows * CAP, lane, wv, nw) && inside)
+        store_or_update<G, UPD>(g, acc, img, u, ix, iy, q0, nq, ns);
 }
 
-// Quad-layout Siddon BP for launches with few tiles: an 8 x 8-pixel tile of one
-// group of 4 slices per workgroup, whose VS waves take one part of the views each
-// (gathers from memory, as k_siddon_fan_bp_q); their sums are added in LDS in wave
-// order and the last wave stores or updates.
-//
-// Bound: the latency of a wave's view loop (about 0.7 us per view).  One slice,
-// k_siddon_fan_bp_q -> VS = 4: 256^2, 30 views 23 -> 11 us (1024 -> 4096 waves);
-// 512^2, 96 views 74 -> 67 us, 288 views 254 -> 195 us; and the update is in the
-// epilogue instead of a launch of its own.
-template <int NB, int VS, bool UPD>
-__global__ __launch_bounds__(64 * VS) void k_siddon_fan_bp_qv(FanK g, const float4* __restrict__ prj,
-                                                              float* __restrict__ img, int view0, int nviews, int ns,
-                                                              SqsUpd u)
+// The same for one group of slices, whose bins cost less to gather from memory than
+// to stage (nothing shares a window's loads): 96 views of 512^2 66 us, staged 79;
+// 30 views of 256^2 12 and 14.
+template <bool UPD>
+__global__ __launch_bounds__(512) void k_siddon_fan_bp_tile1(FanK g, const float4* __restrict__ prj,
+                                                             float* __restrict__ img, int view0, int nviews, int ns,
+                                                             SqsUpd u)
 {
-    __shared__ float4 red[64];
-    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int iy = blockIdx.x * 8 + (lane & 7), ix = blockIdx.y * 8 + (lane >> 3), q0 = blockIdx.z;
-    const int v0 = (int)((long)nviews * wv / VS), v1 = (int)((long)nviews * (wv + 1) / VS);
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
+    const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
     const bool inside = ix < g.nx && iy < g.ny;
+    const int q0 = blockIdx.z;
+    const float4* const P[1] = {prj + (long)q0 * nviews * g.nu};
+    const float4* const sray = g.sray + (long)view0 * g.nu;
+    const float yr = (float)iy - 0.5f * g.ny, xr = (float)ix - 0.5f * g.nx;
     float4 acc[1] = {vzero<float4>()};
-    if (inside)
-        siddon_bp_pixel_slices<float4, NB, 1>(g, prj + ((long)q0 * nviews + v0) * g.nu, 0, 1, view0 + v0, v1 - v0, ix,
-                                              iy, acc);
-    if (add_waves<1>(acc, red, lane, wv, VS) && inside) store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
+    TileRange tr;
+    tr.init(g, lane);
+    const int v0 = (int)((long)nviews * wv / nw), v1 = (int)((long)nviews * (wv + 1) / nw);
+    for (int vi = v0; vi < v1; ++vi) {
+        const int w = (vi - v0) & 63;
+        if (w == 0) tr.batch(g, view0 + vi, lane, tx, ty, 0.0f);
+        const int span = __builtin_amdgcn_readlane(tr.span, w);
+        if (span < 0) continue;
+        int t0, t1;
+        tr.range(w, span, t0, t1);
+        if (!inside) t1 = -1;
+        const bool xv = g.vcls[view0 + vi] == 0;
+        const unsigned row = (unsigned)(vi * g.nu + __builtin_amdgcn_readlane(tr.base, w)) * 16u;
+        siddon_gather_bins<float4, 2, 1>(sray, row, P, row, g.nu, t0, t1, xv ? yr : xr, xv ? (float)ix : (float)iy,
+                                         acc);
+    }
+    if (add_waves<1>(acc, dyn4, lane, wv, nw) && inside) store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
 }
 
 // Exact DD adjoint (dd_adj_tile): a workgroup takes an 8 x 8-pixel tile of G
@@ -511,7 +508,6 @@ template <int G, int CAP, bool WIDE>
 __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const float4* __restrict__ wprj,
                                                                    float* __restrict__ img, int ns)
 {
-    extern __shared__ float4 dyn4[];
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
     const int iy = blockIdx.x * 8 + (lane & 7), ix = blockIdx.y * 8 + (lane >> 3);
     const bool inside = ix < g.nx && iy < g.ny;
@@ -542,7 +538,7 @@ __global__ void k_dd_preweight(FanK g, const float* __restrict__ prj, float* __r
     wprj[i] = prj[i] * f;
 }
 
-// Reference-parity DD BP (DDBPFanKernelX/Y) of geometries without FanK::tile: pixel
+// Reference-parity DD BP (DDBPFanKernelX/Y) of geometries without FanK::tile_dd: pixel
 // edges projected through
 // atan, average of the (pre-weighted) detector row over the footprint.  One
 // lane per pixel of S consecutive slices (grid z counts groups of S): the
@@ -624,7 +620,7 @@ __global__ __launch_bounds__(BX * BY) void k_dd_fan_bp_q(FanK g, const float4* _
 // The footprint of the lane's pixel in one view of a TileProj batch (l: the view's
 // lane): [lo, hi] relative to the tile's first bin, between the projections of the
 // pixel's edges along x (X views) or y, and the view's weight over the footprint's
-// width, kr / (r / r0)^2 / (hi - lo) with fbp, else 1 / (hi - lo).  FanK::tile keeps
+// width, kr / (r / r0)^2 / (hi - lo) with fbp, else 1 / (hi - lo).  FanK::tile_dd keeps
 // the width above 1e-3 bins.
 __device__ __forceinline__ void dd_bp_footprint(const FanK& g, const TileProj& tp, int l, int cls, float inv_da, int fbp,
                                                 float& lo, float& hi, float& k)
@@ -634,8 +630,8 @@ __device__ __forceinline__ void dd_bp_footprint(const FanK& g, const TileProj& t
     const float ed = cls == 0 ? -Q * (0.5f * g.dx) : P * (0.5f * g.dy);
     const float num = fmaf(P, tp.px, Q * tp.py), den = fmaf(P, tp.py, fmaf(-Q, tp.px, 1.0f));
     auto bin = [&](float nn, float dd) {
-        const float z = nn * __builtin_amdgcn_rcpf(dd), s = z * z;   // atan z to 2e-8 at |z| = 0.1
-        return fmaf(z * inv_da, -fmaf(s, fmaf(s, 0.2f, -1.0f / 3.0f), 1.0f), u0);
+        const float z = nn * __builtin_amdgcn_rcpf(dd), s = z * z;   // atan z to 5e-9 at |z| = 0.15
+        return fmaf(z * inv_da, -fmaf(s, fmaf(s, fmaf(s, -1.0f / 7.0f, 0.2f), -1.0f / 3.0f), 1.0f), u0);
     };
     const float b1 = bin(num - en, den - ed), b2 = bin(num + en, den + ed);
     lo = fminf(b1, b2);
@@ -645,7 +641,7 @@ __device__ __forceinline__ void dd_bp_footprint(const FanK& g, const TileProj& t
 }
 
 // The DD BP of an 8 x 8-pixel tile of G interleaved slice groups, for geometries
-// with FanK::tile.  The views are split evenly over the workgroup's nw waves; the
+// with FanK::tile_dd.  The views are split evenly over the workgroup's nw waves; the
 // waves' sums are added in LDS in wave order.  Per view the tile's bins of the G
 // groups' pre-weighted rows, CAP at a time, are loaded once per wave with coalesced
 // dwordx4 loads, issued one step (a view, or a further CAP bins of it) ahead into
@@ -667,7 +663,6 @@ template <int G, int CAP>
 __global__ __launch_bounds__(512, 4) void k_dd_fan_bp_tile(FanK g, const float4* __restrict__ wprj,
                                                            float* __restrict__ img, int ns, int fbp)
 {
-    extern __shared__ float4 dyn4[];
     constexpr int kLoads = (G * CAP + 63) / 64;
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
     const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
@@ -709,7 +704,7 @@ __global__ __launch_bounds__(512, 4) void k_dd_fan_bp_tile(FanK g, const float4*
             do {
                 more = ++view < v1;
                 if (!more) break;
-                if (((view - v0) & 63) == 0) tp.batch(g, view, lane, tx, ty, 0.5 * g.nu - (double)g.off_a, 0.0f);
+                if (((view - v0) & 63) == 0) tp.batch(g, view, lane, tx, ty, 0.5 * g.nu - (double)g.off_a);
                 span = __builtin_amdgcn_readlane(tp.span, (view - v0) & 63);
             } while (span < 0);
             if (more) {
@@ -1108,12 +1103,15 @@ void FanTables::build(const FanGeo& g, const float* deg_host, hipStream_t st)
     const double R = 0.5 * std::sqrt((double)g.nx * g.dx * g.nx * g.dx + (double)g.ny * g.dy * g.ny * g.dy);
     k.unit_angle = R < 0.45 * (double)g.dso ? 1 : 0;
     // the tiles' points (an incomplete tile reaches over the image) lie within Rt of the
-    // centre: half a tile over their distance from the source at most kTileMax, and
-    // the footprint of half a pixel, at least cos(72 deg) of it across the ray
-    // (45 deg of view, 27 of fan), over 1e-3 bins
+    // centre: half a tile over their distance from the source at most 1/4; and for DD
+    // at most kTileMax, and the footprint of a pixel, cos(45 deg of view + the fan's angle) of it across
+    // the ray, over 1e-3 bins
     const double hx = 4.0 * g.dx, hy = 4.0 * g.dy, ht = std::sqrt(hx * hx + hy * hy), Rt = R + 2.0 * ht;
-    k.tile = Rt < 0.45 * (double)g.dso && ht <= fan::kTileMax * ((double)g.dso - Rt) &&
-             0.3 * std::min(g.dx, g.dy) >= 1e-3 * std::fabs((double)g.da) * ((double)g.dso + Rt) ? 1 : 0;
+    const double dso = (double)g.dso;
+    k.tile = Rt < 0.9 * dso && ht <= 0.25 * (dso - Rt) ? 1 : 0;
+    k.tile_dd = k.tile && ht <= fan::kTileMax * (dso - Rt) &&
+                        std::cos(0.7854 + std::asin(Rt / dso)) * std::min(g.dx, g.dy) >=
+                              1e-3 * std::fabs((double)g.da) * (dso + Rt) ? 1 : 0;
 }
 
 bool FanTables::matches(const FanGeo& g, const float* deg_host) const
@@ -1340,37 +1338,6 @@ void go_siddon_bp_q(const FanK& g, const float4* prj, float* img, int ns, int vi
                        dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns);
 }
 
-template <int BX, int BY, int NB, int G, int CAP>
-void go_siddon_bp_ql(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_siddon_fan_bp_ql<BX, BY, NB, G, CAP>),
-                       dim3(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(cdiv(ns, 4), G)), dim3(BX, BY), 0, st, g, prj, img,
-                       view0, nviews, ns, SqsUpd{});
-}
-
-template <int NB, int VS>
-void go_siddon_bp_qv(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_siddon_fan_bp_qv<NB, VS, false>), dim3(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(ns, 4)),
-                       dim3(64, VS), 0, st, g, prj, img, view0, nviews, ns, SqsUpd{});
-}
-
-template <int NB, int VS>
-void go_siddon_bp_qvu(const FanK& g, const float4* prj, int ns, int view0, int nviews, const SqsUpd& u, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_siddon_fan_bp_qv<NB, VS, true>), dim3(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(ns, 4)),
-                       dim3(64, VS), 0, st, g, prj, nullptr, view0, nviews, ns, u);
-}
-
-template <int BX, int BY, int NB, int G, int CAP>
-void go_siddon_bp_qlu(const FanK& g, const float4* prj, int ns, int view0, int nviews, const SqsUpd& u,
-                      hipStream_t st)
-{
-    hipLaunchKernelGGL((k_siddon_fan_bp_ql<BX, BY, NB, G, CAP, true>),
-                       dim3(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(cdiv(ns, 4), G)), dim3(BX, BY), 0, st, g, prj,
-                       nullptr, view0, nviews, ns, u);
-}
-
 using SidFpQFn = void (*)(const FanK&, const float4*, const float4*, float4*, int, int, int, const float4*,
                           const float4*, int, int, hipStream_t);
 using SidBpQFn = void (*)(const FanK&, const float4*, float*, int, int, int, hipStream_t);
@@ -1393,43 +1360,66 @@ const SidFpQPFn kSidFpQP[] = {go_siddon_fp_qp<64, kXcds, 1, 2>,  go_siddon_fp_qp
                               go_siddon_fp_qp<128, kXcds, 2>,    go_siddon_fp_qp<64, kXcds, 2, 2>,
                               go_siddon_fp_qp<128, kXcds, 2, 2>, go_siddon_fp_qp<128, 0, 2>};
 constexpr int kNSidFpQP = sizeof(kSidFpQP) / sizeof(kSidFpQP[0]);
-const SidBpQFn kSidBpQ[] = {go_siddon_bp_ql<8, 8, 2, 8, 24>,  go_siddon_bp_ql<8, 32, 2, 8, 24>,
-                            go_siddon_bp_ql<8, 8, 2, 8, 32>,  go_siddon_bp_ql<8, 8, 2, 8, 21>,
-                            go_siddon_bp_ql<8, 8, 2, 8, 16>,  go_siddon_bp_ql<8, 8, 2, 4, 24>,
-                            go_siddon_bp_ql<8, 8, 2, 2, 32>,
-                            go_siddon_bp_q<16, 16, 2, 8>,     go_siddon_bp_q<8, 8, 2, 8>,
-                            go_siddon_bp_q<16, 16, 2, 4>,     go_siddon_bp_q<8, 8, 2, 4>,
-                            go_siddon_bp_q<8, 8, 2, 2>,       go_siddon_bp_q<16, 16, 2, 2>,
-                            go_siddon_bp_q<8, 8, 2, 1>,       go_siddon_bp_q<16, 16, 2, 1>,
-                            go_siddon_bp_q<8, 8, 3, 4>,       go_siddon_bp_q<8, 8, 3, 2>,
-                            go_siddon_bp_qv<2, 4>,            go_siddon_bp_qv<2, 8>,
-                            go_siddon_bp_qv<2, 2>};
+// per-pixel gathers, for every geometry
+const SidBpQFn kSidBpQ[] = {go_siddon_bp_q<16, 16, 2, 8>, go_siddon_bp_q<8, 8, 2, 8>, go_siddon_bp_q<16, 16, 2, 4>,
+                            go_siddon_bp_q<8, 8, 2, 4>,   go_siddon_bp_q<8, 8, 2, 2>, go_siddon_bp_q<16, 16, 2, 2>,
+                            go_siddon_bp_q<8, 8, 2, 1>,   go_siddon_bp_q<16, 16, 2, 1>, go_siddon_bp_q<8, 8, 3, 4>,
+                            go_siddon_bp_q<8, 8, 3, 2>};
 constexpr int kNSidFpQ = sizeof(kSidFpQ) / sizeof(kSidFpQ[0]);
 constexpr int kNSidBpQ = sizeof(kSidBpQ) / sizeof(kSidBpQ[0]);
-constexpr int kNSidBpStaged = 7;   // the first seven are k_siddon_fan_bp_ql
-constexpr int kNSidBpSplit = 3;    // the last three k_siddon_fan_bp_qv
-using SidBpQUFn = void (*)(const FanK&, const float4*, int, int, int, const SqsUpd&, hipStream_t);
-// the staged shapes of kSidBpQ, in the same order, with the OS-SQS update in the epilogue
-const SidBpQUFn kSidBpQU[kNSidBpStaged] = {
-    go_siddon_bp_qlu<8, 8, 2, 8, 24>, go_siddon_bp_qlu<8, 32, 2, 8, 24>, go_siddon_bp_qlu<8, 8, 2, 8, 32>,
-    go_siddon_bp_qlu<8, 8, 2, 8, 21>, go_siddon_bp_qlu<8, 8, 2, 8, 16>, go_siddon_bp_qlu<8, 8, 2, 4, 24>,
-    go_siddon_bp_qlu<8, 8, 2, 2, 32>};
-const SidBpQUFn kSidBpQVU[kNSidBpSplit] = {go_siddon_bp_qvu<2, 4>, go_siddon_bp_qvu<2, 8>, go_siddon_bp_qvu<2, 2>};
 
-// Candidate i of the interleaved BP for this launch: in listed order, or for one
-// group of slices the view-split shapes first (the staged shapes carry up to 8
-// groups per lane: 43 against 10 us for one slice of 256^2, 30 views); the
-// staged shapes only where 8 groups' rows fit 32-bit offsets.
+using SidBpTileFn = void (*)(const FanK&, const float4*, float*, int, int, int, const SqsUpd*, hipStream_t);
+// u != nullptr: the OS-SQS update in the epilogue instead of img
+template <int G, int CAP>
+void go_siddon_bp_tile(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, const SqsUpd* u,
+                       hipStream_t st)
+{
+    const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
+    // Waves per tile: up to 8 while they do not fill the chip (4096 of 4 and more
+    // groups, 4 a SIMD by their registers; more of the shorter ones of 1 and 2 groups)
+    // and each keeps 8 views, over which its batch of tile projections pays.  us with
+    // nw = 1, 2, 4, 8: one slice of 256^2, 30 views 23, 15, 12, 12, 360 views 279, 184,
+    // 133, 87; 5 slices of 512^2 (G = 2), 1152 views 1117, 1088, 941, 966; 32 slices of
+    // 250^2 (G = 8), 360 views 438, 251, 200, 255; of 512^2, 96 views 153, 177, 170, 202.
+    const long full = G <= 2 ? 16384 : 4096;
+    int nw = 1;
+    while (nw < 8 && (long)grd.x * grd.y * grd.z * nw < full && nviews >= 8 * nw) nw *= 2;
+    const size_t lds = ((G == 1 ? 0 : (size_t)nw * (G + 1) * CAP) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    const SqsUpd upd = u != nullptr ? *u : SqsUpd{};
+    void (*k)(FanK, const float4*, float*, int, int, int, SqsUpd);
+    if constexpr (G == 1) k = u != nullptr ? k_siddon_fan_bp_tile1<true> : k_siddon_fan_bp_tile1<false>;
+    else k = u != nullptr ? k_siddon_fan_bp_tile<G, CAP, true> : k_siddon_fan_bp_tile<G, CAP, false>;
+    hipLaunchKernelGGL(k, grd, dim3(64, nw), lds, st, g, prj, img, view0, nviews, ns, upd);
+}
+constexpr int kNSidBpTile = 7;
+const SidBpTileFn kSidBpTile[kNSidBpTile] = {
+    go_siddon_bp_tile<1, 32>, go_siddon_bp_tile<2, 32>, go_siddon_bp_tile<2, 24>, go_siddon_bp_tile<4, 24>,
+    go_siddon_bp_tile<4, 32>, go_siddon_bp_tile<8, 24>, go_siddon_bp_tile<8, 32>};
+
+// Candidate i of the interleaved BP for this launch: the tile shapes (FanK::tile), the
+// fewest groups per lane that hold the batch first, then fewer, then more, where G
+// groups' rows fit 32-bit offsets; then the gathers, at kNSidBpTile + their index.
 struct SidBpOrder {
-    int first, n, shift;
+    int idx[kNSidBpTile + kNSidBpQ], n = 0;
     SidBpOrder(const FanK& g, int nslices, int nviews)
     {
-        first = 9L * nviews * g.nu * 16L < 0x7fffffffL ? 0 : kNSidBpStaged;
-        n = kNSidBpQ - first;
-        shift = nslices <= 4 ? n - kNSidBpSplit : 0;
+        const int nquads = cdiv(nslices, 4);
+        auto add = [&](int lg) {
+            if (!g.tile || (long)(1 << lg) * nviews * g.nu * 16L >= 0x7fffffffL) return;
+            for (int i = lg == 0 ? 0 : 2 * lg - 1; i <= 2 * lg; i++) idx[n++] = i;
+        };
+        const int best = nquads > 4 ? 3 : nquads > 2 ? 2 : nquads - 1;
+        for (int lg = best; lg >= 0; lg--) add(lg);
+        for (int lg = best + 1; lg < 4; lg++) add(lg);
+        for (int i = 0; i < kNSidBpQ; i++) idx[n++] = kNSidBpTile + i;
     }
-    int operator[](int i) const { return first + (i + shift) % n; }
 };
+
+void go_siddon_bp_any(int c, const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
+{
+    if (c < kNSidBpTile) kSidBpTile[c](g, prj, img, ns, view0, nviews, nullptr, st);
+    else kSidBpQ[c - kNSidBpTile](g, prj, img, ns, view0, nviews, st);
+}
 
 } // namespace
 
@@ -1515,10 +1505,10 @@ void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, i
     if (nslices <= 0 || nviews <= 0) return;
     require_offsets32(g, nviews, sizeof(float4));
     const SidBpOrder order(g, nslices, nviews);
-    const int c = order[tune_choose({TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, 1}, order.n,
-                                    [&](int i) { kSidBpQ[order[i]](g, prj_q, img_xy, nslices, view0, nviews, st); }, st,
-                                    true)];
-    kSidBpQ[c](g, prj_q, img_xy, nslices, view0, nviews, st);
+    const int c = order.idx[tune_choose({TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, 1}, order.n, [&](int i) {
+        go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
+    }, st, true)];
+    go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, st);
     check_launch("siddon_fan_bp_q");
 }
 
@@ -1529,22 +1519,14 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
     require_offsets32(g, nviews, sizeof(float4));
     const SidBpOrder order(g, nslices, nviews);
     // the launch shape is tuned on the plain backprojection (img_xy as its output)
-    const int c = order[tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, order.n,
-                                    [&](int i) { kSidBpQ[order[i]](g, prj_q, img_xy, nslices, view0, nviews, st); }, st,
-                                    true)];
-    if (c >= kNSidBpQ - kNSidBpSplit) {
-        kSidBpQVU[c - (kNSidBpQ - kNSidBpSplit)](g, prj_q, nslices, view0, nviews, u, st);
-        check_launch("siddon_fan_bp_q_update");
-        return true;
-    }
-    if (c < kNSidBpStaged) {
-        kSidBpQU[c](g, prj_q, nslices, view0, nviews, u, st);
-        check_launch("siddon_fan_bp_q_update");
-        return true;
-    }
-    kSidBpQ[c](g, prj_q, img_xy, nslices, view0, nviews, st);
-    check_launch("siddon_fan_bp_q");
-    return false;
+    const int c = order.idx[tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, order.n, [&](int i) {
+        go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
+    }, st, true)];
+    const bool fused = c < kNSidBpTile;
+    if (fused) kSidBpTile[c](g, prj_q, nullptr, nslices, view0, nviews, &u, st);
+    else go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, st);
+    check_launch("siddon_fan_bp_q_update");
+    return fused;
 }
 
 void launch_siddon_fan_fp_f64(const FanK& g, const double* Pyx, const double* Pxy, double* prj_vu,

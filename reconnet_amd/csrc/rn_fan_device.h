@@ -701,16 +701,15 @@ __device__ __forceinline__ float atan_fast(float z)
 }
 
 // The projection of an 8 x 8-pixel tile onto the detector: its centre's angle
-// th0 and distance r0 from the source once per view in FP64, every other point d
-// of the tile relative to it,
+// th0 and distance r0 from the source once per view, every other point d of the
+// tile relative to it,
 //     theta(d) = th0 + atan(z),  z = (P dx + Q dy) / (1 + P dy - Q dx),
 // (P, Q) the tangential direction over r0: |z| is about half the tile over r0
-// (FanK::tile: at most 0.1, on the host), so FP32 gives the angle to about 1e-9
-// rad, an absolute bin coordinate in FP32 1e-7.  A wave owns a tile and works out
-// 64 views at a time, one per lane; a view's numbers then reach the wave as
-// scalars (v_readlane).  Bin coordinates are relative to `base`, the first bin the
-// tile can meet; base + span is the last (span < 0: the tile misses the detector).
-constexpr float kTileMax = 0.1f;
+// (at most 1/4 with FanK::tile, kTileMax with FanK::tile_dd).  A wave owns a tile and works out 64 views
+// at a time, one per lane; a view's numbers then reach the wave as scalars
+// (v_readlane).  Bin coordinates are relative to `base`, the first bin the tile can
+// meet; base + span is the last (span < 0: the tile misses the detector).
+constexpr float kTileMax = 0.15f;
 
 // 1/15!, 1/14!, 1/13!, ..., 1/1!, 1/0!: sin and cos from the highest term down, in
 // memory so that the loop over them keeps no registers between batches
@@ -719,6 +718,13 @@ __constant__ const double kTrig[16] = {
     1.0 / 3628800.0, 1.0 / 362880.0, 1.0 / 40320.0, 1.0 / 5040.0, 1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0,
     1.0 / 6.0, 1.0 / 2.0, 1.0, 1.0};
 
+__device__ __forceinline__ float lane_f(float v, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// The tile's points to FP32 accuracy relative to a centre angle in FP64: an angle
+// to about 1e-9 rad (an absolute bin coordinate in FP32 has 1e-7).
 struct TileProj {
     float P, Q;         // per mm
     float u0;           // bin coordinate of the centre minus base
@@ -732,9 +738,8 @@ struct TileProj {
         py = ((float)(lane & 7) - 3.5f) * g.dy;
     }
     // Views view .. view + 63 (this lane's: view + lane, clamped) of the tile whose
-    // first pixel is (tx, ty); ub: bin coordinate of angle 0; pad: bins added to
-    // the span on either side.
-    __device__ __forceinline__ void batch(const FanK& g, int view, int lane, int tx, int ty, double ub, float pad)
+    // first pixel is (tx, ty); ub: bin coordinate of angle 0.
+    __device__ __forceinline__ void batch(const FanK& g, int view, int lane, int tx, int ty, double ub)
     {
         // (opaque, so that nothing of the tile is kept in registers between batches)
         asm volatile("" : "+s"(tx), "+s"(ty));
@@ -748,9 +753,9 @@ struct TileProj {
         Q = (float)(s * d - c * rx) * ir2;
         kr = g.dso * g.dso * ir2;
         // th0: an FP32 estimate t, then the small angle left, (rx cos t - d sin t) / r0,
-        // with sin t and cos t from their Taylor series (|t| < 0.5: terms past t^15
-        // are below 1e-18)
-        const double t = (double)atan_fast<true>((float)rx / (float)d), q = t * t;
+        // with sin t and cos t from their Taylor series (|t| < 1.2: terms past t^15
+        // are below 1e-12)
+        const double t = (double)atan_fast<false>((float)rx / (float)d), q = t * t;
         double sn = kTrig[0], cn = kTrig[1];
         #pragma unroll 1
         for (int i = 2; i < 16; i += 2) {
@@ -764,7 +769,7 @@ struct TileProj {
         // denominator within that (with dx and dy exchanged) of 1; atan z <= z
         const float m = fabsf(P) * 4.0f * g.dx + fabsf(Q) * 4.0f * g.dy;
         const float n = fabsf(P) * 4.0f * g.dy + fabsf(Q) * 4.0f * g.dx;
-        const double w = (double)(m / ((1.0f - n) * fabsf(g.da)) + pad + 0.02f);
+        const double w = (double)(m / ((1.0f - n) * fabsf(g.da)) + 0.02f);
         const double lo = fmin(fmax(floor(u - w), 0.0), (double)g.nu);
         const double hi = fmax(fmin(floor(u + w), (double)(g.nu - 1)), -1.0);
         base = (int)lo;
@@ -773,10 +778,62 @@ struct TileProj {
     }
 };
 
-__device__ __forceinline__ float lane_f(float v, int l)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
+// The bins whose centre rays can meet each of the tile's pixels (a superset; the
+// others have weight 0): centre coordinate u0 - m (1 - n), m and n the numerator
+// and denominator of z in bins, to the second order, and one half width per view
+// that covers the pixel's box, the remainder's bound and FP32.
+struct TileRange {
+    float P, Q;         // bins per mm
+    float u0, hw;
+    int base, span;
+    float px, py, qx, qy;   // this lane's pixel from the tile centre, mm and mm x da
+
+    __device__ __forceinline__ void init(const FanK& g, int lane)
+    {
+        px = ((float)(lane >> 3) - 3.5f) * g.dx;
+        py = ((float)(lane & 7) - 3.5f) * g.dy;
+        qx = px * g.da;
+        qy = py * g.da;
+    }
+    // as TileProj::batch; pad: further bins on either side
+    __device__ __forceinline__ void batch(const FanK& g, int view, int lane, int tx, int ty, float pad)
+    {
+        asm volatile("" : "+s"(tx), "+s"(ty));
+        const int v = min(view + lane, g.nview - 1);
+        const float c = g.vcos[v], s = g.vsin[v], ida = 1.0f / g.da;
+        const float x = ((float)tx + 3.5f - 0.5f * (float)(g.nx - 1)) * g.dx;
+        const float y = ((float)ty + 3.5f - 0.5f * (float)(g.ny - 1)) * g.dy;
+        const float rx = x * c + y * s, d = y * c - x * s + g.dso;
+        const float ir2 = 1.0f / fmaf(rx, rx, d * d);
+        P = (c * d + s * rx) * ir2;
+        Q = (s * d - c * rx) * ir2;
+        const float u = g.cu - g.off_a - atan_fast<false>(rx / d) * ida;
+        const float m = fabsf(P) * 4.0f * g.dx + fabsf(Q) * 4.0f * g.dy;
+        const float n = fabsf(P) * 4.0f * g.dy + fabsf(Q) * 4.0f * g.dx;
+        const float zm = m / (1.0f - n), a = fabsf(ida);
+        // FP32: the angle to RN_ATAN_FAST_ERR and 1e-6 of its rounded operands, the bin
+        // coordinate to 1e-6 of its size
+        const float eps = 0.02f + pad + (RN_ATAN_FAST_ERR + 1e-6f) * a + 1e-6f * (float)g.nu;
+        hw = 0.125f * zm * a + (n * n * zm + zm * zm * zm) * a + eps;
+        const float w = zm * a + eps;
+        const float lo = fminf(fmaxf(floorf(u - w), 0.0f), (float)g.nu);
+        const float hi = fmaxf(fminf(floorf(u + w), (float)(g.nu - 1)), -1.0f);
+        base = (int)lo;
+        span = (int)hi - base;
+        u0 = u - lo;
+        P *= ida;
+        Q *= ida;
+    }
+    // this lane's first and last bin, relative to base, in the view of lane l
+    __device__ __forceinline__ void range(int l, int span_l, int& t0, int& t1) const
+    {
+        const float p = lane_f(P, l), q = lane_f(Q, l), h = lane_f(hw, l);
+        const float m = fmaf(p, px, q * py), n1 = fmaf(p, qy, fmaf(-q, qx, -1.0f));
+        const float u = fmaf(m, n1, lane_f(u0, l));
+        t0 = max((int)ceilf(u - h), 0);
+        t1 = min((int)floorf(u + h), span_l);
+    }
+};
 
 // First and last bin whose centre ray can meet pixel (ix, iy) of view `view`:
 // the pixel lies in the disc of radius rpix around its centre, whose rays span
@@ -798,20 +855,14 @@ __device__ __forceinline__ void bin_range(const FanK& g, float xc, float yc, flo
 }
 
 // Length of ray r in cell `cell` of line lr (the weight siddon_fp_ray gives
-// it), computed without branches.  WIDE: the interval's FP32 width is known to
-// be positive (no zero-width case to select; the same value as the general
-// form then).
-template <bool WIDE>
+// it), computed without branches: overlap and width of the interval between the
+// line's crossings ea and eb (both have the sign of eb - ea).
 __device__ __forceinline__ float siddon_cell_weight(const float4 r, float lr, float cell)
 {
-    const float ea = fmaf(r.y, lr, r.x), eb = fmaf(r.y, lr + 1.0f, r.x);
-    const float lo = fminf(ea, eb), hi = fmaxf(ea, eb), w = hi - lo;
-    const float ov = fmaxf(fminf(hi, cell + 1.0f) - fmaxf(lo, cell), 0.0f);
-    if (WIDE) return ov * __builtin_amdgcn_rcpf(w) * r.z;
-    const bool pos = w > 0.0f;
-    const float pt = (lo >= cell && lo < cell + 1.0f) ? 1.0f : 0.0f;
-    const float inv = __builtin_amdgcn_rcpf(pos ? w : 1.0f);
-    return (pos ? ov * inv : pt) * r.z;
+    const float ea = fmaf(r.y, lr, r.x), eb = fmaf(r.y, lr + 1.0f, r.x), c1 = cell + 1.0f;
+    const float ov = __builtin_amdgcn_fmed3f(eb, cell, c1) - __builtin_amdgcn_fmed3f(ea, cell, c1);
+    const float pt = (ea >= cell && ea < c1) ? 1.0f : 0.0f;
+    return (ea != eb ? ov * __builtin_amdgcn_rcpf(eb - ea) : pt) * r.z;
 }
 
 // the bins k0 .. k1 of one view for S slices (slice q's row `rboff` bytes
@@ -830,14 +881,14 @@ __device__ __forceinline__ void siddon_gather_bins(const float4* __restrict__ sr
         // cost no vector-memory bandwidth); the others add weight x value
         if (k0 + j <= k1) {
             const unsigned kk = (unsigned)(k0 + j);
-            const float wt = siddon_cell_weight<false>(ld_at(sray, rowoff + kk * 16u), lr, cell);
+            const float wt = siddon_cell_weight(ld_at(sray, rowoff + kk * 16u), lr, cell);
             const unsigned boff = rboff + kk * (unsigned)sizeof(T);
             #pragma unroll
             for (int q = 0; q < S; ++q) vmadd(acc[q], ld_at(pq[q], boff), wt);
         }
     }
     for (int k = k0 + NB; k <= k1; ++k) {
-        const float wt = siddon_cell_weight<false>(ld_at(sray, rowoff + (unsigned)k * 16u), lr, cell);
+        const float wt = siddon_cell_weight(ld_at(sray, rowoff + (unsigned)k * 16u), lr, cell);
         const unsigned boff = rboff + (unsigned)k * (unsigned)sizeof(T);
         #pragma unroll
         for (int q = 0; q < S; ++q) vmadd(acc[q], ld_at(pq[q], boff), wt);
@@ -848,26 +899,27 @@ __device__ __forceinline__ void siddon_gather_bins(const float4* __restrict__ sr
 // row q of `st` holds group q's values and row G the view's ray table, CAP
 // bins per row from the window's first bin (every slot holds written values:
 // the caller clears the rows before its first window); t0 .. t1 are the pixel's bins
-// relative to that first bin.  The first NB bins are taken by every lane with
+// relative to that first bin.  The first two bins are taken by every lane with
 // no branch around the accumulators: a lane past t1 reads slot 0 (a bin of
 // this view's window) with weight 0, which keeps the kernel in registers.
 // The rest in a loop.
-template <int NB, int G, int CAP, bool WIDE>
+template <int G, int CAP>
 __device__ __forceinline__ void siddon_gather_staged(const float4* st, int t0, int t1, float lr, float cell,
                                                      float4 (&acc)[G])
 {
+    const bool on0 = t0 <= t1, on1 = t0 < t1;
+    const int i0 = on0 ? t0 : 0, i1 = on1 ? t0 + 1 : 0;
+    const float c0 = siddon_cell_weight(st[G * CAP + i0], lr, cell);
+    const float c1 = siddon_cell_weight(st[G * CAP + i1], lr, cell);
+    const float w0 = on0 ? c0 : 0.0f, w1 = on1 ? c1 : 0.0f;
     #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const bool on = t0 + j <= t1;
-        const int t = on ? t0 + j : 0;
-        const float wt = on ? siddon_cell_weight<WIDE>(st[G * CAP + t], lr, cell) : 0.0f;
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + i0], w0);
+    #pragma unroll
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + i1], w1);
+    for (int t = t0 + 2; t <= t1; ++t) {
+        const float w = siddon_cell_weight(st[G * CAP + t], lr, cell);
         #pragma unroll
-        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], wt);
-    }
-    for (int t = t0 + NB; t <= t1; ++t) {
-        const float wt = siddon_cell_weight<WIDE>(st[G * CAP + t], lr, cell);
-        #pragma unroll
-        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], wt);
+        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], w);
     }
 }
 

@@ -191,7 +191,7 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
             launch_dd_preweight(t.k, W, w.ry.as<float>(), ns, st);
             P = w.ry.as<float>();
         }
-        if (t.k.tile) {
+        if (t.k.tile_dd) {
             launch_pack_quads(P, w.quad.as<float4>(), nullptr, g.nview, g.nu, ns, false, st);
             launch_dd_fan_bp_tile(t.k, w.quad.as<float4>(), out, ns, fbp, st);
         } else if (ns >= 4) {
