@@ -411,12 +411,12 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
     tr.init(g, lane);
     float4 rg[kLoads], rr;
     int t0 = 0, t1 = -1;   // the step's bins (relative to its first one)
-    float lr = 0.0f, cell = 0.0f;
+    bool xv = true;
     const int v0 = (int)((long)nviews * wv / nw), v1 = (int)((long)nviews * (wv + 1) / nw);
     int vi = v0 - 1, base = 0, span = -1, off = 0;
     for (bool more = true;;) {
         const int a0 = max(t0, 0), a1 = min(t1, CAP - 1);
-        const float l = lr, ce = cell;
+        const float lr = xv ? yr : xr, cell = xv ? xr + 0.5f * g.nx : yr + 0.5f * g.ny;
         if (off + CAP <= span) {
             off += CAP;
             t0 -= CAP;
@@ -434,9 +434,7 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
                 base = __builtin_amdgcn_readlane(tr.base, w);
                 tr.range(w, span, t0, t1);
                 if (!inside) t1 = -1;
-                const bool xv = g.vcls[view0 + vi] == 0;
-                lr = xv ? yr : xr;
-                cell = xv ? (float)ix : (float)iy;
+                xv = g.vcls[view0 + vi] == 0;
             }
         }
         if (more) {
@@ -446,7 +444,7 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
                     rg[j] = ld_at(P, roff[j] + (unsigned)(vi * g.nu + min(base + off + bj[j], g.nu - 1)) * 16u);
             if (lane < CAP) rr = ld_at(sray, (unsigned)(vi * g.nu + min(base + off + lane, g.nu - 1)) * 16u);
         }
-        siddon_gather_staged<G, CAP>(st, a0, a1, l, ce, acc);
+        siddon_gather_staged<G, CAP>(st, a0, a1, lr, cell, acc);
         if (!more) break;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
@@ -495,31 +493,27 @@ __global__ __launch_bounds__(512) void k_siddon_fan_bp_tile1(FanK g, const float
 }
 
 // Exact DD adjoint (dd_adj_tile): a workgroup takes an 8 x 8-pixel tile of G
-// groups of 4 slices with 1 wave, or with kDdAdjSegs waves that walk one view
-// segment each (tiles x groups too few to fill the chip); the segments' sums
-// are added in LDS in segment order, the order of the one-wave shape.
+// groups of 4 slices with kDdAdjSegs waves that walk one view segment each; their
+// sums are added in LDS in segment order.
 //
-// Bound: VALU (about 100 instructions per wave and view for the bin range, its
-// window and the staging, 20 per candidate bin and 4 per bin and group).  32
-// slices of 256^2, 360 views, 512 bins: 0.44 ms (1.69 ms with per-slice gathers
-// from memory, S slices per lane); one slice 0.12 ms; one slice of 128^2, 180
-// views 32 us (256 us).
+// Bound: VALU and LDS reads (per wave and view about 60 instructions for the bin
+// range and the staging, 20 per candidate bin and 4 per bin and group).  ms, per-slice
+// gathers from memory -> bin ranges per pixel through an atan -> now: 32 slices of
+// 256^2, 360 views, 512 bins 1.69 -> 0.41 -> 0.28; of 512^2, 1152 views 16.2 -> 3.1 ->
+// 2.4; one slice of 256^2 0.65 -> 0.122 -> 0.109.
 template <int G, int CAP, bool WIDE>
 __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const float4* __restrict__ wprj,
                                                                    float* __restrict__ img, int ns)
 {
-    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
-    const int iy = blockIdx.x * 8 + (lane & 7), ix = blockIdx.y * 8 + (lane >> 3);
-    const bool inside = ix < g.nx && iy < g.ny;
-    const int nquads = (ns + 3) / 4;
-    const int q0 = blockIdx.z * G;
-    const int nq = min(G, nquads - q0);
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int ty = blockIdx.x * 8, tx = blockIdx.y * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
+    const int q0 = blockIdx.z * G, nq = min(G, (ns + 3) / 4 - q0);
     const long sstride = (long)g.nview * g.nu;
-    const int per = kDdAdjSegs / nw;
     float4 tot[G];
-    dd_adj_tile<G, CAP, 3, WIDE>(g, wprj + q0 * sstride, sstride, nq, 0, g.nview, wv * per, (wv + 1) * per, ix, iy,
-                                 inside, lane, dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
-    if (add_waves<G>(tot, dyn4 + nw * DdAdjStage<G, CAP>::kFloat4, lane, wv, nw) && inside)
+    dd_adj_tile<G, CAP, 3, WIDE, true>(g, wprj + q0 * sstride, sstride, nq, 0, g.nview, wv, wv + 1, tx, ty, lane,
+                                       dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
+    if (add_waves<G>(tot, dyn4 + kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4, lane, wv, kDdAdjSegs) && ix < g.nx &&
+        iy < g.ny)
         store_or_update<G, false>(g, tot, img, SqsUpd{}, ix, iy, q0, nq, ns);
 }
 
@@ -1181,19 +1175,16 @@ void go_siddon_bp(const FanK& g, const float* prj, float* img, int ns, int view0
                        dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns, acc);
 }
 
-// Eight waves per tile, one per view segment, while one would leave the 1024 SIMDs
-// fewer than 8 waves each (32 slices of 256^2, 16 per lane, are 2048 waves: DD
-// adjoint 0.62 ms by one wave per tile, 0.45 by eight; DD BP, one slice of 512^2,
-// 4096 waves: 0.73 by two, 0.65 by eight).
-constexpr long kDdAdjWaves = 8192;
+// DD BP: eight waves per tile while one would leave the 1024 SIMDs fewer than 8 waves
+// each (one slice of 512^2, 4096 waves: 0.73 ms by two, 0.65 by eight).
+constexpr long kDdBpWaves = 8192;
 
 template <int G, int CAP>
 void go_dd_adj(const FanK& g, const float4* wprj, float* img, int ns, hipStream_t st)
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
-    const int nw = (long)grd.x * grd.y * grd.z < kDdAdjWaves ? kDdAdjSegs : 1;
-    const dim3 blk(64, nw);
-    const size_t lds = ((size_t)nw * DdAdjStage<G, CAP>::kFloat4 + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    const dim3 blk(64, kDdAdjSegs);
+    const size_t lds = ((size_t)kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4 + G * 64) * sizeof(float4);
     if (g.dwide) hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, true>), grd, blk, lds, st, g, wprj, img, ns);
     else hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, false>), grd, blk, lds, st, g, wprj, img, ns);
 }
@@ -1260,7 +1251,7 @@ template <int G, int CAP>
 void go_dd_bp_tile(const FanK& g, const float4* wprj, float* img, int ns, int fbp, hipStream_t st)
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
-    const int nw = (long)grd.x * grd.y * grd.z < kDdAdjWaves ? 8 : 1;
+    const int nw = (long)grd.x * grd.y * grd.z < kDdBpWaves ? 8 : 1;
     const size_t lds = ((size_t)nw * G * CAP + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     hipLaunchKernelGGL((k_dd_fan_bp_tile<G, CAP>), grd, dim3(64, nw), lds, st, g, wprj, img, ns, fbp);
 }

@@ -786,14 +786,13 @@ struct TileRange {
     float P, Q;         // bins per mm
     float u0, hw;
     int base, span;
-    float px, py, qx, qy;   // this lane's pixel from the tile centre, mm and mm x da
+    float px, py, da;   // this lane's pixel from the tile centre, mm
 
     __device__ __forceinline__ void init(const FanK& g, int lane)
     {
         px = ((float)(lane >> 3) - 3.5f) * g.dx;
         py = ((float)(lane & 7) - 3.5f) * g.dy;
-        qx = px * g.da;
-        qy = py * g.da;
+        da = g.da;
     }
     // as TileProj::batch; pad: further bins on either side
     __device__ __forceinline__ void batch(const FanK& g, int view, int lane, int tx, int ty, float pad)
@@ -828,7 +827,7 @@ struct TileRange {
     __device__ __forceinline__ void range(int l, int span_l, int& t0, int& t1) const
     {
         const float p = lane_f(P, l), q = lane_f(Q, l), h = lane_f(hw, l);
-        const float m = fmaf(p, px, q * py), n1 = fmaf(p, qy, fmaf(-q, qx, -1.0f));
+        const float m = fmaf(p, px, q * py), n1 = fmaf(fmaf(p, py, -q * px), da, -1.0f);
         const float u = fmaf(m, n1, lane_f(u0, l));
         t0 = max((int)ceilf(u - h), 0);
         t1 = min((int)floorf(u + h), span_l);
@@ -842,14 +841,14 @@ struct TileRange {
 // and view of the geometry (FanK::unit_angle).
 template <bool UNIT>
 __device__ __forceinline__ void bin_range(const FanK& g, float xc, float yc, float rpix, float inv_da, int view,
-                                          int& k0, int& k1)
+                                          float pad, int& k0, int& k1)
 {
     const float ct = g.vcos[view], st = g.vsin[view];
     const float rx = xc * ct + yc * st, ry = -xc * st + yc * ct;
     const float d0 = ry + g.dso;
     const float uc = g.cu - g.off_a - atan_fast<UNIT>(rx * __builtin_amdgcn_rcpf(d0)) * inv_da;
     const float sr = fminf(rpix * __builtin_amdgcn_rsqf(fmaf(rx, rx, d0 * d0)), 1.0f);
-    const float hw = sr * fmaf(2.0f, sr, 1.0f) * fabsf(inv_da) + 0.02f + RN_ATAN_FAST_ERR * fabsf(inv_da);
+    const float hw = sr * fmaf(2.0f, sr, 1.0f) * fabsf(inv_da) + 0.02f + pad + RN_ATAN_FAST_ERR * fabsf(inv_da);
     k0 = max((int)ceilf(uc - hw), 0);
     k1 = min((int)floorf(uc + hw), g.nu - 1);
 }
@@ -861,8 +860,10 @@ __device__ __forceinline__ float siddon_cell_weight(const float4 r, float lr, fl
 {
     const float ea = fmaf(r.y, lr, r.x), eb = fmaf(r.y, lr + 1.0f, r.x), c1 = cell + 1.0f;
     const float ov = __builtin_amdgcn_fmed3f(eb, cell, c1) - __builtin_amdgcn_fmed3f(ea, cell, c1);
+    const bool pos = ea != eb;
     const float pt = (ea >= cell && ea < c1) ? 1.0f : 0.0f;
-    return (ea != eb ? ov * __builtin_amdgcn_rcpf(eb - ea) : pt) * r.z;
+    const float inv = __builtin_amdgcn_rcpf(pos ? eb - ea : 1.0f);
+    return (pos ? ov * inv : pt) * r.z;
 }
 
 // the bins k0 .. k1 of one view for S slices (slice q's row `rboff` bytes
@@ -948,7 +949,7 @@ __device__ __forceinline__ void siddon_bp_views(const FanK& g, const T* __restri
     for (int vi = 0; vi < nviews; ++vi) {
         const int view = view0 + vi;
         int k0, k1;
-        bin_range<UNIT>(g, xc, yc, rpix, inv_da, view, k0, k1);
+        bin_range<UNIT>(g, xc, yc, rpix, inv_da, view, 0.0f, k0, k1);
         const bool xv = g.vcls[view] == 0;
         const float lr = xv ? yr : xr;          // this pixel's line
         const float cell = xv ? (float)ix : (float)iy;
@@ -983,21 +984,22 @@ __device__ __forceinline__ T siddon_bp_pixel(const FanK& g, const T* __restrict_
 // every bin whose footprint meets its segment, the FP's share overlap / width
 // from the same edge rays.  One pass over the candidate bins serves both
 // lines: the bins whose centre lies within half a bin of the angles the
-// pixel's disc spans (bin_range plus half a bin; the others have zero overlap).
+// pixel's box spans (TileRange, or without FanK::tile bin_range, plus half a bin; the
+// others have zero overlap).
 //
 // A wave takes an 8 x 8-pixel tile of G groups of 4 interleaved slices
 // (float4 sinograms [view][nu], already multiplied by the rays' length per
 // line) and stages, per view, the tile's bin window in its own LDS rows: the
 // groups' values and the window's bin edges, (A, B) of one edge ray per entry,
-// each edge shared by the two bins it separates.  As in k_siddon_fan_bp_ql: CAP
-// bins at a time, the first chunk loaded one view ahead into registers, wider
-// windows in further chunks, no barrier (a wave touches only its rows), rows
-// cleared at the start so that lanes without a bin read zeros or an earlier
-// view's bins with weight 0, never unwritten memory.
+// each edge shared by the two bins it separates.  As in k_siddon_fan_bp_tile: CAP
+// bins at a time, loaded one step (a view, or a further CAP bins of it) ahead into
+// registers, no barrier (a wave touches only its rows), rows cleared at the start so
+// that lanes without a bin read zeros or an earlier view's bins with weight 0, never
+// unwritten memory.
 //
 // The views are summed in kDdAdjSegs fixed segments whose sums are then added
-// in order, whatever the launch shape: one wave may walk all of them, or one
-// wave each, with the same bits.
+// in order, by one wave that walks all of them or by one wave each, with the same
+// bits.
 constexpr int kDdAdjSegs = 8;
 
 template <int G, int CAP>
@@ -1013,7 +1015,7 @@ struct DdAdjStage {
 // every footprint of the geometry has a positive FP32 width (FanK::dwide).
 template <int G, int CAP, int NB, bool WIDE>
 __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, float lr, float cell, float up,
-                                              float4 (&acc)[G])
+                                              float4* acc)
 {
     const float2* edge = reinterpret_cast<const float2*>(st + G * CAP);
     const float c1 = cell + 1.0f, lu = lr + 1.0f;
@@ -1052,114 +1054,114 @@ __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, 
 
 // Views [nviews seg0 / kDdAdjSegs, nviews seg1 / kDdAdjSegs) of the G groups at
 // P (groups sstride cells apart, groups k >= nq read group nq - 1 and are
-// discarded by the caller) for this lane's pixel (ix, iy); lanes outside the
-// image (inside = false) stage only.  st: this wave's DdAdjStage LDS.  tot
+// discarded by the caller) for this lane's pixel of the tile whose first pixel is
+// (tx, ty); lanes outside the image stage only.  st: this wave's DdAdjStage LDS.  tot
 // receives the ordered sum of the segments' sums.  Byte offsets from P stay
-// below 2^31 (checked on the host).
-template <int G, int CAP, int NB, bool WIDE>
+// below 2^31 (checked on the host).  ONE: seg1 = seg0 + 1 (the segment's sum needs no
+// registers of its own).
+template <int G, int CAP, int NB, bool WIDE, bool ONE>
 __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restrict__ P, long sstride, int nq,
-                                            int view0, int nviews, int seg0, int seg1, int ix, int iy, bool inside,
-                                            int lane, float4* st, float4 (&tot)[G])
+                                            int view0, int nviews, int seg0, int seg1, int tx, int ty, int lane,
+                                            float4* st, float4 (&tot)[G])
 {
     using S = DdAdjStage<G, CAP>;
-    static_assert(CAP <= 64, "one load for the edges and one more");
+    static_assert(CAP < 64, "one load for the edges");
     constexpr int kLoads = (G * CAP + 63) / 64;
     for (int i = lane; i < S::kFloat4; i += 64) st[i] = vzero<float4>();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int cx = min(ix, g.nx - 1), cy = min(iy, g.ny - 1);
-    const float xc = ((float)cx - 0.5f * (g.nx - 1)) * g.dx, yc = ((float)cy - 0.5f * (g.ny - 1)) * g.dy;
-    const float rpix = 0.5f * sqrtf(g.dx * g.dx + g.dy * g.dy);
-    const float inv_da = 1.0f / g.da;
-    const float ainv = fabsf(inv_da);
-    const float yr = (float)cy - 0.5f * g.ny, xr = (float)cx - 0.5f * g.nx;
-    const float upx = cy + 1 < g.ny ? 0.5f : 0.0f, upy = cx + 1 < g.nx ? 0.5f : 0.0f;
+    const int ix = tx + (lane >> 3), iy = ty + (lane & 7);
+    const bool inside = ix < g.nx && iy < g.ny;
+    const float yr = (float)iy - 0.5f * g.ny, xr = (float)ix - 0.5f * g.nx;
     int bj[kLoads];
     unsigned roff[kLoads];
-    bool has[kLoads];
     #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-        const int i = j * 64 + lane, r = i / CAP;
+        const int i = j * 64 + lane;
         bj[j] = i % CAP;
-        has[j] = r < G;
-        roff[j] = (unsigned)(min(r, nq - 1) * sstride) * 16u;
+        roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
     }
-    float4 acc[G], rg[kLoads];
+    float4 part[ONE ? 1 : G], rg[kLoads];
+    float4* const acc = ONE ? tot : part;   // (resolved at compile time)
     float2 re;
     #pragma unroll
     for (int q = 0; q < G; ++q) tot[q] = acc[q] = vzero<float4>();
-    // the pixel's candidate bins of view row vi (empty outside the image or the detector)
-    auto range = [&](int vi, int& k0, int& k1) {
-        const float ct = g.vcos[view0 + vi], sn = g.vsin[view0 + vi];
-        const float rx = xc * ct + yc * sn, ry = -xc * sn + yc * ct;
-        const float d0 = ry + g.dso;
-        const float z = rx * __builtin_amdgcn_rcpf(d0);
-        const float uc = g.cu - g.off_a - (g.unit_angle ? atan_fast<true>(z) : atan_fast<false>(z)) * inv_da;
-        const float sr = fminf(rpix * __builtin_amdgcn_rsqf(fmaf(rx, rx, d0 * d0)), 1.0f);
-        const float hw = sr * fmaf(2.0f, sr, 1.0f) * ainv + 0.52f + RN_ATAN_FAST_ERR * ainv;
-        k0 = max((int)ceilf(uc - hw), 0);
-        k1 = min((int)floorf(uc + hw), g.nu - 1);
-        if (!inside || k1 < k0) { k0 = g.nu; k1 = -1; }
-    };
-    // loads of the CAP bins from `base` of view row vi and of their CAP + 1 edges
-    // (edge e is the first edge of bin e, the last one the second edge of the
-    // last bin), and their LDS handover
-    auto issue = [&](int vi, int base) {
-        #pragma unroll
-        for (int j = 0; j < kLoads; ++j)
-            if (has[j]) rg[j] = ld_at(P, roff[j] + (unsigned)(vi * g.nu + min(base + bj[j], g.nu - 1)) * 16u);
-        if (lane < CAP + 1) {
-            const int e = min(base + lane, g.nu);
-            const float2* d2 = reinterpret_cast<const float2*>(g.dray);
-            re = ld_at(d2, (unsigned)((view0 + vi) * g.nu) * 16u + (e < g.nu ? (unsigned)e * 16u : (unsigned)g.nu * 16u - 8u));
+    TileRange tr;
+    tr.init(g, lane);
+    const int v0 = (int)((long)nviews * seg0 / kDdAdjSegs), v1 = (int)((long)nviews * seg1 / kDdAdjSegs);
+    // the candidate bins of view row vi: the tile's window [base, base + span] and
+    // this lane's bins t0 .. t1 in it (span < 0: none)
+    int t0 = 0, t1 = -1, base = 0, span = -1;
+    auto prepare = [&](int vi) {
+        if (g.tile) {
+            const int w = (vi - v0) & 63;
+            if (w == 0) tr.batch(g, view0 + vi, lane, tx, ty, 0.5f);
+            span = __builtin_amdgcn_readlane(tr.span, w);
+            if (span < 0) return;
+            base = __builtin_amdgcn_readlane(tr.base, w);
+            tr.range(w, span, t0, t1);
+            if (!inside) t1 = -1;
+        } else {
+            const float rpix = 0.5f * sqrtf(g.dx * g.dx + g.dy * g.dy), inv_da = 1.0f / g.da;
+            int k0, k1;
+            bin_range<false>(g, ((float)ix - 0.5f * (g.nx - 1)) * g.dx, ((float)iy - 0.5f * (g.ny - 1)) * g.dy, rpix,
+                             inv_da, view0 + vi, 0.5f, k0, k1);
+            if (!inside || k1 < k0) { k0 = g.nu; k1 = -1; }
+            base = wave_min(k0);
+            span = wave_max(k1) - base;
+            t0 = k0 - base;
+            t1 = k1 - base;
         }
     };
-    auto handover = [&]() {
+    int vi = v0 - 1, off = 0, seg = seg0;
+    int send = (int)((long)nviews * (seg0 + 1) / kDdAdjSegs);
+    bool xv = true;
+    for (bool more = true;;) {
+        const int a0 = max(t0, 0), a1 = min(t1, CAP - 1);
+        // the step's view: the pixel's line and cell, 1/2 if the line above exists
+        const float lr = xv ? yr : xr, hl = 0.5f * (xv ? g.ny : g.nx);
+        const float cell = xv ? xr + 0.5f * g.nx : yr + 0.5f * g.ny, up = lr + 1.0f < hl ? 0.5f : 0.0f;
+        if (off + CAP <= span) {
+            off += CAP;
+            t0 -= CAP;
+            t1 -= CAP;
+        } else {
+            off = 0;
+            do {
+                more = ++vi < v1;
+                if (!more) break;
+                prepare(vi);
+            } while (span < 0);
+            if (more) xv = g.vcls[view0 + vi] == 0;
+        }
+        if (more) {
+            // CAP bins and their CAP + 1 edges (edge e is the first edge of bin e, the last
+            // one the second edge of the last bin)
+            #pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP)
+                    rg[j] = ld_at(P, roff[j] + (unsigned)(vi * g.nu + min(base + off + bj[j], g.nu - 1)) * 16u);
+            if (lane < CAP + 1) {
+                const int e = min(base + off + lane, g.nu);
+                const float2* d2 = reinterpret_cast<const float2*>(g.dray);
+                re = ld_at(d2, (unsigned)((view0 + vi) * g.nu + e) * 16u - (e < g.nu ? 0u : 8u));
+            }
+        }
+        dd_adj_gather<G, CAP, NB, WIDE>(st, a0, a1, lr, cell, up, acc);
+        if (!ONE && vi >= send) {   // the segment's last step is done
+            #pragma unroll
+            for (int q = 0; q < G; ++q) {
+                vadd(tot[q], acc[q]);
+                acc[q] = vzero<float4>();
+            }
+            while (vi >= send && ++seg < seg1) send = (int)((long)nviews * (seg + 1) / kDdAdjSegs);
+        }
+        if (!more) break;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
         for (int j = 0; j < kLoads; ++j)
-            if (has[j]) st[j * 64 + lane] = rg[j];
+            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane] = rg[j];
         if (lane < CAP + 1) reinterpret_cast<float2*>(st + S::kVals)[lane] = re;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    };
-    const int vend = (int)((long)nviews * seg1 / kDdAdjSegs);
-    int vi = (int)((long)nviews * seg0 / kDdAdjSegs);
-    int k0 = g.nu, k1 = -1;
-    if (vi < vend) range(vi, k0, k1);
-    int wlo = wave_min(k0), whi = wave_max(k1);
-    if (vi < vend && whi >= wlo) issue(vi, wlo);
-    for (int seg = seg0; seg < seg1; ++seg) {
-        const int send = (int)((long)nviews * (seg + 1) / kDdAdjSegs);
-        for (; vi < send; ++vi) {
-            const bool any = whi >= wlo;
-            const int nch = any ? (whi - wlo) / CAP + 1 : 1;   // an empty window: one chunk of weight-0 reads
-            if (any) handover();
-            int n0 = g.nu, n1 = -1, nlo = g.nu, nhi = -1;
-            if (vi + 1 < vend) {
-                range(vi + 1, n0, n1);
-                nlo = wave_min(n0);
-                nhi = wave_max(n1);
-            }
-            const bool pre = nhi >= nlo;
-            if (pre && nch == 1) issue(vi + 1, nlo);
-            const bool xv = g.vcls[view0 + vi] == 0;
-            const float lr = xv ? yr : xr, up = xv ? upx : upy;
-            const float cell = xv ? (float)cx : (float)cy;
-            dd_adj_gather<G, CAP, NB, WIDE>(st, k0 - wlo, min(k1 - wlo, CAP - 1), lr, cell, up, acc);
-            for (int c = 1; c < nch; ++c) {
-                const int base = wlo + c * CAP;
-                issue(vi, base);
-                handover();
-                dd_adj_gather<G, CAP, NB, WIDE>(st, max(k0 - base, 0), min(k1 - base, CAP - 1), lr, cell, up, acc);
-            }
-            if (pre && nch > 1) issue(vi + 1, nlo);
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            k0 = n0; k1 = n1; wlo = nlo; whi = nhi;
-        }
-        #pragma unroll
-        for (int q = 0; q < G; ++q) {
-            vadd(tot[q], acc[q]);
-            acc[q] = vzero<float4>();
-        }
     }
 }
 

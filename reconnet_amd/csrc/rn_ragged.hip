@@ -119,16 +119,16 @@ __global__ __launch_bounds__(256, 4) void k_ragged_dd_adj(const RagSlice* __rest
         if (item >= total) break;
         const RagSlice& d = sl[__builtin_amdgcn_readfirstlane(find_slice(sl, nsl, item))];
         const int local = item - d.item0;
-        const int ix = (local / d.tiles) * 8 + (lane >> 3), iy = (local % d.tiles) * 8 + (lane & 7);
+        const int tx = (local / d.tiles) * 8, ty = (local % d.tiles) * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
         const bool inside = ix < d.g.nx && iy < d.g.ny;
         const long plane = (long)d.g.nx * d.g.ny, sino = (long)d.g.nu * d.g.nview;
         const float4* P = reinterpret_cast<const float4*>(d.pa);
         const int nq = (d.nsl + 3) / 4;
         float4 tot[G];
         if (d.g.dwide)
-            dd_adj_tile<G, CAP, 3, true>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, ix, iy, inside, lane, st, tot);
+            dd_adj_tile<G, CAP, 3, true, false>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, tx, ty, lane, st, tot);
         else
-            dd_adj_tile<G, CAP, 3, false>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, ix, iy, inside, lane, st, tot);
+            dd_adj_tile<G, CAP, 3, false, false>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, tx, ty, lane, st, tot);
         if (!inside) continue;
         #pragma unroll
         for (int k = 0; k < G; ++k) {
