@@ -328,28 +328,6 @@ __device__ __forceinline__ void store_or_update(const FanK& g, const float4 (&ac
     }
 }
 
-// Adds the G values per lane of a workgroup's nw waves in wave order through
-// red [G][64]; true in the wave that holds the sums (every wave calls it).
-template <int G>
-__device__ __forceinline__ bool add_waves(float4 (&v)[G], float4* red, int lane, int wv, int nw)
-{
-    if (nw == 1) return true;
-    for (int w = 0; w < nw; ++w) {
-        if (w == wv) {
-            #pragma unroll
-            for (int k = 0; k < G; ++k) {
-                if (w > 0) {
-                    const float4 r = red[k * 64 + lane];
-                    v[k] = make_float4(r.x + v[k].x, r.y + v[k].y, r.z + v[k].z, r.w + v[k].w);
-                }
-                red[k * 64 + lane] = v[k];
-            }
-        }
-        __syncthreads();
-    }
-    return wv == nw - 1;
-}
-
 // The Siddon BP of an 8 x 8-pixel tile of G interleaved slice groups, for geometries
 // with FanK::tile.  The views are split evenly over the workgroup's nw waves; the
 // waves' sums are added in LDS in wave order.  Per view the tile's bins of the G
@@ -510,8 +488,8 @@ __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const
     const int q0 = blockIdx.z * G, nq = min(G, (ns + 3) / 4 - q0);
     const long sstride = (long)g.nview * g.nu;
     float4 tot[G];
-    dd_adj_tile<G, CAP, 3, WIDE, true>(g, wprj + q0 * sstride, sstride, nq, 0, g.nview, wv, wv + 1, tx, ty, lane,
-                                       dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
+    dd_adj_tile<G, CAP, 3, WIDE>(g, wprj + q0 * sstride, sstride, nq, g.nview, wv, tx, ty, lane,
+                                 dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
     if (add_waves<G>(tot, dyn4 + kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4, lane, wv, kDdAdjSegs) && ix < g.nx &&
         iy < g.ny)
         store_or_update<G, false>(g, tot, img, SqsUpd{}, ix, iy, q0, nq, ns);

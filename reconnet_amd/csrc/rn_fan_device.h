@@ -998,8 +998,7 @@ __device__ __forceinline__ T siddon_bp_pixel(const FanK& g, const T* __restrict_
 // unwritten memory.
 //
 // The views are summed in kDdAdjSegs fixed segments whose sums are then added
-// in order, by one wave that walks all of them or by one wave each, with the same
-// bits.
+// in order, one wave each, so that a batch and its slices alone give the same bits.
 constexpr int kDdAdjSegs = 8;
 
 template <int G, int CAP>
@@ -1015,7 +1014,7 @@ struct DdAdjStage {
 // every footprint of the geometry has a positive FP32 width (FanK::dwide).
 template <int G, int CAP, int NB, bool WIDE>
 __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, float lr, float cell, float up,
-                                              float4* acc)
+                                              float4 (&acc)[G])
 {
     const float2* edge = reinterpret_cast<const float2*>(st + G * CAP);
     const float c1 = cell + 1.0f, lu = lr + 1.0f;
@@ -1052,17 +1051,15 @@ __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, 
     for (int t = t0 + NB; t <= t1; ++t) bin(t, true);
 }
 
-// Views [nviews seg0 / kDdAdjSegs, nviews seg1 / kDdAdjSegs) of the G groups at
-// P (groups sstride cells apart, groups k >= nq read group nq - 1 and are
-// discarded by the caller) for this lane's pixel of the tile whose first pixel is
-// (tx, ty); lanes outside the image stage only.  st: this wave's DdAdjStage LDS.  tot
-// receives the ordered sum of the segments' sums.  Byte offsets from P stay
-// below 2^31 (checked on the host).  ONE: seg1 = seg0 + 1 (the segment's sum needs no
-// registers of its own).
-template <int G, int CAP, int NB, bool WIDE, bool ONE>
+// View segment seg of kDdAdjSegs of the G groups at P (groups sstride cells apart,
+// groups k >= nq read group nq - 1 and are discarded by the caller) for this lane's
+// pixel of the tile whose first pixel is (tx, ty); lanes outside the image stage only.
+// st: this wave's DdAdjStage LDS.  Byte offsets from P stay below 2^31 (checked on the
+// host).
+template <int G, int CAP, int NB, bool WIDE>
 __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restrict__ P, long sstride, int nq,
-                                            int view0, int nviews, int seg0, int seg1, int tx, int ty, int lane,
-                                            float4* st, float4 (&tot)[G])
+                                            int nviews, int seg, int tx, int ty, int lane, float4* st,
+                                            float4 (&acc)[G])
 {
     using S = DdAdjStage<G, CAP>;
     static_assert(CAP < 64, "one load for the edges");
@@ -1080,21 +1077,20 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
         bj[j] = i % CAP;
         roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
     }
-    float4 part[ONE ? 1 : G], rg[kLoads];
-    float4* const acc = ONE ? tot : part;   // (resolved at compile time)
+    float4 rg[kLoads];
     float2 re;
     #pragma unroll
-    for (int q = 0; q < G; ++q) tot[q] = acc[q] = vzero<float4>();
+    for (int q = 0; q < G; ++q) acc[q] = vzero<float4>();
     TileRange tr;
     tr.init(g, lane);
-    const int v0 = (int)((long)nviews * seg0 / kDdAdjSegs), v1 = (int)((long)nviews * seg1 / kDdAdjSegs);
+    const int v0 = (int)((long)nviews * seg / kDdAdjSegs), v1 = (int)((long)nviews * (seg + 1) / kDdAdjSegs);
     // the candidate bins of view row vi: the tile's window [base, base + span] and
     // this lane's bins t0 .. t1 in it (span < 0: none)
     int t0 = 0, t1 = -1, base = 0, span = -1;
     auto prepare = [&](int vi) {
         if (g.tile) {
             const int w = (vi - v0) & 63;
-            if (w == 0) tr.batch(g, view0 + vi, lane, tx, ty, 0.5f);
+            if (w == 0) tr.batch(g, vi, lane, tx, ty, 0.5f);
             span = __builtin_amdgcn_readlane(tr.span, w);
             if (span < 0) return;
             base = __builtin_amdgcn_readlane(tr.base, w);
@@ -1104,7 +1100,7 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
             const float rpix = 0.5f * sqrtf(g.dx * g.dx + g.dy * g.dy), inv_da = 1.0f / g.da;
             int k0, k1;
             bin_range<false>(g, ((float)ix - 0.5f * (g.nx - 1)) * g.dx, ((float)iy - 0.5f * (g.ny - 1)) * g.dy, rpix,
-                             inv_da, view0 + vi, 0.5f, k0, k1);
+                             inv_da, vi, 0.5f, k0, k1);
             if (!inside || k1 < k0) { k0 = g.nu; k1 = -1; }
             base = wave_min(k0);
             span = wave_max(k1) - base;
@@ -1112,8 +1108,7 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
             t1 = k1 - base;
         }
     };
-    int vi = v0 - 1, off = 0, seg = seg0;
-    int send = (int)((long)nviews * (seg0 + 1) / kDdAdjSegs);
+    int vi = v0 - 1, off = 0;
     bool xv = true;
     for (bool more = true;;) {
         const int a0 = max(t0, 0), a1 = min(t1, CAP - 1);
@@ -1131,7 +1126,7 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
                 if (!more) break;
                 prepare(vi);
             } while (span < 0);
-            if (more) xv = g.vcls[view0 + vi] == 0;
+            if (more) xv = g.vcls[vi] == 0;
         }
         if (more) {
             // CAP bins and their CAP + 1 edges (edge e is the first edge of bin e, the last
@@ -1143,18 +1138,10 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
             if (lane < CAP + 1) {
                 const int e = min(base + off + lane, g.nu);
                 const float2* d2 = reinterpret_cast<const float2*>(g.dray);
-                re = ld_at(d2, (unsigned)((view0 + vi) * g.nu + e) * 16u - (e < g.nu ? 0u : 8u));
+                re = ld_at(d2, (unsigned)((vi) * g.nu + e) * 16u - (e < g.nu ? 0u : 8u));
             }
         }
         dd_adj_gather<G, CAP, NB, WIDE>(st, a0, a1, lr, cell, up, acc);
-        if (!ONE && vi >= send) {   // the segment's last step is done
-            #pragma unroll
-            for (int q = 0; q < G; ++q) {
-                vadd(tot[q], acc[q]);
-                acc[q] = vzero<float4>();
-            }
-            while (vi >= send && ++seg < seg1) send = (int)((long)nviews * (seg + 1) / kDdAdjSegs);
-        }
         if (!more) break;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
@@ -1163,6 +1150,28 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
         if (lane < CAP + 1) reinterpret_cast<float2*>(st + S::kVals)[lane] = re;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
+}
+
+// Adds the G values per lane of a workgroup's nw waves in wave order through
+// red [G][64]; true in the wave that holds the sums (every wave calls it).
+template <int G>
+__device__ __forceinline__ bool add_waves(float4 (&v)[G], float4* red, int lane, int wv, int nw)
+{
+    if (nw == 1) return true;
+    for (int w = 0; w < nw; ++w) {
+        if (w == wv) {
+            #pragma unroll
+            for (int k = 0; k < G; ++k) {
+                if (w > 0) {
+                    const float4 r = red[k * 64 + lane];
+                    v[k] = make_float4(r.x + v[k].x, r.y + v[k].y, r.z + v[k].z, r.w + v[k].w);
+                }
+                red[k * 64 + lane] = v[k];
+            }
+        }
+        __syncthreads();
+    }
+    return wv == nw - 1;
 }
 
 } // namespace fan

@@ -105,37 +105,45 @@ __global__ __launch_bounds__(256) void k_ragged_siddon_bp(const RagSlice* __rest
 }
 
 // DD adjoint: pa holds the descriptor's kRagS slices as kRagS / 4 interleaved
-// groups (multiplied by the rays' length per line); a wave takes one tile and
-// stages its bin windows in its own LDS rows (dd_adj_tile).
-__global__ __launch_bounds__(256, 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl, int total,
-                                                          int* __restrict__ counter)
+// groups (multiplied by the rays' length per line); a workgroup takes one tile, its
+// kDdAdjSegs waves one view segment each (dd_adj_tile), and adds the segments' sums
+// in order.  WIDE: FanK::dwide of every descriptor.
+//
+// Bound: as k_dd_fan_adj.  6 slices of 256^2 with 360 views, 6 of 384^2 with 720 and 4
+// of 512^2 with 1152: 1.84 ms, 2.4 with one wave per tile and all its views (the queue
+// then ended in a tail of 1152-view items).
+template <bool WIDE>
+__global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl,
+                                                                      int total, int* __restrict__ counter)
 {
     constexpr int G = kRagS / 4, CAP = 32;
-    __shared__ float4 stage[4 * DdAdjStage<G, CAP>::kFloat4];
-    const int lane = threadIdx.x & 63;
-    float4* st = stage + (threadIdx.x >> 6) * DdAdjStage<G, CAP>::kFloat4;
+    __shared__ float4 stage[kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4];
+    __shared__ float4 red[G * 64];
+    __shared__ int next;
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    float4* st = stage + wv * DdAdjStage<G, CAP>::kFloat4;
     for (;;) {
-        const int item = __builtin_amdgcn_readfirstlane(next_item(counter, lane));
+        // (every wave has read `next` before the barriers of add_waves, which thread 0
+        // passes before it writes the next one)
+        if (lane == 0 && wv == 0) next = atomicAdd(counter, 1);
+        __syncthreads();
+        const int item = __builtin_amdgcn_readfirstlane(next);
         if (item >= total) break;
         const RagSlice& d = sl[__builtin_amdgcn_readfirstlane(find_slice(sl, nsl, item))];
         const int local = item - d.item0;
         const int tx = (local / d.tiles) * 8, ty = (local % d.tiles) * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
-        const bool inside = ix < d.g.nx && iy < d.g.ny;
         const long plane = (long)d.g.nx * d.g.ny, sino = (long)d.g.nu * d.g.nview;
-        const float4* P = reinterpret_cast<const float4*>(d.pa);
-        const int nq = (d.nsl + 3) / 4;
         float4 tot[G];
-        if (d.g.dwide)
-            dd_adj_tile<G, CAP, 3, true, false>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, tx, ty, lane, st, tot);
-        else
-            dd_adj_tile<G, CAP, 3, false, false>(d.g, P, sino, nq, 0, d.g.nview, 0, kDdAdjSegs, tx, ty, lane, st, tot);
-        if (!inside) continue;
-        #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            const float v[4] = {tot[k].x, tot[k].y, tot[k].z, tot[k].w};
+        dd_adj_tile<G, CAP, 3, WIDE>(d.g, reinterpret_cast<const float4*>(d.pa), sino, (d.nsl + 3) / 4, d.g.nview, wv,
+                                     tx, ty, lane, st, tot);
+        if (add_waves<G>(tot, red, lane, wv, kDdAdjSegs) && ix < d.g.nx && iy < d.g.ny) {
             #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (4 * k + c < d.nsl) d.out[(4 * k + c) * plane + (long)ix * d.g.ny + iy] = v[c];
+            for (int k = 0; k < G; ++k) {
+                const float v[4] = {tot[k].x, tot[k].y, tot[k].z, tot[k].w};
+                #pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4 * k + c < d.nsl) d.out[(4 * k + c) * plane + (long)ix * d.g.ny + iy] = v[c];
+            }
         }
     }
 }
@@ -298,6 +306,7 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
     float4* Q = p_->wq.as<float4>();
     p_->host.clear();
     const int chunk = siddon ? kRagSidBp : kRagS;
+    bool wide = true;
     int item = 0;
     for (int k = 0; k < nd; k++) {
         const int s = p_->first[p_->order[k]], cnt = p_->count[p_->order[k]];
@@ -309,6 +318,7 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
         for (int c0 = 0; c0 < cnt; c0 += chunk) {
             RagSlice d{};
             d.g = p_->tables[s].k;
+            wide = wide && d.g.dwide;
             d.nsl = std::min(chunk, cnt - c0);
             d.pa = siddon ? v + c0 * sino : reinterpret_cast<const float*>(Q);    // one chunk for the DD adjoint
             d.pb = nullptr;
@@ -328,8 +338,8 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
         hipLaunchKernelGGL(k_ragged_siddon_bp, dim3(persistent_blocks()), dim3(256), 0, st,
                            p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
     else
-        hipLaunchKernelGGL(k_ragged_dd_adj, dim3(persistent_blocks()), dim3(256), 0, st,
-                           p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
+        hipLaunchKernelGGL(wide ? k_ragged_dd_adj<true> : k_ragged_dd_adj<false>, dim3(persistent_blocks()),
+                           dim3(64, kDdAdjSegs), 0, st, p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
     check_launch("ragged_bp");
     RN_HIP_CHECK(hipStreamSynchronize(st));
 }
