@@ -813,7 +813,9 @@ struct TileRange {
         // FP32: the angle to RN_ATAN_FAST_ERR and 1e-6 of its rounded operands, the bin
         // coordinate to 1e-6 of its size
         const float eps = 0.02f + pad + (RN_ATAN_FAST_ERR + 1e-6f) * a + 1e-6f * (float)g.nu;
-        hw = 0.125f * zm * a + (n * n * zm + zm * zm * zm) * a + eps;
+        // the pixel's corners (an eighth of the tile) move numerator and denominator; the
+        // centre's z is m (1 - n) to n^2 z and atan z is z to z^3
+        hw = (0.125f * zm / (1.0f - n) + n * n * zm + zm * zm * zm) * a + eps;
         const float w = zm * a + eps;
         const float lo = fminf(fmaxf(floorf(u - w), 0.0f), (float)g.nu);
         const float hi = fmaxf(fminf(floorf(u + w), (float)(g.nu - 1)), -1.0f);
