@@ -127,6 +127,10 @@ void launch_permute_rows(const float* in, float* out, const int* perm, int rows,
 // Siddon BP gather of a quad sinogram [q][view][nu] into plain images [s][nx][ny]
 void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, int nslices, int view0,
                             int nviews, hipStream_t st);
+// the same for fewer than 4 slices (one padded group) of geometries with FanK::tile and
+// 8 quad sinograms within 2 GiB; the bits do not depend on the launch shape
+void launch_siddon_fan_bp_few(const FanK& g, const float4* prj_q, float* img_xy, int nslices, int view0,
+                              int nviews, hipStream_t st);
 // The OS-SQS update applied to a backprojected subset gradient: the current
 // image is read from its interleaved copy Qold (padded quads [q][nx][qpitch(ny)])
 // and the normaliser from D4 (quads [q][nx][ny]); the new image goes to Xn

@@ -164,7 +164,9 @@ __global__ __launch_bounds__(BLK) void k_siddon_fan_fp(FanK g, const T* __restri
 // ---------------------------------------------------------------------------
 
 // One lane per pixel of S consecutive slices (the grid's z index counts
-// groups of S): the bin ranges and weights are shared by the slices.
+// groups of S): the bin ranges and weights are shared by the slices.  The views are
+// summed in kBpSegs fixed segments whose sums are added in order, as the waves of the
+// tile kernels and of the ragged batches do, with the same bits.
 template <class T, int BX, int BY, int NB, int S>
 __global__ __launch_bounds__(BX * BY) void k_siddon_fan_bp(FanK g, const T* __restrict__ prj,
                                                        T* __restrict__ img, int view0, int nviews, int ns,
@@ -176,13 +178,22 @@ __global__ __launch_bounds__(BX * BY) void k_siddon_fan_bp(FanK g, const T* __re
     const int nsl = min(S, ns - s0);
     if (ix >= g.nx || iy >= g.ny) return;
     const long sstride = (long)nviews * g.nu;
-    T acc[S];
-    siddon_bp_pixel_slices<T, NB, S>(g, prj + s0 * sstride, sstride, nsl, view0, nviews, ix, iy, acc);
+    T acc[S], tot[S];
+    #pragma unroll
+    for (int q = 0; q < S; ++q) tot[q] = vzero<T>();
+    #pragma unroll 1
+    for (int seg = 0; seg < kBpSegs; ++seg) {
+        const int v0 = (int)((long)nviews * seg / kBpSegs), v1 = (int)((long)nviews * (seg + 1) / kBpSegs);
+        siddon_bp_pixel_slices<T, NB, S>(g, prj + s0 * sstride + (long)v0 * g.nu, sstride, nsl, view0 + v0, v1 - v0,
+                                         ix, iy, acc);
+        #pragma unroll
+        for (int q = 0; q < S; ++q) vadd(tot[q], acc[q]);
+    }
     #pragma unroll
     for (int q = 0; q < S; ++q) {
         if (q >= nsl) break;
         T* o = img + (long)(s0 + q) * g.nx * g.ny + (long)ix * g.ny + iy;
-        *o = accumulate ? *o + acc[q] : acc[q];
+        *o = accumulate ? *o + tot[q] : tot[q];
     }
 }
 
@@ -438,40 +449,22 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
 // The same for one group of slices, whose bins cost less to gather from memory than
 // to stage (nothing shares a window's loads): 96 views of 512^2 66 us, staged 79;
 // 30 views of 256^2 12 and 14.
-template <bool UPD>
+template <int NB, bool UPD>
 __global__ __launch_bounds__(512) void k_siddon_fan_bp_tile1(FanK g, const float4* __restrict__ prj,
                                                              float* __restrict__ img, int view0, int nviews, int ns,
                                                              SqsUpd u)
 {
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
-    const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
-    const bool inside = ix < g.nx && iy < g.ny;
-    const int q0 = blockIdx.z;
-    const float4* const P[1] = {prj + (long)q0 * nviews * g.nu};
-    const float4* const sray = g.sray + (long)view0 * g.nu;
-    const float yr = (float)iy - 0.5f * g.ny, xr = (float)ix - 0.5f * g.nx;
+    const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7), q0 = blockIdx.z;
     float4 acc[1] = {vzero<float4>()};
-    TileRange tr;
-    tr.init(g, lane);
-    const int v0 = (int)((long)nviews * wv / nw), v1 = (int)((long)nviews * (wv + 1) / nw);
-    for (int vi = v0; vi < v1; ++vi) {
-        const int w = (vi - v0) & 63;
-        if (w == 0) tr.batch(g, view0 + vi, lane, tx, ty, 0.0f);
-        const int span = __builtin_amdgcn_readlane(tr.span, w);
-        if (span < 0) continue;
-        int t0, t1;
-        tr.range(w, span, t0, t1);
-        if (!inside) t1 = -1;
-        const bool xv = g.vcls[view0 + vi] == 0;
-        const unsigned row = (unsigned)(vi * g.nu + __builtin_amdgcn_readlane(tr.base, w)) * 16u;
-        siddon_gather_bins<float4, 2, 1>(sray, row, P, row, g.nu, t0, t1, xv ? yr : xr, xv ? (float)ix : (float)iy,
-                                         acc);
-    }
-    if (add_waves<1>(acc, dyn4, lane, wv, nw) && inside) store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
+    siddon_bp_tile1<NB>(g, prj + (long)q0 * nviews * g.nu, view0, (int)((long)nviews * wv / nw),
+                        (int)((long)nviews * (wv + 1) / nw), tx, ty, lane, acc);
+    if (add_waves<1>(acc, dyn4, lane, wv, nw) && ix < g.nx && iy < g.ny)
+        store_or_update<1, UPD>(g, acc, img, u, ix, iy, q0, 1, ns);
 }
 
 // Exact DD adjoint (dd_adj_tile): a workgroup takes an 8 x 8-pixel tile of G
-// groups of 4 slices with kDdAdjSegs waves that walk one view segment each; their
+// groups of 4 slices with kBpSegs waves that walk one view segment each; their
 // sums are added in LDS in segment order.
 //
 // Bound: VALU and LDS reads (per wave and view about 60 instructions for the bin
@@ -480,7 +473,7 @@ __global__ __launch_bounds__(512) void k_siddon_fan_bp_tile1(FanK g, const float
 // 256^2, 360 views, 512 bins 1.69 -> 0.41 -> 0.28; of 512^2, 1152 views 16.2 -> 3.1 ->
 // 2.4; one slice of 256^2 0.65 -> 0.122 -> 0.109.
 template <int G, int CAP, bool WIDE>
-__global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const float4* __restrict__ wprj,
+__global__ __launch_bounds__(64 * kBpSegs, 4) void k_dd_fan_adj(FanK g, const float4* __restrict__ wprj,
                                                                    float* __restrict__ img, int ns)
 {
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
@@ -490,7 +483,7 @@ __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_dd_fan_adj(FanK g, const
     float4 tot[G];
     dd_adj_tile<G, CAP, 3, WIDE>(g, wprj + q0 * sstride, sstride, nq, g.nview, wv, tx, ty, lane,
                                  dyn4 + wv * DdAdjStage<G, CAP>::kFloat4, tot);
-    if (add_waves<G>(tot, dyn4 + kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4, lane, wv, kDdAdjSegs) && ix < g.nx &&
+    if (add_waves<G>(tot, dyn4 + kBpSegs * DdAdjStage<G, CAP>::kFloat4, lane, wv, kBpSegs) && ix < g.nx &&
         iy < g.ny)
         store_or_update<G, false>(g, tot, img, SqsUpd{}, ix, iy, q0, nq, ns);
 }
@@ -1161,8 +1154,8 @@ template <int G, int CAP>
 void go_dd_adj(const FanK& g, const float4* wprj, float* img, int ns, hipStream_t st)
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
-    const dim3 blk(64, kDdAdjSegs);
-    const size_t lds = ((size_t)kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4 + G * 64) * sizeof(float4);
+    const dim3 blk(64, kBpSegs);
+    const size_t lds = ((size_t)kBpSegs * DdAdjStage<G, CAP>::kFloat4 + G * 64) * sizeof(float4);
     if (g.dwide) hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, true>), grd, blk, lds, st, g, wprj, img, ns);
     else hipLaunchKernelGGL((k_dd_fan_adj<G, CAP, false>), grd, blk, lds, st, g, wprj, img, ns);
 }
@@ -1337,11 +1330,13 @@ const SidBpQFn kSidBpQ[] = {go_siddon_bp_q<16, 16, 2, 8>, go_siddon_bp_q<8, 8, 2
 constexpr int kNSidFpQ = sizeof(kSidFpQ) / sizeof(kSidFpQ[0]);
 constexpr int kNSidBpQ = sizeof(kSidBpQ) / sizeof(kSidBpQ[0]);
 
-using SidBpTileFn = void (*)(const FanK&, const float4*, float*, int, int, int, const SqsUpd*, hipStream_t);
+using SidBpTileFn = void (*)(const FanK&, const float4*, float*, int, int, int, const SqsUpd*, bool, hipStream_t);
 // u != nullptr: the OS-SQS update in the epilogue instead of img
-template <int G, int CAP>
+// few: kBpSegs waves per tile whatever its size, so that the bits do not depend on the
+// shape.  CAP = 0: the gathers of one group from memory.
+template <int G, int CAP, int NB = 2>
 void go_siddon_bp_tile(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, const SqsUpd* u,
-                       hipStream_t st)
+                       bool few, hipStream_t st)
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
     // Waves per tile: up to 8 while they do not fill the chip (4096 of 4 and more
@@ -1352,18 +1347,26 @@ void go_siddon_bp_tile(const FanK& g, const float4* prj, float* img, int ns, int
     // 250^2 (G = 8), 360 views 438, 251, 200, 255; of 512^2, 96 views 153, 177, 170, 202.
     const long full = G <= 2 ? 16384 : 4096;
     int nw = 1;
+    if (few) nw = kBpSegs;
     while (nw < 8 && (long)grd.x * grd.y * grd.z * nw < full && nviews >= 8 * nw) nw *= 2;
-    const size_t lds = ((G == 1 ? 0 : (size_t)nw * (G + 1) * CAP) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    const size_t lds = ((CAP == 0 ? 0 : (size_t)nw * (G + 1) * CAP) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     const SqsUpd upd = u != nullptr ? *u : SqsUpd{};
     void (*k)(FanK, const float4*, float*, int, int, int, SqsUpd);
-    if constexpr (G == 1) k = u != nullptr ? k_siddon_fan_bp_tile1<true> : k_siddon_fan_bp_tile1<false>;
+    if constexpr (CAP == 0) k = u != nullptr ? k_siddon_fan_bp_tile1<NB, true> : k_siddon_fan_bp_tile1<NB, false>;
     else k = u != nullptr ? k_siddon_fan_bp_tile<G, CAP, true> : k_siddon_fan_bp_tile<G, CAP, false>;
     hipLaunchKernelGGL(k, grd, dim3(64, nw), lds, st, g, prj, img, view0, nviews, ns, upd);
 }
 constexpr int kNSidBpTile = 7;
 const SidBpTileFn kSidBpTile[kNSidBpTile] = {
-    go_siddon_bp_tile<1, 32>, go_siddon_bp_tile<2, 32>, go_siddon_bp_tile<2, 24>, go_siddon_bp_tile<4, 24>,
+    go_siddon_bp_tile<1, 0>,  go_siddon_bp_tile<2, 32>, go_siddon_bp_tile<2, 24>, go_siddon_bp_tile<4, 24>,
     go_siddon_bp_tile<4, 32>, go_siddon_bp_tile<8, 24>, go_siddon_bp_tile<8, 32>};
+// fewer than 4 slices of a projector call
+const SidBpTileFn kSidBpFew[] = {
+    go_siddon_bp_tile<1, 0>,     go_siddon_bp_tile<1, 0, 3>, go_siddon_bp_tile<1, 0, 1>, go_siddon_bp_tile<1, 0, 4>,
+    go_siddon_bp_tile<1, 32>,    go_siddon_bp_tile<1, 24>,   go_siddon_bp_tile<1, 48>,   go_siddon_bp_tile<2, 32>,
+    go_siddon_bp_tile<2, 24>,    go_siddon_bp_tile<4, 32>,   go_siddon_bp_tile<4, 24>,   go_siddon_bp_tile<8, 32>,
+    go_siddon_bp_tile<8, 24>};
+constexpr int kNSidBpFew = sizeof(kSidBpFew) / sizeof(kSidBpFew[0]);
 
 // Candidate i of the interleaved BP for this launch: the tile shapes (FanK::tile), the
 // fewest groups per lane that hold the batch first, then fewer, then more, where G
@@ -1386,7 +1389,7 @@ struct SidBpOrder {
 
 void go_siddon_bp_any(int c, const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
 {
-    if (c < kNSidBpTile) kSidBpTile[c](g, prj, img, ns, view0, nviews, nullptr, st);
+    if (c < kNSidBpTile) kSidBpTile[c](g, prj, img, ns, view0, nviews, nullptr, false, st);
     else kSidBpQ[c - kNSidBpTile](g, prj, img, ns, view0, nviews, st);
 }
 
@@ -1481,6 +1484,18 @@ void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, i
     check_launch("siddon_fan_bp_q");
 }
 
+void launch_siddon_fan_bp_few(const FanK& g, const float4* prj_q, float* img_xy, int nslices, int view0, int nviews,
+                              hipStream_t st)
+{
+    if (nslices <= 0 || nviews <= 0) return;
+    require_offsets32(g, nviews, sizeof(float));
+    const int c = tune_choose({TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, 1}, kNSidBpFew, [&](int i) {
+        kSidBpFew[i](g, prj_q, img_xy, nslices, view0, nviews, nullptr, true, st);
+    }, st, true);
+    kSidBpFew[c](g, prj_q, img_xy, nslices, view0, nviews, nullptr, true, st);
+    check_launch("siddon_fan_bp_few");
+}
+
 bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* img_xy, int nslices, int view0,
                                    int nviews, const SqsUpd& u, hipStream_t st)
 {
@@ -1492,7 +1507,7 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
         go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
     }, st, true)];
     const bool fused = c < kNSidBpTile;
-    if (fused) kSidBpTile[c](g, prj_q, nullptr, nslices, view0, nviews, &u, st);
+    if (fused) kSidBpTile[c](g, prj_q, nullptr, nslices, view0, nviews, &u, false, st);
     else go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, st);
     check_launch("siddon_fan_bp_q_update");
     return fused;

@@ -710,6 +710,9 @@ __device__ __forceinline__ float atan_fast(float z)
 // (v_readlane).  Bin coordinates are relative to `base`, the first bin the tile can
 // meet; base + span is the last (span < 0: the tile misses the detector).
 constexpr float kTileMax = 0.15f;
+// view segments (one wave each, or in turn) of backprojections whose bits do not depend
+// on the launch shape
+constexpr int kBpSegs = 8;
 
 // 1/15!, 1/14!, 1/13!, ..., 1/1!, 1/0!: sin and cos from the highest term down, in
 // memory so that the loop over them keeps no registers between batches
@@ -979,6 +982,35 @@ __device__ __forceinline__ T siddon_bp_pixel(const FanK& g, const T* __restrict_
     return acc[0];
 }
 
+// Views v0 .. v1 - 1 (rows of prj [view][nu], view0 + v in the tables) of one group of
+// slices for this lane's pixel of the tile whose first pixel is (tx, ty), gathered from
+// memory; every lane of the wave calls it.
+template <int NB>
+__device__ __forceinline__ void siddon_bp_tile1(const FanK& g, const float4* __restrict__ prj, int view0, int v0,
+                                                int v1, int tx, int ty, int lane, float4 (&acc)[1])
+{
+    const int ix = tx + (lane >> 3), iy = ty + (lane & 7);
+    const bool inside = ix < g.nx && iy < g.ny;
+    const float4* const P[1] = {prj};
+    const float4* const sray = g.sray + (long)view0 * g.nu;
+    const float yr = (float)iy - 0.5f * g.ny, xr = (float)ix - 0.5f * g.nx;
+    TileRange tr;
+    tr.init(g, lane);
+    for (int vi = v0; vi < v1; ++vi) {
+        const int w = (vi - v0) & 63;
+        if (w == 0) tr.batch(g, view0 + vi, lane, tx, ty, 0.0f);
+        const int span = __builtin_amdgcn_readlane(tr.span, w);
+        if (span < 0) continue;
+        int t0, t1;
+        tr.range(w, span, t0, t1);
+        if (!inside) t1 = -1;
+        const bool xv = g.vcls[view0 + vi] == 0;
+        const unsigned row = (unsigned)(vi * g.nu + __builtin_amdgcn_readlane(tr.base, w)) * 16u;
+        siddon_gather_bins<float4, NB, 1>(sray, row, P, row, g.nu, t0, t1, xv ? yr : xr, xv ? (float)ix : (float)iy,
+                                          acc);
+    }
+}
+
 // Exact transpose of the DD FP (dd_fp_ray_slices; no reference counterpart:
 // the reference DD BP is not the adjoint of its FP).  The pixel enters line
 // iy (or ix), its lower edge, and line iy + 1 (or ix + 1), its upper edge,
@@ -999,10 +1031,8 @@ __device__ __forceinline__ T siddon_bp_pixel(const FanK& g, const T* __restrict_
 // that lanes without a bin read zeros or an earlier view's bins with weight 0, never
 // unwritten memory.
 //
-// The views are summed in kDdAdjSegs fixed segments whose sums are then added
+// The views are summed in kBpSegs fixed segments whose sums are then added
 // in order, one wave each, so that a batch and its slices alone give the same bits.
-constexpr int kDdAdjSegs = 8;
-
 template <int G, int CAP>
 struct DdAdjStage {
     static constexpr int kVals = G * CAP;                  // float4: the groups' bins
@@ -1053,7 +1083,7 @@ __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, 
     for (int t = t0 + NB; t <= t1; ++t) bin(t, true);
 }
 
-// View segment seg of kDdAdjSegs of the G groups at P (groups sstride cells apart,
+// View segment seg of kBpSegs of the G groups at P (groups sstride cells apart,
 // groups k >= nq read group nq - 1 and are discarded by the caller) for this lane's
 // pixel of the tile whose first pixel is (tx, ty); lanes outside the image stage only.
 // st: this wave's DdAdjStage LDS.  Byte offsets from P stay below 2^31 (checked on the
@@ -1085,7 +1115,7 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
     for (int q = 0; q < G; ++q) acc[q] = vzero<float4>();
     TileRange tr;
     tr.init(g, lane);
-    const int v0 = (int)((long)nviews * seg / kDdAdjSegs), v1 = (int)((long)nviews * (seg + 1) / kDdAdjSegs);
+    const int v0 = (int)((long)nviews * seg / kBpSegs), v1 = (int)((long)nviews * (seg + 1) / kBpSegs);
     // the candidate bins of view row vi: the tile's window [base, base + span] and
     // this lane's bins t0 .. t1 in it (span < 0: none)
     int t0 = 0, t1 = -1, base = 0, span = -1;

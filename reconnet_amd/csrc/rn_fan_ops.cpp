@@ -177,7 +177,10 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
         Q = w.ry.as<float>();
     }
     float* W = w.sino.as<float>();   // [slice][nview][nu]
-    const bool quads = kind == FanBP::Siddon && ns >= 4 && qplanes_fit32(g.nx, g.ny);   // transposed and interleaved in one pass
+    // Siddon: transposed and interleaved in one pass; below 4 slices by tiles only (one
+    // slice, 64^2 0.067 -> 0.022 ms, 256^2 0.26 -> 0.08, 512^2 0.93 -> 0.80)
+    const bool few = kind == FanBP::Siddon && ns < 4 && t.k.tile && 8L * sino * 16L < 0x7fffffffL;
+    const bool quads = few || (kind == FanBP::Siddon && ns >= 4 && qplanes_fit32(g.nx, g.ny));
     if (kind != FanBP::DDAdjoint && !quads) launch_transpose(Q, W, g.nu, g.nview, ns, st);
     float* out = direct_out ? img_ref : w.rx.as<float>();
     switch (kind) {
@@ -211,7 +214,8 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
     case FanBP::Siddon:
         if (quads) {
             launch_pack_quads(Q, nullptr, w.quad.as<float4>(), g.nu, g.nview, ns, false, st);
-            launch_siddon_fan_bp_q(t.k, w.quad.as<float4>(), out, ns, 0, g.nview, st);
+            if (few) launch_siddon_fan_bp_few(t.k, w.quad.as<float4>(), out, ns, 0, g.nview, st);
+            else launch_siddon_fan_bp_q(t.k, w.quad.as<float4>(), out, ns, 0, g.nview, st);
         } else {
             launch_siddon_fan_bp(t.k, W, out, ns, 0, g.nview, false, st);
         }

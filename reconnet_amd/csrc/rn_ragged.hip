@@ -82,52 +82,70 @@ __global__ __launch_bounds__(256) void k_ragged_fp(const RagSlice* __restrict__ 
     }
 }
 
-__global__ __launch_bounds__(256) void k_ragged_siddon_bp(const RagSlice* __restrict__ sl, int nsl, int total,
-                                                          int* __restrict__ counter)
+// The next item of a workgroup.  (Every wave has read `next` before the barriers of
+// add_waves, which thread 0 passes before it writes the next one.)
+__device__ __forceinline__ int next_tile(int* counter, int* next, int lane, int wv)
 {
-    constexpr int S = kRagSidBp;
-    const int lane = threadIdx.x & 63;
+    if (lane == 0 && wv == 0) *next = atomicAdd(counter, 1);
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*next);
+}
+
+// Siddon BP: pa holds the descriptor's kRagSidBp slices as one interleaved group; a
+// workgroup takes one tile, its kBpSegs waves one view segment each, with the arithmetic
+// of k_siddon_fan_bp_tile1 (FanK::tile) or k_siddon_fan_bp, and adds the segments' sums
+// in order.
+__global__ __launch_bounds__(64 * kBpSegs) void k_ragged_siddon_bp(const RagSlice* __restrict__ sl, int nsl, int total,
+                                                                   int* __restrict__ counter)
+{
+    static_assert(kRagSidBp == 4, "one group per descriptor");
+    __shared__ float4 red[64];
+    __shared__ int next;
+    const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     for (;;) {
-        const int item = next_item(counter, lane);
+        const int item = next_tile(counter, &next, lane, wv);
         if (item >= total) break;
-        const RagSlice& d = sl[find_slice(sl, nsl, item)];
+        const RagSlice& d = sl[__builtin_amdgcn_readfirstlane(find_slice(sl, nsl, item))];
         const int local = item - d.item0;
-        const int ix = (local / d.tiles) * 8 + (lane >> 3), iy = (local % d.tiles) * 8 + (lane & 7);
-        if (ix < d.g.nx && iy < d.g.ny) {
-            const long plane = (long)d.g.nx * d.g.ny, sino = (long)d.g.nu * d.g.nview;
-            float acc[S];
-            siddon_bp_pixel_slices<float, 4, S>(d.g, d.pa, sino, d.nsl, 0, d.g.nview, ix, iy, acc);
+        const int tx = (local / d.tiles) * 8, ty = (local % d.tiles) * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
+        const bool inside = ix < d.g.nx && iy < d.g.ny;
+        const int v0 = (int)((long)d.g.nview * wv / kBpSegs), v1 = (int)((long)d.g.nview * (wv + 1) / kBpSegs);
+        const float4* P = reinterpret_cast<const float4*>(d.pa);
+        float4 acc[1] = {vzero<float4>()};
+        if (d.g.tile)
+            siddon_bp_tile1<2>(d.g, P, 0, v0, v1, tx, ty, lane, acc);
+        else if (inside)
+            siddon_bp_pixel_slices<float4, 4, 1>(d.g, P + (long)v0 * d.g.nu, 0, 1, v0, v1 - v0, ix, iy, acc);
+        if (add_waves<1>(acc, red, lane, wv, kBpSegs) && inside) {
+            const long plane = (long)d.g.nx * d.g.ny;
+            const float v[4] = {acc[0].x, acc[0].y, acc[0].z, acc[0].w};
             #pragma unroll
-            for (int q = 0; q < S; ++q)
-                if (q < d.nsl) d.out[q * plane + (long)ix * d.g.ny + iy] = acc[q];
+            for (int c = 0; c < 4; ++c)
+                if (c < d.nsl) d.out[c * plane + (long)ix * d.g.ny + iy] = v[c];
         }
     }
 }
 
 // DD adjoint: pa holds the descriptor's kRagS slices as kRagS / 4 interleaved
 // groups (multiplied by the rays' length per line); a workgroup takes one tile, its
-// kDdAdjSegs waves one view segment each (dd_adj_tile), and adds the segments' sums
+// kBpSegs waves one view segment each (dd_adj_tile), and adds the segments' sums
 // in order.  WIDE: FanK::dwide of every descriptor.
 //
 // Bound: as k_dd_fan_adj.  6 slices of 256^2 with 360 views, 6 of 384^2 with 720 and 4
 // of 512^2 with 1152: 1.84 ms, 2.4 with one wave per tile and all its views (the queue
 // then ended in a tail of 1152-view items).
 template <bool WIDE>
-__global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl,
+__global__ __launch_bounds__(64 * kBpSegs, 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl,
                                                                       int total, int* __restrict__ counter)
 {
     constexpr int G = kRagS / 4, CAP = 32;
-    __shared__ float4 stage[kDdAdjSegs * DdAdjStage<G, CAP>::kFloat4];
+    __shared__ float4 stage[kBpSegs * DdAdjStage<G, CAP>::kFloat4];
     __shared__ float4 red[G * 64];
     __shared__ int next;
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     float4* st = stage + wv * DdAdjStage<G, CAP>::kFloat4;
     for (;;) {
-        // (every wave has read `next` before the barriers of add_waves, which thread 0
-        // passes before it writes the next one)
-        if (lane == 0 && wv == 0) next = atomicAdd(counter, 1);
-        __syncthreads();
-        const int item = __builtin_amdgcn_readfirstlane(next);
+        const int item = next_tile(counter, &next, lane, wv);
         if (item >= total) break;
         const RagSlice& d = sl[__builtin_amdgcn_readfirstlane(find_slice(sl, nsl, item))];
         const int local = item - d.item0;
@@ -136,7 +154,7 @@ __global__ __launch_bounds__(64 * kDdAdjSegs, 4) void k_ragged_dd_adj(const RagS
         float4 tot[G];
         dd_adj_tile<G, CAP, 3, WIDE>(d.g, reinterpret_cast<const float4*>(d.pa), sino, (d.nsl + 3) / 4, d.g.nview, wv,
                                      tx, ty, lane, st, tot);
-        if (add_waves<G>(tot, red, lane, wv, kDdAdjSegs) && ix < d.g.nx && iy < d.g.ny) {
+        if (add_waves<G>(tot, red, lane, wv, kBpSegs) && ix < d.g.nx && iy < d.g.ny) {
             #pragma unroll
             for (int k = 0; k < G; ++k) {
                 const float v[4] = {tot[k].x, tot[k].y, tot[k].z, tot[k].w};
@@ -231,9 +249,9 @@ void RaggedBatch::setup(const std::vector<FanGeo>& geos, const std::vector<const
     p_->desc.alloc(nd * ((kRagS + kRagFp - 1) / kRagFp) * sizeof(RagSlice));
     p_->counter.alloc(sizeof(int));
     p_->wa.alloc(io * sizeof(float));
-    p_->wb.alloc(std::max(io, so) * sizeof(float));
+    p_->wb.alloc(io * sizeof(float));
     p_->wc.alloc(io * sizeof(float));
-    // the DD adjoint's interleaved sinograms: whole groups of 4 slices per descriptor
+    // the interleaved sinograms: whole groups of 4 slices per descriptor
     long qo = 0;
     for (int k = 0; k < nd; k++) {
         const FanGeo& g = geos[p_->first[k]];
@@ -302,7 +320,6 @@ void RaggedBatch::forward(bool siddon, const float* img, float* prj, hipStream_t
 void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_t st)
 {
     const int nd = (int)p_->first.size();
-    float* V = p_->wb.as<float>();   // view-major copies of the sinograms
     float4* Q = p_->wq.as<float4>();
     p_->host.clear();
     const int chunk = siddon ? kRagSidBp : kRagS;
@@ -311,8 +328,7 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
     for (int k = 0; k < nd; k++) {
         const int s = p_->first[p_->order[k]], cnt = p_->count[p_->order[k]];
         const FanGeo& g = p_->tables[s].geo;
-        float* v = V + p_->sino_off[s];
-        if (siddon) launch_transpose(prj + p_->sino_off[s], v, g.nu, g.nview, cnt, st);
+        if (siddon) launch_pack_quads(prj + p_->sino_off[s], nullptr, Q, g.nu, g.nview, cnt, false, st);
         else launch_pack_quads_len(p_->tables[s].k, prj + p_->sino_off[s], Q, cnt, st);
         const long plane = (long)g.nx * g.ny, sino = (long)g.nu * g.nview;
         for (int c0 = 0; c0 < cnt; c0 += chunk) {
@@ -320,7 +336,7 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
             d.g = p_->tables[s].k;
             wide = wide && d.g.dwide;
             d.nsl = std::min(chunk, cnt - c0);
-            d.pa = siddon ? v + c0 * sino : reinterpret_cast<const float*>(Q);    // one chunk for the DD adjoint
+            d.pa = reinterpret_cast<const float*>(Q + c0 / 4 * sino);
             d.pb = nullptr;
             d.out = img + p_->img_off[s] + c0 * plane;
             d.tiles = cdiv(g.ny, 8);
@@ -335,11 +351,11 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
     RN_HIP_CHECK(hipMemcpyAsync(p_->desc.get(), p_->host.data(), nbd * sizeof(RagSlice), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, p_->counter.as<int>());
     if (siddon)
-        hipLaunchKernelGGL(k_ragged_siddon_bp, dim3(persistent_blocks()), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_ragged_siddon_bp, dim3(persistent_blocks()), dim3(64, kBpSegs), 0, st,
                            p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
     else
         hipLaunchKernelGGL(wide ? k_ragged_dd_adj<true> : k_ragged_dd_adj<false>, dim3(persistent_blocks()),
-                           dim3(64, kDdAdjSegs), 0, st, p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
+                           dim3(64, kBpSegs), 0, st, p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
     check_launch("ragged_bp");
     RN_HIP_CHECK(hipStreamSynchronize(st));
 }
