@@ -181,7 +181,8 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
     // slice, 64^2 0.067 -> 0.022 ms, 256^2 0.26 -> 0.08, 512^2 0.93 -> 0.80)
     const bool few = kind == FanBP::Siddon && ns < 4 && t.k.tile && 8L * sino * 16L < 0x7fffffffL;
     const bool quads = few || (kind == FanBP::Siddon && ns >= 4 && qplanes_fit32(g.nx, g.ny));
-    if (kind != FanBP::DDAdjoint && !quads) launch_transpose(Q, W, g.nu, g.nview, ns, st);
+    const bool direct = quads || kind == FanBP::DDAdjoint || (kind == FanBP::DDFBP && t.k.tile_dd);
+    if (!direct) launch_transpose(Q, W, g.nu, g.nview, ns, st);
     float* out = direct_out ? img_ref : w.rx.as<float>();
     switch (kind) {
     case FanBP::DD:
@@ -195,7 +196,8 @@ void fan_backward(const FanTables& t, FanBP kind, int nB, int nC, const float* p
             P = w.ry.as<float>();
         }
         if (t.k.tile_dd) {
-            launch_pack_quads(P, w.quad.as<float4>(), nullptr, g.nview, g.nu, ns, false, st);
+            if (fbp) launch_pack_quads(Q, nullptr, w.quad.as<float4>(), g.nu, g.nview, ns, false, st);
+            else launch_pack_quads(P, w.quad.as<float4>(), nullptr, g.nview, g.nu, ns, false, st);
             launch_dd_fan_bp_tile(t.k, w.quad.as<float4>(), out, ns, fbp, st);
         } else if (ns >= 4) {
             // groups of 4 slices interleaved: one float4 load per bin and group

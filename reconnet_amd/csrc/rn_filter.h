@@ -22,6 +22,7 @@ private:
     int nu_ = 0, nview_ = 0, type_ = 0;
     float da_ = 0, off_a_ = 0, dso_ = 0;
     bool fan_ = true;
+    size_t mfma_off_ = 0;   // k_ramp_mfma's taps in buf_ (floats, 16-byte aligned)
     std::vector<float> host_;
     DevBuf buf_;
 };
