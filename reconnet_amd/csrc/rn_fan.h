@@ -63,6 +63,7 @@ class FanTables {
 public:
     void build(const FanGeo& g, const float* deg_host, hipStream_t st);
     bool matches(const FanGeo& g, const float* deg_host) const;
+    size_t bytes() const { return buf_.size() + ray_.size() + dray_.size(); }
     FanK k{};
     FanGeo geo{};
     std::vector<float> deg;

@@ -68,6 +68,8 @@ public:
     void kernel_times(double* ms_fp, double* ms_bp, double* ms_upd, long* steps) const;
     const FanTables& tables() const { return t_; }
     int nslices() const { return ns_; }
+    // device memory held
+    size_t bytes() const;
 private:
     FanTables t_;
     int ns_ = 0, npers_ = 0, nsub_ = 0;

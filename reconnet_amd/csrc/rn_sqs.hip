@@ -413,8 +413,11 @@ void OsSqs::setup(const FanGeo& g, const float* deg_host, int nslices, int nview
 void OsSqs::set_data(const float* prj_ref, const float* w_ref, hipStream_t st)
 {
     const FanGeo& g = t_.geo;
-    // view-major, then the engine's view order
-    DevBuf tmp((size_t)ns_ * g.nu * g.nview * sizeof(float));
+    // view-major, then the engine's view order (through the quad measurement's buffer,
+    // which is written last)
+    DevBuf own;
+    if (!quads_) own.ensure((size_t)ns_ * g.nu * g.nview * sizeof(float));
+    DevBuf& tmp = quads_ ? B4_ : own;
     launch_transpose(prj_ref, tmp.as<float>(), g.nu, g.nview, ns_, st);
     launch_permute_rows(tmp.as<float>(), B_.as<float>(), perm_dev_.as<int>(), g.nview, g.nu, ns_, st);
     if (w_ref) {
@@ -465,6 +468,15 @@ void OsSqs::sync_transposed(hipStream_t st)
     if (quads_) launch_pack_quads(X_[cur_].as<float>(), Qxy_[cur_].as<float4>(), Qyx_[cur_].as<float4>(), t_.geo.nx,
                                   t_.geo.ny, ns_, true, st);
     else launch_transpose(X_[cur_].as<float>(), Xyx_.as<float>(), t_.geo.nx, t_.geo.ny, ns_, st);
+}
+
+size_t OsSqs::bytes() const
+{
+    size_t n = t_.bytes();
+    for (const DevBuf* b : {&B_, &W_, &D_, &X_[0], &X_[1], &Xyx_, &R_, &G_, &red_, &Qxy_[0], &Qxy_[1], &Qyx_[0],
+                            &Qyx_[1], &B4_, &W4_, &R4_, &D4_, &perm_dev_})
+        n += b->size();
+    return n;
 }
 
 OsSqs::~OsSqs()
