@@ -183,8 +183,8 @@ inline bool qplanes_fit32(int nx, int ny)
 // ---- layout helpers ----
 // out[b][c][r] = in[b][r][c] for a batch of (rows x cols) matrices
 void launch_transpose(const float* in, float* out, int rows, int cols, int batch, hipStream_t st);
-// axis 0: out[i][j] = (in[i-1][j] + in[i][j]) / 2 ; axis 1: out[i][j] = (in[i][j-1] + in[i][j]) / 2
-void launch_avg_prev(const float* in, float* out, int n0, int n1, int batch, int axis, hipStream_t st);
+// ry[i][j] = (in[i-1][j] + in[i][j]) / 2 and rx[j][i] = (in[i][j-1] + in[i][j]) / 2 for a batch
+void launch_avg_planes(const float* in, float* ry, float* rx, int n0, int n1, int batch, hipStream_t st);
 // dst[(b*nout + o)*nc + c][i] = sum_p M[o][p] * src[((b*n + i)*np + p)*nc + c]
 void launch_mix_gather(const float* src, float* dst, const float* M, int nB, int n, int np, int nc, int nout,
                        hipStream_t st);

@@ -140,9 +140,7 @@ void fan_forward(const FanTables& t, FanFP kind, int nB, int nC, const float* im
         else launch_siddon_fan_fp_q(t.k, QX, QY, out_vu, ns, 0, g.nview, st);
     } else if (kind == FanFP::DD) {
         // RY[x][y] = (P[x-1][y] + P[x][y]) / 2 ;  RX = transpose((P[x][y-1] + P[x][y]) / 2)
-        launch_avg_prev(P, w.ry.as<float>(), g.nx, g.ny, ns, 0, st);
-        launch_avg_prev(P, out_vu, g.nx, g.ny, ns, 1, st);
-        launch_transpose(out_vu, w.rx.as<float>(), g.nx, g.ny, ns, st);
+        launch_avg_planes(P, w.ry.as<float>(), w.rx.as<float>(), g.nx, g.ny, ns, st);
         launch_dd_fan_fp(t.k, w.rx.as<float>(), w.ry.as<float>(), out_vu, ns, 0, g.nview, st);
     } else {
         launch_transpose(P, w.rx.as<float>(), g.nx, g.ny, ns, st);

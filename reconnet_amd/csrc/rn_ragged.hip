@@ -185,7 +185,7 @@ struct RaggedBatch::Impl {
     std::vector<int> first, count;   // descriptor k: slices first[k] .. first[k] + count[k] - 1
     std::vector<int> order;          // descriptors by decreasing cost
     long img_total = 0, sino_total = 0;
-    DevBuf desc, counter, wa, wb, wc, wq;
+    DevBuf desc, counter, wa, wb, wq;
     std::vector<RagSlice> host;
 };
 
@@ -250,7 +250,6 @@ void RaggedBatch::setup(const std::vector<FanGeo>& geos, const std::vector<const
     p_->counter.alloc(sizeof(int));
     p_->wa.alloc(io * sizeof(float));
     p_->wb.alloc(io * sizeof(float));
-    p_->wc.alloc(io * sizeof(float));
     // the interleaved sinograms: whole groups of 4 slices per descriptor
     long qo = 0;
     for (int k = 0; k < nd; k++) {
@@ -285,10 +284,7 @@ void RaggedBatch::forward(bool siddon, const float* img, float* prj, hipStream_t
             pb = P;
         } else {
             // RY[x][y] = (P[x-1][y] + P[x][y]) / 2 ;  RX = transpose((P[x][y-1] + P[x][y]) / 2)
-            float* c = p_->wc.as<float>() + p_->img_off[s];
-            launch_avg_prev(P, b, g.nx, g.ny, cnt, 0, st);
-            launch_avg_prev(P, c, g.nx, g.ny, cnt, 1, st);
-            launch_transpose(c, a, g.nx, g.ny, cnt, st);
+            launch_avg_planes(P, b, a, g.nx, g.ny, cnt, st);
             pa = a;
             pb = b;
         }
