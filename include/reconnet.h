@@ -319,7 +319,7 @@ int rn_helical_rebin(const float* fan, float* par, int nBatches, int nChannels,
 /* Launch-shape autotuner (no reference counterpart).  On the first launch of
  * a shape key the projector launchers time their candidate block / tile shapes
  * on the caller's stream and keep the fastest for the process; the choice
- * never changes results.  Enabled unless RECONNET_AUTOTUNE=0 or switched off
+ * changes results by at most the rounding of a regrouped sum.  Enabled unless RECONNET_AUTOTUNE=0 or switched off
  * here.  rn_autotune_report writes "kernel a b c d e -> choice (ms ...)"
  * lines into buf (NUL-terminated, truncated to len) and returns the full
  * length. */
@@ -327,9 +327,8 @@ int rn_autotune_enable(int on);
 int rn_autotune_report(char* buf, int len);
 int rn_autotune_reset(void);
 /* Force candidate `candidate` of kernel `kernel` (1 Siddon FP, 2 Siddon BP,
- * 3 DD FP, 4 DD adjoint, 5 DD BP, 7 DD FBP BP; 8 / 9 Siddon FP / BP,
- * 10 / 11 DD BP / FBP BP and 12 DD FP on the interleaved 4-slice layout used
- * for 4 or more slices; 13 the CNN's 32 -> 32 convolution, 14 the one-launch CNN forward, 15 the
+ * 3 DD FP, 4 DD adjoint, 5 DD BP, 7 DD FBP BP; 8 / 9 the OS-SQS engine's
+ * Siddon FP / BP, 10 / 11 DD BP / FBP BP and 12 DD FP of 4 or more slices; 13 the CNN's 32 -> 32 convolution, 14 the one-launch CNN forward, 15 the
  * helical backprojection, 16 the cone DD forward projector, 17 the pixel-driven BP, 18 the Siddon cone
  * backprojection of upright detectors, 19 the cone DD adjoint) for every shape, bypassing the
  * timing; candidate < 0 removes the pin.  A launch of a kernel with fewer

@@ -1674,9 +1674,9 @@ __global__ __launch_bounds__(256) void k_helical_bp(HelicalGeo h, const float* _
             }
             #pragma unroll
             for (int j = 0; j < ZC; ++j) {
-                const float a = fmaf(av[j], r1[j].x - r0[j].x, r0[j].x), d = fmaf(av[j], r1[j].y - r0[j].y, r0[j].y);
+                const float a = fmaf(whi, r0[j].y, wlo * r0[j].x), d = fmaf(whi, r1[j].y, wlo * r1[j].x);
                 // (a voxel outside its window: its sums are not used)
-                val[j] = fmaf(fmaf(whi, d, wlo * a), w[j], val[j]);
+                val[j] = fmaf(fmaf(av[j], d, (1.0f - av[j]) * a), w[j], val[j]);
                 tw[j] += w[j];
             }
         }

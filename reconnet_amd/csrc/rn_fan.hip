@@ -370,11 +370,11 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
 {
     static_assert(CAP <= 64, "one load for the ray table row");
     // LDS rows 0 .. G - 1: the groups; row G: the ray table
-    constexpr int kRows = G + 1, kLoads = (G * CAP + 63) / 64;
+    constexpr int CS = stage_pitch(CAP), kLds = (G + 1) * CS, kLoads = (G * CAP + 63) / 64;
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
     const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
-    float4* st = dyn4 + wv * kRows * CAP;
-    for (int i = lane; i < kRows * CAP; i += 64) st[i] = vzero<float4>();
+    float4* st = dyn4 + wv * kLds;
+    for (int i = lane; i < kLds; i += 64) st[i] = vzero<float4>();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const bool inside = ix < g.nx && iy < g.ny;   // lanes outside stage but gather nothing
     const int q0 = blockIdx.z * G, nq = min(G, (ns + 3) / 4 - q0);
@@ -386,14 +386,15 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
     #pragma unroll
     for (int q = 0; q < G; ++q) acc[q] = vzero<float4>();
     // staging load j of this lane: element i = 64 j + lane of the group rows, that is
-    // group i / CAP, bin i % CAP of the window (LDS slot i); the ray table row is one
+    // group i / CAP, bin i % CAP of the window; the ray table row is one
     // more load by the first CAP lanes
-    int bj[kLoads];
+    int bj[kLoads], slot[kLoads];   // slot: the zero entries of the rows before
     unsigned roff[kLoads];
     #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
         const int i = j * 64 + lane;
         bj[j] = i % CAP;
+        slot[j] = G == 1 ? 0 : i / CAP;
         roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
     }
     TileRange tr;
@@ -438,11 +439,11 @@ __global__ __launch_bounds__(512, 4) void k_siddon_fan_bp_tile(FanK g, const flo
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
         for (int j = 0; j < kLoads; ++j)
-            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane] = rg[j];
-        if (lane < CAP) st[G * CAP + lane] = rr;
+            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane + slot[j]] = rg[j];
+        if (lane < CAP) st[G * CS + lane] = rr;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
-    if (add_waves<G>(acc, dyn4 + nw * kRows * CAP, lane, wv, nw) && inside)
+    if (add_waves<G>(acc, dyn4 + nw * kLds, lane, wv, nw) && inside)
         store_or_update<G, UPD>(g, acc, img, u, ix, iy, q0, nq, ns);
 }
 
@@ -628,11 +629,11 @@ template <int G, int CAP>
 __global__ __launch_bounds__(512, 4) void k_dd_fan_bp_tile(FanK g, const float4* __restrict__ wprj,
                                                            float* __restrict__ img, int ns, int fbp)
 {
-    constexpr int kLoads = (G * CAP + 63) / 64;
+    constexpr int kLds = G * stage_pitch(CAP), kLoads = (G * CAP + 63) / 64;
     const int lane = threadIdx.x, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.y), nw = blockDim.y;
     const int tx = blockIdx.y * 8, ty = blockIdx.x * 8, ix = tx + (lane >> 3), iy = ty + (lane & 7);
-    float4* st = dyn4 + wv * G * CAP;
-    for (int i = lane; i < G * CAP; i += 64) st[i] = vzero<float4>();
+    float4* st = dyn4 + wv * kLds;
+    for (int i = lane; i < kLds; i += 64) st[i] = vzero<float4>();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const bool inside = ix < g.nx && iy < g.ny;   // lanes outside stage but gather nothing
     const int q0 = blockIdx.z * G, nq = min(G, (ns + 3) / 4 - q0);
@@ -643,12 +644,13 @@ __global__ __launch_bounds__(512, 4) void k_dd_fan_bp_tile(FanK g, const float4*
     for (int q = 0; q < G; ++q) acc[q] = vzero<float4>();
     // staging load j of this lane: element i = 64 j + lane, row i / CAP, bin
     // i % CAP (LDS slot i)
-    int bj[kLoads];
+    int bj[kLoads], slot[kLoads];   // slot: the zero entries of the rows before
     unsigned roff[kLoads];
     #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
         const int i = j * 64 + lane;
         bj[j] = i % CAP;
+        slot[j] = G == 1 ? 0 : i / CAP;
         roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
     }
     const float inv_da = 1.0f / g.da;
@@ -690,10 +692,10 @@ __global__ __launch_bounds__(512, 4) void k_dd_fan_bp_tile(FanK g, const float4*
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
         for (int j = 0; j < kLoads; ++j)
-            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane] = rg[j];
+            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane + slot[j]] = rg[j];
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
-    if (add_waves<G>(acc, dyn4 + nw * G * CAP, lane, wv, nw) && inside)
+    if (add_waves<G>(acc, dyn4 + nw * kLds, lane, wv, nw) && inside)
         store_or_update<G, false>(g, acc, img, SqsUpd{}, ix, iy, q0, nq, ns);
 }
 
@@ -1236,7 +1238,7 @@ void go_dd_bp_tile(const FanK& g, const float4* wprj, float* img, int ns, int fb
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
     const int nw = (long)grd.x * grd.y * grd.z < kDdBpWaves ? 8 : 1;
-    const size_t lds = ((size_t)nw * G * CAP + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    const size_t lds = ((size_t)nw * G * stage_pitch(CAP) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     hipLaunchKernelGGL((k_dd_fan_bp_tile<G, CAP>), grd, dim3(64, nw), lds, st, g, wprj, img, ns, fbp);
 }
 // groups of 4 slices per lane 1, 2, 4, 8; windows of 32 and 24 bins
@@ -1362,7 +1364,7 @@ void go_siddon_bp_tile(const FanK& g, const float4* prj, float* img, int ns, int
     int nw = 1;
     if (few) nw = kBpSegs;
     while (nw < 8 && (long)grd.x * grd.y * grd.z * nw < full && nviews >= 8 * nw) nw *= 2;
-    const size_t lds = ((CAP == 0 ? 0 : (size_t)nw * (G + 1) * CAP) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
+    const size_t lds = ((CAP == 0 ? 0 : (size_t)nw * (G + 1) * stage_pitch(CAP)) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     const SqsUpd upd = u != nullptr ? *u : SqsUpd{};
     void (*k)(FanK, const float4*, float*, int, int, int, SqsUpd);
     if constexpr (CAP == 0) k = u != nullptr ? k_siddon_fan_bp_tile1<NB, true> : k_siddon_fan_bp_tile1<NB, false>;

@@ -72,10 +72,14 @@ __device__ __forceinline__ void seg_acc_rows(const T* const (&rows)[S], unsigned
     }
 }
 
+// Rows of CAP staged bins in LDS are CAP + 1 entries apart; the last one stays zero, and
+// a lane without a bin reads it with weight 0 (a bin of the window would carry a NaN or
+// an infinity to pixels that do not meet it).
+constexpr int stage_pitch(int cap) { return cap + 1; }
+
 // acc[q] += k * the integral over [lo, hi] (h0: the end of the row) of row q of G
-// staged rows (CAP entries from st + q CAP, the first one the interval's origin);
-// two bins without branches (a lane that does not meet one takes its first with
-// weight 0), further ones in a loop.
+// staged rows, their first entry the interval's origin; two bins without branches,
+// further ones in a loop.
 template <int G, int CAP>
 __device__ __forceinline__ void seg_rel_staged(const float4* st, float lo, float hi, float h0, float k,
                                                float4 (&acc)[G])
@@ -83,23 +87,23 @@ __device__ __forceinline__ void seg_rel_staged(const float4* st, float lo, float
     const float l = fmaxf(lo, 0.0f), h = fminf(hi, h0);
     const bool on0 = h > l;
     float f = floorf(l);
-    int t = on0 ? (int)f : 0;
+    int t = on0 ? (int)f : CAP;
     const float c0 = on0 ? (fminf(h, f + 1.0f) - l) * k : 0.0f;
     #pragma unroll
-    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], c0);
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * stage_pitch(CAP) + t], c0);
     f += 1.0f;
     const bool on1 = on0 && h > f;
     const float c1 = on1 ? (fminf(h, f + 1.0f) - f) * k : 0.0f;
-    t += on1 ? 1 : 0;
+    t = on1 ? t + 1 : CAP;
     #pragma unroll
-    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], c1);
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * stage_pitch(CAP) + t], c1);
     f += 1.0f;
     if (!on1) return;
     while (h > f) {
         ++t;
         const float c = (fminf(h, f + 1.0f) - f) * k;
         #pragma unroll
-        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], c);
+        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * stage_pitch(CAP) + t], c);
         f += 1.0f;
     }
 }
@@ -906,26 +910,26 @@ __device__ __forceinline__ void siddon_gather_bins(const float4* __restrict__ sr
 // bins per row from the window's first bin (every slot holds written values:
 // the caller clears the rows before its first window); t0 .. t1 are the pixel's bins
 // relative to that first bin.  The first two bins are taken by every lane with
-// no branch around the accumulators: a lane past t1 reads slot 0 (a bin of
-// this view's window) with weight 0, which keeps the kernel in registers.
-// The rest in a loop.
+// no branch around the accumulators (a lane past t1 reads the zero entry), which keeps
+// the kernel in registers.  The rest in a loop.
 template <int G, int CAP>
 __device__ __forceinline__ void siddon_gather_staged(const float4* st, int t0, int t1, float lr, float cell,
                                                      float4 (&acc)[G])
 {
     const bool on0 = t0 <= t1, on1 = t0 < t1;
-    const int i0 = on0 ? t0 : 0, i1 = on1 ? t0 + 1 : 0;
-    const float c0 = siddon_cell_weight(st[G * CAP + i0], lr, cell);
-    const float c1 = siddon_cell_weight(st[G * CAP + i1], lr, cell);
+    const int i0 = on0 ? t0 : CAP, i1 = on1 ? t0 + 1 : CAP;
+    constexpr int CS = stage_pitch(CAP);
+    const float c0 = siddon_cell_weight(st[G * CS + i0], lr, cell);
+    const float c1 = siddon_cell_weight(st[G * CS + i1], lr, cell);
     const float w0 = on0 ? c0 : 0.0f, w1 = on1 ? c1 : 0.0f;
     #pragma unroll
-    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + i0], w0);
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CS + i0], w0);
     #pragma unroll
-    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + i1], w1);
+    for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CS + i1], w1);
     for (int t = t0 + 2; t <= t1; ++t) {
-        const float w = siddon_cell_weight(st[G * CAP + t], lr, cell);
+        const float w = siddon_cell_weight(st[G * CS + t], lr, cell);
         #pragma unroll
-        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], w);
+        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CS + t], w);
     }
 }
 
@@ -1027,16 +1031,15 @@ __device__ __forceinline__ void siddon_bp_tile1(const FanK& g, const float4* __r
 // groups' values and the window's bin edges, (A, B) of one edge ray per entry,
 // each edge shared by the two bins it separates.  As in k_siddon_fan_bp_tile: CAP
 // bins at a time, loaded one step (a view, or a further CAP bins of it) ahead into
-// registers, no barrier (a wave touches only its rows), rows cleared at the start so
-// that lanes without a bin read zeros or an earlier view's bins with weight 0, never
-// unwritten memory.
+// registers, no barrier (a wave touches only its rows), rows cleared at the start
+// (lanes without a bin read a row's zero entry).
 //
 // The views are summed in kBpSegs fixed segments whose sums are then added
 // in order, one wave each, so that a batch and its slices alone give the same bits.
 template <int G, int CAP>
 struct DdAdjStage {
-    static constexpr int kVals = G * CAP;                  // float4: the groups' bins
-    static constexpr int kEdges = (CAP + 2) / 2;           // float4: CAP + 1 edges of 8 bytes
+    static constexpr int kVals = G * stage_pitch(CAP);     // float4: the groups' bins
+    static constexpr int kEdges = (CAP + 3) / 2;           // float4: CAP + 1 edges of 8 bytes and one unused
     static constexpr int kFloat4 = kVals + kEdges;         // LDS of one wave
 };
 
@@ -1048,7 +1051,7 @@ template <int G, int CAP, int NB, bool WIDE>
 __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, float lr, float cell, float up,
                                               float4 (&acc)[G])
 {
-    const float2* edge = reinterpret_cast<const float2*>(st + G * CAP);
+    const float2* edge = reinterpret_cast<const float2*>(st + DdAdjStage<G, CAP>::kVals);
     const float c1 = cell + 1.0f, lu = lr + 1.0f;
     const int ts = t1 >= t0 ? t0 : 0;
     float2 e = edge[ts];
@@ -1072,13 +1075,13 @@ __device__ __forceinline__ void dd_adj_gather(const float4* st, int t0, int t1, 
         const float wt = weight(b0, b1, p0, p1);
         const float w = on ? wt : 0.0f;
         #pragma unroll
-        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * CAP + t], w);
+        for (int q = 0; q < G; ++q) vmadd(acc[q], st[q * stage_pitch(CAP) + t], w);
         a0 = b0; a1 = b1; q0 = p0; q1 = p1;
     };
     #pragma unroll
     for (int j = 0; j < NB; ++j) {
         const bool on = t0 + j <= t1;
-        bin(on ? t0 + j : 0, on);
+        bin(on ? t0 + j : CAP, on);
     }
     for (int t = t0 + NB; t <= t1; ++t) bin(t, true);
 }
@@ -1101,12 +1104,13 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
     const int ix = tx + (lane >> 3), iy = ty + (lane & 7);
     const bool inside = ix < g.nx && iy < g.ny;
     const float yr = (float)iy - 0.5f * g.ny, xr = (float)ix - 0.5f * g.nx;
-    int bj[kLoads];
+    int bj[kLoads], slot[kLoads];   // slot: the zero entries of the rows before
     unsigned roff[kLoads];
     #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
         const int i = j * 64 + lane;
         bj[j] = i % CAP;
+        slot[j] = G == 1 ? 0 : i / CAP;
         roff[j] = (unsigned)(min(i / CAP, nq - 1) * sstride) * 16u;
     }
     float4 rg[kLoads];
@@ -1178,7 +1182,7 @@ __device__ __forceinline__ void dd_adj_tile(const FanK& g, const float4* __restr
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         #pragma unroll
         for (int j = 0; j < kLoads; ++j)
-            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane] = rg[j];
+            if (64 * (j + 1) <= G * CAP || j * 64 + lane < G * CAP) st[j * 64 + lane + slot[j]] = rg[j];
         if (lane < CAP + 1) reinterpret_cast<float2*>(st + S::kVals)[lane] = re;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }

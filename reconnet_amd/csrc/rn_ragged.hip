@@ -133,9 +133,10 @@ __global__ __launch_bounds__(64 * kBpSegs) void k_ragged_siddon_bp(const RagSlic
 //
 // Bound: as k_dd_fan_adj.  6 slices of 256^2 with 360 views, 6 of 384^2 with 720 and 4
 // of 512^2 with 1152: 1.84 ms, 2.4 with one wave per tile and all its views (the queue
-// then ended in a tail of 1152-view items).
+// then ended in a tail of 1152-view items).  80 registers let three workgroups share a
+// CU (81: two, 2.35 ms).
 template <bool WIDE>
-__global__ __launch_bounds__(64 * kBpSegs, 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl,
+__global__ __launch_bounds__(64 * kBpSegs, WIDE ? 6 : 4) void k_ragged_dd_adj(const RagSlice* __restrict__ sl, int nsl,
                                                                       int total, int* __restrict__ counter)
 {
     constexpr int G = kRagS / 4, CAP = 32;
