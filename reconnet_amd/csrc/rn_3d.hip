@@ -1597,7 +1597,7 @@ __global__ __launch_bounds__(256) void k_helical_bp(HelicalGeo h, const float* _
     // the taper's phase in revolutions: cos((q - Q) / (1 - Q) pi / 2) = cos(2 pi r),
     // r = (q - Q) / (4 (1 - Q)), by the hardware cosine (taper weights enter as
     // sum w P / sum w; its error is far below the parity bound)
-    const float tq = 0.25f / (1.0f - h.Q);
+    const float tq = 0.25f / (1.0f - h.Q), qlive = fmaxf(1.0f, h.Q);
     float acc[ZC];
     #pragma unroll
     for (int j = 0; j < ZC; ++j) acc[j] = 0.0f;
@@ -1628,14 +1628,14 @@ __global__ __launch_bounds__(256) void k_helical_bp(HelicalGeo h, const float* _
             const float zsl = fmaf(-sg, as, tv.w);
             // v / dv, and which voxels see it inside the taper
             float s[ZC];
-            float qmin = 2.0f, qmax = 0.0f;
+            float qmin = qlive, qmax = 0.0f;
             #pragma unroll
             for (int j = 0; j < ZC; ++j) {
                 s[j] = ((zc[j] - tv.z) - zsl) * mag;
                 qmin = fminf(qmin, fabsf(s[j]) * qs);
                 qmax = fmaxf(qmax, fabsf(s[j]) * qs);
             }
-            if (!__any(qmin < 1.0f)) continue;
+            if (!__any(qmin < qlive)) continue;
             const bool anytaper = __any(qmax > h.Q);
             const float pu = fmaf(u, idu, cu);
             const float fu = floorf(pu);
@@ -1664,12 +1664,12 @@ __global__ __launch_bounds__(256) void k_helical_bp(HelicalGeo h, const float* _
                 r1[j] = *reinterpret_cast<const PairF*>(pn + off);
             }
             #pragma unroll
-            for (int j = 0; j < ZC; ++j) w[j] = fabsf(s[j]) * qs < 1.0f ? 1.0f : 0.0f;
+            for (int j = 0; j < ZC; ++j) w[j] = 1.0f;
             if (anytaper) {
                 #pragma unroll
                 for (int j = 0; j < ZC; ++j) {
                     const float q = fabsf(s[j]) * qs, c = __builtin_amdgcn_cosf((q - h.Q) * tq);
-                    w[j] = q <= h.Q ? 1.0f : w[j] * c * c;
+                    w[j] = q <= h.Q ? 1.0f : (q < 1.0f ? c * c : 0.0f);   // (Q = 1: no taper, c is not a number)
                 }
             }
             #pragma unroll

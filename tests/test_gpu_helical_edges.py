@@ -2,7 +2,7 @@
 where its shortcuts can go wrong: rows and columns that fall off the detector on
 either side (a short detector, offsets of several cells), voxels that no view sees
 inside the taper, heights outside the scan, an odd and a single detector row, image
-sizes below and over a wave's 8 x 8 columns."""
+sizes below and over a wave's 8 x 8 columns, no taper at all (Q = 1)."""
 
 import numpy as np
 import pytest
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nx,ny,nz,nu,nv,off_u,off_v,vol_z0,zrot,m_pi,Q", [
     (7, 9, 5, 40, 9, 0.25, 0.0, 8.0, 12.0, 1, 0.5), (17, 8, 9, 12, 4, -3.0, 2.5, -6.0, 10.0, 1, 0.6),
     (12, 13, 3, 50, 1, 0.25, 0.25, 9.0, 3.0, 1, 0.5), (9, 9, 17, 33, 24, 0.0, -6.0, 30.0, 12.0, 2, 0.4),
-    (16, 16, 8, 48, 16, 0.3, -0.5, 10.0, -9.0, 1, 0.9),
+    (16, 16, 8, 48, 16, 0.3, -0.5, 10.0, -9.0, 1, 0.9), (10, 11, 6, 40, 12, 0.25, 0.0, 9.0, 11.0, 1, 1.0),
 ])
 def test_helical_bp_edges(nx, ny, nz, nu, nv, off_u, off_v, vol_z0, zrot, m_pi, Q):
     import oracle as orc
