@@ -1216,7 +1216,6 @@ using DdAdjFn = void (*)(const FanK&, const float4*, float*, int, hipStream_t);
 // groups of 4 slices per lane 1, 2, 4, 8; windows of 32 and 24 bins
 const DdAdjFn kDdAdj[] = {go_dd_adj<1, 32>, go_dd_adj<1, 24>, go_dd_adj<2, 32>, go_dd_adj<2, 24>,
                           go_dd_adj<4, 32>, go_dd_adj<4, 24>, go_dd_adj<8, 32>, go_dd_adj<8, 24>};
-constexpr int kNDdAdj = sizeof(kDdAdj) / sizeof(kDdAdj[0]);
 const DdBpFn kDdBp[] = {go_dd_bp<16, 16, 1>, go_dd_bp<8, 32, 1>, go_dd_bp<32, 8, 1>, go_dd_bp<8, 8, 1>,
                        go_dd_bp<8, 8, 4>,   go_dd_bp<16, 16, 4>, go_dd_bp<8, 8, 8>, go_dd_bp<16, 16, 8>,
                        go_dd_bp<8, 8, 16>};

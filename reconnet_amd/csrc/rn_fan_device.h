@@ -976,16 +976,6 @@ __device__ __forceinline__ void siddon_bp_pixel_slices(const FanK& g, const T* _
     else siddon_bp_views<T, NB, false, S>(g, prj, sstride, nsl, view0, nviews, ix, iy, acc);
 }
 
-// one pixel of one slice
-template <class T, int NB = 4>
-__device__ __forceinline__ T siddon_bp_pixel(const FanK& g, const T* __restrict__ prj, int view0, int nviews,
-                                             int ix, int iy)
-{
-    T acc[1];
-    siddon_bp_pixel_slices<T, NB, 1>(g, prj, 0, 1, view0, nviews, ix, iy, acc);
-    return acc[0];
-}
-
 // Views v0 .. v1 - 1 (rows of prj [view][nu], view0 + v in the tables) of one group of
 // slices for this lane's pixel of the tile whose first pixel is (tx, ty), gathered from
 // memory; every lane of the wave calls it.
