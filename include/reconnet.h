@@ -321,7 +321,8 @@ int rn_helical_rebin(const float* fan, float* par, int nBatches, int nChannels,
  * on the caller's stream and keep the fastest for the process; the choice
  * changes results by at most the rounding of a regrouped sum.  Enabled unless RECONNET_AUTOTUNE=0 or switched off
  * here.  rn_autotune_report writes "kernel a b c d e -> choice (ms ...)"
- * lines into buf (NUL-terminated, truncated to len) and returns the full
+ * lines (a seventh number follows e where equal sizes have several candidate
+ * lists) into buf (NUL-terminated, truncated to len) and returns the full
  * length. */
 int rn_autotune_enable(int on);
 int rn_autotune_report(char* buf, int len);

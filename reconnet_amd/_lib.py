@@ -94,7 +94,8 @@ def autotune_pin(kernel, candidate):
 
 def autotune(enable=None, reset=False):
     """Switch the launch-shape autotuner on/off, clear its cache, and return
-    its current choices as {(kernel, a, b, c, d, e): (choice, [ms per candidate])}."""
+    its current choices as {(kernel, a, b, c, d, e): (choice, [ms per candidate])}; a
+    seventh number in a key tells candidate lists of equal sizes apart."""
     h = lib()
     if enable is not None:
         check(h.rn_autotune_enable(1 if enable else 0), "rn_autotune_enable")

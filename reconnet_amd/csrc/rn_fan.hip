@@ -1249,7 +1249,7 @@ const DdBpQFn kDdBpTile[] = {go_dd_bp_tile<1, 32>, go_dd_bp_tile<1, 24>, go_dd_b
 // fewer; more groups than that last.  Groups are addressed with 32-bit byte offsets:
 // G of them have to fit.
 struct GroupOrder {
-    int idx[8], n = 0;
+    int idx[8] = {}, n = 0;
     GroupOrder(const FanK& g, int nslices)
     {
         const int nquads = cdiv(nslices, 4);
@@ -1386,9 +1386,11 @@ constexpr int kNSidBpFew = sizeof(kSidBpFew) / sizeof(kSidBpFew[0]);
 // fewest groups per lane that hold the batch first, then fewer, then more, where G
 // groups' rows fit 32-bit offsets; then the gathers, at kNSidBpTile + their index.
 struct SidBpOrder {
-    int idx[kNSidBpTile + kNSidBpQ], n = 0;
+    int idx[kNSidBpTile + kNSidBpQ] = {}, n = 0;
+    int layout;   // TuneKey::layout: the list depends on FanK::tile, which the sizes do not tell
     SidBpOrder(const FanK& g, int nslices, int nviews)
     {
+        layout = g.tile ? 1 : 2;
         const int nquads = cdiv(nslices, 4);
         auto add = [&](int lg) {
             if (!g.tile || (long)(1 << lg) * nviews * g.nu * 16L >= 0x7fffffffL) return;
@@ -1491,7 +1493,8 @@ void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, i
     if (nslices <= 0 || nviews <= 0) return;
     require_offsets32(g, nviews, sizeof(float4));
     const SidBpOrder order(g, nslices, nviews);
-    const int c = order.idx[tune_choose({TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, 1}, order.n, [&](int i) {
+    const TuneKey key{TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, order.layout};
+    const int c = order.idx[tune_choose(key, order.n, [&](int i) {
         go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
     }, st, true)];
     go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, st);
@@ -1517,7 +1520,8 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
     require_offsets32(g, nviews, sizeof(float4));
     const SidBpOrder order(g, nslices, nviews);
     // the launch shape is tuned on the plain backprojection (img_xy as its output)
-    const int c = order.idx[tune_choose({TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices}, order.n, [&](int i) {
+    const TuneKey key{TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices, order.layout};
+    const int c = order.idx[tune_choose(key, order.n, [&](int i) {
         go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
     }, st, true)];
     const bool fused = c < kNSidBpTile;

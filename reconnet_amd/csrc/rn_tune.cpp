@@ -73,8 +73,9 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
                                                 std::to_string(ncand));
             return pin->second;
         }
+        // (a choice timed in a list of another length would name another candidate, or none)
         auto it = s.cache.find(key);
-        if (it != s.cache.end()) return it->second.choice;
+        if (it != s.cache.end() && (int)it->second.ms.size() == ncand) return it->second.choice;
         if (ncand <= 1 || !may_tune || !enabled_locked(s)) return 0;
     }
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -105,8 +106,9 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
             break;
         }
     std::lock_guard<std::mutex> lk(s.mu);
-    auto res = s.cache.emplace(key, e);
-    return res.first->second.choice;
+    Entry& kept = s.cache[key];
+    if ((int)kept.ms.size() != ncand) kept = e;
+    return kept.choice;
 }
 
 void tune_set_enabled(bool on)
@@ -131,9 +133,10 @@ std::string tune_report()
     char line[512];
     for (const auto& kv : s.cache) {
         const TuneKey& k = kv.first;
-        int n = std::snprintf(line, sizeof line, "%d %d %d %d %d %d -> %d (", k.kernel, k.a, k.b, k.c, k.d, k.e,
-                              kv.second.choice);
+        int n = std::snprintf(line, sizeof line, "%d %d %d %d %d %d", k.kernel, k.a, k.b, k.c, k.d, k.e);
         out.append(line, n);
+        if (k.layout != 0) out += " " + std::to_string(k.layout);
+        out += " -> " + std::to_string(kv.second.choice) + " (";
         for (size_t i = 0; i < kv.second.ms.size(); i++) {
             // every digit of the float, so the report shows the values the choice compared
             n = std::snprintf(line, sizeof line, "%s%.9g", i ? " " : "", (double)kv.second.ms[i]);

@@ -5,7 +5,9 @@
 // launch of a key the tuner times every candidate with HIP events on the
 // caller's stream (one warm-up and three timed runs each) and keeps the first
 // candidate within 3 % of the fastest (candidates are listed in order of
-// preference); later launches of the key reuse it.  Candidates compute every
+// preference); later launches of the key reuse it.  A key names one candidate
+// list: whatever else decides the list (spacings, distances, the data layout)
+// goes into its layout number.  Candidates compute every
 // output element by the same per-element code; those that split an element's
 // sum over lanes or waves (interleaved Siddon and DD kernels) may round it
 // differently in its last bits.
@@ -26,7 +28,7 @@ namespace rn {
 struct TuneKey {
     int kernel;
     int a, b, c, d, e;
-    int layout = 0;   // one kernel id with several candidate lists: 1 = interleaved slices
+    int layout = 0;   // which of a kernel id's candidate lists, where the sizes do not say it
     bool operator<(const TuneKey& o) const;
 };
 
@@ -60,7 +62,8 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
 
 void tune_set_enabled(bool on);
 bool tune_enabled();
-// "kernel a b c d e -> choice (ms per candidate ...)" lines for every tuned key
+// "kernel a b c d e -> choice (ms per candidate ...)" lines for every tuned key; a
+// layout number other than 0 follows e
 std::string tune_report();
 void tune_reset();
 // Force candidate `candidate` for every key of `kernel` (a TuneKernel; a

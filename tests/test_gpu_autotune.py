@@ -297,3 +297,56 @@ def test_staged_dd_fbp_reads_nothing_outside_its_window():
     assert np.isfinite(out).all()
     for s in range(8):
         assert rel_l2(out[s], ref[s]) <= 1e-5, s
+
+
+def _other_spacing():
+    # sizes of one key: the second geometry's tiles are too large seen from the
+    # source for the tile kernels (FanK::tile)
+    from reconnet_amd.geometry import FanGeometry
+
+    return [FanGeometry(nx=48, ny=48, dx=d, dy=d, nu=70, nview=40, da=a, dsd=1085.6, dso=595.0)
+            for d, a in ((1.0, 1.2 / 1085.6), (10.0, 0.018))]
+
+
+def _lists(kernel):
+    # (candidates timed, choice) of every key of a kernel
+    from reconnet_amd._lib import autotune
+
+    return sorted((len(ms), choice) for k, (choice, ms) in autotune().items() if k[0] == kernel)
+
+
+def test_equal_sizes_with_and_without_tiles_keep_their_own_choice():
+    # the interleaved Siddon BP of two geometries of equal sizes, one with the tile
+    # kernels among its candidates and one without, in one process: a choice belongs to
+    # the list it was timed in.  1e-5: 40 views x 2 bins of FP32 terms, regrouped.
+    from reconnet_amd._lib import autotune
+    from reconnet_amd.sqs import OsSqsTV
+    from reconnet_amd.torch_ops import FanPlan
+
+    rng = np.random.default_rng(5)
+    geos = _other_spacing()
+    y = torch.from_numpy(rng.uniform(0, 1, (5, 70, 40)).astype(np.float32)).cuda()
+
+    def sqs(geo):
+        eng = OsSqsTV(geo, 4, 5)
+        eng.set_data(y)
+        eng.compute_norm()
+        eng.set_image(torch.zeros(5, 48, 48, device="cuda"))
+        eng.run_pass()
+        out = eng.image()
+        eng.close()
+        return out
+
+    runs = [lambda g: FanPlan(g).backward(y, "siddon"), sqs]
+    try:
+        autotune(enable=False, reset=True)
+        refs = [[run(g) for g in geos] for run in runs]
+        for kernel, run, ref in zip((2, 9), runs, refs):
+            autotune(enable=True, reset=True)
+            for g, r in zip(geos + geos[:1], ref + ref[:1]):
+                assert float((run(g) - r).abs().max() / r.abs().max()) <= 1e-5
+            lists = _lists(kernel)
+            assert [n for n, _ in lists] == [10, 17], (kernel, lists)
+            assert all(0 <= c < n for n, c in lists), (kernel, lists)
+    finally:
+        autotune(enable=True, reset=True)
