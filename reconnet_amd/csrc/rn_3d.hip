@@ -1829,8 +1829,9 @@ void siddon_arb_bp(const ArbGeo& g, bool parallel, int nB, int nC, const float* 
         }
         check_launch("siddon_cone_bp");
     };
-    const int c = tune_choose({TK_SIDDON_CONE_BP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC}, 3, launch, st, true);
-    launch(c);
+    // (the list is the geometry's, not the sizes')
+    const TuneKey key{TK_SIDDON_CONE_BP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC, lists ? 0 : 1};
+    launch(tune_choose(key, 3, launch, st, true));
 }
 
 void dd_tomo_fp(const ArbGeo& g, int nB, int nC, const float* img, float* prj,
@@ -2032,9 +2033,9 @@ void ConePlan::dd_adj(int nB, int nC, const float* prj, float* img, DevBuf& work
         }
         check_launch("dd_cone_adj");
     };
-    const int c = tune_choose({TK_DD_CONE_ADJ, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC}, 6 - first, launch, st,
-                              true);
-    launch(c);
+    // (the list is the geometry's, not the sizes')
+    const TuneKey key{TK_DD_CONE_ADJ, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC, windows ? 0 : 1};
+    launch(tune_choose(key, 6 - first, launch, st, true));
 }
 
 void ConePlan::siddon_fp(int nB, int nC, const float* img, float* prj, DevBuf& work, hipStream_t st) const

@@ -350,3 +350,32 @@ def test_equal_sizes_with_and_without_tiles_keep_their_own_choice():
             assert all(0 <= c < n for n, c in lists), (kernel, lists)
     finally:
         autotune(enable=True, reset=True)
+
+
+def test_equal_cone_sizes_with_row_windows_and_row_sums_keep_their_own_choice():
+    # two cone plans of equal sizes, one whose DD adjoint may use row windows or row
+    # sums and one with more than 7 rows per voxel (row sums only), 300 planes: more than
+    # a workgroup's z range; against the oracle (1e-5, the parity bar)
+    import oracle as orc
+    from reconnet_amd._lib import autotune
+    from reconnet_amd.geometry import circular_cone_vectors
+    from reconnet_amd.torch_ops import ConePlan
+    from tests.helpers import rel_l2
+
+    nx, ny, nz, nu, nv, nview = 8, 7, 300, 20, 60, 8
+    p = np.random.default_rng(2).uniform(0, 1, (1, nu, nview, nv, 1)).astype(np.float32)
+    plans = []
+    for dz, dv, dso in ((0.5, 1.0, 120.0), (4.0, 0.5, 90.0)):
+        vecs = circular_cone_vectors(nview, dso, 200.0 + dso, th0=0.3)
+        geo = dict(dx=1.0, dy=1.0, dz=dz, du=1.3, dv=dv, off_u=0.0, off_v=0.0, cx=0.0, cy=0.0, cz=0.0)
+        plans.append((ConePlan(nx, ny, nz, 1.0, 1.0, dz, nu, nv, 1.3, dv, *vecs),
+                      orc.dd_cone_adj(p, *vecs, geo, (nx, ny, nz))))
+    try:
+        autotune(enable=True, reset=True)
+        for plan, ref in plans + plans[:1]:
+            assert rel_l2(plan.backward(torch.from_numpy(p).cuda(), "dd").cpu().numpy(), ref) <= 1e-5
+        lists = _lists(19)
+        assert [n for n, _ in lists] == [3, 6], lists
+        assert all(0 <= c < n for n, c in lists), lists
+    finally:
+        autotune(enable=True, reset=True)
