@@ -1070,57 +1070,69 @@ __global__ __launch_bounds__(256) void k_dd_cone_fp(ArbGeo a, Grid3K g, const fl
             const int cnt = __popcll(gm), n = (wave_max_nn(cnt) + 3) & ~3;
             if (on) {
                 const int pos = __popcll(gm & ((1ull << lg) - 1ull));
-                const int k = min(j + 1, nn - 1);
+                const int k = ob > 0.0f ? j + 1 : j;
                 const unsigned r1 = (unsigned)(vw.xv ? p * g.ny + j : j * g.ny + p);
                 const unsigned r2 = (unsigned)(vw.xv ? p * g.ny + k : k * g.ny + p);
                 const unsigned m = OFF32 ? (unsigned)g.nz * (unsigned)nC * 4u : 1u;
                 ent[pos] = make_float4(__uint_as_float(r1 * m), __uint_as_float(r2 * m), oa * ia, ob * ia);
                 emp[pos] = mp;
             }
-            // entries past the group's count: no weight, on a plane of the batch
+            // entries past the group's count: a cell of the volume, on a plane of the
+            // batch; their values (a NaN or an infinity among them) are dropped
             for (int i = cnt + lg; i < n; i += LV) {
                 ent[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 emp[i] = mpA;
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            // fours of entries that every group has, then the rest
+            auto walk = [&](auto add) {
+                int least = __builtin_amdgcn_readlane(cnt, 0), i = 0;
+                #pragma unroll
+                for (int k = 1; k < NG; ++k) least = min(least, __builtin_amdgcn_readlane(cnt, k * LV));
+                for (; i + 4 <= least; i += 4) {
+                    #pragma unroll
+                    for (int k = 0; k < 4; ++k) acc = add(i + k, acc);
+                }
+                for (; i < n; i += 4) {
+                    #pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float v = add(i + k, acc);
+                        acc = i + k < cnt ? v : acc;
+                    }
+                }
+            };
             if (two) {
-                for (int i = 0; i < n; i += 4) {
-                    #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const float4 e = ent[i + k];
-                        const float m = emp[i + k];
-                        const float z1 = fmaf(m, sl, vw.a0), fl = floorf(z1), h = fabsf(m) * aT3;
-                        const float w1 = fmaxf((z1 - fl) + h - 1.0f, 0.0f), w0 = h - w1;
-                        const char *pa = cell(e.x, (int)fl), *pb2 = cell(e.y, (int)fl);
-                        float a0, a1, b0, b1;
-                        if (C1) {
-                            const F2 x = *reinterpret_cast<const F2*>(pa), y = *reinterpret_cast<const F2*>(pb2);
-                            a0 = x[0]; a1 = x[1]; b0 = y[0]; b1 = y[1];
-                        } else {
-                            a0 = ld(pa); a1 = ld(pa + 4 * nC); b0 = ld(pb2); b1 = ld(pb2 + 4 * nC);
-                        }
-                        acc = fmaf(e.z, fmaf(a1, w1, a0 * w0), acc);
-                        acc = fmaf(e.w, fmaf(b1, w1, b0 * w0), acc);
+                walk([&](int i, float s) {
+                    const float4 e = ent[i];
+                    const float m = emp[i];
+                    const float z1 = fmaf(m, sl, vw.a0), fl = floorf(z1), h = fabsf(m) * aT3;
+                    const float w1 = fmaxf((z1 - fl) + h - 1.0f, 0.0f), w0 = h - w1;
+                    const char *pa = cell(e.x, (int)fl), *pb2 = cell(e.y, (int)fl);
+                    float a0, a1, b0, b1;
+                    if (C1) {
+                        const F2 x = *reinterpret_cast<const F2*>(pa), y = *reinterpret_cast<const F2*>(pb2);
+                        a0 = x[0]; a1 = x[1]; b0 = y[0]; b1 = y[1];
+                    } else {
+                        a0 = ld(pa); a1 = ld(pa + 4 * nC); b0 = ld(pb2); b1 = ld(pb2 + 4 * nC);
                     }
-                }
+                    return fmaf(e.w, fmaf(b1, w1, b0 * w0), fmaf(e.z, fmaf(a1, w1, a0 * w0), s));
+                });
             } else if (three) {
-                for (int i = 0; i < n; i += 4) {
-                    #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const float4 e = ent[i + k];
-                        const float m = emp[i + k];
-                        const float z1 = fmaf(m, sl, vw.a0), fl = floorf(z1), h = fabsf(m) * aT3;
-                        const float t = (z1 - fl) + h;
-                        const float w1 = __builtin_amdgcn_fmed3f(t - 1.0f, 0.0f, 1.0f), w2 = fmaxf(t - 2.0f, 0.0f);
-                        const float w0 = (h - w1) - w2;
-                        const char *pa = cell(e.x, (int)fl), *pb2 = cell(e.y, (int)fl);
-                        const float sa = fmaf(ld(pa + 8 * nC), w2, fmaf(ld(pa + 4 * nC), w1, ld(pa) * w0));
-                        const float sb = fmaf(ld(pb2 + 8 * nC), w2, fmaf(ld(pb2 + 4 * nC), w1, ld(pb2) * w0));
-                        acc = fmaf(e.w, sb, fmaf(e.z, sa, acc));
-                    }
-                }
+                walk([&](int i, float s) {
+                    const float4 e = ent[i];
+                    const float m = emp[i];
+                    const float z1 = fmaf(m, sl, vw.a0), fl = floorf(z1), h = fabsf(m) * aT3;
+                    const float t = (z1 - fl) + h;
+                    const float w1 = __builtin_amdgcn_fmed3f(t - 1.0f, 0.0f, 1.0f), w2 = fmaxf(t - 2.0f, 0.0f);
+                    const float w0 = (h - w1) - w2;
+                    const char *pa = cell(e.x, (int)fl), *pb2 = cell(e.y, (int)fl);
+                    const float sa = fmaf(ld(pa + 8 * nC), w2, fmaf(ld(pa + 4 * nC), w1, ld(pa) * w0));
+                    const float sb = fmaf(ld(pb2 + 8 * nC), w2, fmaf(ld(pb2 + 4 * nC), w1, ld(pb2) * w0));
+                    return fmaf(e.w, sb, fmaf(e.z, sa, s));
+                });
             } else {
                 for (int i = 0; i < n; ++i) {
+                    if (i >= cnt) continue;
                     const float4 e = ent[i];
                     const float m = emp[i];
                     const float y0 = fmaf(m, sl0, vw.a0), y1 = fmaf(m, sl1, vw.a0);
@@ -1133,7 +1145,8 @@ __global__ __launch_bounds__(256) void k_dd_cone_fp(ArbGeo a, Grid3K g, const fl
                         sa = fmaf(ld(cell(e.x, k)), oz, sa);
                         sb = fmaf(ld(cell(e.y, k)), oz, sb);
                     }
-                    acc = fmaf(e.w, sb, fmaf(e.z, sa, acc));
+                    acc = fmaf(e.z, sa, acc);
+                    if (e.w != 0.0f) acc = fmaf(e.w, sb, acc);
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");

@@ -115,3 +115,28 @@ def test_cone_forward_paths(nx, ny, nz, dz, nu, nv, du, dv, nview, dso, nc):
             assert rel_l2(plan.forward(torch.from_numpy(x).cuda(), "dd").cpu().numpy(), ref) <= 1e-5, c
     finally:
         autotune_pin("dd_cone_fp", None)
+
+
+def test_cone_forward_keeps_a_nan_in_its_rays():
+    # a NaN (or infinite) voxel reaches the rays that meet it or a cell next to it
+    # (those of a volume of ones around it, 0 elsewhere) and no others, the corner
+    # columns of the volume among the voxels
+    from reconnet_amd.torch_ops import ConePlan
+
+    n, nz = 21, 16
+    vecs = circular_cone_vectors(7, 120.0, 200.0, th0=0.3)
+    plan = ConePlan(n, n, nz, 1.0, 1.0, 1.0, 50, 18, 1.0, 1.0, *vecs)
+    x = torch.rand((1, n, n, nz, 1), device="cuda")
+    ref = plan.forward(x, "dd")
+    for ix, iy in ((0, 0), (0, n - 1), (n - 1, 0), (10, 10)):
+        for bad in (float("nan"), float("inf")):
+            z = x.clone()
+            z[0, ix, iy, 7, 0] = bad
+            near = torch.zeros_like(x)
+            near[0, max(ix - 1, 0):ix + 2, max(iy - 1, 0):iy + 2, 5:10] = 1.0
+            met = plan.forward(near, "dd") > 0
+            out = plan.forward(z, "dd")
+            assert bool((~met).any()) and torch.equal(out[~met], ref[~met]), (ix, iy, bad)
+            hit = torch.zeros_like(x)
+            hit[0, ix, iy, 7, 0] = 1.0
+            assert not bool(torch.isfinite(out[plan.forward(hit, "dd") > 0]).any())
