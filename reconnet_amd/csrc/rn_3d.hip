@@ -2012,7 +2012,9 @@ void ConePlan::dd_adj(int nB, int nC, const float* prj, float* img, DevBuf& work
     // are better taken from two row sums; the windows of one slice in 4 GiB);
     // 3-5: 1, 2 or 4 voxels per lane from the row-sum table
     const int nvp = g.nv + kConePad + 4;
-    const bool windows = ds_max_ <= kConeMaxDs && (long)g.nu * g.nview * nvp * 4L < (1L << 32);
+    // (the kernel's FP32 value of ds_max_, 4e-7 off at most, stays below kConeMaxDs too: it
+    // drops columns beyond, and two chunks of 4 rows hold a voxel's)
+    const bool windows = ds_max_ <= kConeMaxDs * (1.0 - 1e-5) && (long)g.nu * g.nview * nvp * 4L < (1L << 32);
     const int first = windows ? 0 : 3;
     auto launch = [&](int i) {
         const int c = first + i;
