@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * kBpSegs) void k_ragged_siddon_bp(const RagSlic
 // DD adjoint: pa holds the descriptor's kRagS slices as kRagS / 4 interleaved
 // groups (multiplied by the rays' length per line); a workgroup takes one tile, its
 // kBpSegs waves one view segment each (dd_adj_tile), and adds the segments' sums
-// in order.  WIDE: FanK::dwide of every descriptor.
+// in order.  WIDE: FanK::dwide of the launch's descriptors.
 //
 // Bound: as k_dd_fan_adj.  6 slices of 256^2 with 360 views, 6 of 384^2 with 720 and 4
 // of 512^2 with 1152: 1.84 ms, 2.4 with one wave per tile and all its views (the queue
@@ -320,10 +320,18 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
     float4* Q = p_->wq.as<float4>();
     p_->host.clear();
     const int chunk = siddon ? kRagSidBp : kRagS;
-    bool wide = true;
-    int item = 0;
+    // the DD adjoint's descriptors by FanK::dwide, a launch for each kind: a slice's bits
+    // depend on its own geometry only
+    std::vector<int> order = p_->order;
+    int nwide = nd;
+    if (!siddon)
+        nwide = (int)(std::stable_partition(order.begin(), order.end(), [&](int k) {
+                    return p_->tables[p_->first[k]].k.dwide != 0;
+                }) - order.begin());
+    int items[2] = {0, 0}, split = 0;   // per launch; the second one's first descriptor
     for (int k = 0; k < nd; k++) {
-        const int s = p_->first[p_->order[k]], cnt = p_->count[p_->order[k]];
+        int& item = items[k < nwide ? 0 : 1];
+        const int s = p_->first[order[k]], cnt = p_->count[order[k]];
         const FanGeo& g = p_->tables[s].geo;
         if (siddon) launch_pack_quads(prj + p_->sino_off[s], nullptr, Q, g.nu, g.nview, cnt, false, st);
         else launch_pack_quads_len(p_->tables[s].k, prj + p_->sino_off[s], Q, cnt, st);
@@ -331,7 +339,6 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
         for (int c0 = 0; c0 < cnt; c0 += chunk) {
             RagSlice d{};
             d.g = p_->tables[s].k;
-            wide = wide && d.g.dwide;
             d.nsl = std::min(chunk, cnt - c0);
             d.pa = reinterpret_cast<const float*>(Q + c0 / 4 * sino);
             d.pb = nullptr;
@@ -343,17 +350,23 @@ void RaggedBatch::backward(bool siddon, const float* prj, float* img, hipStream_
             p_->host.push_back(d);
         }
         Q += (long)((cnt + 3) / 4) * sino;
+        if (k < nwide) split = (int)p_->host.size();
     }
     const int nbd = (int)p_->host.size();
     RN_HIP_CHECK(hipMemcpyAsync(p_->desc.get(), p_->host.data(), nbd * sizeof(RagSlice), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, p_->counter.as<int>());
-    if (siddon)
-        hipLaunchKernelGGL(k_ragged_siddon_bp, dim3(persistent_blocks()), dim3(64, kBpSegs), 0, st,
-                           p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
-    else
-        hipLaunchKernelGGL(wide ? k_ragged_dd_adj<true> : k_ragged_dd_adj<false>, dim3(persistent_blocks()),
-                           dim3(64, kBpSegs), 0, st, p_->desc.as<RagSlice>(), nbd, item, p_->counter.as<int>());
-    check_launch("ragged_bp");
+    auto launch = [&](auto kern, int d0, int d1, int total) {
+        if (d1 == d0) return;
+        hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, p_->counter.as<int>());
+        hipLaunchKernelGGL(kern, dim3(persistent_blocks()), dim3(64, kBpSegs), 0, st, p_->desc.as<RagSlice>() + d0,
+                           d1 - d0, total, p_->counter.as<int>());
+        check_launch("ragged_bp");
+    };
+    if (siddon) {
+        launch(k_ragged_siddon_bp, 0, nbd, items[0]);
+    } else {
+        launch(k_ragged_dd_adj<true>, 0, split, items[0]);
+        launch(k_ragged_dd_adj<false>, split, nbd, items[1]);
+    }
     RN_HIP_CHECK(hipStreamSynchronize(st));
 }
 

@@ -51,3 +51,21 @@ def test_transpose_and_batch(nx, ny, d, nu, s, nview, slices):
     lhs = (ax.double() * y.double()).sum((1, 2))
     rhs = (x.double() * outs[0].double()).sum((1, 2))
     assert float(((lhs - rhs).abs() / lhs.abs()).max()) <= 2e-6
+
+
+def test_ragged_batch_of_ordinary_and_very_long_images_equals_single_slices():
+    # a slice whose image reaches past the source's line in some view (870 mm of 1190:
+    # FanK::dwide is 0) leaves the bits of the others as those of calls of their own
+    from reconnet_amd.geometry import FanGeometry
+    from reconnet_amd.ragged import RaggedFanBatch
+    from reconnet_amd.torch_ops import FanPlan
+
+    a, b = (FanGeometry(nx=nx, ny=ny, dx=1.0, dy=dy, nu=140, nview=33, da=da, dsd=1085.6, dso=595.0)
+            for nx, ny, dy, da in ((48, 48, 1.0, 1.2 / 1085.6), (8, 64, 13.6, 0.0143)))
+    geos = [a, b, a, a, b]
+    rng = np.random.default_rng(8)
+    ys = [torch.from_numpy(rng.uniform(0, 1, (g.nu, g.nview)).astype(np.float32)).cuda() for g in geos]
+    out = RaggedFanBatch(geos).backward(torch.cat([y.reshape(-1) for y in ys]), "dd")
+    for g, y, o in zip(geos, ys, out.split([g.nx * g.ny for g in geos])):
+        one = FanPlan(g).backward(y[None].contiguous(), "dd_adjoint").reshape(-1)
+        assert torch.equal(o, one), (g.nx, float((o - one).abs().max()))
