@@ -1639,16 +1639,18 @@ __global__ __launch_bounds__(256) void k_helical_bp(HelicalGeo h, const float* _
             // source height zk - zr2pi asin(u / dso) as tv.z + zsl (tv.z exact in
             // float, so that z - tv.z loses nothing to the source's turn height)
             const float zsl = fmaf(-sg, as, tv.w);
-            // v / dv, and which voxels see it inside the taper
+            // v / dv, and which voxels see it inside the taper or on its bound (beyond the
+            // source's circle u > dso: not numbers, as the sum then)
             float s[ZC];
-            float qmin = qlive, qmax = 0.0f;
+            float qmin, qmax;
             #pragma unroll
             for (int j = 0; j < ZC; ++j) {
                 s[j] = ((zc[j] - tv.z) - zsl) * mag;
-                qmin = fminf(qmin, fabsf(s[j]) * qs);
-                qmax = fmaxf(qmax, fabsf(s[j]) * qs);
+                const float q = fabsf(s[j]) * qs;
+                qmin = j == 0 ? q : fminf(qmin, q);
+                qmax = j == 0 ? q : fmaxf(qmax, q);
             }
-            if (!__any(qmin < qlive)) continue;
+            if (__all(qmin > qlive)) continue;
             const bool anytaper = __any(qmax > h.Q);
             const float pu = fmaf(u, idu, cu);
             const float fu = floorf(pu);
