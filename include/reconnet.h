@@ -322,8 +322,8 @@ int rn_helical_rebin(const float* fan, float* par, int nBatches, int nChannels,
  * changes results by at most the rounding of a regrouped sum.  Enabled unless RECONNET_AUTOTUNE=0 or switched off
  * here.  rn_autotune_report writes "kernel a b c d e -> choice (ms ...)"
  * lines (a seventh number follows e where equal sizes have several candidate
- * lists) into buf (NUL-terminated, truncated to len) and returns the full
- * length. */
+ * lists; inf ms: not a choice for these sizes) into buf (NUL-terminated,
+ * truncated to len) and returns the full length. */
 int rn_autotune_enable(int on);
 int rn_autotune_report(char* buf, int len);
 int rn_autotune_reset(void);

@@ -95,7 +95,8 @@ def autotune_pin(kernel, candidate):
 def autotune(enable=None, reset=False):
     """Switch the launch-shape autotuner on/off, clear its cache, and return
     its current choices as {(kernel, a, b, c, d, e): (choice, [ms per candidate])}; a
-    seventh number in a key tells candidate lists of equal sizes apart."""
+    seventh number in a key tells candidate lists of equal sizes apart.  Candidates
+    that would round a sum differently are not timed: inf."""
     h = lib()
     if enable is not None:
         check(h.rn_autotune_enable(1 if enable else 0), "rn_autotune_enable")

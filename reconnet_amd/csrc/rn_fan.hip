@@ -1336,6 +1336,18 @@ const SidFpQPFn kSidFpQP[] = {go_siddon_fp_qp<64, kXcds, 1, 2>,  go_siddon_fp_qp
                               go_siddon_fp_qp<128, kXcds, 2>,    go_siddon_fp_qp<64, kXcds, 2, 2>,
                               go_siddon_fp_qp<128, kXcds, 2, 2>, go_siddon_fp_qp<128, 0, 2>};
 constexpr int kNSidFpQP = sizeof(kSidFpQP) / sizeof(kSidFpQP[0]);
+// the shapes with a ray's lines split over 2 and over 4 lanes (bit i: candidate i)
+constexpr uint32_t kSidFpQ2 = 0x7, kSidFpQ4 = 0x8, kSidFpQP2 = 0x1807, kSidFpQP4 = 0x18;
+// The split is the sizes', not the tuner's: it decides the last bits.  4 lanes per ray,
+// or 2 where the lines are long and the chip is full without: ms with 2 and with 4,
+// 256^2 x 16, 360 views 0.147, 0.143; 383^2 x 6, 520 views 0.144, 0.139; 512^2 x 32, 96
+// views (weighted residual) 0.228, 0.262; 512^2 x 4, 1152 views 0.326, 0.342; one slice of
+// 64^2, 15 views 0.012, 0.005.
+bool split4(const FanK& g, int nslices, int nviews)
+{
+    const int nl = std::max(g.nx, g.ny);
+    return nl < 400 || (double)cdiv(nslices, 4) * nviews * g.nu * nl < 2.5e8;
+}
 // per-pixel gathers, for every geometry
 const SidBpQFn kSidBpQ[] = {go_siddon_bp_q<16, 16, 2, 8>, go_siddon_bp_q<8, 8, 2, 8>, go_siddon_bp_q<16, 16, 2, 4>,
                             go_siddon_bp_q<8, 8, 2, 4>,   go_siddon_bp_q<8, 8, 2, 2>, go_siddon_bp_q<16, 16, 2, 2>,
@@ -1470,7 +1482,7 @@ void launch_siddon_fan_fp_residual_q(const FanK& g, const float4* Qyx, const flo
     const int nq = cdiv(nslices, 4);
     const int c = tune_choose({TK_SIDDON_FP_Q, g.nx, g.ny, g.nu, nviews, nslices}, kNSidFpQ, [&](int i) {
         kSidFpQ[i](g, Qyx, Qxy, res_q, nq, view0, nviews, meas_q, w_q, res_vstride, res_voff, st);
-    }, st, true);
+    }, st, true, split4(g, nslices, nviews) ? kSidFpQ4 : kSidFpQ2);
     kSidFpQ[c](g, Qyx, Qxy, res_q, nq, view0, nviews, meas_q, w_q, res_vstride, res_voff, st);
     check_launch("siddon_fan_fp_residual_q");
 }
@@ -1482,7 +1494,8 @@ void launch_siddon_fan_fp_q(const FanK& g, const float4* Qyx, const float4* Qxy,
     require_offsets32(g, nviews, sizeof(float));
     RN_REQUIRE(qplanes_fit32(g.nx, g.ny), "padded image plane of one slice group exceeds 2 GiB");
     const int c = tune_choose({TK_SIDDON_FP, g.nx, g.ny, g.nu, nviews, nslices, 1}, kNSidFpQP,
-                              [&](int i) { kSidFpQP[i](g, Qyx, Qxy, prj_vu, nslices, view0, nviews, st); }, st, true);
+                              [&](int i) { kSidFpQP[i](g, Qyx, Qxy, prj_vu, nslices, view0, nviews, st); }, st, true,
+                              split4(g, nslices, nviews) ? kSidFpQP4 : kSidFpQP2);
     kSidFpQP[c](g, Qyx, Qxy, prj_vu, nslices, view0, nviews, st);
     check_launch("siddon_fan_fp_q");
 }

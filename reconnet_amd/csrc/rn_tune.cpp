@@ -2,6 +2,7 @@
 
 #include "rn_tune.h"
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -61,9 +62,12 @@ struct Events {
 } // namespace
 
 int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& launch, hipStream_t st,
-                bool may_tune)
+                bool may_tune, uint32_t pick)
 {
     State& s = state();
+    int first = 0;
+    while (first < 31 && !(pick >> first & 1u)) first++;
+    RN_REQUIRE(ncand <= 32 && first < ncand, "no launch candidate to choose");
     {
         std::lock_guard<std::mutex> lk(s.mu);
         auto pin = s.pinned.find(key.kernel);
@@ -76,18 +80,19 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
         // (a choice timed in a list of another length would name another candidate, or none)
         auto it = s.cache.find(key);
         if (it != s.cache.end() && (int)it->second.ms.size() == ncand) return it->second.choice;
-        if (ncand <= 1 || !may_tune || !enabled_locked(s)) return 0;
+        if (ncand <= 1 || !may_tune || !enabled_locked(s)) return first;
     }
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     RN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
-    if (cap != hipStreamCaptureStatusNone) return 0;
+    if (cap != hipStreamCaptureStatusNone) return first;
 
     Entry e;
-    e.ms.assign(ncand, 0.0f);
+    e.ms.assign(ncand, INFINITY);
     Events ev;
     constexpr int reps = 3;
-    float best = 0.0f;
-    for (int i = 0; i < ncand; i++) {
+    float best = INFINITY;
+    for (int i = first; i < ncand; i++) {
+        if (!(pick >> i & 1u)) continue;
         launch(i);   // warm-up (instruction cache, tables)
         RN_HIP_CHECK(hipEventRecord(ev.a, st));
         for (int r = 0; r < reps; r++) launch(i);
@@ -96,7 +101,7 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
         float ms = 0.0f;
         RN_HIP_CHECK(hipEventElapsedTime(&ms, ev.a, ev.b));
         e.ms[i] = ms / reps;
-        if (i == 0 || e.ms[i] < best) best = e.ms[i];
+        if (e.ms[i] < best) best = e.ms[i];
     }
     // the first candidate within 3 % of the fastest: timing noise does not
     // move the choice away from the earlier-listed (preferred) shapes

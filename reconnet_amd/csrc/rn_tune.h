@@ -8,9 +8,11 @@
 // preference); later launches of the key reuse it.  A key names one candidate
 // list: whatever else decides the list (spacings, distances, the data layout)
 // goes into its layout number.  Candidates compute every
-// output element by the same per-element code; those that split an element's
-// sum over lanes or waves (interleaved Siddon and DD kernels) may round it
-// differently in its last bits.
+// output element by the same per-element code.  Those that split an element's
+// sum over lanes or waves round it differently in its last bits: where the list
+// has several splits, the launch says which candidates have the one its sizes
+// call for, and the choice is among those, so that a call's bits do not depend
+// on a timing.
 //
 // Tuning is skipped (the first candidate, or the cached choice, is used) when
 // the stream is being captured into a graph, when the launch accumulates into
@@ -19,6 +21,7 @@
 
 #include "rn_common.h"
 
+#include <cstdint>
 #include <functional>
 #include <string>
 #include <vector>
@@ -56,9 +59,11 @@ enum TuneKernel {
 
 // Returns the candidate index to launch for `key`; runs the timing when the
 // key is new and tuning is allowed.  `launch(i)` must enqueue candidate i on
-// `st` and be repeatable (its output overwritten, not accumulated).
+// `st` and be repeatable (its output overwritten, not accumulated).  pick: bit i
+// set if candidate i may be chosen; the others serve pins only, are not timed and
+// reported with inf ms.
 int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& launch, hipStream_t st,
-                bool may_tune);
+                bool may_tune, uint32_t pick = 0xffffffffu);
 
 void tune_set_enabled(bool on);
 bool tune_enabled();

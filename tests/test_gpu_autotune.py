@@ -379,3 +379,54 @@ def test_equal_cone_sizes_with_row_windows_and_row_sums_keep_their_own_choice():
         assert all(0 <= c < n for n, c in lists), lists
     finally:
         autotune(enable=True, reset=True)
+
+
+# operator, kernel name, nx, ny, nu, nview, slices
+SAME_BITS = [
+    ("siddon fp", "siddon_fp", 64, 50, 96, 90, 6), ("siddon fp", "siddon_fp", 250, 250, 367, 60, 16),
+    ("siddon fp", "siddon_fp", 400, 380, 300, 300, 32),
+]
+
+
+@pytest.mark.parametrize("op,kernel,nx,ny,nu,nview,slices", SAME_BITS)
+def test_shapes_the_tuner_may_choose_have_the_same_bits(op, kernel, nx, ny, nu, nview, slices):
+    # a choice by timing must not move a result: every candidate that was timed
+    # (the others report inf), and the tuner switched off
+    from reconnet_amd._lib import TUNED_KERNELS, autotune, autotune_pin
+    from reconnet_amd.geometry import FanGeometry
+    from reconnet_amd.sqs import OsSqsTV
+    from reconnet_amd.torch_ops import FanPlan
+
+    d = 350.0 / max(nx, ny)
+    geo = FanGeometry(nx=nx, ny=ny, dx=d, dy=d, nu=nu, nview=nview, da=0.9 / nu, dsd=1085.6, dso=595.0)
+    gen = torch.Generator(device="cuda").manual_seed(nu + slices)
+    rand = lambda *s: torch.rand(s, device="cuda", generator=gen)  # noqa: E731
+    x, y = rand(slices, nx, ny), rand(slices, nu, nview)
+    if op == "sqs":
+        eng = OsSqsTV(geo, 4, slices)
+        eng.set_data(100.0 * y, rand(slices, nu, nview))
+        eng.set_norm(1.0 + rand(slices, nx, ny))
+
+        def run():
+            eng.set_image(x)
+            eng.run_pass(lam=1e-3)
+            return eng.image()
+    else:
+        plan = FanPlan(geo)
+        kind, way = op.split()
+        run = {"fp": lambda: plan.forward(x, kind), "bp": lambda: plan.backward(y, kind)}[way]
+    try:
+        autotune(enable=False, reset=True)
+        ref = run()
+        autotune(enable=True, reset=True)
+        assert torch.equal(run(), ref)
+        for choice, ms in [v for k, v in autotune().items() if k[0] == TUNED_KERNELS[kernel]]:
+            timed = [c for c, m in enumerate(ms) if np.isfinite(m)]
+            assert choice in timed
+            for c in timed:
+                autotune_pin(kernel, c)
+                assert torch.equal(run(), ref), c
+            autotune_pin(kernel, None)
+    finally:
+        autotune_pin(kernel, None)
+        autotune(enable=True, reset=True)
