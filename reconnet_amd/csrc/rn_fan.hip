@@ -217,6 +217,7 @@ __global__ __launch_bounds__(BLK) void k_siddon_fan_fp_q(FanK g, const float4* _
         tile = l % tiles;
         vi = (l / tiles) % nviews;
         sg = l / (tiles * nviews);
+        if (sg * G >= (ns + 3) / 4) return;   // the grid is rounded up to whole rounds of XCDs
     } else {
         tile = blockIdx.x;
         vi = blockIdx.y;
@@ -1280,9 +1281,10 @@ void run_siddon_fp_q(const FanK& g, const float4* Qyx, const float4* Qxy, float4
 {
     const int ngroups = cdiv(cdiv(ns, 4), G);
     const long nblk = (long)cdiv(g.nu, BLK / H) * nviews * ngroups;
-    if (XCD > 0 && nblk % XCD == 0 && nblk <= 0x7fffffffL) {
-        hipLaunchKernelGGL((k_siddon_fan_fp_q<BLK, XCD, G, H, PLAIN>), dim3((unsigned)nblk), dim3(BLK), 0, st, g, Qyx,
-                           Qxy, res, prj, view0, nviews, ns, meas, w, g.nview, res_vstride, res_voff);
+    if (XCD > 0 && nblk + XCD <= 0x7fffffffL) {
+        const long n = cdiv(nblk, XCD > 0 ? XCD : 1) * (long)XCD;
+        hipLaunchKernelGGL((k_siddon_fan_fp_q<BLK, XCD, G, H, PLAIN>), dim3((unsigned)n), dim3(BLK), 0, st, g, Qyx, Qxy,
+                           res, prj, view0, nviews, ns, meas, w, g.nview, res_vstride, res_voff);
     } else {
         hipLaunchKernelGGL((k_siddon_fan_fp_q<BLK, 0, G, H, PLAIN>), dim3(cdiv(g.nu, BLK / H), nviews, ngroups),
                            dim3(BLK), 0, st, g, Qyx, Qxy, res, prj, view0, nviews, ns, meas, w, g.nview, res_vstride,
@@ -1339,14 +1341,13 @@ constexpr int kNSidFpQP = sizeof(kSidFpQP) / sizeof(kSidFpQP[0]);
 // the shapes with a ray's lines split over 2 and over 4 lanes (bit i: candidate i)
 constexpr uint32_t kSidFpQ2 = 0x7, kSidFpQ4 = 0x8, kSidFpQP2 = 0x1807, kSidFpQP4 = 0x18;
 // The split is the sizes', not the tuner's: it decides the last bits.  4 lanes per ray,
-// or 2 where the lines are long and the chip is full without: ms with 2 and with 4,
-// 256^2 x 16, 360 views 0.147, 0.143; 383^2 x 6, 520 views 0.144, 0.139; 512^2 x 32, 96
-// views (weighted residual) 0.228, 0.262; 512^2 x 4, 1152 views 0.326, 0.342; one slice of
-// 64^2, 15 views 0.012, 0.005.
+// or 2 where the lines are long and the rays fill the chip without.  ms with 2 and with
+// 4: one slice of 64^2, 15 views 0.012, 0.005; 256^2 x 16, 360 views 0.147, 0.143; 383^2
+// x 6, 520 views 0.144, 0.139; 512^2, 96 views, one slice 0.060, 0.035, 5 slices 0.070,
+// 0.071, 32 slices 0.228, 0.262; 462 x 512 x 5, 232 views of 328 0.093, 0.101.
 bool split4(const FanK& g, int nslices, int nviews)
 {
-    const int nl = std::max(g.nx, g.ny);
-    return nl < 400 || (double)cdiv(nslices, 4) * nviews * g.nu * nl < 2.5e8;
+    return std::max(g.nx, g.ny) < 480 || (long)cdiv(nslices, 4) * nviews * g.nu < 100000;
 }
 // per-pixel gathers, for every geometry
 const SidBpQFn kSidBpQ[] = {go_siddon_bp_q<16, 16, 2, 8>, go_siddon_bp_q<8, 8, 2, 8>, go_siddon_bp_q<16, 16, 2, 4>,

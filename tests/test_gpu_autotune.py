@@ -384,7 +384,7 @@ def test_equal_cone_sizes_with_row_windows_and_row_sums_keep_their_own_choice():
 # operator, kernel name, nx, ny, nu, nview, slices
 SAME_BITS = [
     ("siddon fp", "siddon_fp", 64, 50, 96, 90, 6), ("siddon fp", "siddon_fp", 250, 250, 367, 60, 16),
-    ("siddon fp", "siddon_fp", 400, 380, 300, 300, 32),
+    ("siddon fp", "siddon_fp", 480, 380, 301, 97, 15),
 ]
 
 
