@@ -256,9 +256,12 @@ __global__ __launch_bounds__(BLK) void k_siddon_fan_fp_q(FanK g, const float4* _
 
 // Quad-layout Siddon BP: one lane per pixel of G groups of 4 slices (one
 // float4 load per bin and group); writes the plain images of the real slices.
-template <int BX, int BY, int NB, int G>
+// SEG: the views in nseg segments, as many as the tile kernels' waves, whose sums are
+// added in order, with the same bits; else all views in one sum.
+template <int BX, int BY, int NB, int G, bool SEG>
 __global__ __launch_bounds__(BX * BY) void k_siddon_fan_bp_q(FanK g, const float4* __restrict__ prj,
-                                                         float* __restrict__ img, int view0, int nviews, int ns)
+                                                         float* __restrict__ img, int view0, int nviews, int ns,
+                                                         int nseg)
 {
     const int iy = blockIdx.x * BX + threadIdx.x;
     const int ix = blockIdx.y * BY + threadIdx.y;
@@ -267,8 +270,23 @@ __global__ __launch_bounds__(BX * BY) void k_siddon_fan_bp_q(FanK g, const float
     const int nq = min(G, nquads - q0);
     if (ix >= g.nx || iy >= g.ny) return;
     const long sstride = (long)nviews * g.nu;
+    const float4* P = prj + q0 * sstride;
     float4 acc[G];
-    siddon_bp_pixel_slices<float4, NB, G>(g, prj + q0 * sstride, sstride, nq, view0, nviews, ix, iy, acc);
+    if constexpr (SEG) {
+        float4 sum[G];
+        #pragma unroll 1
+        for (int seg = 0; seg < nseg; ++seg) {
+            const int v0 = (int)((long)nviews * seg / nseg), v1 = (int)((long)nviews * (seg + 1) / nseg);
+            siddon_bp_pixel_slices<float4, NB, G>(g, P + (long)v0 * g.nu, sstride, nq, view0 + v0, v1 - v0, ix, iy, sum);
+            #pragma unroll
+            for (int k = 0; k < G; ++k) {
+                if (seg == 0) acc[k] = sum[k];
+                else vadd(acc[k], sum[k]);
+            }
+        }
+    } else {
+        siddon_bp_pixel_slices<float4, NB, G>(g, P, sstride, nq, view0, nviews, ix, iy, acc);
+    }
     const long plane = (long)g.nx * g.ny, pix = (long)ix * g.ny + iy;
     #pragma unroll
     for (int k = 0; k < G; ++k) {
@@ -1309,16 +1327,19 @@ void go_siddon_fp_qp(const FanK& g, const float4* Qyx, const float4* Qxy, float*
     run_siddon_fp_q<BLK, XCD, G, H, true>(g, Qyx, Qxy, nullptr, prj, ns, view0, nviews, nullptr, nullptr, 0, 0, st);
 }
 
+// nseg: view segments of every pixel's sum
 template <int BX, int BY, int NB, int G>
-void go_siddon_bp_q(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
+void go_siddon_bp_q(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, int nseg,
+                    hipStream_t st)
 {
-    hipLaunchKernelGGL((k_siddon_fan_bp_q<BX, BY, NB, G>), dim3(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(cdiv(ns, 4), G)),
-                       dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns);
+    const auto k = nseg > 1 ? k_siddon_fan_bp_q<BX, BY, NB, G, true> : k_siddon_fan_bp_q<BX, BY, NB, G, false>;
+    hipLaunchKernelGGL(k, dim3(cdiv(g.ny, BX), cdiv(g.nx, BY), cdiv(cdiv(ns, 4), G)), dim3(BX, BY), 0, st, g, prj, img,
+                       view0, nviews, ns, nseg);
 }
 
 using SidFpQFn = void (*)(const FanK&, const float4*, const float4*, float4*, int, int, int, const float4*,
                           const float4*, int, int, hipStream_t);
-using SidBpQFn = void (*)(const FanK&, const float4*, float*, int, int, int, hipStream_t);
+using SidBpQFn = void (*)(const FanK&, const float4*, float*, int, int, int, int, hipStream_t);
 // G: groups of 4 slices per lane; H: parts of the line range per ray (the
 // split shortens the waves of a launch that would leave a partial second
 // round on the chip); candidates in order of preference (the tuner keeps the
@@ -1357,25 +1378,15 @@ const SidBpQFn kSidBpQ[] = {go_siddon_bp_q<16, 16, 2, 8>, go_siddon_bp_q<8, 8, 2
 constexpr int kNSidFpQ = sizeof(kSidFpQ) / sizeof(kSidFpQ[0]);
 constexpr int kNSidBpQ = sizeof(kSidBpQ) / sizeof(kSidBpQ[0]);
 
-using SidBpTileFn = void (*)(const FanK&, const float4*, float*, int, int, int, const SqsUpd*, bool, hipStream_t);
+using SidBpTileFn = void (*)(const FanK&, const float4*, float*, int, int, int, const SqsUpd*, int, hipStream_t);
 // u != nullptr: the OS-SQS update in the epilogue instead of img
-// few: kBpSegs waves per tile whatever its size, so that the bits do not depend on the
-// shape.  CAP = 0: the gathers of one group from memory.
+// nw: waves per tile, each with an even share of the views.  CAP = 0: the gathers of one
+// group from memory.
 template <int G, int CAP, int NB = 2>
 void go_siddon_bp_tile(const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, const SqsUpd* u,
-                       bool few, hipStream_t st)
+                       int nw, hipStream_t st)
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
-    // Waves per tile: up to 8 while they do not fill the chip (4096 of 4 and more
-    // groups, 4 a SIMD by their registers; more of the shorter ones of 1 and 2 groups)
-    // and each keeps 8 views, over which its batch of tile projections pays.  us with
-    // nw = 1, 2, 4, 8: one slice of 256^2, 30 views 23, 15, 12, 12, 360 views 279, 184,
-    // 133, 87; 5 slices of 512^2 (G = 2), 1152 views 1117, 1088, 941, 966; 32 slices of
-    // 250^2 (G = 8), 360 views 438, 251, 200, 255; of 512^2, 96 views 153, 177, 170, 202.
-    const long full = G <= 2 ? 16384 : 4096;
-    int nw = 1;
-    if (few) nw = kBpSegs;
-    while (nw < 8 && (long)grd.x * grd.y * grd.z * nw < full && nviews >= 8 * nw) nw *= 2;
     const size_t lds = ((CAP == 0 ? 0 : (size_t)nw * (G + 1) * stage_pitch(CAP)) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     const SqsUpd upd = u != nullptr ? *u : SqsUpd{};
     void (*k)(FanK, const float4*, float*, int, int, int, SqsUpd);
@@ -1401,25 +1412,43 @@ constexpr int kNSidBpFew = sizeof(kSidBpFew) / sizeof(kSidBpFew[0]);
 struct SidBpOrder {
     int idx[kNSidBpTile + kNSidBpQ] = {}, n = 0;
     int layout;   // TuneKey::layout: the list depends on FanK::tile, which the sizes do not tell
+    int nw = 1;   // view segments of every candidate's sums (a wave each by tiles)
     SidBpOrder(const FanK& g, int nslices, int nviews)
     {
         layout = g.tile ? 1 : 2;
         const int nquads = cdiv(nslices, 4);
+        const int best = nquads > 4 ? 3 : nquads > 2 ? 2 : nquads - 1;
+        // Waves per tile of the preferred shape: up to 8 while they do not fill the chip
+        // (4096 of 4 and more groups, 4 a SIMD by their registers; more of the shorter
+        // ones of 1 and 2 groups) or leave over 30 % of the last round idle, and each
+        // keeps 8 views, over which its batch of tile projections pays.  Every shape takes
+        // that many: the split decides the last bits.  us with 1, 2, 4, 8: one slice of
+        // 256^2, 30 views 23, 15, 12, 12, 360 views 279, 184, 133, 87; 5 slices of 512^2 (2
+        // groups), 1152 views 1117, 1088, 941, 966; 32 slices of 250^2 (8 groups), 360
+        // views 438, 251, 200, 255; of 383^2 (2304 tiles), 520 views 561, 513, 428, 399; of
+        // 512^2, 96 views 153, 177, 170, 202.  One where 4 and more groups meet bins wider
+        // than 1.6 pixels on half a chip of tiles: the gathers with one sum are the faster
+        // shape then (16 slices of 464 x 512, bins of 2.1 pixels: 248, tiles by 4 waves 324).
+        const long tiles = (long)cdiv(g.nx, 8) * cdiv(g.ny, 8) * cdiv(nquads, 1 << best);
+        const long full = best <= 1 ? 16384 : 4096;
+        auto more = [&](long w) { return w < full || (w < 4 * full && 10 * w < 7 * full * ((w + full - 1) / full)); };
+        const bool wide = best >= 2 && tiles >= 2048 && fabsf(g.da) * g.dso > 1.6f * std::max(g.dx, g.dy);
+        while (g.tile && !wide && nw < 8 && more(tiles * nw) && nviews >= 8 * nw) nw *= 2;
         auto add = [&](int lg) {
             if (!g.tile || (long)(1 << lg) * nviews * g.nu * 16L >= 0x7fffffffL) return;
             for (int i = lg == 0 ? 0 : 2 * lg - 1; i <= 2 * lg; i++) idx[n++] = i;
         };
-        const int best = nquads > 4 ? 3 : nquads > 2 ? 2 : nquads - 1;
         for (int lg = best; lg >= 0; lg--) add(lg);
         for (int lg = best + 1; lg < 4; lg++) add(lg);
         for (int i = 0; i < kNSidBpQ; i++) idx[n++] = kNSidBpTile + i;
     }
 };
 
-void go_siddon_bp_any(int c, const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, hipStream_t st)
+void go_siddon_bp_any(int c, const FanK& g, const float4* prj, float* img, int ns, int view0, int nviews, int nw,
+                      hipStream_t st)
 {
-    if (c < kNSidBpTile) kSidBpTile[c](g, prj, img, ns, view0, nviews, nullptr, false, st);
-    else kSidBpQ[c - kNSidBpTile](g, prj, img, ns, view0, nviews, st);
+    if (c < kNSidBpTile) kSidBpTile[c](g, prj, img, ns, view0, nviews, nullptr, nw, st);
+    else kSidBpQ[c - kNSidBpTile](g, prj, img, ns, view0, nviews, nw, st);
 }
 
 } // namespace
@@ -1509,9 +1538,9 @@ void launch_siddon_fan_bp_q(const FanK& g, const float4* prj_q, float* img_xy, i
     const SidBpOrder order(g, nslices, nviews);
     const TuneKey key{TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, order.layout};
     const int c = order.idx[tune_choose(key, order.n, [&](int i) {
-        go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
+        go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, order.nw, st);
     }, st, true)];
-    go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, st);
+    go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, order.nw, st);
     check_launch("siddon_fan_bp_q");
 }
 
@@ -1521,9 +1550,9 @@ void launch_siddon_fan_bp_few(const FanK& g, const float4* prj_q, float* img_xy,
     if (nslices <= 0 || nviews <= 0) return;
     require_offsets32(g, nviews, sizeof(float));
     const int c = tune_choose({TK_SIDDON_BP, g.nx, g.ny, g.nu, nviews, nslices, 1}, kNSidBpFew, [&](int i) {
-        kSidBpFew[i](g, prj_q, img_xy, nslices, view0, nviews, nullptr, true, st);
+        kSidBpFew[i](g, prj_q, img_xy, nslices, view0, nviews, nullptr, kBpSegs, st);
     }, st, true);
-    kSidBpFew[c](g, prj_q, img_xy, nslices, view0, nviews, nullptr, true, st);
+    kSidBpFew[c](g, prj_q, img_xy, nslices, view0, nviews, nullptr, kBpSegs, st);
     check_launch("siddon_fan_bp_few");
 }
 
@@ -1536,11 +1565,11 @@ bool launch_siddon_fan_bp_q_update(const FanK& g, const float4* prj_q, float* im
     // the launch shape is tuned on the plain backprojection (img_xy as its output)
     const TuneKey key{TK_SIDDON_BP_Q, g.nx, g.ny, g.nu, nviews, nslices, order.layout};
     const int c = order.idx[tune_choose(key, order.n, [&](int i) {
-        go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, st);
+        go_siddon_bp_any(order.idx[i], g, prj_q, img_xy, nslices, view0, nviews, order.nw, st);
     }, st, true)];
     const bool fused = c < kNSidBpTile;
-    if (fused) kSidBpTile[c](g, prj_q, nullptr, nslices, view0, nviews, &u, false, st);
-    else go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, st);
+    if (fused) kSidBpTile[c](g, prj_q, nullptr, nslices, view0, nviews, &u, order.nw, st);
+    else go_siddon_bp_any(c, g, prj_q, img_xy, nslices, view0, nviews, order.nw, st);
     check_launch("siddon_fan_bp_q_update");
     return fused;
 }

@@ -385,6 +385,11 @@ def test_equal_cone_sizes_with_row_windows_and_row_sums_keep_their_own_choice():
 SAME_BITS = [
     ("siddon fp", "siddon_fp", 64, 50, 96, 90, 6), ("siddon fp", "siddon_fp", 250, 250, 367, 60, 16),
     ("siddon fp", "siddon_fp", 480, 380, 301, 97, 15),
+    ("siddon bp", "siddon_bp", 64, 50, 96, 90, 6), ("siddon bp", "siddon_bp", 250, 250, 367, 60, 16),
+    ("siddon bp", "siddon_bp", 250, 250, 367, 40, 32), ("siddon bp", "siddon_bp", 400, 380, 120, 30, 5),
+    ("siddon bp", "siddon_bp", 40, 40, 60, 7, 33), ("sqs", "siddon_fp_q", 96, 70, 140, 60, 2),
+    ("sqs", "siddon_fp_q", 400, 490, 301, 300, 21), ("sqs", "siddon_bp_q", 96, 70, 140, 60, 2),
+    ("sqs", "siddon_bp_q", 400, 400, 180, 100, 32),
 ]
 
 
