@@ -1180,10 +1180,6 @@ void go_siddon_bp(const FanK& g, const float* prj, float* img, int ns, int view0
                        dim3(BX, BY), 0, st, g, prj, img, view0, nviews, ns, acc);
 }
 
-// DD BP: eight waves per tile while one would leave the 1024 SIMDs fewer than 8 waves
-// each (one slice of 512^2, 4096 waves: 0.73 ms by two, 0.65 by eight).
-constexpr long kDdBpWaves = 8192;
-
 template <int G, int CAP>
 void go_dd_adj(const FanK& g, const float4* wprj, float* img, int ns, hipStream_t st)
 {
@@ -1251,16 +1247,17 @@ const DdBpQFn kDdBpQ[] = {go_dd_bp_q<8, 8, 4>,   go_dd_bp_q<16, 16, 2>, go_dd_bp
                           go_dd_bp_q<16, 16, 1>, go_dd_bp_q<8, 8, 1>};
 constexpr int kNDdBpQ = sizeof(kDdBpQ) / sizeof(kDdBpQ[0]);
 
+// nw: waves per tile, each with an even share of the views
 template <int G, int CAP>
-void go_dd_bp_tile(const FanK& g, const float4* wprj, float* img, int ns, int fbp, hipStream_t st)
+void go_dd_bp_tile(const FanK& g, const float4* wprj, float* img, int ns, int fbp, int nw, hipStream_t st)
 {
     const dim3 grd(cdiv(g.ny, 8), cdiv(g.nx, 8), cdiv(cdiv(ns, 4), G));
-    const int nw = (long)grd.x * grd.y * grd.z < kDdBpWaves ? 8 : 1;
     const size_t lds = ((size_t)nw * G * stage_pitch(CAP) + (nw > 1 ? G * 64 : 0)) * sizeof(float4);
     hipLaunchKernelGGL((k_dd_fan_bp_tile<G, CAP>), grd, dim3(64, nw), lds, st, g, wprj, img, ns, fbp);
 }
+using DdBpTileFn = void (*)(const FanK&, const float4*, float*, int, int, int, hipStream_t);
 // groups of 4 slices per lane 1, 2, 4, 8; windows of 32 and 24 bins
-const DdBpQFn kDdBpTile[] = {go_dd_bp_tile<1, 32>, go_dd_bp_tile<1, 24>, go_dd_bp_tile<2, 32>, go_dd_bp_tile<2, 24>,
+const DdBpTileFn kDdBpTile[] = {go_dd_bp_tile<1, 32>, go_dd_bp_tile<1, 24>, go_dd_bp_tile<2, 32>, go_dd_bp_tile<2, 24>,
                              go_dd_bp_tile<4, 32>, go_dd_bp_tile<4, 24>, go_dd_bp_tile<8, 32>, go_dd_bp_tile<8, 24>};
 
 // Candidates of a kernel with G = 1, 2, 4, 8 groups per lane, two each, in the order
@@ -1269,6 +1266,7 @@ const DdBpQFn kDdBpTile[] = {go_dd_bp_tile<1, 32>, go_dd_bp_tile<1, 24>, go_dd_b
 // G of them have to fit.
 struct GroupOrder {
     int idx[8] = {}, n = 0;
+    long tiles;   // tiles times batches of groups of the preferred shape
     GroupOrder(const FanK& g, int nslices)
     {
         const int nquads = cdiv(nslices, 4);
@@ -1278,6 +1276,7 @@ struct GroupOrder {
             idx[n++] = 2 * lg + 1;
         };
         const int best = nquads > 4 ? 3 : nquads > 2 ? 2 : nquads - 1;
+        tiles = (long)cdiv(g.nx, 8) * cdiv(g.ny, 8) * cdiv(nquads, 1 << best);
         for (int lg = best; lg >= 0; lg--) add(lg);
         for (int lg = best + 1; lg < 4; lg++) add(lg);
     }
@@ -1644,12 +1643,16 @@ void launch_dd_fan_bp_tile(const FanK& g, const float4* wprj_q, float* img_xy, i
     if (nslices <= 0) return;
     require_offsets32(g, g.nview, nslices < 4 ? sizeof(float) : sizeof(float4));
     const GroupOrder order(g, nslices);
+    // Eight waves per tile while one of the preferred shape would leave the 1024 SIMDs
+    // fewer than 8 waves each (one slice of 512^2, 4096 waves: 0.73 ms by two, 0.65 by
+    // eight).  Every shape takes that many: the split decides the last bits.
+    const int nw = order.tiles < 8192 ? 8 : 1;
     // the kernel id of the layout the slices' count had without tiles
     const int id = nslices < 4 ? (fbp ? TK_DD_FBP : TK_DD_BP) : (fbp ? TK_DD_FBP_Q : TK_DD_BP_Q);
     const int c = tune_choose({id, g.nx, g.ny, g.nu, g.nview, nslices, 1}, order.n,
-                              [&](int i) { kDdBpTile[order.idx[i]](g, wprj_q, img_xy, nslices, fbp ? 1 : 0, st); }, st,
+                              [&](int i) { kDdBpTile[order.idx[i]](g, wprj_q, img_xy, nslices, fbp ? 1 : 0, nw, st); }, st,
                               true);
-    kDdBpTile[order.idx[c]](g, wprj_q, img_xy, nslices, fbp ? 1 : 0, st);
+    kDdBpTile[order.idx[c]](g, wprj_q, img_xy, nslices, fbp ? 1 : 0, nw, st);
     check_launch("dd_fan_bp_tile");
 }
 

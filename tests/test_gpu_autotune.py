@@ -389,7 +389,9 @@ SAME_BITS = [
     ("siddon bp", "siddon_bp", 250, 250, 367, 40, 32), ("siddon bp", "siddon_bp", 400, 380, 120, 30, 5),
     ("siddon bp", "siddon_bp", 40, 40, 60, 7, 33), ("sqs", "siddon_fp_q", 96, 70, 140, 60, 2),
     ("sqs", "siddon_fp_q", 400, 490, 301, 300, 21), ("sqs", "siddon_bp_q", 96, 70, 140, 60, 2),
-    ("sqs", "siddon_bp_q", 400, 400, 180, 100, 32),
+    ("sqs", "siddon_bp_q", 400, 400, 180, 100, 32), ("dd bp", "dd_bp", 64, 50, 96, 30, 3),
+    ("dd_fbp bp", "dd_fbp_q", 250, 250, 367, 60, 32), ("dd bp", "dd_bp_q", 250, 250, 367, 60, 32),
+    ("dd_fbp bp", "dd_fbp_q", 480, 500, 230, 40, 6), ("dd_fbp bp", "dd_fbp_q", 40, 40, 60, 7, 33),
 ]
 
 
