@@ -17,15 +17,17 @@ struct ArbGeo {
     // path.  Set by callers that hold the views on the host; 0 is always safe.
     int rows_z = 0;
     // rows_z views whose sources lie off the grid: a bound on the detector rows
-    // whose rays meet one voxel (arb_rows_per_voxel), for the cone
-    // backprojection's column lists; 0 (always safe) is no bound.
+    // whose rays meet one voxel, for the cone backprojection's column lists; 0 (always
+    // safe) is no bound.  z_reach: the voxels along z that a view's rows reach at the
+    // grid's centre, on average.  Both from arb_rows.
     float rows_per_voxel = 0.0f;
+    float z_reach = 0.0f;
 };
 
 bool arb_rows_along_z(const float* detU, const float* detV, int nview);
-// host arrays [nview][3]; 0 where the views are not upright or a source is on or near the grid
-float arb_rows_per_voxel(const ArbGeo& g, const float* detCenter, const float* detU, const float* detV,
-                         const float* src);
+// Sets rows_per_voxel and z_reach from host arrays [nview][3]; both 0 where the views
+// are not upright or a source is on or near the grid.
+void arb_rows(ArbGeo& g, const float* detCenter, const float* detU, const float* detV, const float* src);
 
 // Siddon with per-view detCenter / detU / detV and either invRayDir
 // (parallel, SiddonParallel.cu) or the source position (cone, SiddonCone.cu).

@@ -1742,10 +1742,11 @@ bool arb_rows_along_z(const float* detU, const float* detV, int nview)
     return true;
 }
 
-float arb_rows_per_voxel(const ArbGeo& g, const float* C, const float* U, const float* V, const float* S)
+void arb_rows(ArbGeo& g, const float* C, const float* U, const float* V, const float* S)
 {
-    if (!C || !S || !arb_rows_along_z(U, V, g.nview)) return 0.0f;
-    double most = 0.0;
+    g.rows_per_voxel = g.z_reach = 0.0f;
+    if (!C || !S || !arb_rows_along_z(U, V, g.nview)) return;
+    double most = 0.0, reach = 0.0;
     for (int v = 0; v < g.nview; v++) {
         const double dzs = std::fabs((double)V[3 * v + 2] * g.dv);
         // t of the grid's in-plane corners on the view's rays (1 on the detector): affine in (x, y)
@@ -1763,10 +1764,12 @@ float arb_rows_per_voxel(const ArbGeo& g, const float* C, const float* U, const 
         const double cz = std::fabs((double)C[3 * v + 2] - S[3 * v + 2]);
         const double steep = cz / dzs + 0.5 * g.nv + std::fabs((double)g.off_v) + 1.0;
         const double w = g.dz / (t * dzs) + steep * dt / t;
-        if (!(t > 0.02) || !(w <= 1e6)) return 0.0f;
+        if (!(t > 0.02) || !(w <= 1e6)) return;
         most = std::max(most, w);
+        reach += ((g.cx - (double)S[3 * v]) * nx + (g.cy - (double)S[3 * v + 1]) * ny) / A * dzs * g.nv / g.dz;
     }
-    return (float)most;
+    g.rows_per_voxel = (float)most;
+    g.z_reach = (float)(reach / g.nview);
 }
 
 void siddon_arb_fp(const ArbGeo& g, bool parallel, int nB, int nC, const float* img, float* prj,
@@ -1802,7 +1805,7 @@ void siddon_arb_bp(const ArbGeo& g, bool parallel, int nB, int nC, const float* 
         check_launch("siddon_arb_bp");
         return;
     }
-    // upright cone views: column lists with one (x, y) per 16, 8 or 32 lanes where
+    // upright cone views: column lists with one (x, y) per 8, 16 or 32 lanes where
     // a voxel meets few rows (and the windows of one slice fit 4 GiB), else 1, 2
     // or 4 voxels per lane testing every view
     const int nvp = g.nv + kConePad + 4;
@@ -1844,9 +1847,20 @@ void siddon_arb_bp(const ArbGeo& g, bool parallel, int nB, int nC, const float* 
         }
         check_launch("siddon_cone_bp");
     };
-    // (the list is the geometry's, not the sizes')
-    const TuneKey key{TK_SIDDON_CONE_BP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC, lists ? 0 : 1};
-    launch(tune_choose(key, 3, launch, st, true));
+    // Lanes per (x, y) of the lists: a batch of that many views makes a partial sum, so
+    // the geometry decides and not the tuner.  32, or 16 where the rows reach up to 15
+    // voxels (8 up to 6) or just over 32 and the (x, y) fill the chip.  ms with 8, 16
+    // and 32: 190 x 177 x 99, reach 27 1.25, 0.93, 0.95; 207 x 205 x 28, reach 7.7 0.65,
+    // 0.56, 0.87; 151^2 x 20, reach 5.5 0.49, 0.65, 1.03; 202^2 x 113, reach 31 0.94, 0.79,
+    // 0.84; 60^2 x 95, reach 26 0.16, 0.090, 0.065; 128^2 x 64 all reached 1.40, 1.20, 1.06.
+    const long waves = (long)g.nx * g.ny * nB * nC / 4;         // by 16 lanes
+    const float reach = std::min(g.z_reach, (float)g.nz);
+    int lz = 32;
+    if (waves >= 1100 && (reach <= 15.0f || (waves >= 4096 && reach > 30.0f && reach <= 36.0f))) lz = 16;
+    if (waves >= 4096 && reach <= (g.nz <= 8 ? 8.0f : 6.0f)) lz = 8;
+    const uint32_t pick = !lists ? 7u : lz == 16 ? 1u : lz == 8 ? 2u : 4u;
+    const TuneKey key{TK_SIDDON_CONE_BP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC, lists ? lz : 0};
+    launch(tune_choose(key, 3, launch, st, true, pick));
 }
 
 void dd_tomo_fp(const ArbGeo& g, int nB, int nC, const float* img, float* prj,
@@ -1966,7 +1980,7 @@ void ConePlan::setup(const ArbGeo& g, const float* C, const float* U, const floa
     RN_HIP_CHECK(hipStreamSynchronize(st));
     geo = g;
     geo.rows_z = arb_rows_along_z(U, V, n) ? 1 : 0;
-    geo.rows_per_voxel = arb_rows_per_voxel(g, C, U, V, S);
+    arb_rows(geo, C, U, V, S);
 }
 
 void ConePlan::dd_fp(int nB, int nC, const float* img, float* prj, hipStream_t st) const

@@ -376,7 +376,7 @@ void arb_call(const char* name, bool forward, int kind, float* out, const float*
     case 1: { // Siddon cone: v3 = src
         ArbGeo gz = g;
         gz.rows_z = arb_rows_along_z(v1, v2, g.nview) ? 1 : 0;
-        gz.rows_per_voxel = arb_rows_per_voxel(g, v0, v1, v2, v3);
+        arb_rows(gz, v0, v1, v2, v3);
         if (forward) siddon_arb_fp(gz, false, nB, nC, c.a.as<float>(), c.b.as<float>(), d0, d1, d2, d3, c.g, c.st());
         else siddon_arb_bp(gz, false, nB, nC, c.a.as<float>(), c.b.as<float>(), d0, d1, d2, d3, c.g, c.st());
         break;
@@ -477,7 +477,7 @@ extern "C" void cOSSQSConeAbitrary(float* res, const float* img, const float* pr
         RN_REQUIRE(nviewPerSubset > 0 && nSubsets > 0, "subset sizes must be positive");
         ArbGeo g = make_arb(nx, ny, nz, dx, dy, dz, cx, cy, cz, nu, nview, nv, du, dv, off_u, off_v);
         g.rows_z = arb_rows_along_z(detU, detV, nview) ? 1 : 0;
-        if (detCenter && src) g.rows_per_voxel = arb_rows_per_voxel(g, detCenter, detU, detV, src);
+        if (detCenter && src) arb_rows(g, detCenter, detU, detV, src);
         ThreadCtx& c = ctx();
         const size_t nimg = (size_t)nBatches * nx * ny * nz * nChannels;
         const size_t nprj = (size_t)nBatches * nu * nview * nv * nChannels, nvec = 3 * (size_t)nview;

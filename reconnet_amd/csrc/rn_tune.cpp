@@ -23,6 +23,12 @@ struct Entry {
     std::vector<float> ms;
 };
 
+// (a choice timed in a list of another length would name another candidate, or none)
+bool usable(const Entry& e, int ncand, uint32_t pick)
+{
+    return (int)e.ms.size() == ncand && (pick >> e.choice & 1u) != 0;
+}
+
 struct State {
     std::mutex mu;
     std::map<TuneKey, Entry> cache;
@@ -77,9 +83,8 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
                                                 std::to_string(ncand));
             return pin->second;
         }
-        // (a choice timed in a list of another length would name another candidate, or none)
         auto it = s.cache.find(key);
-        if (it != s.cache.end() && (int)it->second.ms.size() == ncand) return it->second.choice;
+        if (it != s.cache.end() && usable(it->second, ncand, pick)) return it->second.choice;
         if (ncand <= 1 || !may_tune || !enabled_locked(s)) return first;
     }
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -112,7 +117,7 @@ int tune_choose(const TuneKey& key, int ncand, const std::function<void(int)>& l
         }
     std::lock_guard<std::mutex> lk(s.mu);
     Entry& kept = s.cache[key];
-    if ((int)kept.ms.size() != ncand) kept = e;
+    if (!usable(kept, ncand, pick)) kept = e;
     return kept.choice;
 }
 

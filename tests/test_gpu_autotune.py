@@ -437,3 +437,27 @@ def test_shapes_the_tuner_may_choose_have_the_same_bits(op, kernel, nx, ny, nu, 
     finally:
         autotune_pin(kernel, None)
         autotune(enable=True, reset=True)
+
+
+@pytest.mark.parametrize("n,nz,nu,nv,height", [(20, 12, 30, 14, 12.0), (150, 20, 60, 8, 128.0), (70, 16, 40, 9, 128.0)])
+def test_cone_siddon_backprojection_has_the_same_bits_with_any_timing(n, nz, nu, nv, height):
+    # 32, 8 and 16 lanes per (x, y): the geometry's choice, whatever the tuner times
+    from reconnet_amd._lib import TUNED_KERNELS, autotune, autotune_pin
+    from reconnet_amd.geometry import circular_cone_vectors
+    from reconnet_amd.torch_ops import ConePlan
+
+    d = 256.0 / n
+    plan = ConePlan(n, n, nz, d, d, height / nz, nu, nv, 614.4 / nu, 64.0 / nv, *circular_cone_vectors(33, 595.0, 1085.6))
+    y = torch.rand((1, nu, 33, nv, 1), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
+    try:
+        autotune(enable=False, reset=True)
+        ref = plan.backward(y, "siddon")
+        autotune(enable=True, reset=True)
+        assert torch.equal(plan.backward(y, "siddon"), ref)
+        (choice, ms), = [v for k, v in autotune().items() if k[0] == TUNED_KERNELS["siddon_cone_bp"]]
+        for c in [c for c, m in enumerate(ms) if np.isfinite(m)]:
+            autotune_pin("siddon_cone_bp", c)
+            assert torch.equal(plan.backward(y, "siddon"), ref), c
+    finally:
+        autotune_pin("siddon_cone_bp", None)
+        autotune(enable=True, reset=True)
