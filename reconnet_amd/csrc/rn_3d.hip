@@ -1276,6 +1276,28 @@ __device__ __forceinline__ float cone_list_sum(const float4* list, int n, const 
     return sum;
 }
 
+// The same without the rows of weight 0: a NaN or an infinity there is not the voxel's.
+__device__ __forceinline__ float cone_list_sum_met(const float4* list, int n, const char* __restrict__ Q, float fz,
+                                                   float lo, float hi)
+{
+    float sum = 0.0f;
+    #pragma unroll 1
+    for (int i = 0; i < n; ++i) {
+        const float4 e = list[i];
+        const float s = fmaf(fz, e.z, e.y), r0 = floorf(s), f = s - r0, t = f + fabsf(e.z);
+        float d = 0.0f;
+        #pragma unroll 1
+        for (float j = 0.0f; j < t; j += 1.0f) {
+            const int r = (int)__builtin_amdgcn_fmed3f(r0 + j, lo, hi);
+            const unsigned off = __float_as_uint(e.w) + (unsigned)(r * 4);   // (r may be negative: added in 32 bits)
+            const float w = fminf(t - j, 1.0f) - (j == 0.0f ? f : 0.0f);
+            d = fmaf(w, *reinterpret_cast<const float*>(Q + off), d);
+        }
+        sum = e.x != 0.0f ? fmaf(e.x, d, sum) : sum;
+    }
+    return sum;
+}
+
 template <int LZ>
 __global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g, const float* __restrict__ Q,
                                                              float* __restrict__ img,
@@ -1378,6 +1400,10 @@ __global__ __launch_bounds__(256, 4) void k_dd_cone_adj_list(ArbGeo a, Grid3K g,
                 if (dmax <= 2.0f) v = cone_list_sum<3>(list, n, Qb, fz, lo, fnv, 0);
                 else if (dmax <= 3.0f) v = cone_list_sum<4>(list, n, Qb, fz, lo, fnv, 0);
                 else v = cone_list_sum<0>(list, n, Qb, fz, lo, fnv, ((int)dmax + 5) / 4);
+                if (__any(z < ze && !(fabsf(v) < INFINITY))) {
+                    const float u = cone_list_sum_met(list, n, Qb, fz, lo, fnv);
+                    v = fabsf(v) < INFINITY ? v : u;
+                }
                 if (z < ze) acc[z - z0] += v;
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
