@@ -792,6 +792,37 @@ __global__ __launch_bounds__(256) void k_wgrad_narrow(const float* __restrict__ 
             red[wv][n * 32 + 2 * (4 * k + i) + 1] = od[i];
         }
     }
+    // A NaN or an infinity in the tensor times the zero of a tap off the image is not that
+    // tap's: such sums are made again without those products (one lane per channel and
+    // pixel parity).
+    bool bad = false;
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) bad = bad || !(fabsf(ev[i]) < INFINITY) || !(fabsf(od[i]) < INFINITY);
+    if (__any(bad && n < 9)) {
+        const int c = lane & 31;
+        float s[9];
+        #pragma unroll
+        for (int t = 0; t < 9; ++t) s[t] = 0.0f;
+        for (int ch = (int)blockIdx.x * 4 + wv; ch < nchunk; ch += (int)gridDim.x * 4) {
+            const int row = ch / chunks_per_row, c0 = (ch - row * chunks_per_row) * kNarrowPx, y = row % H;
+            for (int x = c0 + (lane >> 5); x < min(c0 + kNarrowPx, W); x += 2) {
+                const float d = bf2f(act[((long)row * W + x) * 32 + c]);
+                #pragma unroll
+                for (int t = 0; t < 9; ++t) {
+                    const int dy = sg * (t / 3 - 1), dx = sg * (t % 3 - 1);
+                    if (y + dy >= 0 && y + dy < H && x + dx >= 0 && x + dx < W)
+                        s[t] = fmaf(img[(long)(row + dy) * W + x + dx], d, s[t]);
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        #pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            s[t] += __shfl_xor(s[t], 32);
+            float& r = red[wv][t * 32 + c];
+            if (lane < 32 && !(fabsf(r) < INFINITY)) r = s[t];
+        }
+    }
     if (mode != 0) {
         // the image's sum over the four pixel groups of the shift-0 lanes, in place of the channel sums
         sum += __shfl_xor(sum, 16);

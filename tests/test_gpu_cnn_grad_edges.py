@@ -58,3 +58,33 @@ def test_mid_gradients(shape):
                      for t in range(9)])
     assert np.array_equal(g.cpu().double().numpy(), want)
     assert np.array_equal(gb.cpu().double().numpy(), d.sum((0, 1, 2)))
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 4), (2, 5, 70), (1, 66, 33)])
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_narrow_gradients_of_taps_off_the_image(shape, mode, bad):
+    # a NaN or an infinity of one channel on the image's border reaches the taps whose
+    # image pixel exists and no others; those keep their exact sums
+    from reconnet_amd.cnn import _p, _sigs, _st
+
+    B, H, W = shape
+    rng = np.random.default_rng(W + mode)
+    img = rng.integers(1, 4, shape).astype(np.float64)
+    act = rng.integers(-3, 4, shape + (32,)).astype(np.float64)
+    for y, x, c in ((0, 0, 5), (H - 1, W - 1, 8), (H // 2, 0, 31), (0, W // 2, 0)):
+        a0, ok = act.copy(), np.zeros(shape)
+        a0[B - 1, y, x, c], ok[B - 1, y, x] = 0.0, 1.0
+        want = _shift_sums(img, a0)
+        inside = _shift_sums(np.ones(shape), ok[..., None])[:, 0] > 0      # taps whose image pixel exists
+        a1 = act.copy()
+        a1[B - 1, y, x, c] = bad
+        g = torch.empty(320, device="cuda")
+        xt, at = torch.from_numpy(img).float().cuda(), torch.from_numpy(a1).cuda().to(torch.bfloat16)
+        assert _sigs().rn_cnn_wgrad_narrow(_p(xt), _p(at), _p(g), B, H, W, mode, _st()) == 0
+        got = g.cpu().double().numpy()[:288].reshape(9, 32)
+        if mode == 1:
+            got = got[::-1]
+        assert not np.isfinite(got[inside, c]).any(), (y, x)
+        got[inside, c] = want[inside, c]
+        assert np.array_equal(got, want), (y, x)
