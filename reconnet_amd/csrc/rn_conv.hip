@@ -952,15 +952,22 @@ __global__ __launch_bounds__(256, 2) void k_wgrad_mid(const uint16_t* __restrict
                 d2[kc] = tr_frag(dzS + 16 * kc * 32 + tl);
                 accb = mfma32(d2[kc], ones, accb);
             }
+            // (dz rows of this item only: a zero in the others' place would turn a NaN or an
+            // infinity of the input row into a tap's that has no such product)
+            bf16x8 f[3][2];
             #pragma unroll
             for (int dx = 0; dx < 3; ++dx)
                 #pragma unroll
-                for (int kc = 0; kc < 2; ++kc) {
-                    const bf16x8 f = tr_frag(inS + (16 * kc + dx) * 32 + tl);
-                    acc[dx] = mfma32(d2[kc], f, acc[dx]);             // input row above the dz row
-                    acc[3 + dx] = mfma32(d1[kc], f, acc[3 + dx]);
-                    acc[6 + dx] = mfma32(d0[kc], f, acc[6 + dx]);     // below
-                }
+                for (int kc = 0; kc < 2; ++kc) f[dx][kc] = tr_frag(inS + (16 * kc + dx) * 32 + tl);
+            auto taps = [&](f32x16* a, const bf16x8 (&d)[2]) {
+                #pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+                    #pragma unroll
+                    for (int kc = 0; kc < 2; ++kc) a[dx] = mfma32(d[kc], f[dx][kc], a[dx]);
+            };
+            if (r + 1 < y1) taps(acc, d2);                          // input row above the dz row
+            if (r >= y0 && r < y1) taps(acc + 3, d1);
+            if (r > y0) taps(acc + 6, d0);                          // below
             #pragma unroll
             for (int kc = 0; kc < 2; ++kc) {
                 d0[kc] = d1[kc];

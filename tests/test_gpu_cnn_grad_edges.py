@@ -88,3 +88,26 @@ def test_narrow_gradients_of_taps_off_the_image(shape, mode, bad):
         assert not np.isfinite(got[inside, c]).any(), (y, x)
         got[inside, c] = want[inside, c]
         assert np.array_equal(got, want), (y, x)
+
+
+@pytest.mark.parametrize("shape,row", [((1, 3, 32), 2), ((2, 70, 36), 69), ((1, 70, 36), 8), ((1, 70, 36), 7)])
+def test_mid_gradients_of_an_infinite_input(shape, row):
+    # an infinite input pixel of channel 3, in the last row of the image or on either side
+    # of a wave's rows, makes the taps with a product of it infinite and leaves the others
+    from reconnet_amd.cnn import _p, _sigs, _st
+
+    B, H, W = shape
+    rng = np.random.default_rng(row)
+    a = rng.integers(-2, 3, shape + (32,)).astype(np.float64)
+    d = rng.integers(1, 4, shape + (32,)).astype(np.float64)
+    p = np.pad(a, ((0, 0), (1, 1), (1, 1), (0, 0)))
+    want = np.stack([np.tensordot(d, p[:, t // 3:t // 3 + H, t % 3:t % 3 + W], ((0, 1, 2), (0, 1, 2)))
+                     for t in range(9)])
+    for t in range(9):
+        if 0 <= row - (t // 3 - 1) < H:
+            want[t, :, 3] = np.inf
+    a[B - 1, row, 17, 3] = np.inf
+    at, dt = (torch.from_numpy(v).cuda().to(torch.bfloat16) for v in (a, d))
+    g, gb = torch.empty(9, 32, 32, device="cuda"), torch.empty(32, device="cuda")
+    assert _sigs().rn_cnn_wgrad_mid_bias(_p(at), _p(dt), _p(g), _p(gb), B, H, W, _st()) == 0
+    assert np.array_equal(g.cpu().double().numpy(), want)
