@@ -669,16 +669,6 @@ __device__ __forceinline__ void dd_fp_ray_quads(const FanK& g, const float4* __r
     for (int k = 0; k < G; ++k) acc[k] = vscale(acc[k], L);
 }
 
-// One ray of one slice (siddon_fp_ray_slices with S = 1).
-template <class T>
-__device__ __forceinline__ T siddon_fp_ray(const FanK& g, const T* __restrict__ Pyx, const T* __restrict__ Pxy,
-                                           int view, int iu, bool active = true)
-{
-    T acc[1];
-    siddon_fp_ray_slices<T, 1>(g, Pyx, Pxy, 0, 1, view, iu, active, acc);
-    return acc[0];
-}
-
 // atan from an odd polynomial on [-1, 1] (coefficients fitted here by
 // iteratively reweighted least squares on Chebyshev nodes; maximum error
 // 2.5e-7 rad) and, unless UNIT (|z| <= 1 known), atan(z) = sign(z) pi/2 -
@@ -862,7 +852,7 @@ __device__ __forceinline__ void bin_range(const FanK& g, float xc, float yc, flo
     k1 = min((int)floorf(uc + hw), g.nu - 1);
 }
 
-// Length of ray r in cell `cell` of line lr (the weight siddon_fp_ray gives
+// Length of ray r in cell `cell` of line lr (the weight siddon_fp_ray_slices gives
 // it), computed without branches: overlap and width of the interval between the
 // line's crossings ea and eb (both have the sign of eb - ea).
 __device__ __forceinline__ float siddon_cell_weight(const float4 r, float lr, float cell)
@@ -933,10 +923,10 @@ __device__ __forceinline__ void siddon_gather_staged(const float4* st, int t0, i
     }
 }
 
-// Exact transpose of siddon_fp_ray: pixel (ix, iy) gathers, over views
+// Exact transpose of siddon_fp_ray_slices: pixel (ix, iy) gathers, over views
 // view0 .. view0+nviews-1 of prj ([nviews][nu] per slice, slices sstride
 // elements apart; slices q >= nsl read slice nsl - 1 and are discarded by the
-// caller), the rays that cross it, with the weights siddon_fp_ray gives it.
+// caller), the rays that cross it, with their weights there.
 // The bin range and the weights are computed once per view for all S slices.
 // The first NB bins of a pixel's range are taken without branches, the rest
 // in a loop (NB changes only the speed).
