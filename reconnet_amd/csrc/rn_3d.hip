@@ -1875,14 +1875,16 @@ void siddon_arb_bp(const ArbGeo& g, bool parallel, int nB, int nC, const float* 
     };
     // Lanes per (x, y) of the lists: a batch of that many views makes a partial sum, so
     // the geometry decides and not the tuner.  32, or 16 where the rows reach up to 15
-    // voxels (8 up to 6) or just over 32 and the (x, y) fill the chip.  ms with 8, 16
+    // voxels (8 up to 6) or just over 32 (beyond the centre, where the detector covers
+    // part of the volume) and the (x, y) fill the chip.  ms with 8, 16
     // and 32: 190 x 177 x 99, reach 27 1.25, 0.93, 0.95; 207 x 205 x 28, reach 7.7 0.65,
     // 0.56, 0.87; 151^2 x 20, reach 5.5 0.49, 0.65, 1.03; 202^2 x 113, reach 31 0.94, 0.79,
     // 0.84; 60^2 x 95, reach 26 0.16, 0.090, 0.065; 128^2 x 64 all reached 1.40, 1.20, 1.06.
     const long waves = (long)g.nx * g.ny * nB * nC / 4;         // by 16 lanes
     const float reach = std::min(g.z_reach, (float)g.nz);
+    const float over = g.z_reach < (float)g.nz ? 26.0f : 32.0f;
     int lz = 32;
-    if (waves >= 1100 && (reach <= 15.0f || (waves >= 4096 && reach > 30.0f && reach <= 36.0f))) lz = 16;
+    if (waves >= 1100 && (reach <= 15.0f || (waves >= 4096 && reach > over && reach <= 36.0f))) lz = 16;
     if (waves >= 4096 && reach <= (g.nz <= 8 ? 8.0f : 6.0f)) lz = 8;
     const uint32_t pick = !lists ? 7u : lz == 16 ? 1u : lz == 8 ? 2u : 4u;
     const TuneKey key{TK_SIDDON_CONE_BP, g.nx * g.ny, g.nz, g.nu * g.nv, g.nview, nB * nC, lists ? lz : 0};
