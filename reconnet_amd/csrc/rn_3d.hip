@@ -1676,7 +1676,7 @@ __global__ __launch_bounds__(256) void k_helical_bp(HelicalGeo h, const float* _
                 qmin = j == 0 ? q : fminf(qmin, q);
                 qmax = j == 0 ? q : fmaxf(qmax, q);
             }
-            if (__all(qmin > qlive)) continue;
+            if (!__any(!(qmin > qlive))) continue;
             const bool anytaper = __any(qmax > h.Q);
             const float pu = fmaf(u, idu, cu);
             const float fu = floorf(pu);
