@@ -278,11 +278,11 @@ int rn_tv_iso_sqs(const float* img, float* s1, float* s2, float* var, int nb, in
  * axis (x iff |C.x - S.x| >= |C.y - S.y|) the rectangle footprints of the
  * detector cells; its backward is the exact adjoint.  The Siddon kind is the
  * SiddonCone pair (SiddonCone.cu:117,196).  Device pointers, reference
- * layouts, caller stream.  A plan keeps one scratch buffer (the DD backward's
- * row windows, 4·nBatches·nChannels·nu·nview·(nv + 12) bytes, or its FP64 row
- * sums, 8·nBatches·nChannels·nu·nview·(nv + 1) bytes, where a voxel covers more
- * than 7 rows and while the launch shape is tuned): calls on one plan must not
- * overlap. */
+ * layouts, caller stream.  A plan keeps one scratch buffer: both backwards' row
+ * windows, 4·nBatches·nChannels·nu·nview·(nv + 12) bytes where a voxel covers up
+ * to 7 rows (the Siddon kind's after a table of 64·nview); the DD backward's FP64
+ * row sums, 8·nBatches·nChannels·nu·nview·(nv + 1) bytes, where it covers more and
+ * while the launch shape is tuned.  Calls on one plan must not overlap. */
 enum { RN_CONE_DD = 0, RN_CONE_SIDDON = 1 };
 void* rn_cone_plan_create(int nx, int ny, int nz, float dx, float dy, float dz, float cx, float cy, float cz,
         int nu, int nview, int nv, float du, float dv, float off_u, float off_v,
@@ -318,9 +318,11 @@ int rn_helical_rebin(const float* fan, float* par, int nBatches, int nChannels,
 
 /* Launch-shape autotuner (no reference counterpart).  On the first launch of
  * a shape key the projector launchers time their candidate block / tile shapes
- * on the caller's stream and keep the fastest for the process; the choice
- * changes results by at most the rounding of a regrouped sum.  Enabled unless RECONNET_AUTOTUNE=0 or switched off
- * here.  rn_autotune_report writes "kernel a b c d e -> choice (ms ...)"
+ * on the caller's stream and keep the fastest for the process.  The choice
+ * changes no bit of a result, but for the DD forward projection of 4 and more
+ * slices and the cone DD adjoint, which it changes by at most the rounding of
+ * a regrouped sum.  Enabled unless RECONNET_AUTOTUNE=0 or switched off here.
+ * rn_autotune_report writes "kernel a b c d e -> choice (ms ...)"
  * lines (a seventh number follows e where equal sizes have several candidate
  * lists; inf ms: not a choice for these sizes) into buf (NUL-terminated,
  * truncated to len) and returns the full length. */
@@ -329,10 +331,11 @@ int rn_autotune_report(char* buf, int len);
 int rn_autotune_reset(void);
 /* Force candidate `candidate` of kernel `kernel` (1 Siddon FP, 2 Siddon BP,
  * 3 DD FP, 4 DD adjoint, 5 DD BP, 7 DD FBP BP; 8 / 9 the OS-SQS engine's
- * Siddon FP / BP, 10 / 11 DD BP / FBP BP and 12 DD FP of 4 or more slices; 13 the CNN's 32 -> 32 convolution, 14 the one-launch CNN forward, 15 the
- * helical backprojection, 16 the cone DD forward projector, 17 the pixel-driven BP, 18 the Siddon cone
- * backprojection of upright detectors, 19 the cone DD adjoint) for every shape, bypassing the
- * timing; candidate < 0 removes the pin.  A launch of a kernel with fewer
+ * Siddon FP / BP, 10 / 11 DD BP / FBP BP and 12 DD FP of 4 or more slices; 13 the
+ * CNN's 32 -> 32 convolution, 14 the one-launch CNN forward, 15 the helical
+ * backprojection, 16 the cone DD forward projector, 17 the pixel-driven BP, 18 the
+ * Siddon cone backprojection of upright detectors, 19 the cone DD adjoint) for
+ * every shape, bypassing the timing; candidate < 0 removes the pin.  A launch of a kernel with fewer
  * candidates fails with an error.  Lets tests run every launch shape. */
 int rn_autotune_pin(int kernel, int candidate);
 

@@ -600,7 +600,7 @@ __device__ __forceinline__ int wave_max_nn(int v)
 //
 // Bound: VALU issue (about 25 instructions per entry and 19 per row, 2 rows per
 // entry where a voxel covers less than 2).  190 x 177 x 99 voxels, 240 views, 49
-// x 323: 0.99 ms with 32 lanes per (x, y) (1.06 with 16, 1.28 with 8), and 22 us
+// x 323: 0.93 ms with 16 lanes per (x, y) (0.95 with 32, 1.25 with 8), and 22 us
 // for the row windows; 7.4 ms with 64 lanes along z testing every view, column
 // and row for 2 stacked voxels each (siddon_rows_z_view).
 constexpr int kSidCols = 2;          // list entries per view and round
@@ -1553,9 +1553,9 @@ __global__ void k_cone_update(float* __restrict__ x, const float* __restrict__ b
 // land in one detector neighbourhood).  The sums run in the order above (i
 // ascending, m ascending), the window start in the reference's float arithmetic.
 //
-// Bound: VALU.  256^2 x 128 voxels, three turns of 720 views, 64 x 512 detector: 6.9 ms,
-// 9.1 with the square root, arc sine and row tests per conjugate and every conjugate
-// fetched.
+// Bound: VALU.  256^2 x 128 voxels, three turns of 720 views, 64 x 512 detector: 6.4 ms
+// (6.6 a call), 9.2 a call with the square root, arc sine and row tests per conjugate and
+// every conjugate fetched.
 // ---------------------------------------------------------------------------
 // prj_k: [slice][nview][kHelPad + nv + kHelPad][nu]
 constexpr int kHelPad = 2;

@@ -1001,10 +1001,9 @@ __global__ __launch_bounds__(256, 2) void k_wgrad_mid(const uint16_t* __restrict
 
 // out[i] = sum_r part[r][i]: a workgroup takes 32 adjacent columns (128-byte
 // row segments) with its 1024 threads as 32 row groups of 8 loads in flight,
-// whose sums are added in LDS in a fixed order: 4096 rows of 9216 in 39 us
-// (3.9 TB/s), 1024 rows of 320 or 32 in 4.6 us.  One thread per column walking
-// the rows left at most 36 workgroups, each waiting on one load at a time
-// (624 us on average over the eight reductions of a 16 x 512^2 backward).
+// whose sums are added in LDS in a fixed order: 512 rows of 9248 in 5.0 us (3.8
+// TB/s), 1024 rows of 320 in 4.6.  One thread per column walking the rows left at
+// most 36 workgroups, each waiting on one load at a time.
 constexpr int kRedCols = 32, kRedGroups = 32;
 
 // Columns n0 and up go to out2 (the bias behind a layer's weights; dropped if null).

@@ -378,8 +378,8 @@ __device__ __forceinline__ void store_or_update(const FanK& g, const float4 (&ac
 // Bound: LDS reads (nine per bin with 8 groups, 8 clocks each and shared by four
 // SIMDs) and VALU (about 200 instructions, 64 to 96 of them FMAs).  ms, before (bin
 // ranges per pixel through an atan, window as the lanes' minimum and maximum) ->
-// now: 32 slices of 512^2, 96 views 0.168 -> 0.153; 16 slices, 1152 views 1.50 ->
-// 1.27; 32 slices of 250^2, 360 views 0.40 -> 0.20; 6 slices of 256^2 0.28 -> 0.12.
+// now: 32 slices of 512^2, 96 views 0.168 -> 0.146; 16 slices, 1152 views 1.50 ->
+// 1.27; 32 slices of 250^2, 360 views 0.40 -> 0.15; 6 slices of 256^2 0.28 -> 0.094.
 extern __shared__ float4 dyn4[];
 
 template <int G, int CAP, bool UPD>
@@ -1120,7 +1120,8 @@ bool FanTables::matches(const FanGeo& g, const float* deg_host) const
     return std::memcmp(deg.data(), deg_host, sizeof(float) * g.nview) == 0;
 }
 
-// ---- launch shapes: candidates for the autotuner (identical results for every shape) ----
+// ---- launch shapes: candidates for the autotuner.  The shapes it may choose for a size give
+// the same bits, the interleaved DD forward projection's (lines split over lanes) aside ----
 
 namespace {
 

@@ -12,7 +12,8 @@
 // sum over lanes or waves round it differently in its last bits: where the list
 // has several splits, the launch says which candidates have the one its sizes
 // call for, and the choice is among those, so that a call's bits do not depend
-// on a timing.
+// on a timing.  (Two lists choose among splits: the interleaved DD forward
+// projection's and the cone DD adjoint's.)
 //
 // Tuning is skipped (the first candidate, or the cached choice, is used) when
 // the stream is being captured into a graph, when the launch accumulates into
